@@ -9,7 +9,6 @@
 namespace cjx {
 
 constexpr int kHdrWords = 64;      // 2048 bits: bound on one code header
-constexpr int kBlobWords = 128;    // per DC-group header blob
 constexpr int kAcGlobalWords = 8192;
 constexpr int kMaxAcGroups = 32 * 64;  // at most 32 DC groups of 64 AC groups
 // Codestream head: the constant headers (under 32 words) and the TOC, whose
@@ -55,7 +54,7 @@ struct Layout {
     std::uint32_t framing_words[12];  // container framing, 40 or 48 bytes
 };
 
-// One 8-wave workgroup per histogram (histograms first, first + 1, ...):
+// One 8-wave workgroup per histogram (the AC clusters', then the DC groups'):
 // create_huffman_tree's count floors 1, 2, 4, ... are independent trials, so
 // in round r wave w tries floor 2^(8r + w), and the smallest floor whose tree
 // fits 15 bits wins (the serial builder stops at that same floor); floors up
@@ -123,9 +122,9 @@ __device__ void huffman_depths(HuffmanShared& S, int alpha) {
 }
 
 __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const Wg& wg, const std::uint32_t* __restrict__ hists,
-                                                               CodeSet* __restrict__ cs, int first) {
+                                                               CodeSet* __restrict__ cs) {
     __shared__ HuffmanShared S;
-    const int h{first + static_cast<int>(wg.x)};
+    const int h{static_cast<int>(wg.x)};
     const int t{static_cast<int>(threadIdx.x)};
     const int w{t >> 6};
     for (int i{t}; i < kHistStride; i += 64 * kTrials) {
@@ -175,74 +174,73 @@ __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const 
 }
 
 __global__ __launch_bounds__(64 * kTrials) void huffman_kernel(const std::uint32_t* __restrict__ hists,
-                                                               CodeSet* __restrict__ cs, int first) {
-    huffman_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, hists, cs, first);
+                                                               CodeSet* __restrict__ cs) {
+    huffman_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, hists, cs);
 }
 
-// Per DC group: blob_pre = constant prefix + data alphabet + code header;
-// blob_mid = (count - 1) + constant prefix + alphabet + header.
-// One DC group's header blobs (group g, threads of the workgroup take the
-// clearing; thread 0 writes the bits).
-__device__ void dc_blobs_body(const Geometry& geo, const Constants* __restrict__ k, const CodeSet* __restrict__ cs,
-                              const std::uint32_t* __restrict__ fb_count, DcBlobs* __restrict__ blobs,
-                              std::uint32_t* __restrict__ blob_words, int g) {
-    const int t{static_cast<int>(threadIdx.x)};
-    std::uint32_t* pre{blob_words + static_cast<std::size_t>(2 * g) * kBlobWords};
-    std::uint32_t* mid{pre + kBlobWords};
-    for (int i{t}; i < kBlobWords; i += static_cast<int>(blockDim.x)) {
-        pre[i] = 0;
-        mid[i] = 0;
+// Emission of a frame's tokens, one launch: workgroups below num_ac *
+// kGroupParts write one part of an AC group each, the others one chunk of a
+// DC group.  The DC chunks need far less time than the AC parts and fit
+// beside them in one resident round, so they cost no launch of their own.
+struct EmitArgs {
+    const std::int8_t* acs;
+    const std::uint16_t* item_tokens;
+    const std::uint32_t* tokens;
+    const CodeSet* cs;
+    const Constants* k;
+    const std::uint32_t* fb_count;
+    const std::int32_t* dc;
+    const std::int32_t* qf;
+    const std::int8_t* ytox;
+    const std::int8_t* ytob;
+    std::uint32_t* ac_staging;
+    std::uint64_t* ac_part_bits;
+    std::uint32_t* dc_staging;
+    std::uint32_t* chunk_bits;
+    std::uint32_t dc_chunks;  // per DC group (the largest group's)
+};
+
+union EmitShared {
+    GroupShared ac;
+    DcEmitShared dc;
+};
+
+__device__ __attribute__((always_inline)) inline void emit_kernel_body(const Wg& wg, const Geometry& geo,
+                                                                       const EmitArgs& a) {
+    __shared__ EmitShared S;
+    const std::uint32_t ac_wgs{geo.num_ac * kGroupParts};
+    if (wg.x < ac_wgs) {
+        ac_group_emit_body(S.ac, wg, geo, a.acs, a.item_tokens, a.tokens, &a.cs->depth[0][0], &a.cs->code[0][0],
+                           a.ac_staging, a.ac_part_bits);
+        return;
     }
-    __syncthreads();
-    if (t == 0) {
-        const DcGroupGeo d{dc_group_geo(geo, g)};
-        const int hd{kNumClusters + g}, hm{kNumClusters + static_cast<int>(geo.num_dc) + g};
-        BitSink w{pre, 0, kBlobWords * 32};
-        copy_bits(w, k->dc_pre_words, k->dc_pre_bits);
-        write_var_len_u16(w, cs->alpha[hd] - 1);
-        copy_bits(w, cs->hdr[hd], cs->hdr_bits[hd]);
-        blobs->pre_bits[g] = w.ok() ? w.pos : 0u;
-        if (!w.ok()) {
-            atomicOr(&blobs->overflow, 1u);
-        }
-        blobs->pre_off[g] = static_cast<std::uint32_t>(2 * g) * kBlobWords;
-        BitSink m{mid, 0, kBlobWords * 32};
-        m.write(ceil_log2(static_cast<std::uint32_t>(d.n)), fb_count[g] - 1);
-        copy_bits(m, k->dc_mid_words, k->dc_mid_bits);
-        write_var_len_u16(m, cs->alpha[hm] - 1);
-        copy_bits(m, cs->hdr[hm], cs->hdr_bits[hm]);
-        blobs->mid_bits[g] = m.ok() ? m.pos : 0u;
-        if (!m.ok()) {
-            atomicOr(&blobs->overflow, 1u);
-        }
-        blobs->mid_off[g] = static_cast<std::uint32_t>(2 * g + 1) * kBlobWords;
-    }
+    const std::uint32_t i{wg.x - ac_wgs};
+    const Wg dwg{i % a.dc_chunks, i / a.dc_chunks, a.dc_chunks, geo.num_dc};
+    const int hd{kNumClusters + static_cast<int>(dwg.y)}, hm{hd + static_cast<int>(geo.num_dc)};
+    const DcGroupGeo d{dc_group_geo(geo, static_cast<int>(dwg.y))};
+    // blob_pre: constant prefix, data alphabet, code header; blob_mid:
+    // (first blocks - 1), constant prefix, alphabet, header.
+    DcBlob pre, mid;
+    pre.lead_bits = 0;
+    pre.lead = 0;
+    pre.words = a.k->dc_pre_words;
+    pre.word_bits = a.k->dc_pre_bits;
+    pre.alpha_bits = var_len_u16(a.cs->alpha[hd] - 1, pre.alpha);
+    pre.hdr = a.cs->hdr[hd];
+    pre.hdr_bits = a.cs->hdr_bits[hd];
+    mid.lead_bits = ceil_log2(static_cast<std::uint32_t>(d.n));
+    mid.lead = a.fb_count[dwg.y] - 1;
+    mid.words = a.k->dc_mid_words;
+    mid.word_bits = a.k->dc_mid_bits;
+    mid.alpha_bits = var_len_u16(a.cs->alpha[hm] - 1, mid.alpha);
+    mid.hdr = a.cs->hdr[hm];
+    mid.hdr_bits = a.cs->hdr_bits[hm];
+    dc_emit_body(S.dc, dwg, geo, pre, mid, a.dc, a.acs, a.qf, a.ytox, a.ytob, a.cs->depth[hd], a.cs->code[hd],
+                 a.cs->depth[hm], a.cs->code[hm], a.dc_staging, a.chunk_bits);
 }
 
-// The DC chain's sizing pass: workgroup columns 0 .. chunks_per_group - 1 of
-// group row g size the group's item chunks, column chunks_per_group builds
-// its two header blobs (independent work, one launch).
-__device__ __attribute__((always_inline)) inline void dc_blobs_bits_kernel_body(const Wg& wg, 
-    Geometry geo, const Constants* __restrict__ k, const CodeSet* __restrict__ cs,
-    const std::uint32_t* __restrict__ fb_count, DcBlobs* __restrict__ blobs, std::uint32_t* __restrict__ blob_words,
-    const std::int32_t* __restrict__ dc, const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
-    const std::int8_t* __restrict__ ytox, const std::int8_t* __restrict__ ytob,
-    std::uint64_t* __restrict__ chunk_bits, std::uint32_t chunks_per_group) {
-    if (wg.x == chunks_per_group) {
-        dc_blobs_body(geo, k, cs, fb_count, blobs, blob_words, static_cast<int>(wg.y));
-    } else {
-        dc_chunk_bits_body(wg, geo, dc, acs, qf, ytox, ytob, &cs->depth[kNumClusters][0],
-                           &cs->depth[kNumClusters + geo.num_dc][0], chunk_bits, chunks_per_group);
-    }
-}
-
-__global__ __launch_bounds__(256) void dc_blobs_bits_kernel(
-    Geometry geo, const Constants* __restrict__ k, const CodeSet* __restrict__ cs,
-    const std::uint32_t* __restrict__ fb_count, DcBlobs* __restrict__ blobs, std::uint32_t* __restrict__ blob_words,
-    const std::int32_t* __restrict__ dc, const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
-    const std::int8_t* __restrict__ ytox, const std::int8_t* __restrict__ ytob,
-    std::uint64_t* __restrict__ chunk_bits, std::uint32_t chunks_per_group) {
-    dc_blobs_bits_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, cs, fb_count, blobs, blob_words, dc, acs, qf, ytox, ytob, chunk_bits, chunks_per_group);
+__global__ __launch_bounds__(kPartThreads) void emit_kernel(Geometry geo, EmitArgs a) {
+    emit_kernel_body(Wg{blockIdx.x, 0, gridDim.x, 1}, geo, a);
 }
 
 // U32 field coder choice (field_coder.h:46-107) as one code word: selector
@@ -289,11 +287,11 @@ __device__ __forceinline__ void u32_code(const Distr* d, std::uint32_t value, st
 __device__ __attribute__((always_inline)) inline void layout_kernel_body(const Wg& wg, Geometry geo, const Constants* __restrict__ k,
                                                      const CodeSet* __restrict__ cs,
                                                      const std::uint64_t* __restrict__ ac_part_bits,
-                                                     const std::uint32_t* __restrict__ dc_group_bytes,
-                                                     const std::uint64_t* __restrict__ dc_single_bits,
+                                                     std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
+                                                     std::uint32_t* __restrict__ dc_group_bytes,
+                                                     std::uint64_t* __restrict__ dc_group_bits,
                                                      std::uint32_t* __restrict__ ac_group_bytes,
                                                      std::uint64_t* __restrict__ ac_group_bits,
-                                                     const DcBlobs* __restrict__ blobs,
                                                      Layout* __restrict__ lay, std::uint64_t* __restrict__ ac_base,
                                                      std::uint64_t* __restrict__ dc_base,
                                                      std::uint64_t* __restrict__ total_out) {
@@ -305,10 +303,10 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
     // The reads that depend on nothing computed here, issued together before
     // the first wait: each thread's first word of the AcGlobal prefix and of
     // the head (the head's constant words are one per thread), its code
-    // header's alphabet size or bit count, its DC group sizes for the TOC
-    // (entry t: group t - 1) and for the section positions (group t).
+    // header's alphabet size or bit count, and its wave's first DC group's
+    // chunk sizes.
     static_assert(kHeadConstWords == 256, "one head word per thread");
-    const std::uint32_t overflow0{blobs->overflow};
+    __shared__ std::uint32_t dc_bits_s[32];
     const std::uint32_t pre_bits{k->ac_prefix_bits};
     const std::uint32_t hb{k->head_bits};
     const std::uint32_t dc_global_bits{k->dc_global_bits};
@@ -316,9 +314,35 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
     const std::uint32_t head_w0{k->head_words[t]};
     const std::uint32_t alpha_t{t < kNumClusters ? cs->alpha[t] : 0u};
     const std::uint32_t hdr_bits_t{t >= kNumClusters && t < 2 * kNumClusters ? cs->hdr_bits[t - kNumClusters] : 0u};
-    const std::uint32_t dc_bytes_t{static_cast<std::uint32_t>(t) < geo.num_dc ? dc_group_bytes[t] : 0u};
-    const std::uint32_t dc_bytes_prev{t >= 1 && static_cast<std::uint32_t>(t - 1) < geo.num_dc ? dc_group_bytes[t - 1]
-                                                                                                  : 0u};
+    // DC groups: wave w takes groups w, w + 4, ...; the group's chunk sizes
+    // become their exclusive prefix sums (the assembly's chunk offsets).  All
+    // of a group's sizes (at most kDcRounds per lane) are read at once.
+    constexpr int kDcRounds{(kDcMaxChunks + 63) / 64};
+    for (int g{t >> 6}; g < static_cast<int>(geo.num_dc); g += 4) {
+        const int lane{t & 63};
+        const DcGroupGeo d{dc_group_geo(geo, g)};
+        const int used{static_cast<int>((d.items + kDcChunk - 1) / kDcChunk)};
+        std::uint32_t* const cb{chunk_bits + static_cast<std::size_t>(g) * dc_chunks};
+        std::uint32_t v[kDcRounds];
+#pragma unroll
+        for (int r{0}; r < kDcRounds; ++r) {
+            v[r] = 64 * r + lane < used ? cb[64 * r + lane] : 0u;
+        }
+        std::uint32_t sum{0};
+#pragma unroll
+        for (int r{0}; r < kDcRounds; ++r) {
+            const std::uint32_t incl{wave_incl_scan_u32(v[r])};
+            if (64 * r + lane < used) {
+                cb[64 * r + lane] = sum + incl - v[r];
+            }
+            sum += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+        }
+        if (lane == 0) {
+            dc_bits_s[g] = sum;
+            dc_group_bits[g] = sum;
+            dc_group_bytes[g] = (sum + 7) / 8;
+        }
+    }
     // AC group sizes: the sums of their parts' bits.
     for (int g{t}; g < static_cast<int>(geo.num_ac); g += 256) {
         std::uint64_t sum{0};
@@ -336,7 +360,8 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
         hw[i] = 0;
     }
     __syncthreads();
-    std::uint32_t overflow{overflow0};
+    std::uint32_t overflow{0};
+    const auto dc_bytes = [&](std::uint32_t g) { return (dc_bits_s[g] + 7) / 8; };
 
     // AcGlobal.
     for (std::uint32_t i{static_cast<std::uint32_t>(t)}; i < (pre_bits + 31) / 32; i += 256) {
@@ -346,14 +371,7 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
     }
     std::uint32_t len{0}, val{0};
     if (t < kNumClusters) {
-        const std::uint32_t n{alpha_t - 1};
-        if (n == 0) {
-            len = 1;
-        } else {
-            const std::uint32_t nb{31u - static_cast<std::uint32_t>(__builtin_clz(n))};
-            len = 5 + nb;
-            val = 1u | (nb << 1) | ((n - (1u << nb)) << 5);
-        }
+        len = var_len_u16(alpha_t - 1, val);
     } else if (t < 2 * kNumClusters) {
         len = hdr_bits_t;
     }
@@ -390,12 +408,12 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
         std::uint32_t size{0}, code{0}, clen{0};
         if (e < entries) {
             if (single) {
-                const std::uint64_t bits{dc_global_bits + dc_single_bits[0] + abits + agbits[0]};
+                const std::uint64_t bits{dc_global_bits + dc_bits_s[0] + abits + agbits[0]};
                 size = static_cast<std::uint32_t>((bits + 7) / 8);
             } else if (e == 0) {
                 size = dcg;
             } else if (e <= geo.num_dc) {
-                size = dc_bytes_prev;  // e = t: the TOC's DC entries all lie in its first 256
+                size = dc_bytes(e - 1);
             } else if (e == geo.num_dc + 1) {
                 size = acg;
             } else {
@@ -426,14 +444,14 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
     if (single) {
         if (t == 0) {
             dc_base[0] = dcg_bit + dc_global_bits;
-            ac_global_bit = dcg_bit + dc_global_bits + dc_single_bits[0];
+            ac_global_bit = dcg_bit + dc_global_bits + dc_bits_s[0];
             ac_base[0] = ac_global_bit + abits;
         }
     } else {
         const std::uint64_t first{dcg_bit + static_cast<std::uint64_t>(dcg) * 8};
         std::uint64_t dc_total{0};
         const std::uint32_t g{static_cast<std::uint32_t>(t)};
-        const std::uint64_t dsz{g < geo.num_dc ? static_cast<std::uint64_t>(dc_bytes_t) * 8 : 0ull};
+        const std::uint64_t dsz{g < geo.num_dc ? static_cast<std::uint64_t>(dc_bytes(g)) * 8 : 0ull};
         const std::uint64_t dpre{block_excl_scan(dsz, sh, dc_total)};
         if (g < geo.num_dc) {
             dc_base[g] = first + dpre;
@@ -502,15 +520,17 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
 __global__ __launch_bounds__(256) void layout_kernel(Geometry geo, const Constants* __restrict__ k,
                                                      const CodeSet* __restrict__ cs,
                                                      const std::uint64_t* __restrict__ ac_part_bits,
-                                                     const std::uint32_t* __restrict__ dc_group_bytes,
-                                                     const std::uint64_t* __restrict__ dc_single_bits,
+                                                     std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
+                                                     std::uint32_t* __restrict__ dc_group_bytes,
+                                                     std::uint64_t* __restrict__ dc_group_bits,
                                                      std::uint32_t* __restrict__ ac_group_bytes,
                                                      std::uint64_t* __restrict__ ac_group_bits,
-                                                     const DcBlobs* __restrict__ blobs,
                                                      Layout* __restrict__ lay, std::uint64_t* __restrict__ ac_base,
                                                      std::uint64_t* __restrict__ dc_base,
                                                      std::uint64_t* __restrict__ total_out) {
-    layout_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, cs, ac_part_bits, dc_group_bytes, dc_single_bits, ac_group_bytes, ac_group_bits, blobs, lay, ac_base, dc_base, total_out);
+    layout_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, cs, ac_part_bits, chunk_bits,
+                       dc_chunks, dc_group_bytes, dc_group_bits, ac_group_bytes, ac_group_bits, lay, ac_base, dc_base,
+                       total_out);
 }
 
 // The file is a sequence of bit strings ("pieces") laid end to end, each at
@@ -520,8 +540,9 @@ __global__ __launch_bounds__(256) void layout_kernel(Geometry geo, const Constan
 // that overlap it and stored whole, so the output needs no clearing and no
 // atomics.
 struct Pieces {
-    const std::uint32_t* dc_staging;
-    std::uint64_t dc_slot_words;
+    const std::uint32_t* dc_staging;  // dc_chunks slots of kDcSlotWords per group
+    const std::uint32_t* chunk_off;   // the chunks' bit offsets in their group
+    std::uint32_t dc_chunks;
     const std::uint32_t* ac_staging;  // kGroupParts slots of kPartSlotWords per group
     const std::uint64_t* dc_bits;
     const std::uint64_t* ac_bits;
@@ -532,13 +553,16 @@ struct Pieces {
 
 constexpr int kMaxPieces = 4 + 32 + kMaxAcGroups;
 
-// A piece's bits are one run at `src`, or, for an AC group (`parts` set),
-// the concatenation of its parts' runs.
+// A piece's bits are one run at `src`; or, for an AC group (`parts` set), the
+// concatenation of its parts' runs; or, for a DC group (`offs` set), of its
+// chunks' runs.
 struct Piece {
     std::uint64_t dst;
     std::uint64_t nbits;
     const std::uint32_t* src;
     const std::uint64_t* parts;
+    const std::uint32_t* offs;
+    int chunks;
 };
 
 // `len` (1..32) bits of a run from bit `o`.
@@ -552,10 +576,34 @@ __device__ __forceinline__ std::uint32_t run_bits(const std::uint32_t* src, std:
 }
 
 __device__ __forceinline__ std::uint32_t piece_bits(const Piece& pc, std::uint64_t o, std::uint32_t len) {
+    std::uint32_t v{0}, got{0};
+    if (pc.offs != nullptr) {
+        // The last chunk starting at or before bit o, then on from there.
+        const std::uint32_t bits{static_cast<std::uint32_t>(pc.nbits)};
+        std::uint32_t at{static_cast<std::uint32_t>(o)};
+        int c{0}, hi{pc.chunks - 1};
+        while (c < hi) {
+            const int mid{(c + hi + 1) >> 1};
+            if (pc.offs[mid] <= at) {
+                c = mid;
+            } else {
+                hi = mid - 1;
+            }
+        }
+        for (; c < pc.chunks && got < len; ++c) {
+            const std::uint32_t first{pc.offs[c]}, last{c + 1 < pc.chunks ? pc.offs[c + 1] : bits};
+            const std::uint32_t take{min(last - at, len - got)};
+            if (take != 0) {
+                v |= run_bits(pc.src + static_cast<std::size_t>(c) * kDcSlotWords, at - first, take) << got;
+                got += take;
+                at += take;
+            }
+        }
+        return v;
+    }
     if (pc.parts == nullptr) {
         return run_bits(pc.src, o, len);
     }
-    std::uint32_t v{0}, got{0};
     std::uint64_t start{0};
     for (int p{0}; p < kGroupParts && got < len; ++p) {
         const std::uint64_t pb{pc.parts[p]};
@@ -575,25 +623,31 @@ __device__ __forceinline__ std::uint32_t piece_bits(const Piece& pc, std::uint64
 __device__ __forceinline__ Piece piece_at(const Geometry& geo, const Constants* k, const Layout* lay,
                                           const Pieces& P, int i) {
     const int nd{static_cast<int>(geo.num_dc)};
+    const auto run = [](std::uint64_t dst, std::uint64_t nbits, const std::uint32_t* src) {
+        return Piece{dst, nbits, src, nullptr, nullptr, 0};
+    };
     if (i == 0) {
-        return {0, static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->framing_words, nullptr};
+        return run(0, static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->framing_words);
     }
     if (i == 1) {
-        return {static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->head_total_bits, lay->head_words, nullptr};
+        return run(static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->head_total_bits, lay->head_words);
     }
     if (i == 2) {
-        return {lay->dc_global_bit, k->dc_global_bits, k->dc_global_words, nullptr};
+        return run(lay->dc_global_bit, k->dc_global_bits, k->dc_global_words);
     }
     if (i < 3 + nd) {
         const int g{i - 3};
-        return {P.dc_base[g], P.dc_bits[g], P.dc_staging + static_cast<std::size_t>(g) * P.dc_slot_words, nullptr};
+        const DcGroupGeo d{dc_group_geo(geo, g)};
+        const std::size_t c0{static_cast<std::size_t>(g) * P.dc_chunks};
+        return {P.dc_base[g], P.dc_bits[g], P.dc_staging + c0 * kDcSlotWords, nullptr, P.chunk_off + c0,
+                static_cast<int>((d.items + kDcChunk - 1) / kDcChunk)};
     }
     if (i == 3 + nd) {
-        return {lay->ac_global_bit, lay->ac_global_bits, lay->ac_global_words, nullptr};
+        return run(lay->ac_global_bit, lay->ac_global_bits, lay->ac_global_words);
     }
     const int g{i - 4 - nd};
     return {P.ac_base[g], P.ac_bits[g], P.ac_staging + static_cast<std::size_t>(g) * kGroupParts * kPartSlotWords,
-            P.ac_part_bits + static_cast<std::size_t>(g) * kGroupParts};
+            P.ac_part_bits + static_cast<std::size_t>(g) * kGroupParts, nullptr, 0};
 }
 
 __device__ __attribute__((always_inline)) inline void assemble_kernel_body(const Wg& wg, Geometry geo, const Constants* __restrict__ k,

@@ -23,11 +23,9 @@ namespace cjx {
 struct Constants;
 struct CodeSet;
 struct Layout;
-struct DcBlobs;
 
 enum BatchStage : int {
-    kBRegion = 0, kBQuantize, kBDcMaps, kBDcHist, kBHuffDc, kBDcBlobs, kBDcScan, kBDcEmit,
-    kBTokens, kBReduce, kBHuffAc, kBAcEmit, kBLayout, kBAssemble, kBStages
+    kBRegion = 0, kBQuantize, kBTokens, kBHistograms, kBHuffman, kBEmit, kBLayout, kBAssemble, kBStages
 };
 
 struct StageGrid {
@@ -58,8 +56,6 @@ struct FrameJob {
     std::uint32_t* fb_count;
     CodeSet* codes;
     const Constants* k;
-    DcBlobs* blobs;
-    std::uint32_t* blob_words;
     std::uint32_t* tokens;
     std::uint16_t* item_tokens;
     std::uint32_t* item_list;
@@ -70,7 +66,7 @@ struct FrameJob {
     std::uint64_t* ac_part_bits;
     std::uint32_t* ac_group_bytes;
     std::uint64_t* ac_group_bits;
-    std::uint64_t* chunk_bits;
+    std::uint32_t* chunk_bits;
     std::uint32_t* dc_group_bytes;
     std::uint64_t* dc_group_bits;
     Layout* lay;
@@ -94,14 +90,11 @@ struct BatchShape {
 // Stage grids of one frame for a shape (nx, ny only; `first` is the caller's).
 void batch_stage_grids(const Geometry& geo, const BatchShape& shape, StageGrid (&grid)[kBStages]);
 
-// Queues the 14 batched launches of a batch (all frames in `mode`): the
-// region kernel, the AC chain, the layout and the assembly on `s`, the DC
-// chain on `s_dc`, forked after the region kernel (event `fork`) and joined
-// before the layout (event `join`).  A persistent region stage
-// (shape.region_wgs != 0) claims its regions through the eight device
-// counters at `counters`, which a one-workgroup launch clears first.
-void launch_batch(hipStream_t s, hipStream_t s_dc, hipEvent_t fork, hipEvent_t join, const FrameJob* jobs,
-                  int count, const std::uint32_t (&total)[kBStages], std::uint32_t mode, const BatchShape& shape,
-                  std::uint32_t* counters);
+// Queues the eight batched launches of a batch (all frames in `mode`) on `s`.
+// A persistent region stage (shape.region_wgs != 0) claims its regions
+// through the eight device counters at `counters`, which a one-workgroup
+// launch clears first.
+void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
+                  std::uint32_t mode, const BatchShape& shape, std::uint32_t* counters);
 
 }  // namespace cjx

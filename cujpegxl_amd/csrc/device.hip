@@ -127,14 +127,21 @@ bool check_aq_math(unsigned long long* mismatches) {
 std::size_t sizeof_constants() { return sizeof(Constants); }
 std::size_t sizeof_codeset() { return sizeof(CodeSet); }
 std::size_t sizeof_layout() { return sizeof(Layout); }
-std::size_t sizeof_dc_blobs() { return sizeof(DcBlobs); }
-std::uint32_t dc_chunks_per_group() { return (2 + 6 * 65536 + 2 * 1024 + kDcChunk - 1) / kDcChunk; }
-std::uint32_t blob_words_per_group() { return 2 * kBlobWords; }
+std::uint32_t dc_chunks_per_group(const Geometry& geo) {
+    // Group 0 is the largest (dc_group_geo).
+    const std::uint32_t w{geo.bw < 256 ? geo.bw : 256}, h{geo.bh < 256 ? geo.bh : 256};
+    const std::uint32_t items{2 + 6 * w * h + 2 * ((w + 7) / 8) * ((h + 7) / 8)};
+    return (items + kDcChunk - 1) / kDcChunk;
+}
+std::size_t dc_chunk_slot_words() { return kDcSlotWords; }
 
 bool constants_fit(std::uint32_t head_bits, std::uint32_t ac_prefix_bits, std::uint32_t dc_pre_bits,
                    std::uint32_t dc_mid_bits) {
+    // A DC header blob: at most 16 + 20 bits of values and one code header
+    // beside the constant bits.
+    constexpr std::uint32_t blob{32u * kBlobWords - 36u - 32u * kHdrWords};
     return head_bits <= 32u * kHeadConstWords && ac_prefix_bits <= 32u * (kAcGlobalWords / 2) &&
-           dc_pre_bits <= 32u * 64 && dc_mid_bits <= 32u * 64;
+           dc_pre_bits <= blob && dc_mid_bits <= blob;
 }
 
 void fill_constants(void* dst, const std::uint32_t* head, std::uint32_t head_bits,
@@ -189,15 +196,10 @@ void launch_dct8_uniform(hipStream_t s, const Geometry& geo, const FrameParams& 
 void launch_tile_quantize(hipStream_t s, const Geometry& geo, const FrameParams& prm,
                           const std::uint16_t* coeffs, const std::int8_t* acs, const std::int32_t* qf,
                           const float* cfl_part, std::int16_t* ac, std::uint8_t* nz_grid,
-                          std::uint16_t* nz_count, const ItemList& list) {
+                          std::uint16_t* nz_count, const ItemList& list, std::int32_t* dc, std::int8_t* ytox,
+                          std::int8_t* ytob) {
     tile_quantize_kernel<<<geo.cmw * geo.cmh, 256, 0, s>>>(geo, prm, coeffs, acs, qf, cfl_part, ac, nz_grid,
-                                                           nz_count, list);
-}
-
-void launch_dc_maps(hipStream_t s, const Geometry& geo, const FrameParams& prm, const std::uint16_t* coeffs,
-                    const std::int8_t* acs, const float* cfl_part, std::int32_t* dc, std::int8_t* ytox,
-                    std::int8_t* ytob) {
-    dc_maps_kernel<<<grid_for(geo.nblocks, 256), 256, 0, s>>>(geo, prm, coeffs, acs, cfl_part, dc, ytox, ytob);
+                                                           nz_count, list, dc, ytox, ytob);
 }
 
 void launch_nz(hipStream_t s, const Geometry& geo, const std::int16_t* ac, const std::int8_t* acs,
@@ -213,8 +215,9 @@ void launch_fill_u32(hipStream_t s, std::uint32_t* p, std::size_t n, std::uint32
 
 void launch_ac_tokens(hipStream_t s, const Geometry& geo, const std::int16_t* ac, const std::int8_t* acs,
                       const std::uint8_t* nz_grid, const std::uint16_t* nz_count, std::uint32_t* tokens,
-                      std::uint16_t* item_tokens, std::uint32_t* partial, std::uint32_t* hist,
-                      const ItemList& list) {
+                      std::uint16_t* item_tokens, std::uint32_t* partial, std::uint32_t* hists,
+                      const ItemList& list, const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox,
+                      const std::int8_t* ytob, std::uint32_t* fb_count) {
     // One resident round of workgroups (occupancy x CUs of the current
     // device, at most kTokenGrid): a second partial round would double the
     // kernel's time for a few waves.
@@ -233,23 +236,17 @@ void launch_ac_tokens(hipStream_t s, const Geometry& geo, const std::int16_t* ac
     const unsigned int grid{waves < resident ? waves : resident};
     ac_tokens_kernel<<<grid, 256, 0, s>>>(geo, ac, acs, nz_grid, nz_count, tokens, item_tokens, partial, list.items,
                                           list.count);
-    ac_hist_reduce_kernel<<<dim3(kNumClusters * kAcSymbols / 256, 80), 256, 0, s>>>(partial, static_cast<int>(grid),
-                                                                                    hist);
+    const std::uint32_t chunks{dc_chunks_per_group(geo)};
+    histograms_kernel<<<kReduceWgs + chunks * geo.num_dc, 256, 0, s>>>(geo, chunks, partial, static_cast<int>(grid),
+                                                                       hists, dc, acs, qf, ytox, ytob, fb_count);
 }
 
 std::size_t ac_partial_words() {
     return static_cast<std::size_t>(kTokenGrid) * kNumClusters * kAcSymbols;
 }
 
-void launch_dc_hist(hipStream_t s, const Geometry& geo, const std::int32_t* dc, const std::int8_t* acs,
-                    const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                    std::uint32_t* dc_hist, std::uint32_t* meta_hist, std::uint32_t* fb_count) {
-    const dim3 grid{dc_chunks_per_group(), geo.num_dc};
-    dc_hist_kernel<<<grid, 256, 0, s>>>(geo, dc, acs, qf, ytox, ytob, dc_hist, meta_hist, fb_count);
-}
-
-void launch_huffman(hipStream_t s, int first, int count, const std::uint32_t* hists, CodeSet* cs) {
-    huffman_kernel<<<count, 64 * kTrials, 0, s>>>(hists, cs, first);
+void launch_huffman(hipStream_t s, int count, const std::uint32_t* hists, CodeSet* cs) {
+    huffman_kernel<<<count, 64 * kTrials, 0, s>>>(hists, cs);
 }
 
 bool build_codes_host(const std::uint32_t* hists, std::uint32_t count, std::uint32_t* alpha, std::uint8_t* depth,
@@ -264,7 +261,7 @@ bool build_codes_host(const std::uint32_t* hists, std::uint32_t count, std::uint
             hipMemcpy(dh, hists, hbytes, hipMemcpyHostToDevice) == hipSuccess};
     auto* host{new CodeSet};
     if (ok) {
-        huffman_kernel<<<count, 64 * kTrials, 0, nullptr>>>(dh, dcs, 0);
+        huffman_kernel<<<count, 64 * kTrials, 0, nullptr>>>(dh, dcs);
         ok = hipGetLastError() == hipSuccess && hipMemcpy(host, dcs, sizeof(CodeSet), hipMemcpyDeviceToHost) == hipSuccess;
     }
     if (ok) {
@@ -291,59 +288,36 @@ std::size_t ac_group_parts() {
     return kGroupParts;
 }
 
-void launch_ac_group_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs,
-                          const std::uint16_t* item_tokens, const std::uint32_t* tokens, const CodeSet* cs,
-                          std::uint32_t* staging, std::uint64_t* part_bits, hipEvent_t done) {
-    hipExtLaunchKernelGGL(ac_group_emit_kernel, dim3(geo.num_ac * kGroupParts), dim3(kPartThreads), 0, s, nullptr,
-                          done, 0, geo, acs, item_tokens, tokens, &cs->depth[0][0], &cs->code[0][0], staging,
-                          part_bits);
-}
-
-std::size_t dc_group_slot_words() {
-    // Every DC item is at most 32 bits; plus the two header blobs.
-    return static_cast<std::size_t>(dc_chunks_per_group()) * kDcChunk + 2 * kBlobWords + 64;
-}
-
-void launch_dc_sizes(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                     const std::uint32_t* fb_count, DcBlobs* blobs, std::uint32_t* blob_words, const std::int32_t* dc,
-                     const std::int8_t* acs, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                     std::uint64_t* chunk_bits, std::uint32_t* group_bytes, std::uint64_t* group_bits,
-                     std::uint32_t* staging) {
-    const std::uint32_t cpg{dc_chunks_per_group()};
-    dc_blobs_bits_kernel<<<dim3(cpg + 1, geo.num_dc), 256, 0, s>>>(geo, k, cs, fb_count, blobs, blob_words, dc, acs,
-                                                                   qf, ytox, ytob, chunk_bits, cpg);
-    dc_chunk_scan_kernel<<<geo.num_dc, 1024, 0, s>>>(geo, chunk_bits, cpg, blobs, group_bytes, group_bits, staging,
-                                                     dc_group_slot_words());
+void launch_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs, const std::uint16_t* item_tokens,
+                 const std::uint32_t* tokens, const CodeSet* cs, const Constants* k, const std::uint32_t* fb_count,
+                 const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
+                 std::uint32_t* ac_staging, std::uint64_t* ac_part_bits, std::uint32_t* dc_staging,
+                 std::uint32_t* chunk_bits) {
+    const std::uint32_t chunks{dc_chunks_per_group(geo)};
+    emit_kernel<<<geo.num_ac * kGroupParts + chunks * geo.num_dc, kPartThreads, 0, s>>>(
+        geo, EmitArgs{acs, item_tokens, tokens, cs, k, fb_count, dc, qf, ytox, ytob, ac_staging, ac_part_bits,
+                      dc_staging, chunk_bits, chunks});
 }
 
 void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                   const std::uint64_t* ac_part_bits, const std::uint32_t* dc_group_bytes,
-                   const std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
-                   const DcBlobs* blobs, Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base,
-                   std::uint64_t* total_out, hipEvent_t done) {
+                   const std::uint64_t* ac_part_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
+                   std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
+                   Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base, std::uint64_t* total_out,
+                   hipEvent_t done) {
     hipExtLaunchKernelGGL(layout_kernel, dim3(1), dim3(256), 0, s, nullptr, done, 0, geo, k, cs, ac_part_bits,
-                          dc_group_bytes, dc_group_bits, ac_group_bytes, ac_group_bits, blobs, lay, ac_base, dc_base,
-                          total_out);
+                          chunk_bits, dc_chunks_per_group(geo), dc_group_bytes, dc_group_bits, ac_group_bytes,
+                          ac_group_bits, lay, ac_base, dc_base, total_out);
 }
 
 void launch_assemble(hipStream_t s, const Geometry& geo, const Constants* k, const Layout* lay,
                      const std::uint32_t* dc_staging, const std::uint32_t* ac_staging, const std::uint64_t* dc_bits,
-                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits, const std::uint64_t* dc_base,
-                     const std::uint64_t* ac_base, std::uint8_t* out, std::uint64_t cap_bytes, hipEvent_t done) {
-    const Pieces P{dc_staging, dc_group_slot_words(), ac_staging, dc_bits, ac_bits, ac_part_bits, dc_base, ac_base};
+                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits,
+                     const std::uint32_t* chunk_off, const std::uint64_t* dc_base, const std::uint64_t* ac_base,
+                     std::uint8_t* out, std::uint64_t cap_bytes, hipEvent_t done) {
+    const Pieces P{dc_staging, chunk_off, dc_chunks_per_group(geo), ac_staging, dc_bits, ac_bits, ac_part_bits,
+                   dc_base, ac_base};
     hipExtLaunchKernelGGL(assemble_kernel, dim3(2048), dim3(256), 0, s, nullptr, done, 0, geo, k, lay, P,
                           reinterpret_cast<std::uint32_t*>(out), cap_bytes);
-}
-
-void launch_dc_emit(hipStream_t s, const Geometry& geo, const std::int32_t* dc, const std::int8_t* acs,
-                    const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                    const CodeSet* cs, const DcBlobs* blobs, const std::uint32_t* blob_words,
-                    const std::uint64_t* chunk_off, std::uint32_t* staging, hipEvent_t done) {
-    const std::uint32_t cpg{dc_chunks_per_group()};
-    hipExtLaunchKernelGGL(dc_emit_kernel, dim3(cpg, geo.num_dc), dim3(256), 0, s, nullptr, done, 0, geo, dc, acs, qf,
-                          ytox, ytob, &cs->depth[kNumClusters][0], &cs->code[kNumClusters][0],
-                          &cs->depth[kNumClusters + geo.num_dc][0], &cs->code[kNumClusters + geo.num_dc][0], blobs,
-                          blob_words, chunk_off, cpg, staging, dc_group_slot_words());
 }
 
 }  // namespace cjx

@@ -243,10 +243,8 @@ void Encoder::release() {
         (void)hipSetDevice(device_);
     }
     // A frame queued by encode_async and never finished may still run.
-    for (hipStream_t s : {stream_, dc_stream_}) {
-        if (s != nullptr) {
-            (void)hipStreamSynchronize(s);
-        }
+    if (stream_ != nullptr) {
+        (void)hipStreamSynchronize(stream_);
     }
     pending_ = false;
     for (void* p : allocations_) {
@@ -274,15 +272,11 @@ void Encoder::release() {
             e = nullptr;
         }
     }
-    for (hipEvent_t* e : {&ev_fork_, &ev_dc_done_, &ev_size_, &ev_end_, &ev_done_, &ev_caller_, &ev_input_free_}) {
+    for (hipEvent_t* e : {&ev_size_, &ev_end_, &ev_done_, &ev_caller_, &ev_input_free_}) {
         if (*e != nullptr) {
             (void)hipEventDestroy(*e);
             *e = nullptr;
         }
-    }
-    if (dc_stream_ != nullptr) {
-        (void)hipStreamDestroy(dc_stream_);
-        dc_stream_ = nullptr;
     }
     if (stream_ != nullptr) {
         (void)hipStreamDestroy(stream_);
@@ -307,13 +301,12 @@ void Encoder::null_buffers() {
     nz_grid_ = nullptr;
     nz_count_ = nullptr;
     hists_ = fb_count_ = nullptr;
-    codes_ = constants_ = blobs_ = layout_ = nullptr;
-    blob_words_ = nullptr;
+    codes_ = constants_ = layout_ = nullptr;
     tokens_ = nullptr;
     item_tokens_ = nullptr;
     item_list_ = item_count_ = hist_partial_ = ac_staging_ = dc_staging_ = nullptr;
-    ac_part_bits_ = ac_group_bits_ = chunk_bits_ = dc_group_bits_ = ac_base_ = dc_base_ = nullptr;
-    ac_group_bytes_ = dc_group_bytes_ = nullptr;
+    ac_part_bits_ = ac_group_bits_ = dc_group_bits_ = ac_base_ = dc_base_ = nullptr;
+    ac_group_bytes_ = dc_group_bytes_ = chunk_bits_ = nullptr;
     out_ = nullptr;
     out_cap_ = 0;
     features_ = nullptr;
@@ -363,8 +356,7 @@ bool Encoder::setup(int device) {
     if (!g_tables_ok[device & 63]) {
         return false;
     }
-    if (hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&dc_stream_, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess) {
         return false;
     }
     for (hipEvent_t* e : {&ev_done_, &ev_caller_, &ev_input_free_}) {
@@ -373,7 +365,7 @@ bool Encoder::setup(int device) {
         }
     }
     // Bound to kernels' completion at launch (timing-capable events).
-    for (hipEvent_t* e : {&ev_fork_, &ev_size_, &ev_dc_done_, &ev_end_}) {
+    for (hipEvent_t* e : {&ev_size_, &ev_end_}) {
         if (hipEventCreate(e) != hipSuccess) {
             return false;
         }
@@ -402,6 +394,7 @@ void Encoder::carve(Get& get) {
     const std::size_t tiles{static_cast<std::size_t>(geo_.cmw) * geo_.cmh};
     const std::size_t regions{static_cast<std::size_t>(geo_.rw) * geo_.rh};
     const std::size_t nh{static_cast<std::size_t>(kNumClusters) + 2 * geo_.num_dc};
+    const std::size_t dc_chunks{static_cast<std::size_t>(geo_.num_dc) * dc_chunks_per_group(geo_)};
     get(coeffs_, 3 * nblk * 64 * sizeof(std::uint16_t));
     get(acs_, nblk);
     get(qf_, nblk * sizeof(std::int32_t));
@@ -416,19 +409,17 @@ void Encoder::carve(Get& get) {
     get(fb_count_, 64 * sizeof(std::uint32_t));
     get(codes_, sizeof_codeset());
     get(constants_, sizeof_constants());
-    get(blobs_, sizeof_dc_blobs());
-    get(blob_words_, static_cast<std::size_t>(geo_.num_dc) * blob_words_per_group() * sizeof(std::uint32_t));
     get(tokens_, 3 * nblk * 64 * sizeof(std::uint32_t));
     get(item_tokens_, 3 * nblk * sizeof(std::uint16_t));
     get(item_list_, 3 * nblk * sizeof(std::uint32_t));
     get(item_count_, 2 * sizeof(std::uint32_t));
     get(hist_partial_, ac_partial_words() * sizeof(std::uint32_t));
     get(ac_staging_, static_cast<std::size_t>(geo_.num_ac) * ac_group_slot_words() * sizeof(std::uint32_t));
-    get(dc_staging_, static_cast<std::size_t>(geo_.num_dc) * dc_group_slot_words() * sizeof(std::uint32_t));
+    get(dc_staging_, dc_chunks * dc_chunk_slot_words() * sizeof(std::uint32_t));
     get(ac_part_bits_, geo_.num_ac * ac_group_parts() * sizeof(std::uint64_t));
     get(ac_group_bytes_, geo_.num_ac * sizeof(std::uint32_t));
     get(ac_group_bits_, geo_.num_ac * sizeof(std::uint64_t));
-    get(chunk_bits_, static_cast<std::size_t>(geo_.num_dc) * dc_chunks_per_group() * sizeof(std::uint64_t));
+    get(chunk_bits_, dc_chunks * sizeof(std::uint32_t));
     get(dc_group_bytes_, geo_.num_dc * sizeof(std::uint32_t));
     get(dc_group_bits_, geo_.num_dc * sizeof(std::uint64_t));
     get(layout_, sizeof_layout());
@@ -535,8 +526,6 @@ bool Encoder::fill_job(FrameJob& j, hipStream_t s, std::uint8_t* out_dev, std::s
     j.fb_count = fb_count_;
     j.codes = static_cast<CodeSet*>(codes_);
     j.k = static_cast<const Constants*>(constants_);
-    j.blobs = static_cast<DcBlobs*>(blobs_);
-    j.blob_words = blob_words_;
     j.tokens = tokens_;
     j.item_tokens = item_tokens_;
     j.item_list = item_list_;
@@ -572,8 +561,7 @@ bool Encoder::region_only(const std::uint8_t* luma, std::size_t luma_pitch, cons
 }
 #endif
 
-// One frame queued on `s` in dependency order (the two entropy chains one
-// after the other); nothing waits on the host unless the constant bit
+// One frame queued on `s`; nothing waits on the host unless the constant bit
 // strings change (a new shape or distance), which copies them in order on
 // `s` and waits for that copy.
 bool Encoder::encode_on(hipStream_t s, const std::uint8_t* luma, std::size_t luma_pitch, const std::uint8_t* chroma,
@@ -584,27 +572,20 @@ bool Encoder::encode_on(hipStream_t s, const std::uint8_t* luma, std::size_t lum
     }
     auto* codes{static_cast<CodeSet*>(codes_)};
     auto* k{static_cast<const Constants*>(constants_)};
-    auto* blobs{static_cast<DcBlobs*>(blobs_)};
     auto* lay{static_cast<Layout*>(layout_)};
     launch_region(s, geo_, prm_, luma, luma_pitch, chroma, chroma_pitch, coeffs_, acs_, qf_, cfl_part_, item_count_,
                   entropy_clears());
     launch_tile_quantize(s, geo_, prm_, coeffs_, acs_, qf_, cfl_part_, ac_, nz_grid_, nz_count_,
-                         ItemList{item_list_, item_count_});
-    launch_dc_maps(s, geo_, prm_, coeffs_, acs_, cfl_part_, dc_, ytox_, ytob_);
-    launch_dc_hist(s, geo_, dc_, acs_, qf_, ytox_, ytob_, hists_ + kNumClusters * kHistStride,
-                   hists_ + (kNumClusters + geo_.num_dc) * kHistStride, fb_count_);
-    launch_huffman(s, kNumClusters, static_cast<int>(2 * geo_.num_dc), hists_, codes);
-    launch_dc_sizes(s, geo_, k, codes, fb_count_, blobs, blob_words_, dc_, acs_, qf_, ytox_, ytob_, chunk_bits_,
-                    dc_group_bytes_, dc_group_bits_, dc_staging_);
-    launch_dc_emit(s, geo_, dc_, acs_, qf_, ytox_, ytob_, codes, blobs, blob_words_, chunk_bits_, dc_staging_);
+                         ItemList{item_list_, item_count_}, dc_, ytox_, ytob_);
     launch_ac_tokens(s, geo_, ac_, acs_, nz_grid_, nz_count_, tokens_, item_tokens_, hist_partial_, hists_,
-                     ItemList{item_list_, item_count_});
-    launch_huffman(s, 0, kNumClusters, hists_, codes);
-    launch_ac_group_emit(s, geo_, acs_, item_tokens_, tokens_, codes, ac_staging_, ac_part_bits_);
-    launch_layout(s, geo_, k, codes, ac_part_bits_, dc_group_bytes_, dc_group_bits_, ac_group_bytes_,
-                  ac_group_bits_, blobs, lay, ac_base_, dc_base_, size_dev);
+                     ItemList{item_list_, item_count_}, dc_, qf_, ytox_, ytob_, fb_count_);
+    launch_huffman(s, kNumClusters + static_cast<int>(2 * geo_.num_dc), hists_, codes);
+    launch_emit(s, geo_, acs_, item_tokens_, tokens_, codes, k, fb_count_, dc_, qf_, ytox_, ytob_, ac_staging_,
+                ac_part_bits_, dc_staging_, chunk_bits_);
+    launch_layout(s, geo_, k, codes, ac_part_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_, ac_group_bytes_,
+                  ac_group_bits_, lay, ac_base_, dc_base_, size_dev);
     launch_assemble(s, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_group_bits_, ac_part_bits_,
-                    dc_base_, ac_base_, out_dev, cap);
+                    chunk_bits_, dc_base_, ac_base_, out_dev, cap);
     return hipGetLastError() == hipSuccess;
 }
 
@@ -694,9 +675,9 @@ bool Encoder::build_constants(std::uint32_t global_scale, std::uint32_t quant_dc
     return true;
 }
 
-void Encoder::mark(Stage s, hipStream_t on) {
+void Encoder::mark(Stage s) {
     if (profiling_ == 1 || (profiling_ == 2 && (s == Stage::kRegion || s == Stage::kQuantize))) {
-        (void)hipEventRecord(events_[static_cast<int>(s)], on != nullptr ? on : stream_);
+        (void)hipEventRecord(events_[static_cast<int>(s)], stream_);
     }
 }
 
@@ -744,7 +725,7 @@ std::uint8_t* Encoder::mapped_output(std::uint8_t* dst) const {
 // any other output (or none yet, for encode_async) gets the first two chunks
 // staged in the pinned buffer (bytes past the end are never used).
 bool Encoder::queue_readback(std::uint8_t* direct) {
-    mark(Stage::kReadback, tail_);
+    mark(Stage::kReadback);
     staged_ = 0;
     direct_dst_ = direct;
     if (direct == nullptr) {
@@ -761,8 +742,8 @@ bool Encoder::queue_readback(std::uint8_t* direct) {
 bool Encoder::stage_chunk(int slot, std::size_t n) {
     stage_len_[slot] = n;
     const bool ok{hipMemcpyAsync(stage_host_ + slot * kStageChunk, reinterpret_cast<const std::uint8_t*>(out_) + staged_,
-                                 n, hipMemcpyDeviceToHost, tail_) == hipSuccess &&
-                  hipEventRecord(stage_ready_[slot], tail_) == hipSuccess};
+                                 n, hipMemcpyDeviceToHost, stream_) == hipSuccess &&
+                  hipEventRecord(stage_ready_[slot], stream_) == hipSuccess};
     staged_ += n;
     return ok;
 }
@@ -790,7 +771,7 @@ bool Encoder::wait_done() {
         end_bound_ = false;
         return spin_on(ev_end_);
     }
-    return hipEventRecord(ev_done_, tail_) == hipSuccess && spin_on(ev_done_);
+    return hipEventRecord(ev_done_, stream_) == hipSuccess && spin_on(ev_done_);
 }
 
 // The readback's second half: waits for the size, then moves the bytes into
@@ -801,13 +782,13 @@ bool Encoder::finish(std::uint8_t* dst, std::size_t cap, std::size_t* size) {
         return false;
     }
     pending_ = false;
-    // Block until the DC chain (off the critical path, done tens of
-    // microseconds before the layout), then poll for the size, or for the
-    // frame's end when no size event was bound (the assembly writes the
-    // file into `dst`): a blocking wait on a late event would add its
-    // wake-up latency, and the event's interrupt, to the frame.
+    // Poll for the size, or for the frame's end when no size event was bound
+    // (the assembly writes the file into `dst`): a blocking wait would add
+    // its wake-up latency, and the event's interrupt, to the frame, and an
+    // event in mid-chain for a first blocking wait costs about 5 us of idle
+    // device time after the kernel that carries it.
     const bool ended{!size_bound_};
-    if (hipEventSynchronize(ev_dc_done_) != hipSuccess || !(ended ? wait_done() : spin_on(ev_size_))) {
+    if (!(ended ? wait_done() : spin_on(ev_size_))) {
         return false;
     }
     const std::uint64_t total{*total_host_};
@@ -818,7 +799,7 @@ bool Encoder::finish(std::uint8_t* dst, std::size_t cap, std::size_t* size) {
             // The assembly kernel writes the file into `dst`; the frame's end
             // (waited for above without a size event, else below) completes it.
         } else if (host_pinned(dst)) {
-            ok = hipMemcpyAsync(dst, out_, total, hipMemcpyDeviceToHost, tail_) == hipSuccess;
+            ok = hipMemcpyAsync(dst, out_, total, hipMemcpyDeviceToHost, stream_) == hipSuccess;
         } else {
             std::size_t done{0};
             for (int slot{0}; slot < 2 && staged_ < total && stage_len_[slot] == 0; ++slot) {
@@ -842,7 +823,7 @@ bool Encoder::finish(std::uint8_t* dst, std::size_t cap, std::size_t* size) {
     stage_len_[0] = stage_len_[1] = 0;
     direct_dst_ = nullptr;
     if (!ended || copied) {
-        mark(Stage::kCount, tail_);
+        mark(Stage::kCount);
         if (!wait_done()) {
             return false;
         }
@@ -878,30 +859,26 @@ bool Encoder::submit_nv12(const std::uint8_t* luma, std::size_t luma_pitch, cons
         return false;
     }
     // With profiling on, the region kernel's own start and end times open the
-    // region and quantize stages.  Its end is the fork point of the DC chain
-    // (it leaves the coefficients the DC values come from and the CfL
-    // partials the colour maps come from, and clears the entropy stage's
-    // accumulators).
+    // region and quantize stages.
     const bool timed{profiling_ != 0};
-    const hipEvent_t region_end{timed ? events_[static_cast<int>(Stage::kQuantize)] : ev_fork_};
     launch_region(stream_, geo_, prm_, luma, luma_pitch, chroma, chroma_pitch, coeffs_, acs_, qf_, cfl_part_,
                   item_count_, entropy_clears(),
-                  timed ? events_[static_cast<int>(Stage::kRegion)] : nullptr, region_end,
-                  export_ ? features_ : nullptr);
+                  timed ? events_[static_cast<int>(Stage::kRegion)] : nullptr,
+                  timed ? events_[static_cast<int>(Stage::kQuantize)] : nullptr, export_ ? features_ : nullptr);
     // The planes are read by the region kernel only: later work on the
     // caller's stream may overwrite them once it has finished.
     if (release_caller && (hipEventRecord(ev_input_free_, stream_) != hipSuccess ||
                            hipStreamWaitEvent(caller, ev_input_free_, 0) != hipSuccess)) {
         return false;
     }
-    // The quantizer lists the non-empty items for the tokenizer.
+    // The quantizer lists the non-empty items for the tokenizer and leaves
+    // the DC values and colour maps.
     launch_tile_quantize(stream_, geo_, prm_, coeffs_, acs_, qf_, cfl_part_, ac_, nz_grid_, nz_count_,
-                         ItemList{item_list_, item_count_});
+                         ItemList{item_list_, item_count_}, dc_, ytox_, ytob_);
     // A mapped page-locked output receives the file from the assembly kernel.
     std::uint8_t* const direct{mapped_output(dst)};
     return run_entropy(direct != nullptr ? direct : reinterpret_cast<std::uint8_t*>(out_),
-                       direct != nullptr ? cap : out_cap_, region_end, true, true,
-                       direct == nullptr || profiling_ != 0) &&
+                       direct != nullptr ? cap : out_cap_, true, direct == nullptr || profiling_ != 0) &&
            queue_readback(direct != nullptr ? dst : nullptr);
 }
 
@@ -910,7 +887,6 @@ bool Encoder::encode_nv12(const std::uint8_t* luma, std::size_t luma_pitch, cons
     if (!submit_nv12(luma, luma_pitch, chroma, chroma_pitch, nullptr, false, out, cap)) {
         pending_ = false;
         (void)hipStreamSynchronize(stream_);
-        (void)hipStreamSynchronize(dc_stream_);
         return false;
     }
     return finish(out, cap, size);
@@ -929,10 +905,9 @@ bool Encoder::encode_dct8_uniform(const std::uint8_t* luma, std::size_t luma_pit
                         ytob_);
     mark(Stage::kQuantize);
     launch_nz(stream_, geo_, ac_, acs_, nz_grid_, nz_count_, entropy_clears());
-    if (!run_entropy(reinterpret_cast<std::uint8_t*>(out_), out_cap_, nullptr, false) || !queue_readback(nullptr)) {
+    if (!run_entropy(reinterpret_cast<std::uint8_t*>(out_), out_cap_, false) || !queue_readback(nullptr)) {
         pending_ = false;
         (void)hipStreamSynchronize(stream_);
-        (void)hipStreamSynchronize(dc_stream_);
         return false;
     }
     return finish(out, cap, size);
@@ -944,7 +919,6 @@ bool Encoder::encode_async(const std::uint8_t* luma, std::size_t luma_pitch, con
     if (!ok && pending_) {
         pending_ = false;
         (void)hipStreamSynchronize(stream_);
-        (void)hipStreamSynchronize(dc_stream_);
     }
     return ok;
 }
@@ -1041,86 +1015,60 @@ bool Encoder::encode_coefficients(const std::int16_t* ac, const std::int32_t* dc
     mark(Stage::kRegion);
     mark(Stage::kQuantize);
     launch_nz(stream_, geo_, ac_, acs_, nz_grid_, nz_count_, entropy_clears());
-    if (!run_entropy(reinterpret_cast<std::uint8_t*>(out_), out_cap_, nullptr, false) || !queue_readback(nullptr)) {
+    if (!run_entropy(reinterpret_cast<std::uint8_t*>(out_), out_cap_, false) || !queue_readback(nullptr)) {
         pending_ = false;
         (void)hipStreamSynchronize(stream_);
-        (void)hipStreamSynchronize(dc_stream_);
         return false;
     }
     return finish(out, cap, size);
 }
 
-// The histograms (AC clusters, then DC and AcMetadata per DC group), the
-// first-block counts and the DC header-blob table start every frame at zero.
+// The histograms (AC clusters, then DC and AcMetadata per DC group) and the
+// first-block counts start every frame at zero.
 Clears Encoder::entropy_clears() const {
     Clears c{};
     c.ptr[0] = hists_;
     c.words[0] = static_cast<std::uint32_t>((kNumClusters + 2 * geo_.num_dc) * kHistStride);
     c.ptr[1] = fb_count_;
     c.words[1] = 64;
-    c.ptr[2] = static_cast<std::uint32_t*>(blobs_);
-    c.words[2] = static_cast<std::uint32_t>(sizeof_dc_blobs() / 4);
     return c;
 }
 
-bool Encoder::run_entropy(std::uint8_t* out, std::size_t cap, hipEvent_t fork, bool listed, bool maps,
-                          bool size_event) {
+// The entropy stage on the encoder's one stream: six launches, the DC
+// groups' work beside the AC groups' in each (histograms beside the partial
+// histograms' sum, codes beside codes, chunks beside parts).  A DC chain of
+// its own on a second stream was six launches and two cross-stream
+// dependencies (about 5 us each), and ran after the AC chain's start of its
+// stage, not beside it, wherever the two streams shared a hardware queue
+// (four per process: two encoders fill them).  Whole frames, before -> after,
+// with three encoders alive and the DC values in the quantizer included:
+// 320x240 159 -> 123 us, 7680x4320 1,145 -> 1,125 us, 3840x2160 unchanged at
+// 364 us, a batch of 16 mixed frames 1,527 -> 1,486 us.  `size_event` binds
+// ev_size_ to the layout kernel (the host then reads the size before the
+// frame's end).
+bool Encoder::run_entropy(std::uint8_t* out, std::size_t cap, bool listed, bool size_event) {
     auto* codes{static_cast<CodeSet*>(codes_)};
     auto* k{static_cast<const Constants*>(constants_)};
-    auto* blobs{static_cast<DcBlobs*>(blobs_)};
     auto* lay{static_cast<Layout*>(layout_)};
-    // The DC chain (histograms, codes, header blobs, chunk sizes, emission)
-    // depends on nothing of the AC chain: it runs on the second stream from
-    // `fork` (the stream's work so far when null) and joins before the layout.
-    // With `maps` it first derives the DC values from the coefficients and
-    // the tiles' colour maps from the CfL partials.  `size_event` binds ev_size_ to the layout kernel (the host
-    // then reads the size before the frame's end).
     mark(Stage::kHistograms);
-    const int ndc{static_cast<int>(2 * geo_.num_dc)};
-    if (fork == nullptr) {
-        fork = ev_fork_;
-        if (hipEventRecord(fork, stream_) != hipSuccess) {
-            return false;
-        }
-    }
-    if (hipStreamWaitEvent(dc_stream_, fork, 0) != hipSuccess) {
-        return false;
-    }
-    if (maps) {
-        launch_dc_maps(dc_stream_, geo_, prm_, coeffs_, acs_, cfl_part_, dc_, ytox_, ytob_);
-    }
-    launch_dc_hist(dc_stream_, geo_, dc_, acs_, qf_, ytox_, ytob_, hists_ + kNumClusters * kHistStride,
-                   hists_ + (kNumClusters + geo_.num_dc) * kHistStride, fb_count_);
-    launch_huffman(dc_stream_, kNumClusters, ndc, hists_, codes);
-    launch_dc_sizes(dc_stream_, geo_, k, codes, fb_count_, blobs, blob_words_, dc_, acs_, qf_, ytox_, ytob_,
-                    chunk_bits_, dc_group_bytes_, dc_group_bits_, dc_staging_);
-    // The DC chain's end is the emission kernel's own completion (the join
-    // below and the host's first wait use it).
-    launch_dc_emit(dc_stream_, geo_, dc_, acs_, qf_, ytox_, ytob_, codes, blobs, blob_words_, chunk_bits_,
-                   dc_staging_, ev_dc_done_);
     launch_ac_tokens(stream_, geo_, ac_, acs_, nz_grid_, nz_count_, tokens_, item_tokens_, hist_partial_, hists_,
-                     listed ? ItemList{item_list_, item_count_} : ItemList{nullptr, nullptr});
+                     listed ? ItemList{item_list_, item_count_} : ItemList{nullptr, nullptr}, dc_, qf_, ytox_, ytob_,
+                     fb_count_);
     mark(Stage::kCodes);
-    launch_huffman(stream_, 0, kNumClusters, hists_, codes);
+    launch_huffman(stream_, kNumClusters + static_cast<int>(2 * geo_.num_dc), hists_, codes);
     mark(Stage::kSizes);
-    launch_ac_group_emit(stream_, geo_, acs_, item_tokens_, tokens_, codes, ac_staging_, ac_part_bits_);
-    // Join: the AC stream waits for the DC chain's end (which, forked at the
-    // region kernel's end, is done well before the AC emission: the wait on
-    // a completed event is the cheap one) and runs the layout, the assembly
-    // and the readback.
-    if (hipStreamWaitEvent(stream_, ev_dc_done_, 0) != hipSuccess) {
-        return false;
-    }
-    tail_ = stream_;
+    launch_emit(stream_, geo_, acs_, item_tokens_, tokens_, codes, k, fb_count_, dc_, qf_, ytox_, ytob_, ac_staging_,
+                ac_part_bits_, dc_staging_, chunk_bits_);
     size_bound_ = size_event;
     // Without a size event the output is written by the assembly kernel and
     // nothing follows it: its own completion ends the frame.
     end_bound_ = !size_event;
-    launch_layout(stream_, geo_, k, codes, ac_part_bits_, dc_group_bytes_, dc_group_bits_, ac_group_bytes_,
-                  ac_group_bits_, blobs, lay, ac_base_, dc_base_, total_dev_, size_event ? ev_size_ : nullptr);
-    mark(Stage::kEmit, tail_);
+    launch_layout(stream_, geo_, k, codes, ac_part_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_,
+                  ac_group_bytes_, ac_group_bits_, lay, ac_base_, dc_base_, total_dev_,
+                  size_event ? ev_size_ : nullptr);
+    mark(Stage::kEmit);
     launch_assemble(stream_, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_group_bits_, ac_part_bits_,
-                    dc_base_, ac_base_, out, cap, end_bound_ ? ev_end_ : nullptr);
+                    chunk_bits_, dc_base_, ac_base_, out, cap, end_bound_ ? ev_end_ : nullptr);
     return hipGetLastError() == hipSuccess;
 }
 

@@ -132,10 +132,8 @@ private:
     // Uploads the constant bit strings on `s` (the encoder's stream when
     // null) unless they are already those of (global_scale, quant_dc).
     bool build_constants(std::uint32_t global_scale, std::uint32_t quant_dc, hipStream_t s = nullptr);
-    // `fork_bound`: the quantizer's launch has bound `ev_fork_` already;
-    // `listed`: it also listed the non-empty items for the tokenizer.
-    bool run_entropy(std::uint8_t* out, std::size_t cap, hipEvent_t fork, bool listed, bool maps = false,
-                     bool size_event = true);
+    // `listed`: the quantizer listed the non-empty items for the tokenizer.
+    bool run_entropy(std::uint8_t* out, std::size_t cap, bool listed, bool size_event = true);
     std::uint8_t* mapped_output(std::uint8_t* dst) const;
     Clears entropy_clears() const;
     // Queues a frame after the work on `caller` (null: the null stream);
@@ -147,7 +145,7 @@ private:
     bool stage_chunk(int slot, std::size_t n);
     bool upload_nv12(const std::uint8_t* luma, std::size_t luma_pitch, const std::uint8_t* chroma,
                      std::size_t chroma_pitch);
-    void mark(Stage s, hipStream_t on = nullptr);
+    void mark(Stage s);
     bool wait_done();
     static bool spin_on(hipEvent_t e);
 
@@ -158,14 +156,11 @@ private:
     Geometry geo_{};
     FrameParams prm_{};
     hipStream_t stream_{nullptr};
-    hipStream_t dc_stream_{nullptr};  // DC entropy chain, joined by events
-    hipEvent_t ev_fork_{nullptr}, ev_dc_done_{nullptr};  // fork onto / join from the DC stream
-    hipEvent_t ev_size_{nullptr};                        // the total size has reached the host
-    hipEvent_t ev_done_{nullptr};                        // the frame's last copy has finished
+    hipEvent_t ev_size_{nullptr};  // the total size has reached the host
+    hipEvent_t ev_done_{nullptr};  // the frame's last copy has finished
     hipEvent_t ev_end_{nullptr};  // the assembly kernel's completion, when it ends the frame
     bool end_bound_{false};       // ev_end_ is bound to this frame's assembly kernel
     bool size_bound_{true};  // ev_size_ is bound to this frame's layout kernel
-    hipStream_t tail_{nullptr};  // layout, assembly and readback: the DC stream, after both chains
     hipEvent_t ev_caller_{nullptr}, ev_input_free_{nullptr};  // ordering against a caller's stream
     bool pending_{false};            // a frame's readback is queued, finish() not yet called
     std::size_t staged_{0};          // output bytes queued into the staging chunks
@@ -193,19 +188,17 @@ private:
     std::uint32_t* fb_count_{nullptr};
     void* codes_{nullptr};
     void* constants_{nullptr};
-    void* blobs_{nullptr};
-    std::uint32_t* blob_words_{nullptr};
     std::uint32_t* tokens_{nullptr};       // token records in coefficient-slot layout
     std::uint16_t* item_tokens_{nullptr};  // tokens per (block, channel) item
     std::uint32_t* item_list_{nullptr};    // first-block items (quantizer -> tokenizer), ItemList
     std::uint32_t* item_count_{nullptr};   // entries at its front and back
     std::uint32_t* hist_partial_{nullptr}; // per-workgroup AC histograms
     std::uint32_t* ac_staging_{nullptr};   // each AC group's stream at group-relative bits
-    std::uint32_t* dc_staging_{nullptr};   // each DC group's section at group-relative bits
+    std::uint32_t* dc_staging_{nullptr};   // each DC group's chunks at chunk-relative bits
     std::uint64_t* ac_part_bits_{nullptr};   // bits of each part (row band) of each AC group
     std::uint32_t* ac_group_bytes_{nullptr};
     std::uint64_t* ac_group_bits_{nullptr};
-    std::uint64_t* chunk_bits_{nullptr};
+    std::uint32_t* chunk_bits_{nullptr};   // bits of each chunk, then (layout) their offsets
     std::uint32_t* dc_group_bytes_{nullptr};
     std::uint64_t* dc_group_bits_{nullptr};
     void* layout_{nullptr};

@@ -486,8 +486,8 @@ __global__ __launch_bounds__(256) void ac_tokens_kernel(Geometry geo, const std:
 
 // Sums `parts` partial histograms of 32 x 64 bins into the 32 x 256 cluster
 // histograms: grid (bins / 256, slices); each thread adds its slice.
-__device__ __attribute__((always_inline)) inline void ac_hist_reduce_kernel_body(const Wg& wg, const std::uint32_t* __restrict__ partial, int parts,
-                                                             std::uint32_t* __restrict__ hist) {
+__device__ __forceinline__ void ac_hist_reduce_body(const Wg& wg, const std::uint32_t* __restrict__ partial, int parts,
+                                                    std::uint32_t* __restrict__ hist) {
     const int bin{static_cast<int>(wg.x) * 256 + static_cast<int>(threadIdx.x)};
     const int per{(parts + static_cast<int>(wg.ny) - 1) / static_cast<int>(wg.ny)};
     const int p0{static_cast<int>(wg.y) * per};
@@ -499,11 +499,6 @@ __device__ __attribute__((always_inline)) inline void ac_hist_reduce_kernel_body
     if (sum != 0) {
         atomicAdd(&hist[(bin / kAcSymbols) * kHistStride + bin % kAcSymbols], sum);
     }
-}
-
-__global__ __launch_bounds__(256) void ac_hist_reduce_kernel(const std::uint32_t* __restrict__ partial, int parts,
-                                                             std::uint32_t* __restrict__ hist) {
-    ac_hist_reduce_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, partial, parts, hist);
 }
 
 // Block-wide exclusive scan of one value per thread (blockDim.x multiple of 64).
@@ -563,12 +558,11 @@ struct GroupShared {
     std::uint32_t overflow;
 };
 
-__device__ __attribute__((always_inline)) inline void ac_group_emit_kernel_body(const Wg& wg, 
-    Geometry geo, const std::int8_t* __restrict__ acs, const std::uint16_t* __restrict__ item_tokens,
-    const std::uint32_t* __restrict__ tokens, const std::uint8_t* __restrict__ depth,
-    const std::uint16_t* __restrict__ codes, std::uint32_t* __restrict__ staging,
-    std::uint64_t* __restrict__ part_bits) {
-    __shared__ GroupShared S;
+__device__ __forceinline__ void ac_group_emit_body(
+    GroupShared& S, const Wg& wg, const Geometry& geo, const std::int8_t* __restrict__ acs,
+    const std::uint16_t* __restrict__ item_tokens, const std::uint32_t* __restrict__ tokens,
+    const std::uint8_t* __restrict__ depth, const std::uint16_t* __restrict__ codes,
+    std::uint32_t* __restrict__ staging, std::uint64_t* __restrict__ part_bits) {
     const int tid{static_cast<int>(threadIdx.x)};
     const int g{static_cast<int>(wg.x) / kGroupParts};
     const int part{static_cast<int>(wg.x) % kGroupParts};
@@ -752,14 +746,6 @@ __device__ __attribute__((always_inline)) inline void ac_group_emit_kernel_body(
     }
 }
 
-__global__ __launch_bounds__(kPartThreads) void ac_group_emit_kernel(
-    Geometry geo, const std::int8_t* __restrict__ acs, const std::uint16_t* __restrict__ item_tokens,
-    const std::uint32_t* __restrict__ tokens, const std::uint8_t* __restrict__ depth,
-    const std::uint16_t* __restrict__ codes, std::uint32_t* __restrict__ staging,
-    std::uint64_t* __restrict__ part_bits) {
-    ac_group_emit_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, acs, item_tokens, tokens, depth, codes, staging, part_bits);
-}
-
 // ---- DC groups -------------------------------------------------------------
 
 // Item kinds of a DcGroup section, in order (vardct_frame.cc:543-554):
@@ -798,10 +784,6 @@ __device__ __forceinline__ std::int32_t gradient_predict(bool hl, bool ht, std::
         return lo;
     }
     return static_cast<std::int32_t>(static_cast<std::int64_t>(left) + top - tl);
-}
-
-__device__ __forceinline__ std::uint32_t codes_or_zero(const std::uint16_t* codes, std::uint32_t idx) {
-    return codes != nullptr ? static_cast<std::uint32_t>(codes[idx]) : 0u;
 }
 
 // Walks the items of a DcGroup section in order.  Sections: 0 blob_pre,
@@ -927,16 +909,20 @@ __device__ __forceinline__ int dc_cursor_token(const Geometry& geo, const DcGrou
 
 constexpr int kDcChunk = 1024;               // items per workgroup in the DC passes
 constexpr int kDcPerThread = kDcChunk / 256;  // consecutive items per thread
+// Chunks of the largest DC group (256 x 256 blocks).
+constexpr int kDcMaxChunks = (2 + 6 * 65536 + 2 * 1024 + kDcChunk - 1) / kDcChunk;
+// Staging slot of one chunk: every item's token is at most 32 bits, plus the
+// two header blobs.
+constexpr int kBlobWords = 128;
+constexpr int kDcSlotWords = kDcChunk + 2 * kBlobWords;
 
 // DC and AcMetadata token histograms per group, plus the first-block count.
-__device__ __attribute__((always_inline)) inline void dc_hist_kernel_body(const Wg& wg, Geometry geo, const std::int32_t* __restrict__ dc,
-                                                      const std::int8_t* __restrict__ acs,
-                                                      const std::int32_t* __restrict__ qf,
-                                                      const std::int8_t* __restrict__ ytox,
-                                                      const std::int8_t* __restrict__ ytob,
-                                                      std::uint32_t* __restrict__ dc_hist,
-                                                      std::uint32_t* __restrict__ meta_hist,
-                                                      std::uint32_t* __restrict__ fb_count) {
+__device__ __forceinline__ void dc_hist_body(const Wg& wg, const Geometry& geo, const std::int32_t* __restrict__ dc,
+                                             const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
+                                             const std::int8_t* __restrict__ ytox,
+                                             const std::int8_t* __restrict__ ytob,
+                                             std::uint32_t* __restrict__ dc_hist, std::uint32_t* __restrict__ meta_hist,
+                                             std::uint32_t* __restrict__ fb_count) {
     __shared__ std::uint32_t h[2 * kHistStride];
     __shared__ std::uint32_t cnt;
     const int g{static_cast<int>(wg.y)};
@@ -982,234 +968,183 @@ __device__ __attribute__((always_inline)) inline void dc_hist_kernel_body(const 
     }
 }
 
-__global__ __launch_bounds__(256) void dc_hist_kernel(Geometry geo, const std::int32_t* __restrict__ dc,
-                                                      const std::int8_t* __restrict__ acs,
-                                                      const std::int32_t* __restrict__ qf,
-                                                      const std::int8_t* __restrict__ ytox,
-                                                      const std::int8_t* __restrict__ ytob,
-                                                      std::uint32_t* __restrict__ dc_hist,
-                                                      std::uint32_t* __restrict__ meta_hist,
-                                                      std::uint32_t* __restrict__ fb_count) {
-    dc_hist_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, dc, acs, qf, ytox, ytob, dc_hist, meta_hist, fb_count);
+// The partial AC histograms' sum and the DC groups' histograms in one launch
+// (independent work, a few microseconds each): workgroups below
+// kReduceWgs reduce, the others take one chunk of one DC group each.
+constexpr std::uint32_t kReduceBins = kNumClusters * kAcSymbols / 256;
+constexpr std::uint32_t kReduceSlices = 80;
+constexpr std::uint32_t kReduceWgs = kReduceBins * kReduceSlices;
+
+__device__ __forceinline__ void histograms_kernel_body(const Wg& wg, const Geometry& geo, std::uint32_t dc_chunks,
+                                                       const std::uint32_t* __restrict__ partial, int parts,
+                                                       std::uint32_t* __restrict__ hists,
+                                                       const std::int32_t* __restrict__ dc,
+                                                       const std::int8_t* __restrict__ acs,
+                                                       const std::int32_t* __restrict__ qf,
+                                                       const std::int8_t* __restrict__ ytox,
+                                                       const std::int8_t* __restrict__ ytob,
+                                                       std::uint32_t* __restrict__ fb_count) {
+    if (wg.x < kReduceWgs) {
+        ac_hist_reduce_body(Wg{wg.x % kReduceBins, wg.x / kReduceBins, kReduceBins, kReduceSlices}, partial, parts,
+                            hists);
+    } else {
+        const std::uint32_t i{wg.x - kReduceWgs};
+        dc_hist_body(Wg{i % dc_chunks, i / dc_chunks, dc_chunks, geo.num_dc}, geo, dc, acs, qf, ytox, ytob,
+                     hists + kNumClusters * kHistStride, hists + (kNumClusters + geo.num_dc) * kHistStride, fb_count);
+    }
 }
 
-struct DcBlobs {
-    // Per group: blob bit lengths and word offsets into `words`.
-    std::uint32_t pre_bits[64], mid_bits[64];
-    std::uint32_t pre_off[64], mid_off[64];
-    std::uint32_t overflow;  // a header blob exceeded its slot
+__global__ __launch_bounds__(256) void histograms_kernel(Geometry geo, std::uint32_t dc_chunks,
+                                                         const std::uint32_t* __restrict__ partial, int parts,
+                                                         std::uint32_t* __restrict__ hists,
+                                                         const std::int32_t* __restrict__ dc,
+                                                         const std::int8_t* __restrict__ acs,
+                                                         const std::int32_t* __restrict__ qf,
+                                                         const std::int8_t* __restrict__ ytox,
+                                                         const std::int8_t* __restrict__ ytob,
+                                                         std::uint32_t* __restrict__ fb_count) {
+    histograms_kernel_body(Wg{blockIdx.x, 0, gridDim.x, 1}, geo, dc_chunks, partial, parts, hists, dc, acs, qf, ytox,
+                           ytob, fb_count);
+}
+
+// The file's variable-length code of a 16-bit count (alphabet sizes).
+__device__ __forceinline__ std::uint32_t var_len_u16(std::uint32_t n, std::uint32_t& val) {
+    if (n == 0) {
+        val = 0;
+        return 1;
+    }
+    const std::uint32_t nb{31u - static_cast<std::uint32_t>(__builtin_clz(n))};
+    val = 1u | (nb << 1) | ((n - (1u << nb)) << 5);
+    return 5 + nb;
+}
+
+struct DcEmitShared {
+    std::uint32_t lut[2 * kHistStride];  // DC, then AcMetadata: depth | code << 16
+    std::uint32_t buf[kDcSlotWords];
+    std::uint64_t sh[5];
+    std::uint32_t blob_at[2];  // chunk-relative bit positions of the header blobs
 };
 
-// Code length and code of the cursor's item (0 bits for an absent item).
-__device__ __forceinline__ std::uint32_t dc_cursor_code(const Geometry& geo, const DcGroupGeo& d,
-                                                        const DcCursor& c, int g, const std::int32_t* dc,
-                                                        const std::int8_t* acs, const std::int32_t* qf,
-                                                        const std::int8_t* ytox, const std::int8_t* ytob,
-                                                        const std::uint8_t* dc_depth, const std::uint16_t* dc_codes,
-                                                        const std::uint8_t* meta_depth,
-                                                        const std::uint16_t* meta_codes, std::uint32_t& val) {
-    std::uint32_t sym, nb, bits;
-    const int kind{dc_cursor_token(geo, d, c, dc, acs, qf, ytox, ytob, sym, nb, bits)};
-    if (kind == 2) {
-        val = 0;
-        return 0;
-    }
-    const std::uint32_t idx{static_cast<std::uint32_t>(g) * kHistStride + sym};
-    const std::uint32_t dd{(kind == 0 ? dc_depth : meta_depth)[idx]};
-    val = codes_or_zero(kind == 0 ? dc_codes : meta_codes, idx) | (bits << dd);
-    return dd + nb;
-}
+// Constant bits, then a value, then a code's alphabet size and header: a
+// header blob's pieces (the first blob has no value).
+struct DcBlob {
+    std::uint32_t lead_bits, lead;  // value ahead of the constant bits
+    const std::uint32_t* words;
+    std::uint32_t word_bits;
+    std::uint32_t alpha_bits, alpha;
+    const std::uint32_t* hdr;
+    std::uint32_t hdr_bits;
+    __device__ __forceinline__ std::uint32_t bits() const { return lead_bits + word_bits + alpha_bits + hdr_bits; }
+};
 
-// Chunk bit totals of every DC group (grid: chunks x groups).
-// Bits of one chunk of a DC group's items, the two header blobs not
-// counted (the scan adds them: their sizes are built beside this pass).
-__device__ void dc_chunk_bits_body(
-    const Wg& wg, const Geometry& geo, const std::int32_t* __restrict__ dc, const std::int8_t* __restrict__ acs,
-    const std::int32_t* __restrict__ qf, const std::int8_t* __restrict__ ytox,
-    const std::int8_t* __restrict__ ytob, const std::uint8_t* __restrict__ dc_depth,
-    const std::uint8_t* __restrict__ meta_depth, std::uint64_t* __restrict__ chunk_bits,
-    std::uint32_t chunks_per_group) {
-    __shared__ std::uint64_t sh[5];
-    const int g{static_cast<int>(wg.y)};
-    const DcGroupGeo d{dc_group_geo(geo, g)};
-    const std::uint32_t k0{wg.x * kDcChunk + threadIdx.x * kDcPerThread};
-    const std::uint32_t k1{min(k0 + kDcPerThread, d.items)};
-    std::uint64_t run{0};
-    if (k0 < k1) {
-        DcCursor c{dc_cursor_at(d, k0)};
-        for (std::uint32_t k{k0}; k < k1; ++k, dc_cursor_next(d, c)) {
-            if (c.sec == 0 || c.sec == 2) {
-                continue;
-            }
-            std::uint32_t val;
-            run += dc_cursor_code(geo, d, c, g, dc, acs, qf, ytox, ytob, dc_depth, nullptr, meta_depth, nullptr,
-                                  val);
-        }
-    }
-    std::uint64_t total{0};
-    block_excl_scan(run, sh, total);
-    if (threadIdx.x == 0) {
-        chunk_bits[static_cast<std::size_t>(g) * chunks_per_group + wg.x] = total;
-    }
-}
-
-// Exclusive scan of chunk totals per group (one workgroup per group).
-// Also clears the words of the group's staging slot that its emission will
-// OR into.
-__device__ __attribute__((always_inline)) inline void dc_chunk_scan_kernel_body(const Wg& wg, Geometry geo, std::uint64_t* __restrict__ chunk_bits,
-                                                             std::uint32_t chunks_per_group,
-                                                             const DcBlobs* __restrict__ blobs,
-                                                             std::uint32_t* __restrict__ group_bytes,
-                                                             std::uint64_t* __restrict__ group_bits,
-                                                             std::uint32_t* __restrict__ staging,
-                                                             std::uint64_t slot_words) {
-    __shared__ std::uint64_t sh[17];
-    const int g{static_cast<int>(wg.x)};
-    const DcGroupGeo d{dc_group_geo(geo, g)};
-    const std::uint32_t used{(d.items + kDcChunk - 1) / kDcChunk};
+__device__ __forceinline__ void put_blob(std::uint32_t* buf, const DcBlob& b, std::uint32_t at) {
     const std::uint32_t t{threadIdx.x};
-    std::uint64_t v{0};
-    if (t < used) {
-        v = chunk_bits[static_cast<std::size_t>(g) * chunks_per_group + t];
-        // The blobs are items 0 and 1 + 3 n of the group.
-        v += t == 0 ? blobs->pre_bits[g] : 0u;
-        v += t == (1u + 3u * static_cast<std::uint32_t>(d.n)) / kDcChunk ? blobs->mid_bits[g] : 0u;
-    }
-    std::uint64_t total{0};
-    const std::uint64_t ex{block_excl_scan(v, sh, total)};
-    if (t < used) {
-        chunk_bits[static_cast<std::size_t>(g) * chunks_per_group + t] = ex;
-    }
     if (t == 0) {
-        group_bytes[g] = static_cast<std::uint32_t>((total + 7) / 8);
-        group_bits[g] = total;
+        lds_or_bits(buf, kDcSlotWords, at, b.lead, b.lead_bits);
+        lds_or_bits(buf, kDcSlotWords, at + b.lead_bits + b.word_bits, b.alpha, b.alpha_bits);
     }
-    std::uint32_t* const slot{staging + static_cast<std::size_t>(g) * slot_words};
-    const std::uint64_t nw{(total + 31) / 32 < slot_words ? (total + 31) / 32 : slot_words};
-    for (std::uint64_t i{t}; i < nw; i += 1024) {
-        slot[i] = 0;
+    const std::uint32_t w0{at + b.lead_bits}, h0{w0 + b.word_bits + b.alpha_bits};
+    for (std::uint32_t i{32 * t}; i < b.word_bits; i += 32 * 256) {
+        lds_or_bits(buf, kDcSlotWords, w0 + i, b.words[i >> 5], b.word_bits - i < 32 ? b.word_bits - i : 32u);
+    }
+    for (std::uint32_t i{32 * t}; i < b.hdr_bits; i += 32 * 256) {
+        lds_or_bits(buf, kDcSlotWords, h0 + i, b.hdr[i >> 5], b.hdr_bits - i < 32 ? b.hdr_bits - i : 32u);
     }
 }
 
-__global__ __launch_bounds__(1024) void dc_chunk_scan_kernel(Geometry geo, std::uint64_t* __restrict__ chunk_bits,
-                                                             std::uint32_t chunks_per_group,
-                                                             const DcBlobs* __restrict__ blobs,
-                                                             std::uint32_t* __restrict__ group_bytes,
-                                                             std::uint64_t* __restrict__ group_bits,
-                                                             std::uint32_t* __restrict__ staging,
-                                                             std::uint64_t slot_words) {
-    dc_chunk_scan_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, chunk_bits, chunks_per_group, blobs, group_bytes, group_bits, staging, slot_words);
-}
-
-// Emission of one chunk of a DC group into the group's staging slot, at
-// group-relative bit positions: the chunk's items occupy one contiguous bit
-// range, assembled in LDS (interior words plain-stored, the two boundary
-// words ORed into the cleared slot); a range longer than the LDS copy is
-// emitted with global atomics instead.
-constexpr int kDcEmitWords = 2048;
-
-__device__ __attribute__((always_inline)) inline void dc_emit_kernel_body(const Wg& wg, 
-    Geometry geo, const std::int32_t* __restrict__ dc, const std::int8_t* __restrict__ acs,
-    const std::int32_t* __restrict__ qf, const std::int8_t* __restrict__ ytox,
-    const std::int8_t* __restrict__ ytob, const std::uint8_t* __restrict__ dc_depth,
-    const std::uint16_t* __restrict__ dc_codes, const std::uint8_t* __restrict__ meta_depth,
-    const std::uint16_t* __restrict__ meta_codes, const DcBlobs* __restrict__ blobs,
-    const std::uint32_t* __restrict__ blob_words, const std::uint64_t* __restrict__ chunk_off,
-    std::uint32_t chunks_per_group, std::uint32_t* __restrict__ staging, std::uint64_t slot_words) {
-    __shared__ std::uint64_t sh[5];
-    __shared__ std::uint32_t buf[kDcEmitWords];
+// Emission of one chunk of a DC group's items at chunk-relative bit positions
+// into the chunk's own staging slot, with its bit count (the layout scans the
+// counts, the assembly reads the chunks back to back): one pass, since no
+// chunk's place has to be known.  The two header blobs of a group are items
+// of its chunks (the first item, and the one after the DC residuals).  The
+// group's two codes are read into LDS first; an item is tokenized once.
+__device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, const Geometry& geo,
+                                             const DcBlob& pre, const DcBlob& mid, const std::int32_t* __restrict__ dc,
+                                             const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
+                                             const std::int8_t* __restrict__ ytox,
+                                             const std::int8_t* __restrict__ ytob,
+                                             const std::uint8_t* __restrict__ dc_depth,
+                                             const std::uint16_t* __restrict__ dc_codes,
+                                             const std::uint8_t* __restrict__ meta_depth,
+                                             const std::uint16_t* __restrict__ meta_codes,
+                                             std::uint32_t* __restrict__ staging,
+                                             std::uint32_t* __restrict__ chunk_bits) {
     const int g{static_cast<int>(wg.y)};
     const int tid{static_cast<int>(threadIdx.x)};
     const DcGroupGeo d{dc_group_geo(geo, g)};
     if (wg.x * kDcChunk >= d.items) {
-        return;
+        return;  // the layout counts a group's own chunks
+    }
+    static_assert(kHistStride == 256, "one code of each per thread");
+    S.lut[tid] = static_cast<std::uint32_t>(dc_depth[tid]) | (static_cast<std::uint32_t>(dc_codes[tid]) << 16);
+    S.lut[256 + tid] =
+        static_cast<std::uint32_t>(meta_depth[tid]) | (static_cast<std::uint32_t>(meta_codes[tid]) << 16);
+    for (int i{tid}; i < kDcSlotWords; i += 256) {
+        S.buf[i] = 0;
     }
     const std::uint32_t k0{wg.x * kDcChunk + threadIdx.x * kDcPerThread};
-    const std::uint32_t k1{min(k0 + kDcPerThread, d.items)};
-    std::uint64_t run{0};
-    if (k0 < k1) {
-        DcCursor c{dc_cursor_at(d, k0)};
-        for (std::uint32_t k{k0}; k < k1; ++k, dc_cursor_next(d, c)) {
-            if (c.sec == 0 || c.sec == 2) {
-                run += c.sec == 0 ? blobs->pre_bits[g] : blobs->mid_bits[g];
-                continue;
+    int kind[kDcPerThread];  // 0 DC, 1 AcMetadata, 2 absent, 3 first blob, 4 second blob
+    std::uint32_t sym[kDcPerThread]{}, nb[kDcPerThread]{}, ext[kDcPerThread]{};
+    {
+        DcCursor c{dc_cursor_at(d, k0 < d.items ? k0 : 0u)};
+#pragma unroll
+        for (int j{0}; j < kDcPerThread; ++j) {
+            kind[j] = 2;
+            if (k0 + static_cast<std::uint32_t>(j) < d.items) {
+                if (c.sec == 0 || c.sec == 2) {
+                    kind[j] = c.sec == 0 ? 3 : 4;
+                } else {
+                    kind[j] = dc_cursor_token(geo, d, c, dc, acs, qf, ytox, ytob, sym[j], nb[j], ext[j]);
+                }
+                dc_cursor_next(d, c);
             }
-            std::uint32_t val;
-            run += dc_cursor_code(geo, d, c, g, dc, acs, qf, ytox, ytob, dc_depth, nullptr, meta_depth, nullptr,
-                                  val);
         }
+    }
+    __syncthreads();
+    std::uint32_t len[kDcPerThread], val[kDcPerThread];
+    std::uint32_t run{0};
+#pragma unroll
+    for (int j{0}; j < kDcPerThread; ++j) {
+        len[j] = 0;
+        val[j] = 0;
+        if (kind[j] < 2) {
+            const std::uint32_t e{S.lut[kind[j] * kHistStride + static_cast<int>(sym[j])]};
+            const std::uint32_t dd{e & 0xffffu};
+            len[j] = dd + nb[j];
+            val[j] = (e >> 16) | (ext[j] << dd);
+        } else if (kind[j] > 2) {
+            len[j] = kind[j] == 3 ? pre.bits() : mid.bits();
+        }
+        run += len[j];
     }
     std::uint64_t total{0};
-    const std::uint64_t rel0{block_excl_scan(run, sh, total)};
-    std::uint32_t* const out_words{staging + static_cast<std::size_t>(g) * slot_words};
-    const std::uint64_t cap_words{slot_words};
-    const std::uint64_t start{chunk_off[static_cast<std::size_t>(g) * chunks_per_group + wg.x]};
-    const std::uint64_t w0{start >> 5};
-    const std::uint64_t nw{((start + total + 31) >> 5) - w0};
-    const bool staged{nw <= static_cast<std::uint64_t>(kDcEmitWords)};
-    if (staged) {
-        for (int i{tid}; i < static_cast<int>(nw); i += 256) {
-            buf[i] = 0;
+    std::uint32_t at{static_cast<std::uint32_t>(block_excl_scan(run, S.sh, total))};
+#pragma unroll
+    for (int j{0}; j < kDcPerThread; ++j) {
+        if (kind[j] < 2) {
+            lds_or_bits(S.buf, kDcSlotWords, at, val[j], len[j]);
+        } else if (kind[j] > 2) {
+            S.blob_at[kind[j] - 3] = at;
         }
+        at += len[j];
     }
     __syncthreads();
-    const std::uint64_t lbase{w0 << 5};
-    auto put = [&](std::uint64_t at, std::uint32_t v, std::uint32_t len) {
-        if (staged) {
-            lds_or_bits(buf, kDcEmitWords, static_cast<std::uint32_t>(at - lbase), v, len);
-        } else {
-            or_bits(out_words, cap_words, at, v, len);
-        }
-    };
-    std::uint64_t pos{start + rel0};
-    if (k0 < k1) {
-        DcCursor c{dc_cursor_at(d, k0)};
-        for (std::uint32_t k{k0}; k < k1; ++k, dc_cursor_next(d, c)) {
-            if (c.sec == 0 || c.sec == 2) {
-                const std::uint32_t nbits{c.sec == 0 ? blobs->pre_bits[g] : blobs->mid_bits[g]};
-                const std::uint32_t* src{blob_words + (c.sec == 0 ? blobs->pre_off[g] : blobs->mid_off[g])};
-                for (std::uint32_t i{0}; i < nbits; i += 32) {
-                    put(pos + i, src[i >> 5], nbits - i < 32 ? nbits - i : 32u);
-                }
-                pos += nbits;
-                continue;
-            }
-            std::uint32_t val;
-            const std::uint32_t len{dc_cursor_code(geo, d, c, g, dc, acs, qf, ytox, ytob, dc_depth, dc_codes,
-                                                   meta_depth, meta_codes, val)};
-            put(pos, val, len);
-            pos += len;
-        }
+    if (wg.x == 0) {
+        put_blob(S.buf, pre, S.blob_at[0]);
     }
-    if (!staged) {
-        return;
+    if (wg.x == (1u + 3u * static_cast<std::uint32_t>(d.n)) / kDcChunk) {
+        put_blob(S.buf, mid, S.blob_at[1]);
     }
     __syncthreads();
-    for (int i{tid}; i < static_cast<int>(nw); i += 256) {
-        const std::uint64_t gi{w0 + static_cast<std::uint64_t>(i)};
-        if (gi >= cap_words) {
-            continue;
-        }
-        const std::uint32_t v{buf[i]};
-        if (i == 0 || i == static_cast<int>(nw) - 1) {
-            if (v != 0) {
-                atomicOr(&out_words[gi], v);
-            }
-        } else {
-            out_words[gi] = v;
-        }
+    const std::size_t chunk{static_cast<std::size_t>(g) * wg.nx + wg.x};
+    std::uint32_t* const slot{staging + chunk * kDcSlotWords};
+    const int nw{static_cast<int>((total + 31) / 32)};
+    for (int i{tid}; i < nw && i < kDcSlotWords; i += 256) {
+        slot[i] = S.buf[i];
     }
-}
-
-__global__ __launch_bounds__(256) void dc_emit_kernel(
-    Geometry geo, const std::int32_t* __restrict__ dc, const std::int8_t* __restrict__ acs,
-    const std::int32_t* __restrict__ qf, const std::int8_t* __restrict__ ytox,
-    const std::int8_t* __restrict__ ytob, const std::uint8_t* __restrict__ dc_depth,
-    const std::uint16_t* __restrict__ dc_codes, const std::uint8_t* __restrict__ meta_depth,
-    const std::uint16_t* __restrict__ meta_codes, const DcBlobs* __restrict__ blobs,
-    const std::uint32_t* __restrict__ blob_words, const std::uint64_t* __restrict__ chunk_off,
-    std::uint32_t chunks_per_group, std::uint32_t* __restrict__ staging, std::uint64_t slot_words) {
-    dc_emit_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, dc, acs, qf, ytox, ytob, dc_depth, dc_codes, meta_depth, meta_codes, blobs, blob_words, chunk_off, chunks_per_group, staging, slot_words);
+    if (tid == 0) {
+        chunk_bits[chunk] = static_cast<std::uint32_t>(total);
+    }
 }
 
 }  // namespace cjx

@@ -6,13 +6,12 @@
 // adaptive-quantization field, the RD transform selection over the 21 DCT8/16/32
 // candidates of the sharpened Y, the chosen DCTs of all three channels and the
 // CfL regression partials.  Only the FP16 coefficients, the transform map,
-// the quant field and three floats per region reach HBM.  The DC chain of the
-// entropy stage starts after this kernel (with dc_maps_kernel: LLF -> DC of
-// every block, and the 64x64 tiles' colour maps from the partials).
+// the quant field and three floats per region reach HBM.
 //
 // tile_quantize_kernel: one workgroup per 64x64 CfL tile: the tile's colour
-// maps (the same function), quantization of every coefficient with the CfL
-// residual and the per-block non-zero counts the entropy coder predicts from.
+// maps, quantization of every coefficient with the CfL residual, the
+// per-block non-zero counts the entropy coder predicts from, and the DC of
+// every block (from the LLF coefficients it reads anyway).
 //
 // Element layout used throughout a region: thread (wave w, lane L) at
 // iteration k owns element i = 256k + 64w + L of [0, 1024).  Element ids nest:
@@ -1848,6 +1847,10 @@ struct TileShared {
     unsigned int nz[64][3];
     int own[64];              // packed owner: local position | (n << 8)
     float maps[2];
+    // LLF coefficients: (fx, fy) of the transform at local position op in
+    // slot op + 8 fx + fy (the blocks it covers, so no two transforms meet).
+    float llf[3][64];
+    double resample[4 + 16];  // g_tables.llf2, llf4
 };
 
 __device__ __forceinline__ int owner_in_tile(const std::int8_t* acs, int bw, int bx, int by, int& ox,
@@ -1869,80 +1872,35 @@ __device__ __forceinline__ int owner_in_tile(const std::int8_t* acs, int bw, int
     return 8;
 }
 
-// The first kernel of the DC chain: thread i derives the DC of block i
-// (frontend_quantize.cu:181-199, dc_from_llf_strided: the owner transform's
+// DC coefficient of channel c of the block at local position p of a tile
+// (frontend_quantize.cu:181-199, dc_from_llf_strided): the owner transform's
 // (n/8)^2 lowest frequencies, resampled to the block, from the FP16
-// coefficients; then the DC quantization, B against Y's round trip) and,
-// for i below the tile count, the colour maps of tile i for the AcMetadata
-// (the quantizer derives its tile's maps with the same function).
-__device__ __attribute__((always_inline)) inline void dc_maps_kernel_body(const Wg& wg, Geometry geo, FrameParams prm,
-                                                      const std::uint16_t* __restrict__ coeffs,
-                                                      const std::int8_t* __restrict__ acs,
-                                                      const float* __restrict__ cfl_part, std::int32_t* __restrict__ dc,
-                                                      std::int8_t* __restrict__ ytox, std::int8_t* __restrict__ ytob) {
-    const int i{static_cast<int>(wg.x * blockDim.x + threadIdx.x)};
-    if (i < static_cast<int>(geo.cmw * geo.cmh)) {
-        float r[4][3];
-        tile_partials(geo, cfl_part, i % static_cast<int>(geo.cmw), i / static_cast<int>(geo.cmw), r);
-        int mx, mb;
-        cfl_tile_maps(r, mx, mb);
-        ytox[i] = static_cast<std::int8_t>(mx);
-        ytob[i] = static_cast<std::int8_t>(mb);
+// coefficients.
+__device__ __forceinline__ float block_dc(const TileShared& S, int p, int c) {
+    const int own{S.own[p]};
+    const int n{own >> 8}, op{own & 255};
+    const int m{n >> 3}, dx{(p & 7) - (op & 7)}, dy{(p >> 3) - (op >> 3)};
+    if (m == 1) {
+        return S.llf[c][op];
     }
-    if (i >= static_cast<int>(geo.nblocks)) {
-        return;
-    }
-    const int bw{static_cast<int>(geo.bw)};
-    const int bx{i % bw}, by{i / bw};
-    int ox, oy;
-    const int n{owner_in_tile(acs, bw, bx, by, ox, oy)};
-    const int m{n / 8}, dx{bx - ox}, dy{by - oy};
-    const std::size_t nblk{geo.nblocks};
-    const std::size_t cplane{nblk * 64};
-    float dcv[3];
-    for (int c{0}; c < 3; ++c) {
-        // Element e of the owner's transform sits in slot e % 64 of the
-        // covered block e / 64 (row-major over the m x m blocks).
-        const auto llf = [&](int e) {
-            const int qc{e >> 6};
-            const std::size_t blk{static_cast<std::size_t>(oy + qc / m) * bw + ox + qc % m};
-            return static_cast<float>(__builtin_bit_cast(_Float16, coeffs[c * cplane + blk * 64 + (e & 63)]));
-        };
-        if (m == 1) {
-            dcv[c] = llf(0);
-        } else {
-            const double* t{m == 2 ? g_tables.llf2 : g_tables.llf4};
-            double sum{0.0};
-            for (int fx{0}; fx < m; ++fx) {
-                for (int fy{0}; fy < m; ++fy) {
-                    sum += t[fx * m + dx] * t[fy * m + dy] * static_cast<double>(llf(fx * n + fy));
-                }
-            }
-            dcv[c] = static_cast<float>(static_cast<double>(m) * sum);
+    const double* const t{S.resample + (m == 2 ? 0 : 4)};
+    double sum{0.0};
+#pragma unroll 1
+    for (int fx{0}; fx < m; ++fx) {
+#pragma unroll 2
+        for (int fy{0}; fy < m; ++fy) {
+            sum += t[fx * m + dx] * t[fy * m + dy] * static_cast<double>(S.llf[c][op + 8 * fx + fy]);
         }
     }
-    const float dcq_x{4096.0f * prm.dc_scale}, dcq_y{512.0f * prm.dc_scale};
-    const float dcq_b{256.0f * prm.dc_scale};
-    const int qdy{static_cast<int>(__builtin_rintf(dcv[1] * dcq_y))};
-    const float y_dc_round{static_cast<float>(qdy) / dcq_y};
-    dc[nblk + i] = qdy;
-    dc[i] = static_cast<int>(__builtin_rintf(dcv[0] * dcq_x));
-    dc[2 * nblk + i] = static_cast<int>(__builtin_rintf((dcv[2] - 1.0f * y_dc_round) * dcq_b));
-}
-
-__global__ __launch_bounds__(256) void dc_maps_kernel(Geometry geo, FrameParams prm,
-                                                      const std::uint16_t* __restrict__ coeffs,
-                                                      const std::int8_t* __restrict__ acs,
-                                                      const float* __restrict__ cfl_part, std::int32_t* __restrict__ dc,
-                                                      std::int8_t* __restrict__ ytox, std::int8_t* __restrict__ ytob) {
-    dc_maps_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, prm, coeffs, acs, cfl_part, dc, ytox, ytob);
+    return static_cast<float>(static_cast<double>(m) * sum);
 }
 
 __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(const Wg& wg, 
     Geometry geo, FrameParams prm, const std::uint16_t* __restrict__ coeffs,
     const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
     const float* __restrict__ cfl_part, std::int16_t* __restrict__ ac,
-    std::uint8_t* __restrict__ nz_grid, std::uint16_t* __restrict__ nz_count, ItemList list) {
+    std::uint8_t* __restrict__ nz_grid, std::uint16_t* __restrict__ nz_count, ItemList list,
+    std::int32_t* __restrict__ dc, std::int8_t* __restrict__ ytox, std::int8_t* __restrict__ ytob) {
     __shared__ TileShared S;
     const int tid{static_cast<int>(threadIdx.x)};
     const int w{tid >> 6};
@@ -1962,6 +1920,10 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
         }
         S.own[tid] = ((oy - ty * 8) * 8 + (ox - tx * 8)) | (n << 8);
     }
+    if (tid >= 128 && tid < 148) {
+        const int i{tid - 128};
+        S.resample[i] = i < 4 ? g_tables.llf2[i] : g_tables.llf4[i - 4];
+    }
     if (tid == 64) {  // wave 1, beside wave 0's owners
         float r[4][3];
         tile_partials(geo, cfl_part, tx, ty, r);
@@ -1969,6 +1931,8 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
         cfl_tile_maps(r, mx, mb);
         S.maps[0] = 0.0f + static_cast<float>(mx) * (1.0f / 84);
         S.maps[1] = 1.0f + static_cast<float>(mb) * (1.0f / 84);
+        ytox[tile] = static_cast<std::int8_t>(mx);
+        ytob[tile] = static_cast<std::int8_t>(mb);
     }
     __syncthreads();
 
@@ -2010,6 +1974,19 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
             const float qgsf{static_cast<float>(qf[static_cast<std::size_t>(oy) * bw + ox]) *
                              prm.global_scale_float};
             const float rq{1.0f / qgsf};
+            // The lane's LLF coefficients (the first m of its four, in the
+            // rows fx < m) to where block_dc reads them.
+            const int fx{e0 >> (n == 32 ? 5 : (n == 16 ? 4 : 3))};
+            if ((e0 & (n - 1)) == 0 && fx < m) {
+#pragma unroll
+                for (int i{0}; i < 4; ++i) {
+                    if (i < m) {
+                        S.llf[0][op + 8 * fx + i] = f16_at(hx, i);
+                        S.llf[1][op + 8 * fx + i] = f16_at(hy, i);
+                        S.llf[2][op + 8 * fx + i] = f16_at(hb, i);
+                    }
+                }
+            }
             const int cs{n * n};
             const float* const wt{n == 32 ? &g_tables.dequant32[0][0]
                                           : (n == 16 ? &g_tables.dequant16[0][0] : &g_tables.dequant8[0][0])};
@@ -2060,6 +2037,24 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
     }
     __syncthreads();
 
+    if (w > 0) {
+        // The DC values, beside wave 0's lists: waves 1, 2 and 3 take X, Y
+        // and B (against Y's round trip).
+        const int bx{tx * 8 + (lane & 7)}, by{ty * 8 + (lane >> 3)};
+        if (bx < bw && by < bh) {
+            const float scale_y{512.0f * prm.dc_scale};
+            float v{block_dc(S, lane, w - 1)};
+            float scale{w == 1 ? 4096.0f * prm.dc_scale : scale_y};
+            if (w == 3) {
+                const float qy{__builtin_rintf(block_dc(S, lane, 1) * scale_y)};
+                const float y_dc_round{static_cast<float>(static_cast<int>(qy)) / scale_y};
+                v = v - 1.0f * y_dc_round;
+                scale = 256.0f * prm.dc_scale;
+            }
+            dc[static_cast<std::size_t>(w - 1) * nblk + static_cast<std::size_t>(by) * bw + bx] =
+                static_cast<int>(__builtin_rintf(v * scale));
+        }
+    }
     if (tid < 64) {
         const int p{tid};
         const int bx{tx * 8 + (p & 7)}, by{ty * 8 + (p >> 3)};
@@ -2127,8 +2122,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void t
     Geometry geo, FrameParams prm, const std::uint16_t* __restrict__ coeffs,
     const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
     const float* __restrict__ cfl_part, std::int16_t* __restrict__ ac,
-    std::uint8_t* __restrict__ nz_grid, std::uint16_t* __restrict__ nz_count, ItemList list) {
-    tile_quantize_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, prm, coeffs, acs, qf, cfl_part, ac, nz_grid, nz_count, list);
+    std::uint8_t* __restrict__ nz_grid, std::uint16_t* __restrict__ nz_count, ItemList list,
+    std::int32_t* __restrict__ dc, std::int8_t* __restrict__ ytox, std::int8_t* __restrict__ ytob) {
+    tile_quantize_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, prm, coeffs, acs, qf, cfl_part, ac,
+                              nz_grid, nz_count, list, dc, ytox, ytob);
 }
 
 // ---------------------------------------------------------------------------

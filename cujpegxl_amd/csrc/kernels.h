@@ -13,14 +13,14 @@ namespace cjx {
 struct Constants;
 struct CodeSet;
 struct Layout;
-struct DcBlobs;
 
 std::size_t sizeof_constants();
 std::size_t sizeof_codeset();
 std::size_t sizeof_layout();
-std::size_t sizeof_dc_blobs();
-std::uint32_t dc_chunks_per_group();
-std::uint32_t blob_words_per_group();
+// Chunks of a frame's largest DC group (the stride of its chunk tables), and
+// words of one chunk's staging slot.
+std::uint32_t dc_chunks_per_group(const Geometry& geo);
+std::size_t dc_chunk_slot_words();
 // Host view of Constants to fill before upload.
 void fill_constants(void* dst, const std::uint32_t* head, std::uint32_t head_bits,
                     const std::uint32_t* dc_global, std::uint32_t dc_global_bits,
@@ -61,12 +61,8 @@ void launch_dct8_uniform(hipStream_t s, const Geometry& geo, const FrameParams& 
 void launch_tile_quantize(hipStream_t s, const Geometry& geo, const FrameParams& prm,
                           const std::uint16_t* coeffs, const std::int8_t* acs, const std::int32_t* qf,
                           const float* cfl_part, std::int16_t* ac, std::uint8_t* nz_grid,
-                          std::uint16_t* nz_count, const ItemList& list);
-// LLF -> DC of every block from the FP16 coefficients, and the 64x64
-// tiles' colour maps from the regions' CfL partials.
-void launch_dc_maps(hipStream_t s, const Geometry& geo, const FrameParams& prm, const std::uint16_t* coeffs,
-                    const std::int8_t* acs, const float* cfl_part, std::int32_t* dc, std::int8_t* ytox,
-                    std::int8_t* ytob);
+                          std::uint16_t* nz_count, const ItemList& list, std::int32_t* dc, std::int8_t* ytox,
+                          std::int8_t* ytob);
 void launch_nz(hipStream_t s, const Geometry& geo, const std::int16_t* ac, const std::int8_t* acs,
                std::uint8_t* nz_grid, std::uint16_t* nz_count, const Clears& clr);
 void launch_fill_u32(hipStream_t s, std::uint32_t* p, std::size_t n, std::uint32_t v);
@@ -74,48 +70,39 @@ void launch_fill_u32(hipStream_t s, std::uint32_t* p, std::size_t n, std::uint32
 // root against the compiler's correctly rounded forms, over every float
 // input of their domains (check_aq_math_kernel); false on a HIP error.
 bool check_aq_math(unsigned long long* mismatches);
+// The AC tokens, then the histograms of every AC cluster and DC group.
 void launch_ac_tokens(hipStream_t s, const Geometry& geo, const std::int16_t* ac, const std::int8_t* acs,
                       const std::uint8_t* nz_grid, const std::uint16_t* nz_count, std::uint32_t* tokens,
-                      std::uint16_t* item_tokens, std::uint32_t* partial, std::uint32_t* hist,
-                      const ItemList& list);
+                      std::uint16_t* item_tokens, std::uint32_t* partial, std::uint32_t* hists,
+                      const ItemList& list, const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox,
+                      const std::int8_t* ytob, std::uint32_t* fb_count);
 std::size_t ac_partial_words();
-void launch_dc_hist(hipStream_t s, const Geometry& geo, const std::int32_t* dc, const std::int8_t* acs,
-                    const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                    std::uint32_t* dc_hist, std::uint32_t* meta_hist, std::uint32_t* fb_count);
 // Builds the codes of `count` host histograms on the current device and copies
 // the results back (stage harness; allocates).
 bool build_codes_host(const std::uint32_t* hists, std::uint32_t count, std::uint32_t* alpha, std::uint8_t* depth,
                       std::uint16_t* bits, std::uint32_t* hdr_words, std::uint32_t* hdr_bits);
-void launch_huffman(hipStream_t s, int first, int count, const std::uint32_t* hists, CodeSet* cs);
+void launch_huffman(hipStream_t s, int count, const std::uint32_t* hists, CodeSet* cs);
 // Words of one AC group's staging slot (bound on its token stream).
 std::size_t ac_group_slot_words();
 // AC groups are emitted in this many parts (row bands).
 std::size_t ac_group_parts();
-void launch_ac_group_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs,
-                          const std::uint16_t* item_tokens, const std::uint32_t* tokens, const CodeSet* cs,
-                          std::uint32_t* staging, std::uint64_t* part_bits, hipEvent_t done = nullptr);
-// Words of one DC group's staging slot.
-std::size_t dc_group_slot_words();
-// The DC chain's sizing: header blobs and chunk bits in one launch, then
-// the per-group scan of chunk offsets (which adds the blobs' bits).
-void launch_dc_sizes(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                     const std::uint32_t* fb_count, DcBlobs* blobs, std::uint32_t* blob_words, const std::int32_t* dc,
-                     const std::int8_t* acs, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                     std::uint64_t* chunk_bits, std::uint32_t* group_bytes, std::uint64_t* group_bits,
-                     std::uint32_t* staging);
+// The AC groups' parts and the DC groups' chunks into their staging slots,
+// with their bit counts.
+void launch_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs, const std::uint16_t* item_tokens,
+                 const std::uint32_t* tokens, const CodeSet* cs, const Constants* k, const std::uint32_t* fb_count,
+                 const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
+                 std::uint32_t* ac_staging, std::uint64_t* ac_part_bits, std::uint32_t* dc_staging,
+                 std::uint32_t* chunk_bits);
+// `chunk_bits` becomes the chunks' bit offsets in their groups.
 void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                   const std::uint64_t* ac_part_bits, const std::uint32_t* dc_group_bytes,
-                   const std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
-                   const DcBlobs* blobs, Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base,
-                   std::uint64_t* total_out, hipEvent_t done = nullptr);
+                   const std::uint64_t* ac_part_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
+                   std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
+                   Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base, std::uint64_t* total_out,
+                   hipEvent_t done = nullptr);
 void launch_assemble(hipStream_t s, const Geometry& geo, const Constants* k, const Layout* lay,
                      const std::uint32_t* dc_staging, const std::uint32_t* ac_staging, const std::uint64_t* dc_bits,
-                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits, const std::uint64_t* dc_base,
-                     const std::uint64_t* ac_base, std::uint8_t* out, std::uint64_t cap_bytes,
-                     hipEvent_t done = nullptr);
-void launch_dc_emit(hipStream_t s, const Geometry& geo, const std::int32_t* dc, const std::int8_t* acs,
-                    const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                    const CodeSet* cs, const DcBlobs* blobs, const std::uint32_t* blob_words,
-                    const std::uint64_t* chunk_off, std::uint32_t* staging, hipEvent_t done = nullptr);
+                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits, const std::uint32_t* chunk_off,
+                     const std::uint64_t* dc_base, const std::uint64_t* ac_base, std::uint8_t* out,
+                     std::uint64_t cap_bytes, hipEvent_t done = nullptr);
 
 }  // namespace cjx

@@ -1,0 +1,47 @@
+"""GPU: the section layout at DC group edges.  A frame's DC groups are coded
+in chunks of 1,024 items, each at its own bit positions, and joined by the
+assembly: sizes whose last groups are one block wide or high (fewer chunks
+than the largest group, items of one chunk straddling the header blobs), and
+a batch that mixes them.  Files equal the oracle's byte for byte."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import cujpegxl_amd as cj
+from cujpegxl_amd.synth import synthetic_nv12
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(2056, 264, 0.8), (264, 2056, 1.5), (2064, 2056, 1.0), (264, 8, 1.0), (4104, 64, 3.0)]
+
+
+def device_frame(w, h, seed):
+    luma, chroma = synthetic_nv12(w, h, seed)
+    dev = cj.DeviceBuffer.from_array(np.concatenate([luma.ravel(), chroma.ravel()]))
+    return luma, chroma, dev, (dev.ptr, dev.ptr + w * h, w, w)
+
+
+@pytest.mark.parametrize("w,h,d", SIZES)
+def test_dc_group_edges(jo, w, h, d):
+    luma, chroma, dev, planes = device_frame(w, h, 7)
+    enc = cj.Encoder(w, h, d)
+    want = jo.encode_nv12(luma, chroma, w, h, d)
+    for _ in range(2):
+        assert enc.encode_device(*planes) == want
+    enc.close()
+    dev.close()
+
+
+def test_batch_of_dc_group_edges(jo):
+    frames = [device_frame(w, h, 11 + i) for i, (w, h, _) in enumerate(SIZES)]
+    b = cj.Batch([(w, h) for w, h, _ in SIZES], [d for _, _, d in SIZES])
+    b.set_inputs([f[3] for f in frames])
+    want = [jo.encode_nv12(f[0], f[1], w, h, d) for f, (w, h, d) in zip(frames, SIZES)]
+    for _ in range(2):
+        b.run(1)
+        assert b.files() == want
+    b.close()
+    for f in frames:
+        f[2].close()
