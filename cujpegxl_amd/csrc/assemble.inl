@@ -37,6 +37,8 @@ struct CodeSet {
     std::uint32_t hdr[96][kHdrWords];
     std::uint32_t hdr_bits[96];
     std::uint32_t alpha[96];
+    // The AC codes as the emission reads them: depth | code << 16.
+    alignas(16) std::uint32_t lut[kNumClusters * kAcSymbols];
 };
 
 struct Layout {
@@ -164,6 +166,10 @@ __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const 
         cs->depth[h][i] = S.depth[i];
         cs->code[h][i] = S.code[i];
     }
+    if (h < kNumClusters && t < kAcSymbols) {
+        cs->lut[h * kAcSymbols + t] =
+            static_cast<std::uint32_t>(S.depth[t]) | (static_cast<std::uint32_t>(S.code[t]) << 16);
+    }
     if (t < kHdrWords) {
         cs->hdr[h][t] = S.hdr[t];
     }
@@ -178,10 +184,9 @@ __global__ __launch_bounds__(64 * kTrials) void huffman_kernel(const std::uint32
     huffman_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, hists, cs);
 }
 
-// Emission of a frame's tokens, one launch: workgroups below num_ac *
-// kGroupParts write one part of an AC group each, the others one chunk of a
-// DC group.  The DC chunks need far less time than the AC parts and fit
-// beside them in one resident round, so they cost no launch of their own.
+// Emission of a frame's tokens, one launch: workgroups below ac_wgs write
+// runs of an AC group's band, the others one chunk of a DC group.  The DC chunks need no more time than a run and fit beside the
+// runs, so they cost no launch of their own.
 struct EmitArgs {
     const std::int8_t* acs;
     const std::uint16_t* item_tokens;
@@ -194,10 +199,11 @@ struct EmitArgs {
     const std::int8_t* ytox;
     const std::int8_t* ytob;
     std::uint32_t* ac_staging;
-    std::uint64_t* ac_part_bits;
+    std::uint16_t* ac_run_bits;
     std::uint32_t* dc_staging;
     std::uint32_t* chunk_bits;
     std::uint32_t dc_chunks;  // per DC group (the largest group's)
+    std::uint32_t ac_wgs;     // workgroups of the AC groups
 };
 
 union EmitShared {
@@ -208,13 +214,12 @@ union EmitShared {
 __device__ __attribute__((always_inline)) inline void emit_kernel_body(const Wg& wg, const Geometry& geo,
                                                                        const EmitArgs& a) {
     __shared__ EmitShared S;
-    const std::uint32_t ac_wgs{geo.num_ac * kGroupParts};
-    if (wg.x < ac_wgs) {
-        ac_group_emit_body(S.ac, wg, geo, a.acs, a.item_tokens, a.tokens, &a.cs->depth[0][0], &a.cs->code[0][0],
-                           a.ac_staging, a.ac_part_bits);
+    if (wg.x < a.ac_wgs) {
+        ac_group_emit_body(S.ac, wg, geo, a.acs, a.item_tokens, a.tokens, a.cs->lut, a.ac_staging, a.ac_run_bits,
+                           static_cast<int>(a.ac_wgs / (geo.num_ac * kGroupBands)));
         return;
     }
-    const std::uint32_t i{wg.x - ac_wgs};
+    const std::uint32_t i{wg.x - a.ac_wgs};
     const Wg dwg{i % a.dc_chunks, i / a.dc_chunks, a.dc_chunks, geo.num_dc};
     const int hd{kNumClusters + static_cast<int>(dwg.y)}, hm{hd + static_cast<int>(geo.num_dc)};
     const DcGroupGeo d{dc_group_geo(geo, static_cast<int>(dwg.y))};
@@ -239,7 +244,7 @@ __device__ __attribute__((always_inline)) inline void emit_kernel_body(const Wg&
                  a.cs->depth[hm], a.cs->code[hm], a.dc_staging, a.chunk_bits);
 }
 
-__global__ __launch_bounds__(kPartThreads) void emit_kernel(Geometry geo, EmitArgs a) {
+__global__ __launch_bounds__(kEmitThreads) void emit_kernel(Geometry geo, EmitArgs a) {
     emit_kernel_body(Wg{blockIdx.x, 0, gridDim.x, 1}, geo, a);
 }
 
@@ -286,7 +291,7 @@ __device__ __forceinline__ void u32_code(const Distr* d, std::uint32_t value, st
 // one section without padding in between.
 __device__ __attribute__((always_inline)) inline void layout_kernel_body(const Wg& wg, Geometry geo, const Constants* __restrict__ k,
                                                      const CodeSet* __restrict__ cs,
-                                                     const std::uint64_t* __restrict__ ac_part_bits,
+                                                     const std::uint16_t* __restrict__ ac_run_bits,
                                                      std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
                                                      std::uint32_t* __restrict__ dc_group_bytes,
                                                      std::uint64_t* __restrict__ dc_group_bits,
@@ -332,8 +337,8 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
 #pragma unroll
         for (int r{0}; r < kDcRounds; ++r) {
             const std::uint32_t incl{wave_incl_scan_u32(v[r])};
-            if (64 * r + lane < used) {
-                cb[64 * r + lane] = sum + incl - v[r];
+            if (64 * r + lane < static_cast<int>(dc_chunks)) {
+                cb[64 * r + lane] = sum + incl - v[r];  // chunks past the group's end: empty, at its end
             }
             sum += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
         }
@@ -343,15 +348,25 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
             dc_group_bytes[g] = (sum + 7) / 8;
         }
     }
-    // AC group sizes: the sums of their parts' bits.
+    // AC group sizes: the sums of their runs' bits, eight to a 16-byte read.
     for (int g{t}; g < static_cast<int>(geo.num_ac); g += 256) {
-        std::uint64_t sum{0};
-        for (int p{0}; p < kGroupParts; ++p) {
-            sum += ac_part_bits[g * kGroupParts + p];
+        const uint4* const rb{reinterpret_cast<const uint4*>(ac_run_bits + static_cast<std::size_t>(g) * kGroupRuns)};
+        constexpr int kVecs{kGroupRuns / 8};
+        uint4 v[kVecs];
+#pragma unroll
+        for (int i{0}; i < kVecs; ++i) {
+            v[i] = rb[i];
+        }
+        std::uint32_t sum{0};
+#pragma unroll
+        for (int i{0}; i < kVecs; ++i) {
+            for (const std::uint32_t w : {v[i].x, v[i].y, v[i].z, v[i].w}) {
+                sum += (w & 0xffffu) + (w >> 16);
+            }
         }
         agbits[g] = sum;
         ac_group_bits[g] = sum;
-        ac_group_bytes[g] = static_cast<std::uint32_t>((sum + 7) / 8);
+        ac_group_bytes[g] = (sum + 7) / 8;
     }
     for (int i{t}; i < kAcGlobalWords; i += 256) {
         agw[i] = 0;
@@ -519,7 +534,7 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
 
 __global__ __launch_bounds__(256) void layout_kernel(Geometry geo, const Constants* __restrict__ k,
                                                      const CodeSet* __restrict__ cs,
-                                                     const std::uint64_t* __restrict__ ac_part_bits,
+                                                     const std::uint16_t* __restrict__ ac_run_bits,
                                                      std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
                                                      std::uint32_t* __restrict__ dc_group_bytes,
                                                      std::uint64_t* __restrict__ dc_group_bits,
@@ -528,185 +543,211 @@ __global__ __launch_bounds__(256) void layout_kernel(Geometry geo, const Constan
                                                      Layout* __restrict__ lay, std::uint64_t* __restrict__ ac_base,
                                                      std::uint64_t* __restrict__ dc_base,
                                                      std::uint64_t* __restrict__ total_out) {
-    layout_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, cs, ac_part_bits, chunk_bits,
+    layout_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, cs, ac_run_bits, chunk_bits,
                        dc_chunks, dc_group_bytes, dc_group_bits, ac_group_bytes, ac_group_bits, lay, ac_base, dc_base,
                        total_out);
 }
 
-// The file is a sequence of bit strings ("pieces") laid end to end, each at
-// the position the layout gave it: framing, head (headers and TOC), DcGlobal,
-// the DC groups, AcGlobal, the AC groups.  Gaps between pieces (section
-// padding) are zero bits.  Each output word is built once from the pieces
-// that overlap it and stored whole, so the output needs no clearing and no
-// atomics.
-struct Pieces {
+// The file is a sequence of bit strings ("runs") laid end to end, each at the
+// position the layout gave it or that follows from it: framing, head (headers
+// and TOC), DcGlobal, the chunks of the DC groups, AcGlobal, the runs of the
+// AC groups.  Gaps between runs (section padding, under 8 bits) are zero bits.
+// One wave takes a run and stores the 64-byte lines whose first bit lies
+// between its start and the next run's, so that every output word is built
+// and stored once (no clearing, no atomics, full lines over the host link);
+// only the last of them takes bits of the runs that follow.
+struct Sources {
     const std::uint32_t* dc_staging;  // dc_chunks slots of kDcSlotWords per group
     const std::uint32_t* chunk_off;   // the chunks' bit offsets in their group
     std::uint32_t dc_chunks;
-    const std::uint32_t* ac_staging;  // kGroupParts slots of kPartSlotWords per group
+    const std::uint32_t* ac_staging;   // kGroupRuns slots of kRunWords per group
+    const std::uint16_t* ac_run_bits;  // the runs' bit counts
     const std::uint64_t* dc_bits;
-    const std::uint64_t* ac_bits;
-    const std::uint64_t* ac_part_bits;
     const std::uint64_t* dc_base;
     const std::uint64_t* ac_base;
 };
 
-constexpr int kMaxPieces = 4 + 32 + kMaxAcGroups;
+// Runs of a frame: framing, head, DcGlobal, AcGlobal and the groups'.
+__host__ __device__ __forceinline__ std::uint32_t frame_runs(const Geometry& geo, std::uint32_t dc_chunks) {
+    return 4 + geo.num_dc * dc_chunks + geo.num_ac * kGroupRuns;
+}
 
-// A piece's bits are one run at `src`; or, for an AC group (`parts` set), the
-// concatenation of its parts' runs; or, for a DC group (`offs` set), of its
-// chunks' runs.
-struct Piece {
+struct Run {
     std::uint64_t dst;
-    std::uint64_t nbits;
+    std::uint32_t nbits;
     const std::uint32_t* src;
-    const std::uint64_t* parts;
-    const std::uint32_t* offs;
-    int chunks;
 };
 
-// `len` (1..32) bits of a run from bit `o`.
-__device__ __forceinline__ std::uint32_t run_bits(const std::uint32_t* src, std::uint64_t o, std::uint32_t len) {
-    const std::uint32_t sh{static_cast<std::uint32_t>(o & 31u)};
-    std::uint32_t x{src[o >> 5] >> sh};
-    if (sh != 0 && len > 32 - sh) {
-        x |= src[(o >> 5) + 1] << (32 - sh);
-    }
-    return len < 32 ? x & ((1u << len) - 1u) : x;
-}
-
-__device__ __forceinline__ std::uint32_t piece_bits(const Piece& pc, std::uint64_t o, std::uint32_t len) {
-    std::uint32_t v{0}, got{0};
-    if (pc.offs != nullptr) {
-        // The last chunk starting at or before bit o, then on from there.
-        const std::uint32_t bits{static_cast<std::uint32_t>(pc.nbits)};
-        std::uint32_t at{static_cast<std::uint32_t>(o)};
-        int c{0}, hi{pc.chunks - 1};
-        while (c < hi) {
-            const int mid{(c + hi + 1) >> 1};
-            if (pc.offs[mid] <= at) {
-                c = mid;
-            } else {
-                hi = mid - 1;
-            }
-        }
-        for (; c < pc.chunks && got < len; ++c) {
-            const std::uint32_t first{pc.offs[c]}, last{c + 1 < pc.chunks ? pc.offs[c + 1] : bits};
-            const std::uint32_t take{min(last - at, len - got)};
-            if (take != 0) {
-                v |= run_bits(pc.src + static_cast<std::size_t>(c) * kDcSlotWords, at - first, take) << got;
-                got += take;
-                at += take;
-            }
-        }
-        return v;
-    }
-    if (pc.parts == nullptr) {
-        return run_bits(pc.src, o, len);
-    }
-    std::uint64_t start{0};
-    for (int p{0}; p < kGroupParts && got < len; ++p) {
-        const std::uint64_t pb{pc.parts[p]};
-        if (o < start + pb) {
-            const std::uint64_t off{o - start};
-            const std::uint32_t take{static_cast<std::uint32_t>(
-                pb - off < static_cast<std::uint64_t>(len - got) ? pb - off : static_cast<std::uint64_t>(len - got))};
-            v |= run_bits(pc.src + static_cast<std::size_t>(p) * kPartSlotWords, off, take) << got;
-            got += take;
-            o += take;
-        }
-        start += pb;
-    }
-    return v;
-}
-
-__device__ __forceinline__ Piece piece_at(const Geometry& geo, const Constants* k, const Layout* lay,
-                                          const Pieces& P, int i) {
-    const int nd{static_cast<int>(geo.num_dc)};
-    const auto run = [](std::uint64_t dst, std::uint64_t nbits, const std::uint32_t* src) {
-        return Piece{dst, nbits, src, nullptr, nullptr, 0};
-    };
+// Run i < 4 + num_dc * dc_chunks: every run but the AC groups'.
+__device__ __forceinline__ Run front_run(const Geometry& geo, const Constants* k, const Layout* lay, const Sources& P,
+                                         std::uint32_t i) {
     if (i == 0) {
-        return run(0, static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->framing_words);
+        return {0, lay->framing_bytes * 8, lay->framing_words};
     }
     if (i == 1) {
-        return run(static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->head_total_bits, lay->head_words);
+        return {static_cast<std::uint64_t>(lay->framing_bytes) * 8, lay->head_total_bits, lay->head_words};
     }
     if (i == 2) {
-        return run(lay->dc_global_bit, k->dc_global_bits, k->dc_global_words);
+        return {lay->dc_global_bit, k->dc_global_bits, k->dc_global_words};
     }
-    if (i < 3 + nd) {
-        const int g{i - 3};
-        const DcGroupGeo d{dc_group_geo(geo, g)};
-        const std::size_t c0{static_cast<std::size_t>(g) * P.dc_chunks};
-        return {P.dc_base[g], P.dc_bits[g], P.dc_staging + c0 * kDcSlotWords, nullptr, P.chunk_off + c0,
-                static_cast<int>((d.items + kDcChunk - 1) / kDcChunk)};
+    if (i == 3 + geo.num_dc * P.dc_chunks) {
+        return {lay->ac_global_bit, lay->ac_global_bits, lay->ac_global_words};
     }
-    if (i == 3 + nd) {
-        return run(lay->ac_global_bit, lay->ac_global_bits, lay->ac_global_words);
-    }
-    const int g{i - 4 - nd};
-    return {P.ac_base[g], P.ac_bits[g], P.ac_staging + static_cast<std::size_t>(g) * kGroupParts * kPartSlotWords,
-            P.ac_part_bits + static_cast<std::size_t>(g) * kGroupParts, nullptr, 0};
+    const std::uint32_t c{i - 3}, g{c / P.dc_chunks};
+    const std::uint32_t off{P.chunk_off[c]};
+    const std::uint32_t end{(c + 1) % P.dc_chunks != 0 ? P.chunk_off[c + 1] : static_cast<std::uint32_t>(P.dc_bits[g])};
+    return {P.dc_base[g] + off, end - off, P.dc_staging + static_cast<std::size_t>(c) * kDcSlotWords};
 }
 
-__device__ __attribute__((always_inline)) inline void assemble_kernel_body(const Wg& wg, Geometry geo, const Constants* __restrict__ k,
-                                                       const Layout* __restrict__ lay, Pieces P,
-                                                       std::uint32_t* __restrict__ out_words,
-                                                       std::uint64_t cap_bytes) {
-    __shared__ std::uint64_t end_bit[kMaxPieces];
+// The runs of one AC group, in a wave: lane l holds the sizes of runs 2 l and
+// 2 l + 1 and where they end, so that a run's place takes no memory access.
+struct AcRuns {
+    std::uint32_t g, pair, incl;
+    std::uint64_t base;
+};
+
+__device__ __forceinline__ AcRuns ac_runs(const Sources& P, std::uint32_t g) {
+    static_assert(kGroupRuns % 2 == 0 && kGroupRuns <= 128, "two run sizes per lane");
+    const std::uint32_t lane{threadIdx.x & 63u};
+    AcRuns a;
+    a.g = g;
+    a.base = P.ac_base[g];
+    a.pair = 2 * lane < kGroupRuns
+                 ? reinterpret_cast<const std::uint32_t*>(P.ac_run_bits)[g * (kGroupRuns / 2) + lane]
+                 : 0u;
+    a.incl = wave_incl_scan_u32((a.pair & 0xffffu) + (a.pair >> 16));
+    return a;
+}
+
+__device__ __forceinline__ Run ac_run(const AcRuns& a, const Sources& P, std::uint32_t r) {
+    const int at{static_cast<int>(r >> 1)};
+    const std::uint32_t end{static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(a.incl), at))};
+    const std::uint32_t pair{static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(a.pair), at))};
+    const std::uint32_t lo{pair & 0xffffu}, hi{pair >> 16};
+    const std::uint32_t nbits{(r & 1) != 0 ? hi : lo};
+    return {a.base + (end - hi - ((r & 1) != 0 ? 0u : lo)), nbits,
+            P.ac_staging + (static_cast<std::size_t>(a.g) * kGroupRuns + r) * kRunWords};
+}
+
+// First run at or after r with bits; kGroupRuns when there is none.
+__device__ __forceinline__ std::uint32_t next_ac_run(const AcRuns& a, std::uint32_t r) {
+    const std::uint64_t even{__ballot((a.pair & 0xffffu) != 0)}, odd{__ballot((a.pair >> 16) != 0)};
+    const std::uint32_t e0{(r + 1) >> 1}, o0{r >> 1};  // first even / odd run at or after r, by lane
+    const std::uint64_t e{e0 < 64 ? even >> e0 << e0 : 0ull}, o{o0 < 64 ? odd >> o0 << o0 : 0ull};
+    const std::uint32_t er{e != 0 ? 2 * static_cast<std::uint32_t>(__builtin_ctzll(e)) : kGroupRuns};
+    const std::uint32_t orr{o != 0 ? 2 * static_cast<std::uint32_t>(__builtin_ctzll(o)) + 1 : kGroupRuns};
+    return er < orr ? er : orr;
+}
+
+// The bits of `r` that fall into the 32-bit word at bit b0 of the file.
+__device__ __forceinline__ std::uint32_t run_word(const Run& r, std::uint64_t b0) {
+    const std::uint64_t end{r.dst + r.nbits};
+    const std::uint64_t s{r.dst > b0 ? r.dst : b0};
+    const std::uint64_t e{end < b0 + 32 ? end : b0 + 32};
+    if (s >= e) {
+        return 0;
+    }
+    const std::uint32_t o{static_cast<std::uint32_t>(s - r.dst)}, len{static_cast<std::uint32_t>(e - s)};
+    const std::uint32_t sh{o & 31u};
+    std::uint32_t x{r.src[o >> 5] >> sh};
+    if (sh != 0 && len > 32 - sh) {
+        x |= r.src[(o >> 5) + 1] << (32 - sh);
+    }
+    if (len < 32) {
+        x &= (1u << len) - 1u;
+    }
+    return x << static_cast<std::uint32_t>(s - b0);
+}
+
+__device__ __attribute__((always_inline)) inline void assemble_kernel_body(const Wg& wg, const Geometry& geo,
+                                                                           const Constants* __restrict__ k,
+                                                                           const Layout* __restrict__ lay,
+                                                                           const Sources& P,
+                                                                           std::uint32_t* __restrict__ out_words,
+                                                                           std::uint64_t cap_bytes) {
     if (lay->overflow != 0) {
         return;
     }
-    const int n{4 + static_cast<int>(geo.num_dc) + static_cast<int>(geo.num_ac)};
-    for (int i{static_cast<int>(threadIdx.x)}; i < n; i += 256) {
-        const Piece pc{piece_at(geo, k, lay, P, i)};
-        end_bit[i] = pc.dst + pc.nbits;
-    }
-    __syncthreads();
+    const std::uint32_t runs{frame_runs(geo, P.dc_chunks)};
     // Whole words up to the capacity, then the bytes of a partial last word
     // that still fit (the output may be the caller's mapped host buffer).
     std::uint64_t words{(lay->total_bytes + 3) / 4};
     const std::uint64_t cap_words{(cap_bytes + 3) / 4};
     words = words < cap_words ? words : cap_words;
-    for (std::uint64_t w{wg.x * 256ull + threadIdx.x}; w < words; w += wg.nx * 256ull) {
-        const std::uint64_t b0{w * 32};
-        // First piece ending after b0 (pieces are ordered and disjoint).
-        int lo{0}, hi{n};
-        while (lo < hi) {
-            const int mid{(lo + hi) >> 1};
-            if (end_bit[mid] > b0) {
-                hi = mid;
-            } else {
-                lo = mid + 1;
-            }
+    const std::uint32_t lane{threadIdx.x & 63u};
+    const std::uint32_t wave{static_cast<std::uint32_t>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(wg.x * 4 + (threadIdx.x >> 6))))};
+    const std::uint32_t front{4 + geo.num_dc * P.dc_chunks};
+    for (std::uint32_t i{wave}; i < runs; i += wg.nx * 4) {
+        AcRuns group{};
+        Run own;
+        if (i < front) {
+            own = front_run(geo, k, lay, P, i);
+        } else {
+            group = ac_runs(P, (i - front) / kGroupRuns);
+            own = ac_run(group, P, (i - front) % kGroupRuns);
         }
-        std::uint32_t v{0};
-        for (int i{lo}; i < n; ++i) {
-            const Piece pc{piece_at(geo, k, lay, P, i)};
-            if (pc.dst >= b0 + 32) {
-                break;
+        // Padding never crosses a line: the next run's first line is the
+        // first line at or after this run's end.
+        const std::uint64_t own_end{own.dst + own.nbits};
+        const std::uint64_t w0{(own.dst + 511) / 512 * 16};
+        std::uint64_t w1{(own_end + 511) / 512 * 16};
+        w1 = w1 < words ? w1 : words;
+        for (std::uint64_t base{w0}; base < w1; base += 64) {
+            const std::uint64_t w{base + lane};
+            std::uint32_t v{w < w1 ? run_word(own, w * 32) : 0u};
+            const std::uint64_t last{(base + 64 < w1 ? base + 64 : w1) * 32};  // bits this step stores end here
+            if (own_end < last) {
+                for (std::uint32_t j{i + 1}; j < runs; ++j) {
+                    Run r;
+                    if (j < front) {
+                        if (j >= 3 && j + 1 < front) {
+                            const std::uint32_t g{(j - 3) / P.dc_chunks};
+                            const DcGroupGeo d{dc_group_geo(geo, static_cast<int>(g))};
+                            if ((j - 3) % P.dc_chunks * kDcChunk >= d.items) {
+                                j = 3 + (g + 1) * P.dc_chunks - 1;  // past a smaller group's last chunk
+                                continue;
+                            }
+                        }
+                        r = front_run(geo, k, lay, P, j);
+                    } else {
+                        const std::uint32_t g{(j - front) / kGroupRuns};
+                        if (j == front || g != group.g) {
+                            group = ac_runs(P, g);
+                        }
+                        const std::uint32_t n{next_ac_run(group, (j - front) % kGroupRuns)};
+                        if (n == kGroupRuns) {
+                            j = front + (g + 1) * kGroupRuns - 1;
+                            continue;
+                        }
+                        j = front + g * kGroupRuns + n;
+                        r = ac_run(group, P, n);
+                    }
+                    if (r.dst >= last) {
+                        break;
+                    }
+                    if (w < w1) {
+                        v |= run_word(r, w * 32);
+                    }
+                }
             }
-            const std::uint64_t s{pc.dst > b0 ? pc.dst : b0};
-            const std::uint64_t e{pc.dst + pc.nbits < b0 + 32 ? pc.dst + pc.nbits : b0 + 32};
-            if (s >= e) {
+            if (w >= w1) {
                 continue;
             }
-            v |= piece_bits(pc, s - pc.dst, static_cast<std::uint32_t>(e - s)) << static_cast<std::uint32_t>(s - b0);
-        }
-        if ((w + 1) * 4 <= cap_bytes) {
-            out_words[w] = v;
-        } else {
-            auto* ob{reinterpret_cast<std::uint8_t*>(out_words)};
-            for (std::uint64_t b{w * 4}; b < cap_bytes; ++b) {
-                ob[b] = static_cast<std::uint8_t>(v >> (8 * (b - w * 4)));
+            if ((w + 1) * 4 <= cap_bytes) {
+                out_words[w] = v;
+            } else {
+                auto* ob{reinterpret_cast<std::uint8_t*>(out_words)};
+                for (std::uint64_t b{w * 4}; b < cap_bytes; ++b) {
+                    ob[b] = static_cast<std::uint8_t>(v >> (8 * (b - w * 4)));
+                }
             }
         }
     }
 }
 
 __global__ __launch_bounds__(256) void assemble_kernel(Geometry geo, const Constants* __restrict__ k,
-                                                       const Layout* __restrict__ lay, Pieces P,
+                                                       const Layout* __restrict__ lay, Sources P,
                                                        std::uint32_t* __restrict__ out_words,
                                                        std::uint64_t cap_bytes) {
     assemble_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, lay, P, out_words, cap_bytes);

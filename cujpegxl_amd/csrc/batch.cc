@@ -128,8 +128,12 @@ bool BatchEncoder::apply_shape(const BatchShape& shape) {
     }
     shape_ = shape;
     std::fill(std::begin(total_), std::end(total_), 0u);
+    std::uint32_t bands{0};
+    for (const FrameJob& j : jobs_) {
+        bands += j.geo.num_ac * ac_group_bands();
+    }
     for (FrameJob& j : jobs_) {
-        batch_stage_grids(j.geo, shape_, j.grid);
+        batch_stage_grids(j.geo, shape_, emit_band_wgs(bands), j.grid);
         for (int s{0}; s < kBStages; ++s) {
             j.grid[s].first = total_[s];
             total_[s] += j.grid[s].nx * j.grid[s].ny;

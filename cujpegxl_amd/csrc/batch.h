@@ -63,7 +63,7 @@ struct FrameJob {
     std::uint32_t* hist_partial;
     std::uint32_t* ac_staging;
     std::uint32_t* dc_staging;
-    std::uint64_t* ac_part_bits;
+    std::uint16_t* ac_run_bits;
     std::uint32_t* ac_group_bytes;
     std::uint64_t* ac_group_bits;
     std::uint32_t* chunk_bits;
@@ -76,19 +76,22 @@ struct FrameJob {
     std::uint64_t cap;        // its capacity in bytes
     std::uint64_t* size_out;  // the file size (device address)
     Clears clr;
+    std::uint32_t dc_chunks;  // chunks of the frame's largest DC group
 };
 
 // Tunable launch shapes of the batched stages (the autotuner's search space).
 struct BatchShape {
     std::uint32_t token_cap;         // tokenizer workgroups per frame, at most
-    std::uint32_t assemble_words;    // output words per assembly thread (sets its grid)
+    std::uint32_t assemble_words;    // output words per assembly thread of the largest file (bounds its grid)
     // Region stage: 0 for one workgroup per region, else a persistent grid of
     // this many workgroups (a multiple of 8) that claim the regions in turn.
     std::uint32_t region_wgs;
 };
 
-// Stage grids of one frame for a shape (nx, ny only; `first` is the caller's).
-void batch_stage_grids(const Geometry& geo, const BatchShape& shape, StageGrid (&grid)[kBStages]);
+// Stage grids of one frame for a shape and an emission with `band_wgs`
+// workgroups per band (nx, ny only; `first` is the caller's).
+void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32_t band_wgs,
+                       StageGrid (&grid)[kBStages]);
 
 // Queues the eight batched launches of a batch (all frames in `mode`) on `s`.
 // A persistent region stage (shape.region_wgs != 0) claims its regions

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void tokens_batch_kernel(const FrameJob* __res
 __global__ __launch_bounds__(256) void histograms_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBHistograms, wg)};
-    histograms_kernel_body(wg, j.geo, (wg.nx - kReduceWgs) / j.geo.num_dc, j.hist_partial,
+    histograms_kernel_body(wg, j.geo, j.dc_chunks, j.hist_partial,
                            static_cast<int>(j.grid[kBTokens].nx), j.hists, j.dc, j.acs, j.qf, j.ytox, j.ytob,
                            j.fb_count);
 }
@@ -102,31 +102,32 @@ __global__ __launch_bounds__(64 * kTrials) void huffman_batch_kernel(const Frame
     huffman_kernel_body(wg, j.hists, j.codes);
 }
 
-__global__ __launch_bounds__(kPartThreads) void emit_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
+__global__ __launch_bounds__(kEmitThreads) void emit_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBEmit, wg)};
     emit_kernel_body(wg, j.geo, EmitArgs{j.acs, j.item_tokens, j.tokens, j.codes, j.k, j.fb_count, j.dc, j.qf, j.ytox,
-                                         j.ytob, j.ac_staging, j.ac_part_bits, j.dc_staging, j.chunk_bits,
-                                         (wg.nx - j.geo.num_ac * kGroupParts) / j.geo.num_dc});
+                                         j.ytob, j.ac_staging, j.ac_run_bits, j.dc_staging, j.chunk_bits,
+                                         j.dc_chunks, wg.nx - j.dc_chunks * j.geo.num_dc});
 }
 
 __global__ __launch_bounds__(256) void layout_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBLayout, wg)};
-    layout_kernel_body(wg, j.geo, j.k, j.codes, j.ac_part_bits, j.chunk_bits,
-                       (j.grid[kBEmit].nx - j.geo.num_ac * kGroupParts) / j.geo.num_dc, j.dc_group_bytes,
+    layout_kernel_body(wg, j.geo, j.k, j.codes, j.ac_run_bits, j.chunk_bits,
+                       j.dc_chunks, j.dc_group_bytes,
                        j.dc_group_bits, j.ac_group_bytes, j.ac_group_bits, j.lay, j.ac_base, j.dc_base, j.size_out);
 }
 
 __global__ __launch_bounds__(256) void assemble_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBAssemble, wg)};
-    const Pieces P{j.dc_staging, j.chunk_bits, (j.grid[kBEmit].nx - j.geo.num_ac * kGroupParts) / j.geo.num_dc,
-                   j.ac_staging, j.dc_group_bits, j.ac_group_bits, j.ac_part_bits, j.dc_base, j.ac_base};
+    const Sources P{j.dc_staging, j.chunk_bits, j.dc_chunks,
+                    j.ac_staging, j.ac_run_bits, j.dc_group_bits, j.dc_base, j.ac_base};
     assemble_kernel_body(wg, j.geo, j.k, j.lay, P, j.out, j.cap);
 }
 
-void batch_stage_grids(const Geometry& geo, const BatchShape& shape, StageGrid (&g)[kBStages]) {
+void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32_t band_wgs,
+                       StageGrid (&g)[kBStages]) {
     const auto set = [&](BatchStage s, std::uint32_t nx, std::uint32_t ny) {
         g[s] = StageGrid{0, nx > 0 ? nx : 1, ny > 0 ? ny : 1, 0};
     };
@@ -139,13 +140,14 @@ void batch_stage_grids(const Geometry& geo, const BatchShape& shape, StageGrid (
     set(kBTokens, waves < cap ? waves : cap, 1);
     set(kBHistograms, kReduceWgs + dc_wgs, 1);
     set(kBHuffman, kNumClusters + 2 * geo.num_dc, 1);
-    set(kBEmit, geo.num_ac * kGroupParts + dc_wgs, 1);
+    set(kBEmit, geo.num_ac * kGroupBands * band_wgs + dc_wgs, 1);
     set(kBLayout, 1, 1);
     const std::uint64_t nb{geo.nblocks};
     const std::uint64_t words{(3 * nb * 384 + 48 * nb + (geo.num_ac + geo.num_dc) * 2048ull + 16384 + 3) / 4};
     const std::uint64_t per_wg{256ull * (shape.assemble_words > 0 ? shape.assemble_words : 1)};
     const std::uint64_t ag{(words + per_wg - 1) / per_wg};
-    set(kBAssemble, static_cast<std::uint32_t>(ag < 2048 ? ag : 2048), 1);
+    const std::uint32_t run_wgs{(frame_runs(geo, dc_chunks_per_group(geo)) + 3) / 4};
+    set(kBAssemble, ag < run_wgs ? static_cast<std::uint32_t>(ag) : run_wgs, 1);
 }
 
 void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
@@ -167,7 +169,7 @@ void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uin
     tokens_batch_kernel<<<total[kBTokens], 256, 0, s>>>(jobs, count);
     histograms_batch_kernel<<<total[kBHistograms], 256, 0, s>>>(jobs, count);
     huffman_batch_kernel<<<total[kBHuffman], 64 * kTrials, 0, s>>>(jobs, count);
-    emit_batch_kernel<<<total[kBEmit], kPartThreads, 0, s>>>(jobs, count);
+    emit_batch_kernel<<<total[kBEmit], kEmitThreads, 0, s>>>(jobs, count);
     layout_batch_kernel<<<total[kBLayout], 256, 0, s>>>(jobs, count);
     assemble_batch_kernel<<<total[kBAssemble], 256, 0, s>>>(jobs, count);
 }

@@ -281,43 +281,59 @@ bool build_codes_host(const std::uint32_t* hists, std::uint32_t count, std::uint
 
 
 std::size_t ac_group_slot_words() {
-    return static_cast<std::size_t>(kGroupParts) * kPartSlotWords;
+    return static_cast<std::size_t>(kGroupRuns) * kRunWords;
 }
 
-std::size_t ac_group_parts() {
-    return kGroupParts;
+std::size_t ac_group_runs() {
+    return kGroupRuns;
+}
+
+std::uint32_t ac_group_bands() {
+    return kGroupBands;
+}
+
+// Workgroups per band of four block rows: enough to give every band's runs
+// to different workgroups while the chip has idle slots (256 CUs x 8), one
+// where the bands alone fill it (each workgroup numbers the band's tokens
+// again).  Measured: 320x240 8.4 us with four, 27 us with one that keeps all
+// items; 3840x2160 (1,080 bands) 25.3 us with one, 27.2 with two, 35 with
+// four; 7680x4320 75 us with one, 80 with two.
+std::uint32_t emit_band_wgs(std::uint32_t bands) {
+    const std::uint32_t n{2048 / (bands > 0 ? bands : 1)};
+    return n < 1 ? 1 : (n > 4 ? 4 : n);
 }
 
 void launch_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs, const std::uint16_t* item_tokens,
                  const std::uint32_t* tokens, const CodeSet* cs, const Constants* k, const std::uint32_t* fb_count,
                  const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                 std::uint32_t* ac_staging, std::uint64_t* ac_part_bits, std::uint32_t* dc_staging,
+                 std::uint32_t* ac_staging, std::uint16_t* ac_run_bits, std::uint32_t* dc_staging,
                  std::uint32_t* chunk_bits) {
     const std::uint32_t chunks{dc_chunks_per_group(geo)};
-    emit_kernel<<<geo.num_ac * kGroupParts + chunks * geo.num_dc, kPartThreads, 0, s>>>(
-        geo, EmitArgs{acs, item_tokens, tokens, cs, k, fb_count, dc, qf, ytox, ytob, ac_staging, ac_part_bits,
-                      dc_staging, chunk_bits, chunks});
+    const std::uint32_t bands{geo.num_ac * kGroupBands};
+    const std::uint32_t ac_wgs{bands * emit_band_wgs(bands)};
+    emit_kernel<<<ac_wgs + chunks * geo.num_dc, kEmitThreads, 0, s>>>(
+        geo, EmitArgs{acs, item_tokens, tokens, cs, k, fb_count, dc, qf, ytox, ytob, ac_staging, ac_run_bits,
+                      dc_staging, chunk_bits, chunks, ac_wgs});
 }
 
 void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                   const std::uint64_t* ac_part_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
+                   const std::uint16_t* ac_run_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
                    std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
                    Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base, std::uint64_t* total_out,
                    hipEvent_t done) {
-    hipExtLaunchKernelGGL(layout_kernel, dim3(1), dim3(256), 0, s, nullptr, done, 0, geo, k, cs, ac_part_bits,
+    hipExtLaunchKernelGGL(layout_kernel, dim3(1), dim3(256), 0, s, nullptr, done, 0, geo, k, cs, ac_run_bits,
                           chunk_bits, dc_chunks_per_group(geo), dc_group_bytes, dc_group_bits, ac_group_bytes,
                           ac_group_bits, lay, ac_base, dc_base, total_out);
 }
 
 void launch_assemble(hipStream_t s, const Geometry& geo, const Constants* k, const Layout* lay,
                      const std::uint32_t* dc_staging, const std::uint32_t* ac_staging, const std::uint64_t* dc_bits,
-                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits,
-                     const std::uint32_t* chunk_off, const std::uint64_t* dc_base, const std::uint64_t* ac_base,
-                     std::uint8_t* out, std::uint64_t cap_bytes, hipEvent_t done) {
-    const Pieces P{dc_staging, chunk_off, dc_chunks_per_group(geo), ac_staging, dc_bits, ac_bits, ac_part_bits,
-                   dc_base, ac_base};
-    hipExtLaunchKernelGGL(assemble_kernel, dim3(2048), dim3(256), 0, s, nullptr, done, 0, geo, k, lay, P,
-                          reinterpret_cast<std::uint32_t*>(out), cap_bytes);
+                     const std::uint16_t* ac_run_bits, const std::uint32_t* chunk_off, const std::uint64_t* dc_base,
+                     const std::uint64_t* ac_base, std::uint8_t* out, std::uint64_t cap_bytes, hipEvent_t done) {
+    const std::uint32_t chunks{dc_chunks_per_group(geo)};
+    const Sources P{dc_staging, chunk_off, chunks, ac_staging, ac_run_bits, dc_bits, dc_base, ac_base};
+    hipExtLaunchKernelGGL(assemble_kernel, dim3((frame_runs(geo, chunks) + 3) / 4), dim3(256), 0, s, nullptr, done, 0,
+                          geo, k, lay, P, reinterpret_cast<std::uint32_t*>(out), cap_bytes);
 }
 
 }  // namespace cjx

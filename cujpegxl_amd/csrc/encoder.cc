@@ -305,7 +305,8 @@ void Encoder::null_buffers() {
     tokens_ = nullptr;
     item_tokens_ = nullptr;
     item_list_ = item_count_ = hist_partial_ = ac_staging_ = dc_staging_ = nullptr;
-    ac_part_bits_ = ac_group_bits_ = dc_group_bits_ = ac_base_ = dc_base_ = nullptr;
+    ac_run_bits_ = nullptr;
+    ac_group_bits_ = dc_group_bits_ = ac_base_ = dc_base_ = nullptr;
     ac_group_bytes_ = dc_group_bytes_ = chunk_bits_ = nullptr;
     out_ = nullptr;
     out_cap_ = 0;
@@ -416,7 +417,7 @@ void Encoder::carve(Get& get) {
     get(hist_partial_, ac_partial_words() * sizeof(std::uint32_t));
     get(ac_staging_, static_cast<std::size_t>(geo_.num_ac) * ac_group_slot_words() * sizeof(std::uint32_t));
     get(dc_staging_, dc_chunks * dc_chunk_slot_words() * sizeof(std::uint32_t));
-    get(ac_part_bits_, geo_.num_ac * ac_group_parts() * sizeof(std::uint64_t));
+    get(ac_run_bits_, geo_.num_ac * ac_group_runs() * sizeof(std::uint16_t));
     get(ac_group_bytes_, geo_.num_ac * sizeof(std::uint32_t));
     get(ac_group_bits_, geo_.num_ac * sizeof(std::uint64_t));
     get(chunk_bits_, dc_chunks * sizeof(std::uint32_t));
@@ -533,7 +534,7 @@ bool Encoder::fill_job(FrameJob& j, hipStream_t s, std::uint8_t* out_dev, std::s
     j.hist_partial = hist_partial_;
     j.ac_staging = ac_staging_;
     j.dc_staging = dc_staging_;
-    j.ac_part_bits = ac_part_bits_;
+    j.ac_run_bits = ac_run_bits_;
     j.ac_group_bytes = ac_group_bytes_;
     j.ac_group_bits = ac_group_bits_;
     j.chunk_bits = chunk_bits_;
@@ -546,6 +547,7 @@ bool Encoder::fill_job(FrameJob& j, hipStream_t s, std::uint8_t* out_dev, std::s
     j.cap = cap;
     j.size_out = size_dev;
     j.clr = entropy_clears();
+    j.dc_chunks = dc_chunks_per_group(geo_);
     return true;
 }
 
@@ -581,11 +583,11 @@ bool Encoder::encode_on(hipStream_t s, const std::uint8_t* luma, std::size_t lum
                      ItemList{item_list_, item_count_}, dc_, qf_, ytox_, ytob_, fb_count_);
     launch_huffman(s, kNumClusters + static_cast<int>(2 * geo_.num_dc), hists_, codes);
     launch_emit(s, geo_, acs_, item_tokens_, tokens_, codes, k, fb_count_, dc_, qf_, ytox_, ytob_, ac_staging_,
-                ac_part_bits_, dc_staging_, chunk_bits_);
-    launch_layout(s, geo_, k, codes, ac_part_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_, ac_group_bytes_,
+                ac_run_bits_, dc_staging_, chunk_bits_);
+    launch_layout(s, geo_, k, codes, ac_run_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_, ac_group_bytes_,
                   ac_group_bits_, lay, ac_base_, dc_base_, size_dev);
-    launch_assemble(s, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_group_bits_, ac_part_bits_,
-                    chunk_bits_, dc_base_, ac_base_, out_dev, cap);
+    launch_assemble(s, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_run_bits_, chunk_bits_,
+                    dc_base_, ac_base_, out_dev, cap);
     return hipGetLastError() == hipSuccess;
 }
 
@@ -1058,17 +1060,17 @@ bool Encoder::run_entropy(std::uint8_t* out, std::size_t cap, bool listed, bool 
     launch_huffman(stream_, kNumClusters + static_cast<int>(2 * geo_.num_dc), hists_, codes);
     mark(Stage::kSizes);
     launch_emit(stream_, geo_, acs_, item_tokens_, tokens_, codes, k, fb_count_, dc_, qf_, ytox_, ytob_, ac_staging_,
-                ac_part_bits_, dc_staging_, chunk_bits_);
+                ac_run_bits_, dc_staging_, chunk_bits_);
     size_bound_ = size_event;
     // Without a size event the output is written by the assembly kernel and
     // nothing follows it: its own completion ends the frame.
     end_bound_ = !size_event;
-    launch_layout(stream_, geo_, k, codes, ac_part_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_,
+    launch_layout(stream_, geo_, k, codes, ac_run_bits_, chunk_bits_, dc_group_bytes_, dc_group_bits_,
                   ac_group_bytes_, ac_group_bits_, lay, ac_base_, dc_base_, total_dev_,
                   size_event ? ev_size_ : nullptr);
     mark(Stage::kEmit);
-    launch_assemble(stream_, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_group_bits_, ac_part_bits_,
-                    chunk_bits_, dc_base_, ac_base_, out, cap, end_bound_ ? ev_end_ : nullptr);
+    launch_assemble(stream_, geo_, k, lay, dc_staging_, ac_staging_, dc_group_bits_, ac_run_bits_, chunk_bits_,
+                    dc_base_, ac_base_, out, cap, end_bound_ ? ev_end_ : nullptr);
     return hipGetLastError() == hipSuccess;
 }
 

@@ -193,9 +193,9 @@ private:
     std::uint32_t* item_list_{nullptr};    // first-block items (quantizer -> tokenizer), ItemList
     std::uint32_t* item_count_{nullptr};   // entries at its front and back
     std::uint32_t* hist_partial_{nullptr}; // per-workgroup AC histograms
-    std::uint32_t* ac_staging_{nullptr};   // each AC group's stream at group-relative bits
+    std::uint32_t* ac_staging_{nullptr};   // each AC group's runs at run-relative bits
     std::uint32_t* dc_staging_{nullptr};   // each DC group's chunks at chunk-relative bits
-    std::uint64_t* ac_part_bits_{nullptr};   // bits of each part (row band) of each AC group
+    std::uint16_t* ac_run_bits_{nullptr};    // bits of each run of each AC group
     std::uint32_t* ac_group_bytes_{nullptr};
     std::uint64_t* ac_group_bits_{nullptr};
     std::uint32_t* chunk_bits_{nullptr};   // bits of each chunk, then (layout) their offsets

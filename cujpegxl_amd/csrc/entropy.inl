@@ -526,223 +526,219 @@ __device__ std::uint64_t block_excl_scan(std::uint64_t v, std::uint64_t* sh, std
     return r;
 }
 
-// ---- AC groups emitted in parts -----------------------------------------------
+// Exclusive scan of one value per thread over a workgroup of kWaves waves:
+// the waves' totals go through `sh` (kWaves words), every thread adds those of
+// the waves below its own.  `sh` must not be in use by a scan that a thread
+// may still read (callers alternate two buffers, or have a barrier between).
+template <int kWaves>
+__device__ __forceinline__ std::uint32_t block_excl_scan_u32(std::uint32_t v, std::uint32_t* sh,
+                                                             std::uint32_t& total) {
+    const int lane{static_cast<int>(threadIdx.x) & 63}, wv{static_cast<int>(threadIdx.x) >> 6};
+    const std::uint32_t x{wave_incl_scan_u32(v)};
+    if (lane == 63) {
+        sh[wv] = x;
+    }
+    __syncthreads();
+    std::uint32_t base{0};
+    total = 0;
+#pragma unroll
+    for (int i{0}; i < kWaves; ++i) {
+        const std::uint32_t t{sh[i]};
+        base += i < wv ? t : 0u;
+        total += t;
+    }
+    return base + x - v;
+}
+
+// ---- AC groups emitted in runs ------------------------------------------------
 //
-// Each AC group is cut into kGroupParts parts of kPartRows block rows (each a
-// contiguous run of the group's stream), and one 256-thread workgroup writes
-// a part's token stream at part-relative bit positions into the part's
-// staging slot: the part's items in decoder order (block rows, blocks left to
-// right, channels Y, X, B) and their token counts give a flat token numbering
-// (token f belongs to the last item whose prefix is <= f); block scans of the
-// token lengths give the positions; the stream is assembled in LDS and stored
-// once.  The part's bit count falls out of the same pass (a group's size is
-// the sum of its parts').  A stream longer than the LDS copy is emitted again
-// with atomicOr into the zeroed slot.
-constexpr int kGroupParts = 8;
-constexpr int kPartRows = kAcGroupBlocks / kGroupParts;
-constexpr int kPartThreads = 256;
-constexpr int kPartItems = 3 * kAcGroupBlocks * kPartRows;
-constexpr int kPartWords = 2048;
-constexpr int kGroupPerThread = 8;
-// Bound on one part's stream: 28 bits (15-bit code + 13 extra bits) per
-// coefficient slot of its blocks in three channels.
-constexpr std::size_t kPartSlotWords = 3ull * kAcGroupBlocks * kPartRows * 64 * 28 / 32 + 64;
+// An AC group is cut into eight bands of four block rows (which the
+// transforms never cross), and a band's tokens, in decoder order (block rows,
+// blocks left to right, channels Y, X, B), into runs of kRunTokens.  Each run
+// is written at run-relative bit positions into a staging slot of its own,
+// with its bit count; the assembly reads the runs back to back.  `band_wgs`
+// workgroups of 256 threads share a band: each numbers the band's tokens (a
+// scan over its items' counts, items without tokens dropped) and takes runs
+// j, j + band_wgs, ...: a thread finds its first token's item by a binary
+// search, reads eight consecutive tokens and their codes, a block scan of
+// the lengths gives the positions, and the stream is assembled in LDS.
+//
+// The work is a chain of latencies (counts, scan, search, token reads, scan,
+// LDS atomics: about 12,000 clocks a run), so the runs of a band go to
+// different workgroups instead of one after another, and the walk over a
+// thread's tokens meets no item without tokens (up to 96 in a row where
+// every transform is larger than 8x8).  One workgroup per band with all items
+// kept took 27 us at 320x240 and 35 us at 3840x2160; this form 8.4 and 25 us.
+constexpr int kGroupBands = 8;
+constexpr int kBandRows = kAcGroupBlocks / kGroupBands;
+constexpr int kBandItems = 3 * kAcGroupBlocks * kBandRows;
+constexpr int kEmitThreads = 256;
+constexpr int kPerThread = 8;
+constexpr int kRunTokens = kEmitThreads * kPerThread;
+// A band has at most one token per coefficient slot.
+constexpr int kBandRuns = (kBandItems * 64 + kRunTokens - 1) / kRunTokens;
+constexpr int kGroupRuns = kGroupBands * kBandRuns;
+// A token is at most 28 bits (15-bit code, 13 extra bits).
+constexpr int kRunWords = kRunTokens * 28 / 32;
+static_assert(kRunWords * 32 < 65536, "a run's bit count fits 16 bits");
+static_assert(kBandItems * 64 < 65536, "a band's token count fits 16 bits");
+static_assert(kBandItems <= 2 * kEmitThreads, "two items per thread");
+static_assert(kGroupRuns * sizeof(std::uint16_t) % 16 == 0, "16-byte reads of a group's run sizes");
 
 struct GroupShared {
     std::uint32_t lut[kNumClusters * kAcSymbols];  // depth | code << 16
-    std::uint32_t prefix[kPartItems + 1];
-    std::uint32_t slot0[kPartItems];  // token slot of the item's first token
-    std::int8_t m[kPartItems];
-    std::uint32_t buf[kPartWords];
-    std::uint64_t sh[17];
-    std::uint32_t overflow;
+    // Items with tokens: {first token's number, token slot | log2(side / 8)
+    // (a slot is a multiple of 64)}; one more entry ends the numbering.
+    uint2 item[kBandItems + 1];
+    std::uint32_t buf[kRunWords];
+    std::uint32_t sh[2][kEmitThreads / 64];
 };
 
 __device__ __forceinline__ void ac_group_emit_body(
     GroupShared& S, const Wg& wg, const Geometry& geo, const std::int8_t* __restrict__ acs,
     const std::uint16_t* __restrict__ item_tokens, const std::uint32_t* __restrict__ tokens,
-    const std::uint8_t* __restrict__ depth, const std::uint16_t* __restrict__ codes,
-    std::uint32_t* __restrict__ staging, std::uint64_t* __restrict__ part_bits) {
+    const std::uint32_t* __restrict__ lut, std::uint32_t* __restrict__ staging,
+    std::uint16_t* __restrict__ run_bits_out, int band_wgs) {
     const int tid{static_cast<int>(threadIdx.x)};
-    const int g{static_cast<int>(wg.x) / kGroupParts};
-    const int part{static_cast<int>(wg.x) % kGroupParts};
+    const int g{static_cast<int>(wg.x) / (kGroupBands * band_wgs)};
+    const int band{static_cast<int>(wg.x) / band_wgs % kGroupBands};
+    const int first{static_cast<int>(wg.x) % band_wgs};
     const int bx0{(g % static_cast<int>(geo.xg)) * kAcGroupBlocks};
-    const int by0{(g / static_cast<int>(geo.xg)) * kAcGroupBlocks + part * kPartRows};
+    const int by0{(g / static_cast<int>(geo.xg)) * kAcGroupBlocks + band * kBandRows};
     const int gbw{min(kAcGroupBlocks, static_cast<int>(geo.bw) - bx0)};
-    const int gbh{min(kPartRows, static_cast<int>(geo.bh) - by0)};
-    if (gbh <= 0) {
-        if (tid == 0) {
-            part_bits[wg.x] = 0;
-        }
-        return;
-    }
-    const int row_items{3 * gbw};
-    const int items{row_items * gbh};
-    std::uint32_t* const slot{staging + static_cast<std::size_t>(wg.x) * kPartSlotWords};
+    const int gbh{min(kBandRows, static_cast<int>(geo.bh) - by0)};
+    const int items{gbh > 0 ? 3 * gbw * gbh : 0};
+    const std::size_t run0{(static_cast<std::size_t>(g) * kGroupBands + band) * kBandRuns};
 
-    // 1. Token prefix over the part's items (at most two per thread).  Every
-    //    read of this step (the items' transforms and token counts, the code
-    //    table) is issued before the first wait; a covered block's count is
-    //    read too and then taken as 0.
-    static_assert(kPartItems <= 2 * kPartThreads, "two items per thread");
-    static_assert((kNumClusters * kAcSymbols) % kPartThreads == 0, "code table entries per thread");
-    constexpr int kLutPerThread{kNumClusters * kAcSymbols / kPartThreads};
+    // 1. The band's items with tokens, and their token numbers.  Every read
+    //    (the items' transforms and token counts, the code table) is issued
+    //    before the first wait; a covered block's count is read too and then
+    //    taken as 0.
     int item_n[2]{0, 0};
-    std::uint32_t item_cnt[2]{0u, 0u};
+    std::uint32_t item_cnt[2]{0u, 0u}, item_slot[2]{0u, 0u};
 #pragma unroll
     for (int k{0}; k < 2; ++k) {
-        const int i{k * kPartThreads + tid};
+        const int i{2 * tid + k};
         if (i < items) {
-            const int row{i / row_items}, rem{i % row_items};
+            const int row{i / (3 * gbw)}, rem{i % (3 * gbw)};
+            const int ci{rem % 3};
             const std::size_t pos{static_cast<std::size_t>(by0 + row) * geo.bw + bx0 + rem / 3};
             item_n[k] = acs[pos];
-            item_cnt[k] = item_tokens[pos * 3 + rem % 3];
+            item_cnt[k] = item_tokens[pos * 3 + ci];
+            item_slot[k] = static_cast<std::uint32_t>(
+                token_slot(geo, ci == 0 ? 1 : (ci == 1 ? 0 : 2), bx0 + rem / 3, by0 + row, 1, 0));
         }
     }
-    std::uint32_t lut[kLutPerThread];
-#pragma unroll
-    for (int k{0}; k < kLutPerThread; ++k) {
-        const int i{k * kPartThreads + tid};
-        const int at{(i / kAcSymbols) * kHistStride + i % kAcSymbols};
-        lut[k] = static_cast<std::uint32_t>(depth[at]) | (static_cast<std::uint32_t>(codes[at]) << 16);
-    }
-    std::uint32_t carry{0};
+    static_assert(kNumClusters * kAcSymbols == 2 * 4 * kEmitThreads, "two 16-byte reads of the code table");
+    const uint4 code0{reinterpret_cast<const uint4*>(lut)[tid]};
+    const uint4 code1{reinterpret_cast<const uint4*>(lut)[kEmitThreads + tid]};
+    std::uint32_t packed{0};  // tokens | items with tokens << 16
 #pragma unroll
     for (int k{0}; k < 2; ++k) {
-        const int base{k * kPartThreads};
-        if (base >= items) {
-            break;
-        }
-        const int i{base + tid};
-        std::uint32_t cnt{0};
-        if (i < items) {
-            const int row{i / row_items}, rem{i % row_items};
-            const int n{item_n[k]};
-            const int ci{rem % 3};
-            S.m[i] = static_cast<std::int8_t>(n / 8);
-            S.slot0[i] = static_cast<std::uint32_t>(
-                token_slot(geo, ci == 0 ? 1 : (ci == 1 ? 0 : 2), bx0 + rem / 3, by0 + row, 1, 0));
-            cnt = n != 0 ? item_cnt[k] : 0u;
-        }
-        std::uint64_t total{0};
-        const std::uint64_t p{block_excl_scan(cnt, S.sh, total)};
-        if (i < items) {
-            S.prefix[i] = carry + static_cast<std::uint32_t>(p);
-        }
-        carry += static_cast<std::uint32_t>(total);
+        item_cnt[k] = item_n[k] != 0 ? item_cnt[k] : 0u;
+        packed += item_cnt[k] + (item_cnt[k] != 0 ? 0x10000u : 0u);
     }
+    std::uint32_t total{0};
+    std::uint32_t at{block_excl_scan_u32<kEmitThreads / 64>(packed, S.sh[0], total)};
+#pragma unroll
+    for (int k{0}; k < 2; ++k) {
+        if (item_cnt[k] != 0) {
+            S.item[at >> 16] = uint2{at & 0xffffu, item_slot[k] | static_cast<std::uint32_t>(item_n[k] >> 4)};
+            at += item_cnt[k] + 0x10000u;
+        }
+    }
+    const std::uint32_t ntok{total & 0xffffu};
+    const int nitems{static_cast<int>(total >> 16)};
     if (tid == 0) {
-        S.prefix[items] = carry;
-        S.overflow = 0;
+        S.item[nitems] = uint2{ntok, 0u};
     }
-#pragma unroll
-    for (int k{0}; k < kLutPerThread; ++k) {
-        S.lut[k * kPartThreads + tid] = lut[k];
-    }
-    for (int i{tid}; i < kPartWords; i += kPartThreads) {
-        S.buf[i] = 0;
-    }
-    __syncthreads();
+    reinterpret_cast<uint4*>(S.lut)[tid] = code0;
+    reinterpret_cast<uint4*>(S.lut)[kEmitThreads + tid] = code1;
 
-    // 2. Token lengths, positions and bits; twice if the LDS copy overflows.
-    // Each thread takes kGroupPerThread consecutive tokens: one binary search
-    // for the first, then a forward walk over the item prefix.
-    std::uint64_t run{0};
-    for (int pass{0}; pass < 2; ++pass) {
-        const bool global{pass == 1};
-        if (global) {
-            if (S.overflow == 0) {
-                break;
+    // 2. The runs.
+    for (int r{first}; r < kBandRuns; r += band_wgs) {
+        const std::uint32_t f0{static_cast<std::uint32_t>(r) * kRunTokens};
+        if (f0 >= ntok) {
+            if (tid == 0) {
+                run_bits_out[run0 + r] = 0;
             }
-            const std::uint64_t nw{(run + 31) / 32};
-            for (std::uint64_t i{static_cast<std::uint64_t>(tid)}; i < nw && i < kPartSlotWords; i += kPartThreads) {
-                slot[i] = 0;
-            }
-            __syncthreads();
-            run = 0;
+            continue;
         }
-        for (std::uint32_t f0{0}; f0 < carry; f0 += kPartThreads * kGroupPerThread) {
-            const std::uint32_t fb{f0 + static_cast<std::uint32_t>(tid) * kGroupPerThread};
-            std::uint32_t rec[kGroupPerThread];
-            int lo{0};
-            if (fb < carry) {
-                int hi{items - 1};
-                while (lo < hi) {
-                    const int mid{(lo + hi + 1) >> 1};
-                    if (S.prefix[mid] <= fb) {
-                        lo = mid;
-                    } else {
-                        hi = mid - 1;
-                    }
+        __syncthreads();  // the items are in LDS; the last run's words have been stored
+        for (int i{tid}; i < kRunWords; i += kEmitThreads) {
+            S.buf[i] = 0;
+        }
+        const std::uint32_t fb{f0 + static_cast<std::uint32_t>(tid) * kPerThread};
+        std::uint32_t rec[kPerThread];
+        int lo{0};
+        if (fb < ntok) {
+            int hi{nitems - 1};
+            while (lo < hi) {
+                const int mid{(lo + hi + 1) >> 1};
+                if (S.item[mid].x <= fb) {
+                    lo = mid;
+                } else {
+                    hi = mid - 1;
                 }
             }
+        }
+        uint2 cur{S.item[lo]};
+        std::uint32_t next{S.item[lo + 1].x};
 #pragma unroll
-            for (int j{0}; j < kGroupPerThread; ++j) {
-                const std::uint32_t f{fb + static_cast<std::uint32_t>(j)};
-                rec[j] = 0xffffffffu;
-                if (f < carry) {
-                    while (S.prefix[lo + 1] <= f) {
-                        ++lo;
-                    }
-                    const std::uint32_t k{f - S.prefix[lo]};
-                    const std::uint32_t m{static_cast<std::uint32_t>(S.m[lo])};
-                    const std::uint32_t q{k >> 6};
-                    rec[j] = tokens[S.slot0[lo] + (q >> (m >> 1)) * (geo.bw * 64) + ((q & (m - 1)) << 6) + (k & 63u)];
+        for (int j{0}; j < kPerThread; ++j) {
+            const std::uint32_t f{fb + static_cast<std::uint32_t>(j)};
+            rec[j] = 0xffffffffu;
+            if (f < ntok) {
+                if (f >= next) {  // every item has a token: at most one step
+                    ++lo;
+                    cur = S.item[lo];
+                    next = S.item[lo + 1].x;
                 }
+                const std::uint32_t k{f - cur.x};
+                const std::uint32_t l2m{cur.y & 63u};
+                const std::uint32_t q{k >> 6};
+                rec[j] = tokens[(cur.y & ~63u) + (q >> l2m) * (geo.bw * 64) + ((q & ((1u << l2m) - 1u)) << 6) +
+                                (k & 63u)];
             }
-            std::uint32_t len[kGroupPerThread], val[kGroupPerThread];
-            std::uint32_t sum{0};
+        }
+        std::uint32_t len[kPerThread], val[kPerThread];
+        std::uint32_t sum{0};
 #pragma unroll
-            for (int j{0}; j < kGroupPerThread; ++j) {
-                len[j] = 0;
-                val[j] = 0;
-                const std::uint32_t r{rec[j]};
-                if (r != 0xffffffffu) {
-                    const std::uint32_t e{S.lut[(r & 31u) * kAcSymbols + ((r >> 5) & (kAcSymbols - 1))]};
-                    const std::uint32_t d{e & 0xffffu};
-                    len[j] = d + ((r >> 13) & 31u);
-                    val[j] = ((e >> 16) | ((r >> 18) << d)) & ((1u << len[j]) - 1u);
-                }
-                sum += len[j];
+        for (int j{0}; j < kPerThread; ++j) {
+            len[j] = 0;
+            val[j] = 0;
+            const std::uint32_t rc{rec[j]};
+            if (rc != 0xffffffffu) {
+                const std::uint32_t e{S.lut[(rc & 31u) * kAcSymbols + ((rc >> 5) & (kAcSymbols - 1))]};
+                const std::uint32_t d{e & 0xffffu};
+                len[j] = d + ((rc >> 13) & 31u);
+                val[j] = ((e >> 16) | ((rc >> 18) << d)) & ((1u << len[j]) - 1u);
             }
-            std::uint64_t chunk{0};
-            std::uint64_t at{run + block_excl_scan(sum, S.sh, chunk)};
+            sum += len[j];
+        }
+        std::uint32_t bits{0};
+        // The barrier inside also orders the clearing of S.buf before the ORs.
+        std::uint32_t pos{block_excl_scan_u32<kEmitThreads / 64>(sum, S.sh[1], bits)};
 #pragma unroll
-            for (int j{0}; j < kGroupPerThread; ++j) {
-                if (len[j] != 0) {
-                    const std::uint64_t wi{at >> 5};
-                    const std::uint32_t b{static_cast<std::uint32_t>(at & 31u)};
-                    const bool two{b + len[j] > 32};
-                    if (global) {
-                        if (wi < kPartSlotWords) {
-                            atomicOr(&slot[wi], val[j] << b);
-                        }
-                        if (two && wi + 1 < kPartSlotWords) {
-                            atomicOr(&slot[wi + 1], val[j] >> (32 - b));
-                        }
-                    } else if (wi + (two ? 1 : 0) < static_cast<std::uint64_t>(kPartWords)) {
-                        atomicOr(&S.buf[wi], val[j] << b);
-                        if (two) {
-                            atomicOr(&S.buf[wi + 1], val[j] >> (32 - b));
-                        }
-                    } else {
-                        S.overflow = 1;
-                    }
+        for (int j{0}; j < kPerThread; ++j) {
+            if (len[j] != 0) {
+                const std::uint32_t wi{pos >> 5}, b{pos & 31u};
+                atomicOr(&S.buf[wi], val[j] << b);
+                if (b + len[j] > 32) {
+                    atomicOr(&S.buf[wi + 1], val[j] >> (32 - b));
                 }
-                at += len[j];
             }
-            run += chunk;
+            pos += len[j];
         }
         __syncthreads();
-    }
-    if (S.overflow == 0) {
-        const std::uint64_t nw{(run + 31) / 32};
-        for (std::uint64_t i{static_cast<std::uint64_t>(tid)}; i < nw; i += kPartThreads) {
+        std::uint32_t* const slot{staging + (run0 + r) * kRunWords};
+        const int nw{static_cast<int>((bits + 31) / 32)};
+        for (int i{tid}; i < nw; i += kEmitThreads) {
             slot[i] = S.buf[i];
         }
-    }
-    if (tid == 0) {
-        part_bits[wg.x] = run;
+        if (tid == 0) {
+            run_bits_out[run0 + r] = static_cast<std::uint16_t>(bits);
+        }
     }
 }
 
@@ -1021,23 +1017,26 @@ __device__ __forceinline__ std::uint32_t var_len_u16(std::uint32_t n, std::uint3
 struct DcEmitShared {
     std::uint32_t lut[2 * kHistStride];  // DC, then AcMetadata: depth | code << 16
     std::uint32_t buf[kDcSlotWords];
-    std::uint64_t sh[5];
+    std::uint32_t sh[kEmitThreads / 64];
     std::uint32_t blob_at[2];  // chunk-relative bit positions of the header blobs
 };
 
-// Constant bits, then a value, then a code's alphabet size and header: a
-// header blob's pieces (the first blob has no value).
+// A header blob's pieces: a value (none in the first blob), constant bits, a
+// code's alphabet size and its header.
 struct DcBlob {
-    std::uint32_t lead_bits, lead;  // value ahead of the constant bits
+    std::uint32_t lead_bits, lead;
     const std::uint32_t* words;
     std::uint32_t word_bits;
     std::uint32_t alpha_bits, alpha;
     const std::uint32_t* hdr;
     std::uint32_t hdr_bits;
-    __device__ __forceinline__ std::uint32_t bits() const { return lead_bits + word_bits + alpha_bits + hdr_bits; }
 };
 
-__device__ __forceinline__ void put_blob(std::uint32_t* buf, const DcBlob& b, std::uint32_t at) {
+__device__ __forceinline__ std::uint32_t blob_bits(DcBlob b) {
+    return b.lead_bits + b.word_bits + b.alpha_bits + b.hdr_bits;
+}
+
+__device__ __forceinline__ void put_blob(std::uint32_t* buf, DcBlob b, std::uint32_t at) {
     const std::uint32_t t{threadIdx.x};
     if (t == 0) {
         lds_or_bits(buf, kDcSlotWords, at, b.lead, b.lead_bits);
@@ -1059,7 +1058,7 @@ __device__ __forceinline__ void put_blob(std::uint32_t* buf, const DcBlob& b, st
 // of its chunks (the first item, and the one after the DC residuals).  The
 // group's two codes are read into LDS first; an item is tokenized once.
 __device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, const Geometry& geo,
-                                             const DcBlob& pre, const DcBlob& mid, const std::int32_t* __restrict__ dc,
+                                             DcBlob pre, DcBlob mid, const std::int32_t* __restrict__ dc,
                                              const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
                                              const std::int8_t* __restrict__ ytox,
                                              const std::int8_t* __restrict__ ytob,
@@ -1101,6 +1100,7 @@ __device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, cons
         }
     }
     __syncthreads();
+    const std::uint32_t pre_bits{blob_bits(pre)}, mid_bits{blob_bits(mid)};
     std::uint32_t len[kDcPerThread], val[kDcPerThread];
     std::uint32_t run{0};
 #pragma unroll
@@ -1113,12 +1113,12 @@ __device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, cons
             len[j] = dd + nb[j];
             val[j] = (e >> 16) | (ext[j] << dd);
         } else if (kind[j] > 2) {
-            len[j] = kind[j] == 3 ? pre.bits() : mid.bits();
+            len[j] = kind[j] == 3 ? pre_bits : mid_bits;
         }
         run += len[j];
     }
-    std::uint64_t total{0};
-    std::uint32_t at{static_cast<std::uint32_t>(block_excl_scan(run, S.sh, total))};
+    std::uint32_t total{0};
+    std::uint32_t at{block_excl_scan_u32<kEmitThreads / 64>(run, S.sh, total)};
 #pragma unroll
     for (int j{0}; j < kDcPerThread; ++j) {
         if (kind[j] < 2) {
@@ -1129,11 +1129,12 @@ __device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, cons
         at += len[j];
     }
     __syncthreads();
-    if (wg.x == 0) {
-        put_blob(S.buf, pre, S.blob_at[0]);
-    }
-    if (wg.x == (1u + 3u * static_cast<std::uint32_t>(d.n)) / kDcChunk) {
-        put_blob(S.buf, mid, S.blob_at[1]);
+    const std::uint32_t mid_chunk{(1u + 3u * static_cast<std::uint32_t>(d.n)) / kDcChunk};
+#pragma unroll
+    for (int i{0}; i < 2; ++i) {
+        if (wg.x == (i == 0 ? 0u : mid_chunk)) {
+            put_blob(S.buf, i == 0 ? pre : mid, S.blob_at[i]);
+        }
     }
     __syncthreads();
     const std::size_t chunk{static_cast<std::size_t>(g) * wg.nx + wg.x};
@@ -1143,7 +1144,7 @@ __device__ __forceinline__ void dc_emit_body(DcEmitShared& S, const Wg& wg, cons
         slot[i] = S.buf[i];
     }
     if (tid == 0) {
-        chunk_bits[chunk] = static_cast<std::uint32_t>(total);
+        chunk_bits[chunk] = total;
     }
 }
 

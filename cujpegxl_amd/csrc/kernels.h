@@ -84,25 +84,28 @@ bool build_codes_host(const std::uint32_t* hists, std::uint32_t count, std::uint
 void launch_huffman(hipStream_t s, int count, const std::uint32_t* hists, CodeSet* cs);
 // Words of one AC group's staging slot (bound on its token stream).
 std::size_t ac_group_slot_words();
-// AC groups are emitted in this many parts (row bands).
-std::size_t ac_group_parts();
-// The AC groups' parts and the DC groups' chunks into their staging slots,
+// Workgroups the emission gives each of `bands` bands in one launch.
+std::uint32_t emit_band_wgs(std::uint32_t bands);
+// Runs of one AC group (see entropy.inl's emission).
+std::size_t ac_group_runs();
+std::uint32_t ac_group_bands();
+// The AC groups' runs and the DC groups' chunks into their staging slots,
 // with their bit counts.
 void launch_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs, const std::uint16_t* item_tokens,
                  const std::uint32_t* tokens, const CodeSet* cs, const Constants* k, const std::uint32_t* fb_count,
                  const std::int32_t* dc, const std::int32_t* qf, const std::int8_t* ytox, const std::int8_t* ytob,
-                 std::uint32_t* ac_staging, std::uint64_t* ac_part_bits, std::uint32_t* dc_staging,
+                 std::uint32_t* ac_staging, std::uint16_t* ac_run_bits, std::uint32_t* dc_staging,
                  std::uint32_t* chunk_bits);
 // `chunk_bits` becomes the chunks' bit offsets in their groups.
 void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
-                   const std::uint64_t* ac_part_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
+                   const std::uint16_t* ac_run_bits, std::uint32_t* chunk_bits, std::uint32_t* dc_group_bytes,
                    std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
                    Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base, std::uint64_t* total_out,
                    hipEvent_t done = nullptr);
 void launch_assemble(hipStream_t s, const Geometry& geo, const Constants* k, const Layout* lay,
                      const std::uint32_t* dc_staging, const std::uint32_t* ac_staging, const std::uint64_t* dc_bits,
-                     const std::uint64_t* ac_bits, const std::uint64_t* ac_part_bits, const std::uint32_t* chunk_off,
-                     const std::uint64_t* dc_base, const std::uint64_t* ac_base, std::uint8_t* out,
-                     std::uint64_t cap_bytes, hipEvent_t done = nullptr);
+                     const std::uint16_t* ac_run_bits, const std::uint32_t* chunk_off, const std::uint64_t* dc_base,
+                     const std::uint64_t* ac_base, std::uint8_t* out, std::uint64_t cap_bytes,
+                     hipEvent_t done = nullptr);
 
 }  // namespace cjx
