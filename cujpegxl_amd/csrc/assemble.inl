@@ -282,49 +282,101 @@ __device__ __forceinline__ void u32_code(const Distr* d, std::uint32_t value, st
     len = 2 + nb;
 }
 
+// Exclusive scans of two values per thread at once (one barrier), over
+// kWaves waves; `sh` holds 2 kWaves words and must not be in use.
+template <int kWaves>
+__device__ __forceinline__ void block_excl_scan2(std::uint32_t& a, std::uint32_t& b, std::uint32_t* sh,
+                                                 std::uint32_t& total_a, std::uint32_t& total_b) {
+    const int lane{static_cast<int>(threadIdx.x) & 63}, wv{static_cast<int>(threadIdx.x) >> 6};
+    const std::uint32_t xa{wave_incl_scan_u32(a)}, xb{wave_incl_scan_u32(b)};
+    if (lane == 63) {
+        sh[wv] = xa;
+        sh[kWaves + wv] = xb;
+    }
+    __syncthreads();
+    std::uint32_t base_a{0}, base_b{0};
+    total_a = total_b = 0;
+#pragma unroll
+    for (int i{0}; i < kWaves; ++i) {
+        const std::uint32_t ta{sh[i]}, tb{sh[kWaves + i]};
+        base_a += i < wv ? ta : 0u;
+        base_b += i < wv ? tb : 0u;
+        total_a += ta;
+        total_b += tb;
+    }
+    a = base_a + xa - a;
+    b = base_b + xb - b;
+}
+
 // AcGlobal, section sizes, TOC, head, framing and every section's position,
-// by one 256-thread workgroup.  AcGlobal (constant prefix, 32 alphabet sizes,
-// 32 code headers) and the head (constant bits, TOC) are assembled in LDS:
-// every piece's bit offset comes from a block scan of the piece lengths, and
-// the section bases from scans of the section sizes.  `single` frames (one AC
-// group) concatenate DcGlobal, the DC group, AcGlobal and the AC tokens into
-// one section without padding in between.
-__device__ __attribute__((always_inline)) inline void layout_kernel_body(const Wg& wg, Geometry geo, const Constants* __restrict__ k,
-                                                     const CodeSet* __restrict__ cs,
-                                                     const std::uint16_t* __restrict__ ac_run_bits,
-                                                     std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
-                                                     std::uint32_t* __restrict__ dc_group_bytes,
-                                                     std::uint64_t* __restrict__ dc_group_bits,
-                                                     std::uint32_t* __restrict__ ac_group_bytes,
-                                                     std::uint64_t* __restrict__ ac_group_bits,
-                                                     Layout* __restrict__ lay, std::uint64_t* __restrict__ ac_base,
-                                                     std::uint64_t* __restrict__ dc_base,
-                                                     std::uint64_t* __restrict__ total_out) {
-    __shared__ std::uint32_t agw[kAcGlobalWords];
-    __shared__ std::uint32_t hw[kHeadWords];
-    __shared__ std::uint64_t agbits[kMaxAcGroups];
-    __shared__ std::uint64_t sh[17];
+// by one workgroup.  AcGlobal (constant prefix, 32 alphabet sizes, 32 code
+// headers) and the head (constant bits, TOC) are assembled in LDS: the pieces'
+// bit offsets come from one wave scan (64 pieces), the TOC's and the
+// sections' from one scan over the TOC entries, which are in section order.
+// `single` frames (one AC group) concatenate DcGlobal, the DC group, AcGlobal
+// and the AC tokens into one section without padding in between.
+//
+// One workgroup's chain of latencies bounds it, so every global read is
+// issued before the first wait (the code headers whole: 8 KB), 16 waves share
+// the loops, and only the words in use are cleared and stored.  With 256
+// threads, serial scans and the 66 KB worst case cleared and stored it took
+// 11.3 us at 320x240, 12.3 at 3840x2160 and 19.0 at 7680x4320; this form 5.3,
+// 6.5 and 9.0.
+constexpr int kLayoutThreads = 1024;
+constexpr int kLayoutWaves = kLayoutThreads / 64;
+constexpr int kMaxSections = 2 + 32 + kMaxAcGroups;
+
+struct LayoutShared {
+    std::uint32_t agw[kAcGlobalWords];
+    std::uint32_t hw[kHeadWords];
+    std::uint32_t ac_bits[kMaxAcGroups];
+    std::uint32_t dc_bits[32];
+    std::uint32_t piece_off[2 * kNumClusters];
+    std::uint32_t pos[kMaxSections];  // section starts, bytes after the head
+    std::uint32_t sh[2][2 * kLayoutWaves];
+    std::uint32_t ac_global_bits;
+};
+
+__device__ __attribute__((always_inline)) inline void layout_kernel_body(
+    const Wg& wg, const Geometry& geo, const Constants* __restrict__ k, const CodeSet* __restrict__ cs,
+    const std::uint16_t* __restrict__ ac_run_bits, std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,
+    std::uint32_t* __restrict__ dc_group_bytes, std::uint64_t* __restrict__ dc_group_bits,
+    std::uint32_t* __restrict__ ac_group_bytes, std::uint64_t* __restrict__ ac_group_bits, Layout* __restrict__ lay,
+    std::uint64_t* __restrict__ ac_base, std::uint64_t* __restrict__ dc_base, std::uint64_t* __restrict__ total_out) {
+    __shared__ LayoutShared S;
     const int t{static_cast<int>(threadIdx.x)};
-    // The reads that depend on nothing computed here, issued together before
-    // the first wait: each thread's first word of the AcGlobal prefix and of
-    // the head (the head's constant words are one per thread), its code
-    // header's alphabet size or bit count, and its wave's first DC group's
-    // chunk sizes.
-    static_assert(kHeadConstWords == 256, "one head word per thread");
-    __shared__ std::uint32_t dc_bits_s[32];
+    const int lane{t & 63}, wv{t >> 6};
+    // The reads that depend on nothing computed here.
+    static_assert(kHeadConstWords <= kLayoutThreads, "one head word per thread");
+    static_assert(kNumClusters * kHdrWords == 2 * kLayoutThreads, "two code header words per thread");
+    static_assert(2 * kNumClusters == 64, "AcGlobal's pieces fill one wave");
     const std::uint32_t pre_bits{k->ac_prefix_bits};
     const std::uint32_t hb{k->head_bits};
     const std::uint32_t dc_global_bits{k->dc_global_bits};
     const std::uint32_t prefix_w0{k->ac_prefix_words[t]};
-    const std::uint32_t head_w0{k->head_words[t]};
-    const std::uint32_t alpha_t{t < kNumClusters ? cs->alpha[t] : 0u};
-    const std::uint32_t hdr_bits_t{t >= kNumClusters && t < 2 * kNumClusters ? cs->hdr_bits[t - kNumClusters] : 0u};
-    // DC groups: wave w takes groups w, w + 4, ...; the group's chunk sizes
+    const std::uint32_t head_w0{t < kHeadConstWords ? k->head_words[t] : 0u};
+    const std::uint32_t hdr_w[2]{(&cs->hdr[0][0])[t], (&cs->hdr[0][0])[kLayoutThreads + t]};
+    const std::uint32_t hdr_len[2]{cs->hdr_bits[t / kHdrWords], cs->hdr_bits[(kLayoutThreads + t) / kHdrWords]};
+    const std::uint32_t piece{wv == 0 ? (t < kNumClusters ? cs->alpha[t] : cs->hdr_bits[t - kNumClusters]) : 0u};
+    // AC group sizes: the sums of their runs' bits, eight to a 16-byte read.
+    for (int g{t}; g < static_cast<int>(geo.num_ac); g += kLayoutThreads) {
+        const uint4* const rb{reinterpret_cast<const uint4*>(ac_run_bits + static_cast<std::size_t>(g) * kGroupRuns)};
+        std::uint32_t sum{0};
+#pragma unroll
+        for (int i{0}; i < kGroupRuns / 8; ++i) {
+            const uint4 v{rb[i]};
+            sum += (v.x & 0xffffu) + (v.x >> 16) + (v.y & 0xffffu) + (v.y >> 16) + (v.z & 0xffffu) + (v.z >> 16) +
+                   (v.w & 0xffffu) + (v.w >> 16);
+        }
+        S.ac_bits[g] = sum;
+        ac_group_bits[g] = sum;
+        ac_group_bytes[g] = (sum + 7) / 8;
+    }
+    // DC groups: wave w takes groups 15 - w, 31 - w; the group's chunk sizes
     // become their exclusive prefix sums (the assembly's chunk offsets).  All
     // of a group's sizes (at most kDcRounds per lane) are read at once.
     constexpr int kDcRounds{(kDcMaxChunks + 63) / 64};
-    for (int g{t >> 6}; g < static_cast<int>(geo.num_dc); g += 4) {
-        const int lane{t & 63};
+    for (int g{kLayoutWaves - 1 - wv}; g < static_cast<int>(geo.num_dc); g += kLayoutWaves) {
         const DcGroupGeo d{dc_group_geo(geo, g)};
         const int used{static_cast<int>((d.items + kDcChunk - 1) / kDcChunk)};
         std::uint32_t* const cb{chunk_bits + static_cast<std::size_t>(g) * dc_chunks};
@@ -343,184 +395,153 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
             sum += static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
         }
         if (lane == 0) {
-            dc_bits_s[g] = sum;
+            S.dc_bits[g] = sum;
             dc_group_bits[g] = sum;
             dc_group_bytes[g] = (sum + 7) / 8;
         }
     }
-    // AC group sizes: the sums of their runs' bits, eight to a 16-byte read.
-    for (int g{t}; g < static_cast<int>(geo.num_ac); g += 256) {
-        const uint4* const rb{reinterpret_cast<const uint4*>(ac_run_bits + static_cast<std::size_t>(g) * kGroupRuns)};
-        constexpr int kVecs{kGroupRuns / 8};
-        uint4 v[kVecs];
-#pragma unroll
-        for (int i{0}; i < kVecs; ++i) {
-            v[i] = rb[i];
+    // AcGlobal's pieces: alphabet sizes (lanes 0-31), headers (lanes 32-63).
+    std::uint32_t alpha_code{0}, alpha_len{0};
+    if (wv == 0) {
+        if (t < kNumClusters) {
+            alpha_len = var_len_u16(piece - 1, alpha_code);
         }
-        std::uint32_t sum{0};
-#pragma unroll
-        for (int i{0}; i < kVecs; ++i) {
-            for (const std::uint32_t w : {v[i].x, v[i].y, v[i].z, v[i].w}) {
-                sum += (w & 0xffffu) + (w >> 16);
-            }
+        const std::uint32_t len{t < kNumClusters ? alpha_len : piece};
+        const std::uint32_t incl{wave_incl_scan_u32(len)};
+        S.piece_off[t] = pre_bits + incl - len;
+        if (t == 63) {
+            S.ac_global_bits = pre_bits + incl;
         }
-        agbits[g] = sum;
-        ac_group_bits[g] = sum;
-        ac_group_bytes[g] = (sum + 7) / 8;
     }
-    for (int i{t}; i < kAcGlobalWords; i += 256) {
-        agw[i] = 0;
-    }
-    for (int i{t}; i < kHeadWords; i += 256) {
-        hw[i] = 0;
+    // The head's words in use at most: the constant bits, one bit, padding
+    // and 32 bits per TOC entry.
+    const bool single{geo.num_ac == 1};
+    const std::uint32_t entries{single ? 1u : 2u + geo.num_dc + geo.num_ac};
+    const int head_words{min(kHeadWords, static_cast<int>((hb + 8 + 32 * entries + 31) / 32))};
+    for (int i{t}; i < head_words; i += kLayoutThreads) {
+        const std::uint32_t at{32u * static_cast<std::uint32_t>(i)};
+        const std::uint32_t rem{at < hb ? hb - at : 0u};
+        S.hw[i] = rem >= 32 ? head_w0 : (head_w0 & ((1u << rem) - 1u));  // constant words: i == t
     }
     __syncthreads();
-    std::uint32_t overflow{0};
-    const auto dc_bytes = [&](std::uint32_t g) { return (dc_bits_s[g] + 7) / 8; };
 
-    // AcGlobal.
-    for (std::uint32_t i{static_cast<std::uint32_t>(t)}; i < (pre_bits + 31) / 32; i += 256) {
-        const std::uint32_t rem{pre_bits - 32 * i};
-        const std::uint32_t w{i == static_cast<std::uint32_t>(t) ? prefix_w0 : k->ac_prefix_words[i]};
-        agw[i] = rem >= 32 ? w : (w & ((1u << rem) - 1u));
+    // AcGlobal: cleared past the prefix, then the alphabets and headers.
+    const std::uint32_t abits{S.ac_global_bits};
+    std::uint32_t overflow{abits > static_cast<std::uint32_t>(kAcGlobalWords) * 32 ? 1u : 0u};
+    const int ac_words{min(kAcGlobalWords, static_cast<int>((abits + 31) / 32))};
+    for (int i{t}; i < ac_words; i += kLayoutThreads) {
+        const std::uint32_t at{32u * static_cast<std::uint32_t>(i)};
+        const std::uint32_t rem{at < pre_bits ? pre_bits - at : 0u};
+        const std::uint32_t w{rem == 0 ? 0u : (i == t ? prefix_w0 : k->ac_prefix_words[i])};
+        S.agw[i] = rem >= 32 ? w : (w & ((1u << rem) - 1u));
     }
-    std::uint32_t len{0}, val{0};
-    if (t < kNumClusters) {
-        len = var_len_u16(alpha_t - 1, val);
-    } else if (t < 2 * kNumClusters) {
-        len = hdr_bits_t;
-    }
-    std::uint64_t pieces{0};
-    const std::uint64_t off{pre_bits + block_excl_scan(len, sh, pieces)};
-    const std::uint64_t abits{pre_bits + pieces};
-    if (abits > static_cast<std::uint64_t>(kAcGlobalWords) * 32) {
-        overflow = 1;
-    } else if (t < kNumClusters) {
-        lds_or_bits(agw, kAcGlobalWords, static_cast<std::uint32_t>(off), val, len);
-    } else if (t < 2 * kNumClusters) {
-        const std::uint32_t* src{cs->hdr[t - kNumClusters]};
-        for (std::uint32_t i{0}; i < len; i += 32) {
-            lds_or_bits(agw, kAcGlobalWords, static_cast<std::uint32_t>(off) + i, src[i >> 5],
-                        len - i < 32 ? len - i : 32u);
-        }
-    }
-
-    // Head: constant bits, no permutation (one 0 bit), byte-aligned TOC.
-    for (std::uint32_t i{static_cast<std::uint32_t>(t)}; i < (hb + 31) / 32; i += 256) {
-        const std::uint32_t rem{hb - 32 * i};
-        const std::uint32_t w{head_w0};  // i == t: the head has at most 256 words
-        hw[i] = rem >= 32 ? w : (w & ((1u << rem) - 1u));
-    }
+    // TOC entries, in section order.  Sizes sum below 2^32 (a frame has at
+    // most 32 DC groups).
     const Distr toc[4]{{false, 0, 10}, {false, 1024, 14}, {false, 17408, 22}, {false, 4211712, 30}};
-    const bool single{geo.num_ac == 1};
     const std::uint32_t dcg{(dc_global_bits + 7) / 8};
-    const std::uint32_t acg{static_cast<std::uint32_t>((abits + 7) / 8)};
-    const std::uint32_t entries{single ? 1u : 2u + geo.num_dc + geo.num_ac};
-    std::uint64_t at{(hb + 1u + 7u) & ~7u};
-    std::uint64_t body{0};
-    for (std::uint32_t e0{0}; e0 < entries; e0 += 256) {
+    const std::uint32_t acg{(abits + 7) / 8};
+    std::uint32_t at{(hb + 1u + 7u) & ~7u};
+    std::uint32_t body{0};
+    int buf{0};
+    for (std::uint32_t e0{0}; e0 < entries; e0 += kLayoutThreads, buf ^= 1) {
         const std::uint32_t e{e0 + static_cast<std::uint32_t>(t)};
         std::uint32_t size{0}, code{0}, clen{0};
         if (e < entries) {
             if (single) {
-                const std::uint64_t bits{dc_global_bits + dc_bits_s[0] + abits + agbits[0]};
-                size = static_cast<std::uint32_t>((bits + 7) / 8);
+                size = (dc_global_bits + S.dc_bits[0] + abits + S.ac_bits[0] + 7) / 8;
             } else if (e == 0) {
                 size = dcg;
             } else if (e <= geo.num_dc) {
-                size = dc_bytes(e - 1);
+                size = (S.dc_bits[e - 1] + 7) / 8;
             } else if (e == geo.num_dc + 1) {
                 size = acg;
             } else {
-                size = static_cast<std::uint32_t>((agbits[e - geo.num_dc - 2] + 7) / 8);
+                size = (S.ac_bits[e - geo.num_dc - 2] + 7) / 8;
             }
             u32_code(toc, size, code, clen);
         }
-        std::uint64_t chunk_bits{0}, chunk_bytes{0};
-        const std::uint64_t p{at + block_excl_scan(clen, sh, chunk_bits)};
-        (void)block_excl_scan(size, sh, chunk_bytes);
-        if (clen != 0 && p + clen <= static_cast<std::uint64_t>(kHeadWords) * 32) {
-            lds_or_bits(hw, kHeadWords, static_cast<std::uint32_t>(p), code, clen);
+        std::uint32_t p{clen}, q{size}, chunk_bits_sum{0}, chunk_bytes{0};
+        // The barrier inside also orders the clearing above before the ORs.
+        block_excl_scan2<kLayoutWaves>(p, q, S.sh[buf], chunk_bits_sum, chunk_bytes);
+        if (clen != 0) {
+            if (at + p + clen <= static_cast<std::uint32_t>(kHeadWords) * 32) {
+                lds_or_bits(S.hw, kHeadWords, at + p, code, clen);
+            }
+            S.pos[e] = body + q;
         }
-        at += chunk_bits;
+        at += chunk_bits_sum;
         body += chunk_bytes;
     }
-    at = (at + 7) & ~7ull;
-    if (at > static_cast<std::uint64_t>(kHeadWords) * 32) {
+    if (overflow == 0) {
+        if (t < kNumClusters) {
+            lds_or_bits(S.agw, kAcGlobalWords, S.piece_off[t], alpha_code, alpha_len);
+        }
+#pragma unroll
+        for (int j{0}; j < 2; ++j) {
+            const int idx{j * kLayoutThreads + t};
+            const std::uint32_t bit{32u * static_cast<std::uint32_t>(idx % kHdrWords)};
+            if (bit < hdr_len[j]) {
+                lds_or_bits(S.agw, kAcGlobalWords, S.piece_off[kNumClusters + idx / kHdrWords] + bit, hdr_w[j],
+                            hdr_len[j] - bit < 32 ? hdr_len[j] - bit : 32u);
+            }
+        }
+    }
+    at = (at + 7) & ~7u;
+    if (at > static_cast<std::uint32_t>(kHeadWords) * 32) {
         overflow = 1;
     }
-    const std::uint32_t head_bytes{static_cast<std::uint32_t>(at / 8)};
-    const std::uint64_t cs_bytes{head_bytes + body};
+    const std::uint32_t head_bytes{at / 8};
+    const std::uint64_t cs_bytes{static_cast<std::uint64_t>(head_bytes) + body};
     const std::uint32_t framing{cs_bytes >= 0x100000000ull - 8 ? 48u : 40u};
 
     // Section positions (absolute bits in the file).
     const std::uint64_t dcg_bit{(static_cast<std::uint64_t>(framing) + head_bytes) * 8};
+    __syncthreads();
+    const auto section = [&](std::uint32_t e) { return dcg_bit + static_cast<std::uint64_t>(S.pos[e]) * 8; };
     std::uint64_t ac_global_bit{0};
     if (single) {
+        ac_global_bit = dcg_bit + dc_global_bits + S.dc_bits[0];
         if (t == 0) {
             dc_base[0] = dcg_bit + dc_global_bits;
-            ac_global_bit = dcg_bit + dc_global_bits + dc_bits_s[0];
             ac_base[0] = ac_global_bit + abits;
         }
     } else {
-        const std::uint64_t first{dcg_bit + static_cast<std::uint64_t>(dcg) * 8};
-        std::uint64_t dc_total{0};
-        const std::uint32_t g{static_cast<std::uint32_t>(t)};
-        const std::uint64_t dsz{g < geo.num_dc ? static_cast<std::uint64_t>(dc_bytes(g)) * 8 : 0ull};
-        const std::uint64_t dpre{block_excl_scan(dsz, sh, dc_total)};
-        if (g < geo.num_dc) {
-            dc_base[g] = first + dpre;
+        ac_global_bit = section(geo.num_dc + 1);
+        if (t < static_cast<int>(geo.num_dc)) {
+            dc_base[t] = section(1 + static_cast<std::uint32_t>(t));
         }
-        ac_global_bit = first + dc_total;
-        std::uint64_t run{ac_global_bit + static_cast<std::uint64_t>(acg) * 8};
-        for (std::uint32_t g0{0}; g0 < geo.num_ac; g0 += 256) {
-            const std::uint32_t ga{g0 + static_cast<std::uint32_t>(t)};
-            const std::uint64_t asz{ga < geo.num_ac ? (agbits[ga] + 7) / 8 * 8 : 0ull};
-            std::uint64_t chunk{0};
-            const std::uint64_t apre{block_excl_scan(asz, sh, chunk)};
-            if (ga < geo.num_ac) {
-                ac_base[ga] = run + apre;
-            }
-            run += chunk;
+        for (std::uint32_t g{static_cast<std::uint32_t>(t)}; g < geo.num_ac; g += kLayoutThreads) {
+            ac_base[g] = section(geo.num_dc + 2 + g);
         }
     }
     // Container framing (container.cc:35-54): the 32-byte signature and ftyp
     // box, then the jxlc box header (8 bytes, or 16 with a 64-bit size).
-    // Lane i forms bytes 4i..4i+3.
-    if (t < static_cast<int>(framing / 4)) {
-        constexpr std::uint8_t sig[32]{0,   0,   0, 0x0c, 'J', 'X', 'L', ' ', 0x0d, 0x0a, 0x87,
-                                       0x0a, 0,  0, 0,    0x14, 'f', 't', 'y', 'p', 'j',  'x',
-                                       'l', ' ', 0, 0,    0,    0,   'j', 'x', 'l', ' '};
+    // Lane i of the last wave forms bytes 4i..4i+3.
+    const int fl{t - (kLayoutThreads - 64)};
+    if (fl >= 0 && fl < static_cast<int>(framing / 4)) {
+        constexpr std::uint32_t sig[8]{0x0c000000u, 0x204c584au, 0x0a870a0du, 0x14000000u,
+                                       0x70797466u, 0x206c786au, 0x00000000u, 0x206c786au};
         const bool large{framing == 48};
         const std::uint64_t box{cs_bytes + (large ? 16 : 8)};
-        const std::uint32_t field{large ? 1u : static_cast<std::uint32_t>(box)};
-        std::uint32_t word{0};
-        for (int j{0}; j < 4; ++j) {
-            const int i{4 * t + j};
-            std::uint8_t b;
-            if (i < 32) {
-                b = sig[i];
-            } else if (i < 36) {
-                b = static_cast<std::uint8_t>(field >> (8 * (35 - i)));
-            } else if (i < 40) {
-                b = static_cast<std::uint8_t>("jxlc"[i - 36]);
-            } else {
-                b = static_cast<std::uint8_t>(box >> (8 * (47 - i)));
-            }
-            word |= static_cast<std::uint32_t>(b) << (8 * j);
+        std::uint32_t word{fl < 8 ? sig[fl & 7] : 0u};
+        if (fl == 8) {
+            word = __builtin_bswap32(large ? 1u : static_cast<std::uint32_t>(box));
+        } else if (fl == 9) {
+            word = 0x636c786au;  // "jxlc"
+        } else if (fl >= 10) {
+            word = __builtin_bswap32(static_cast<std::uint32_t>(fl == 10 ? box >> 32 : box));
         }
-        lay->framing_words[t] = word;
+        lay->framing_words[fl] = word;
     }
-    __syncthreads();
-    for (int i{t}; i < kAcGlobalWords; i += 256) {
-        lay->ac_global_words[i] = agw[i];
+    for (int i{t}; i < ac_words; i += kLayoutThreads) {
+        lay->ac_global_words[i] = S.agw[i];
     }
-    for (int i{t}; i < kHeadWords; i += 256) {
-        lay->head_words[i] = hw[i];
+    for (int i{t}; i < static_cast<int>((at + 31) / 32) && i < kHeadWords; i += kLayoutThreads) {
+        lay->head_words[i] = S.hw[i];
     }
     if (t == 0) {
-        lay->ac_global_bits = static_cast<std::uint32_t>(abits);
-        lay->head_total_bits = static_cast<std::uint32_t>(at);
+        lay->ac_global_bits = abits;
+        lay->head_total_bits = at;
         lay->head_bytes = head_bytes;
         lay->framing_bytes = framing;
         lay->codestream_bytes = cs_bytes;
@@ -532,7 +553,7 @@ __device__ __attribute__((always_inline)) inline void layout_kernel_body(const W
     }
 }
 
-__global__ __launch_bounds__(256) void layout_kernel(Geometry geo, const Constants* __restrict__ k,
+__global__ __launch_bounds__(kLayoutThreads) void layout_kernel(Geometry geo, const Constants* __restrict__ k,
                                                      const CodeSet* __restrict__ cs,
                                                      const std::uint16_t* __restrict__ ac_run_bits,
                                                      std::uint32_t* __restrict__ chunk_bits, std::uint32_t dc_chunks,

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kEmitThreads) void emit_batch_kernel(const FrameJob
                                          j.dc_chunks, wg.nx - j.dc_chunks * j.geo.num_dc});
 }
 
-__global__ __launch_bounds__(256) void layout_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
+__global__ __launch_bounds__(kLayoutThreads) void layout_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBLayout, wg)};
     layout_kernel_body(wg, j.geo, j.k, j.codes, j.ac_run_bits, j.chunk_bits,
@@ -170,7 +170,7 @@ void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uin
     histograms_batch_kernel<<<total[kBHistograms], 256, 0, s>>>(jobs, count);
     huffman_batch_kernel<<<total[kBHuffman], 64 * kTrials, 0, s>>>(jobs, count);
     emit_batch_kernel<<<total[kBEmit], kEmitThreads, 0, s>>>(jobs, count);
-    layout_batch_kernel<<<total[kBLayout], 256, 0, s>>>(jobs, count);
+    layout_batch_kernel<<<total[kBLayout], kLayoutThreads, 0, s>>>(jobs, count);
     assemble_batch_kernel<<<total[kBAssemble], 256, 0, s>>>(jobs, count);
 }
 

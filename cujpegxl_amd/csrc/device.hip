@@ -321,7 +321,7 @@ void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const
                    std::uint64_t* dc_group_bits, std::uint32_t* ac_group_bytes, std::uint64_t* ac_group_bits,
                    Layout* lay, std::uint64_t* ac_base, std::uint64_t* dc_base, std::uint64_t* total_out,
                    hipEvent_t done) {
-    hipExtLaunchKernelGGL(layout_kernel, dim3(1), dim3(256), 0, s, nullptr, done, 0, geo, k, cs, ac_run_bits,
+    hipExtLaunchKernelGGL(layout_kernel, dim3(1), dim3(kLayoutThreads), 0, s, nullptr, done, 0, geo, k, cs, ac_run_bits,
                           chunk_bits, dc_chunks_per_group(geo), dc_group_bytes, dc_group_bits, ac_group_bytes,
                           ac_group_bits, lay, ac_base, dc_base, total_out);
 }

@@ -45,3 +45,19 @@ def test_batch_of_dc_group_edges(jo):
     b.close()
     for f in frames:
         f[2].close()
+
+
+def test_more_sections_than_layout_threads(jo):
+    # 4 x 256 AC groups and 32 DC groups: 1,058 sections, two rounds of the
+    # layout's 1,024 threads.
+    w, h, d = 776, 65536, 2.0
+    luma, chroma = synthetic_nv12(w, 512, 21)
+    luma, chroma = np.tile(luma, (128, 1)), np.tile(chroma, (128, 1))
+    jo.set_threads(8)
+    want = jo.encode_nv12(luma, chroma, w, h, d)
+    jo.set_threads(1)
+    dev = cj.DeviceBuffer.from_array(np.concatenate([luma.ravel(), chroma.ravel()]))
+    enc = cj.Encoder(w, h, d)
+    assert enc.encode_device(dev.ptr, dev.ptr + w * h, w, w) == want
+    enc.close()
+    dev.close()
