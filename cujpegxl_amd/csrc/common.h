@@ -142,6 +142,12 @@ struct DeviceTables {
     std::uint16_t mf8[2][256];
     std::uint16_t mf16[2][256];
     std::uint16_t mf32[2][1024];
+    // Basis values as the exact matrix-core steps take them: lane l, step s
+    // holds A[l % 16][4 s + l / 16] of blockdiag(A8, A8), A16 and rows
+    // 16 f .. 16 f + 15 of A32.
+    alignas(16) float ex8[64][4];
+    float ex16[64][4];
+    float ex32[2][64][8];
 };
 
 extern __constant__ __align__(16) DeviceTables g_tables;

@@ -142,13 +142,6 @@ __device__ __forceinline__ void lds_or_bits(std::uint32_t* words, std::uint32_t 
     }
 }
 
-// Orders one wave's LDS accesses: writes before the barrier are seen by
-// every lane's reads after it.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 struct AcItem {
     int n;             // transform side, 0 if covered
     int c;             // XYB channel

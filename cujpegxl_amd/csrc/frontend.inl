@@ -27,6 +27,13 @@ constexpr int kTileW = 32 + 2 * kHalo;  // 36
 // each side.
 constexpr int kChromaW = kTileW / 2 + 2;  // 20
 
+// Orders one wave's LDS accesses: writes before the barrier are seen by
+// every lane's reads after it.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Grid-strided zeroing of the Clears buffers by every thread of a launch
 // (of the frame's workgroups, in a batched launch).
 __device__ __forceinline__ void clear_words(const Clears& c, const Wg& wg) {
@@ -306,60 +313,11 @@ __device__ __forceinline__ void dct_line(const float* __restrict__ src, int k0, 
     }
 }
 
-// Separable DCT lines on the matrix cores.  One K=1 step of
-// v_mfma_f32_16x16x1_4b_f32 adds A[b][i] * B[b][j] to D[b][i][j] for four
-// independent 16x16 blocks b, rounding like fmaf (the hardware's result for
-// every K=1 step equals fmaf(a, b, d) bit for bit), so N steps over c
-// reproduce dct_line's fmaf chain exactly.  Lanes 16b..16b+15 supply block b:
-// lane 16b + t gives A[b][t] = a_row[c] and B[b][t] = b_row[c].  On return
-// lane l holds D[b][4 (l / 16) + u][l % 16] in element 4 b + u.  The B row
-// is read like dct_line's source (columns from col0, groups permuted by swz).
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-template <int N>
-__device__ __forceinline__ v16f mfma_lines(const float* __restrict__ a_row, const float* __restrict__ b_row,
-                                           int col0 = 0, int swz = 0) {
-    // The lane's whole basis row is read before the chain starts (one
-    // memory latency instead of one per four steps).
-    float4 ar[N / 4];
-#pragma unroll
-    for (int c{0}; c < N / 4; ++c) {
-        ar[c] = *reinterpret_cast<const float4*>(a_row + 4 * c);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the chain
-    v16f acc;
-#pragma unroll
-    for (int i{0}; i < 16; ++i) {
-        acc[i] = 0.0f;
-    }
-#pragma unroll
-    for (int c{0}; c < N; c += 4) {
-        const float4 a{ar[c / 4]};
-        const float4 b{*reinterpret_cast<const float4*>(b_row + ((((col0 + c) >> 2) ^ swz) << 2))};
-        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a.x, b.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a.y, b.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a.z, b.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a.w, b.w, acc, 0, 0, 0);
-    }
-    return acc;
-}
-
-// Row-pass buffer geometry (floats): line (block b, frequency k) of size n
-// starts at b * BS + k * RS.  RS is a multiple of 4 (16-byte loads) chosen so
-// that eight consecutive lines start in eight different 4-bank groups.
-template <int N>
-struct RowBuf;
-template <>
-struct RowBuf<8> {
+// Row-pass lines of the DCT8s (dct8_uniform_kernel): line (block b, frequency
+// k) starts at b * BS + k * RS; RS a multiple of 4 (16-byte loads) such that
+// eight consecutive lines start in eight different 4-bank groups.
+struct RowBuf8 {
     static constexpr int RS = 12, BS = 104;
-};
-template <>
-struct RowBuf<16> {
-    static constexpr int RS = 20, BS = 320;
-};
-template <>
-struct RowBuf<32> {
-    static constexpr int RS = 36, BS = 1152;
 };
 
 // Sharpened planes: rows of 32 floats without padding, the row's eight
@@ -373,29 +331,24 @@ __device__ __forceinline__ int sp_swz(int row) {
 __device__ __forceinline__ int sp_index(int row, int col) {
     return row * kSP + (((col >> 2) ^ sp_swz(row)) << 2) + (col & 3);
 }
-// Row-pass lines of the three selection sizes side by side.
-constexpr int kLines32 = 0;
-constexpr int kLines16 = kLines32 + RowBuf<32>::BS;
-constexpr int kLines8 = kLines16 + 4 * RowBuf<16>::BS;
-constexpr int kScratch = kLines8 + 16 * RowBuf<8>::BS;
-
-// Element arrays are written in transposed (column) order by the transforms
-// and read in element order: one pad slot per 32 elements keeps the
-// column-order writes of 16 lanes in distinct banks.
-constexpr int kCoefPadded = 1024 + 2 * 32;  // FP16 arrays: two halfs (one bank) per 32
+// Coefficient arrays are written four elements at a time in transposed
+// (column) order by the transforms and read in element order: four pad halfs
+// per 32 elements keep the 8-byte accesses aligned and spread the columns.
+constexpr int kCoefPadded = 1024 + 4 * 32;
 __device__ __forceinline__ int cpad(int e) {
-    return e + 2 * (e >> 5);
+    return e + 4 * (e >> 5);
 }
 
 // Arrays whose lifetimes do not overlap share storage, which keeps the
 // workgroup under 32 KB of LDS (five resident workgroups per CU):
 // - steps 1-3: the XYB tile, then the AQ terms (step 3) past its end;
-//   steps 4-5: the row-pass lines;
+//   step 4: the DCT32's selection terms, the features, the network's hidden
+//   units;
 // - the powers' table and the chroma window in step 1, then the
 //   sharpened planes, from step 2 until their last row pass (Y in
 //   step 4, X and B in step 5); each plane's space then holds coefficients:
 //   X's and B's the chosen transforms (step 5 on), Y's (the last plane, and
-//   256 bytes past it) the DCT16 and DCT32 candidates (step 4 on).  The DCT8
+//   512 bytes past it) the DCT16 and DCT32 candidates (step 4 on).  The DCT8
 //   candidates of Y have their own array.
 constexpr int kPlaneHalfs = 2 * 32 * kSP;
 static_assert(kCoefPadded <= kPlaneHalfs, "a coefficient array per plane");
@@ -410,7 +363,12 @@ struct RegionShared {
                 float blk[16][3];  // per block: HF sum, gamma, blue sum
             } aq;                  // AQ terms (step 3)
         } f;
-        float scratch[kScratch];  // row-pass lines (steps 4-5)
+        struct {
+            float t32[2][4][64][4];  // DCT32 terms (errors, rates) of each wave's quadrant
+            float feat[112];         // network features (block sums first; learned mode and export)
+            float hid[72];           // the network's hidden units and outputs
+        } s;                         // step 4
+        float scratch[3072];  // dct8_uniform_kernel: row-pass lines, then Y's quantized values
     } u;
     union {
         alignas(16) float sharp[3][32 * kSP];
@@ -427,7 +385,6 @@ struct RegionShared {
     float cost32p[4];      // matrix-core form: the DCT32 cost's part from each wave
     float cfl[4][3];
     int acs[16];           // region-local raster
-    float feat[112];       // network features (block sums first; learned mode and export)
     int blkqf[16];         // quant field of the region's blocks (export)
     int choice[4];         // the heuristic's choice per quad (export)
     int learned_ok;        // the network's decision was confident
@@ -680,6 +637,131 @@ __device__ __forceinline__ void gaborish_tile(RegionShared& S, int tid) {
 }
 
 // ---------------------------------------------------------------------------
+// The plain form's DCTs on the matrix cores, exact.  v_mfma_f32_16x16x4_f32
+// adds A[i][k] B[k][j], k = 0..3, to D[i][j] as the fmaf chain in k order (the
+// hardware's result equals the chain bit for bit: 100 M results of 4 to 64
+// steps, denormal products and exact cancellations among them), so a sequence
+// of steps over c gives dct_line's chain.  Lane l supplies A[l % 16][l / 16]
+// and B[l / 16][l % 16] and holds D[4 (l / 16) + u][l % 16], u = 0..3.
+//
+// A row pass T = P A^T takes the pixels as the first operand and the basis
+// row of the lane's frequency as the second, the column pass C = A T the same
+// basis values as the first operand.  Between them T moves from "row 4 g + u
+// in register u of lane group g" to "row 4 u + g" (the natural order of the
+// chain): a 4 x 4 transpose of registers and lane groups, four permlane
+// swaps, no LDS.  A 16 x 16 quad is one tile per pass: a DCT16, or four DCT8s
+// with a block-diagonal basis (a chain's zero steps add +0 to a sum that is
+// never -0).  A DCT32 quadrant takes two row-pass tiles.  Every wave works on
+// one quad and one quadrant.  (Before: K = 1 steps with the DCT32 in wave 0
+// alone, 1,024 clocks a pass, the DCT8s on the VALU, and the row passes
+// through LDS lines; REGION_FIGURES.)
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f4v ex_step(float a, float b, f4v acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ void ex_swap32(float& a, float& b) {
+    const auto r{__builtin_amdgcn_permlane32_swap(f2u(a), f2u(b), false, false)};
+    a = u2f(r[0]);
+    b = u2f(r[1]);
+}
+
+__device__ __forceinline__ void ex_swap16(float& a, float& b) {
+    const auto r{__builtin_amdgcn_permlane16_swap(f2u(a), f2u(b), false, false)};
+    a = u2f(r[0]);
+    b = u2f(r[1]);
+}
+
+// Register u of lane group g <-> register g of lane group u.
+__device__ __forceinline__ void ex_turn(float (&t)[4]) {
+    ex_swap32(t[0], t[2]);
+    ex_swap32(t[1], t[3]);
+    ex_swap16(t[0], t[1]);
+    ex_swap16(t[2], t[3]);
+}
+
+// Pixels (row, col0 + 4 s + l / 16), s = 0 .. kSteps - 1 (col0 0 or 16, 0
+// only with eight steps): the 16-byte group index of step s is step 0's with
+// s XORed in.
+template <int kSteps>
+__device__ __forceinline__ void ex_pixels(const float* plane, int row, int col0, int lane, float (&p)[kSteps]) {
+    const int base{row * kSP + (((col0 >> 2) ^ sp_swz(row)) << 2) + (lane >> 4)};
+#pragma unroll
+    for (int s{0}; s < kSteps; ++s) {
+        p[s] = plane[base ^ (4 * s)];
+    }
+}
+
+__device__ __forceinline__ f4v ex_rows(const float (&p)[4], const float4& b) {
+    f4v t{0.0f, 0.0f, 0.0f, 0.0f};
+    t = ex_step(p[0], b.x, t);
+    t = ex_step(p[1], b.y, t);
+    t = ex_step(p[2], b.z, t);
+    return ex_step(p[3], b.w, t);
+}
+
+__device__ __forceinline__ f4v ex_cols(const float4& a, const f4v& rows, f4v acc) {
+    float t[4]{rows[0], rows[1], rows[2], rows[3]};
+    ex_turn(t);
+    acc = ex_step(a.x, t[0], acc);
+    acc = ex_step(a.y, t[1], acc);
+    acc = ex_step(a.z, t[2], acc);
+    return ex_step(a.w, t[3], acc);
+}
+
+// The 16x16 quad at (row0, col0) of `plane` through the lane's basis values:
+// lane l returns C[4 (l / 16) + u][l % 16] (row = vertical frequency).
+__device__ __forceinline__ f4v ex_quad(const float* plane, int row0, int col0, const float4& b, int lane) {
+    float p[4];
+    ex_pixels<4>(plane, row0 + (lane & 15), col0, lane, p);
+    return ex_cols(b, ex_rows(p, b), f4v{0.0f, 0.0f, 0.0f, 0.0f});
+}
+
+// Lane values of the 32-point basis for frequencies 16 f .. 16 f + 15.
+struct Ex32 {
+    float4 lo, hi;
+};
+__device__ __forceinline__ Ex32 ex_basis32(int f, int lane) {
+    const float4* const b{reinterpret_cast<const float4*>(&g_tables.ex32[f][lane][0])};
+    return {b[0], b[1]};
+}
+
+// DCT32 of the region's plane: the row-pass tiles of horizontal frequencies
+// 16 fxb .. (rows 0..15 and 16..31), the two chains side by side.
+__device__ __forceinline__ void ex_rows32(const float* plane, const Ex32& b, int lane, f4v (&t)[2]) {
+    float p[2][8];
+    ex_pixels<8>(plane, lane & 15, 0, lane, p[0]);
+    ex_pixels<8>(plane, 16 + (lane & 15), 0, lane, p[1]);
+    const float bv[8]{b.lo.x, b.lo.y, b.lo.z, b.lo.w, b.hi.x, b.hi.y, b.hi.z, b.hi.w};
+    t[0] = t[1] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s{0}; s < 8; ++s) {
+        t[0] = ex_step(p[0][s], bv[s], t[0]);
+        t[1] = ex_step(p[1][s], bv[s], t[1]);
+    }
+}
+
+__device__ __forceinline__ f4v ex_cols32(const Ex32& a, const f4v (&t)[2]) {
+    return ex_cols(a.hi, t[1], ex_cols(a.lo, t[0], f4v{0.0f, 0.0f, 0.0f, 0.0f}));
+}
+
+// Output tiles (0, 16 fxb) and (16, 16 fxb) (vertical, horizontal frequency
+// origins) into c[0], c[1].
+__device__ __forceinline__ void ex_dct32(const float* plane, int fxb, int lane, f4v (&c)[2]) {
+    f4v t[2];
+    ex_rows32(plane, ex_basis32(fxb, lane), lane, t);
+    c[0] = ex_cols32(ex_basis32(0, lane), t);
+    c[1] = ex_cols32(ex_basis32(1, lane), t);
+}
+
+// Lane l - 16's value, for lanes of the odd rows of 16.
+__device__ __forceinline__ float from_row_above(float v) {
+    const auto r{__builtin_amdgcn_permlane16_swap(f2u(v), f2u(v), false, false)};
+    return u2f(r[0]);
+}
+
+// ---------------------------------------------------------------------------
 // Matrix-core DCT form with FP16 operands (kModeMfma16).  Every transform is
 // built from v_mfma_f32_16x16x16_f16 steps: D[i][j] += sum_k A[i][k] B[k][j]
 // over a 16x16x16 tile, lane l supplying A[l % 16][4 (l / 16) + 0..3] and
@@ -695,7 +777,6 @@ __device__ __forceinline__ void gaborish_tile(RegionShared& S, int tid) {
 // (exact) into |x| <= 1 (sharpened XYB stays within 2.97 * 0.9) and the
 // results by 4.
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr float kMfScale = 0.25f;
 
 struct MfOp {
@@ -859,25 +940,25 @@ __device__ __forceinline__ float grad_weight(int k) {
     return w[k];
 }
 
-// Block b's raw sums (var, grad, dist, rate, mean) into S.feat[6 b ..]; the
+// Block b's raw sums (var, grad, dist, rate, mean) into S.u.s.feat[6 b ..]; the
 // cost sits in S.cost8.
 __device__ __forceinline__ void feature_store(RegionShared& S, int b, float var, float grad, float dist, float rate,
                                               float mean) {
-    S.feat[6 * b + 0] = var;
-    S.feat[6 * b + 1] = grad;
-    S.feat[6 * b + 3] = dist;
-    S.feat[6 * b + 4] = rate;
-    S.feat[6 * b + 5] = mean;
+    S.u.s.feat[6 * b + 0] = var;
+    S.u.s.feat[6 * b + 1] = grad;
+    S.u.s.feat[6 * b + 3] = dist;
+    S.u.s.feat[6 * b + 4] = rate;
+    S.u.s.feat[6 * b + 5] = mean;
 }
 
-// The raw sums -> the 96 features in S.feat (every thread calls this;
+// The raw sums -> the 96 features in S.u.s.feat (every thread calls this;
 // barriers inside).
 __device__ __forceinline__ void feature_finish(RegionShared& S, int tid, int bx0, int by0, int bw, int bh) {
     float f[6]{};
     if (tid < 16) {
         const int bx{tid & 3}, by{tid >> 2};
         if (bx0 + bx < bw && by0 + by < bh) {
-            const float* s{&S.feat[6 * tid]};
+            const float* s{&S.u.s.feat[6 * tid]};
             const float c8{S.cost8[((by >> 1) * 2 + (bx >> 1)) * 4 + (by & 1) * 2 + (bx & 1)]};
             f[0] = log2_det(1.0f + 4096.0f * fmaxf(s[0], 0.0f));
             f[1] = log2_det(1.0f + 1024.0f * fmaxf(s[1], 0.0f));
@@ -891,7 +972,7 @@ __device__ __forceinline__ void feature_finish(RegionShared& S, int tid, int bx0
     if (tid < 16) {
 #pragma unroll
         for (int k{0}; k < 6; ++k) {
-            S.feat[6 * tid + k] = f[k];
+            S.u.s.feat[6 * tid + k] = f[k];
         }
     }
     __syncthreads();
@@ -906,7 +987,7 @@ __device__ __forceinline__ bool mlp_decide(RegionShared& S, const FrameParams& p
                                            int tid, int bx0, int by0, int bw, int bh) {
     {
         const int j{tid >> 2}, k{tid & 3};
-        const float* const x{&S.feat[24 * k]};
+        const float* const x{&S.u.s.feat[24 * k]};
         float s{0.0f};
 #pragma unroll
         for (int i{0}; i < 24; i += 8) {
@@ -993,7 +1074,7 @@ __device__ __forceinline__ void export_features(const RegionShared& S, float* ou
                                                 int by0, int bw, int bh) {
     float* const row{out + static_cast<std::size_t>(region) * kFeatRow};
     if (tid < 96) {
-        row[tid] = S.feat[tid];
+        row[tid] = S.u.s.feat[tid];
     } else if (tid < 108) {
         const int k{tid - 96};
         float v{0.0f};
@@ -1168,198 +1249,145 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
 
     CJX_REGION_CUT_AT(3)
     // 4. Transform selection on the sharpened Y (transform_select_impl.cuh:49-201).
-    //    Plain: the three sizes run side by side (wave 0 the DCT32 and wave 1
-    //    the four DCT16s on the matrix cores, waves 2-3 the sixteen DCT8s on
-    //    the VALU); each wave keeps its coefficients' selection terms in
-    //    registers and sums them there (per lane in register order, then a
-    //    lane tree).  Learned: the DCT8s and their costs, the region's
+    //    Wave w transforms quad w as four DCT8s and as one DCT16, and quadrant
+    //    w of the DCT32 (vertical frequencies 16 (w / 2).., horizontal ones
+    //    16 (w % 2)..), on the matrix cores; the terms stay in registers and
+    //    are summed there.  Learned: the DCT8s and their costs, the region's
     //    features and the network first; the DCT16 and DCT32 candidates only
     //    where the network is not confident (the heuristic decides there).
-    __syncthreads();  // the XYB tile is dead from here on; its space holds row-pass lines
+    __syncthreads();  // the XYB tile is dead from here on
     CJX_REGION_CUT_AT(6)
-    float* const lines{S.u.scratch};
     const int grp{lane >> 4}, t16{lane & 15};
     const float* const yp{plane_of(S, 1)};
+    const int qrow{(wu >> 1) * 16}, qcol{(wu & 1) * 16};  // the wave's quad
     const bool want_features{kLearned || feat_out != nullptr};
-    float td[16], tr[16];
-    // Plain pieces: row passes of the DCT32 / DCT16 candidates (waves 0-1)
-    // and of the DCT8s (waves 2-3), then the column passes with the costs.
-    const auto rows_big = [&]() {
-        if (wu == 0) {
-            // DCT32 as four 16x16 quadrants: block (fh, rh) = (grp >> 1, grp & 1).
-            const int row{16 * (grp & 1) + t16};
-            const v16f acc{mfma_lines<32>(g_tables.basis32 + (16 * (grp >> 1) + t16) * 32, yp + row * kSP, 0,
-                                          sp_swz(row))};
-#pragma unroll
-            for (int b{0}; b < 4; ++b) {
-#pragma unroll
-                for (int u{0}; u < 4; ++u) {
-                    const int f{16 * (b >> 1) + 4 * grp + u}, r{16 * (b & 1) + t16};
-                    lines[kLines32 + f * RowBuf<32>::RS + r] = acc[4 * b + u];
-                }
-            }
-        } else {
-            // Block q = quad q.
-            const int row{(grp >> 1) * 16 + t16};
-            const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16, yp + row * kSP, (grp & 1) * 16, sp_swz(row))};
-#pragma unroll
-            for (int q{0}; q < 4; ++q) {
-#pragma unroll
-                for (int u{0}; u < 4; ++u) {
-                    lines[kLines16 + q * RowBuf<16>::BS + (4 * grp + u) * RowBuf<16>::RS + t16] = acc[4 * q + u];
-                }
-            }
-        }
+    // Four consecutive elements e0 .. e0 + 3 (e0 a multiple of 4) of an array.
+    const auto store4 = [](_Float16* dst, int e0, const f4v& c) {
+        const h4v h{static_cast<_Float16>(c[0]), static_cast<_Float16>(c[1]), static_cast<_Float16>(c[2]),
+                    static_cast<_Float16>(c[3])};
+        *reinterpret_cast<h4v*>(dst + cpad(e0)) = h;
     };
-    const auto rows8 = [&]() {
-        // 16 blocks x 8 rows over 128 lanes, all 8 frequencies per lane.
-        const int job{((wu - 2) << 6) | lane};
-        const int b{job >> 3}, r{job & 7};
-        float o[8];
-        const int row{(b >> 2) * 8 + r};
-        dct_line<8, 8>(yp + row * kSP, 0, o, (b & 3) * 8, sp_swz(row));
+    // Plain pieces.  The costs' summation orders are fixed: a DCT8 column's
+    // eight terms in order, then its block's eight columns as a lane tree; a
+    // DCT16 lane's four terms (one column, fy = 4 g ..), then the wave tree;
+    // for the DCT32 the four quadrants' terms of a lane (16 in order, wave 0's
+    // quadrant first), then the wave tree.
+    const auto ex_dct8_costs = [&](const f4v& c8) {
+        // Lane group g holds rows 4 g + u of the quad: rows 0-3 of a block's
+        // column in the even group, 4-7 in the odd one, which takes the even
+        // one's running sums over.
+        float v[4], wq[4], wi[4], d[4], rt[4];
+        bool llf[4];
+        int j, e0;
+        mf_quad_element(lane, 0, 8, j, e0);
 #pragma unroll
-        for (int f{0}; f < 8; ++f) {
-            lines[kLines8 + b * RowBuf<8>::BS + f * RowBuf<8>::RS + r] = o[f];
+        for (int u{0}; u < 4; ++u) {
+            v[u] = c8[u];
+            llf[u] = u == 0 && (lane & 7) == 0 && (grp & 1) == 0;  // the DC
         }
-    };
-    // Column passes: 16 terms per lane on waves 0-1, 8 on waves 2-3; costs
-    // straight from the registers: per lane the sum of its terms in register
-    // order, then the wave tree (DCT32; DCT16 per block) or an 8-lane tree
-    // (DCT8: a block's 64 terms sit in 8 consecutive lanes, one column each).
-    const auto cols_big = [&]() {
-        if (wu == 0) {
-            const v16f acc{mfma_lines<32>(g_tables.basis32 + (16 * (grp >> 1) + t16) * 32,
-                                          &lines[kLines32 + (16 * (grp & 1) + t16) * RowBuf<32>::RS])};
-            float v[16], wq[16], wi[16];
-            int e[16];
-            bool llf[16];
-#pragma unroll
-            for (int b{0}; b < 4; ++b) {
-                const int e0{(16 * (b & 1) + t16) * 32 + 16 * (b >> 1) + 4 * grp};
-                selection_weights4(g_tables.wsel32, g_tables.wsel_inv32, e0, 4 * b, wq, wi);
-#pragma unroll
-                for (int u{0}; u < 4; ++u) {
-                    e[4 * b + u] = e0 + u;
-                    v[4 * b + u] = acc[4 * b + u];
-                    llf[4 * b + u] = b == 0 && lane < 4;  // fx, fy < 4
-                }
-            }
-            selection_terms(v, llf, wq, wi, prm, td, tr);
-#pragma unroll
-            for (int i{0}; i < 16; ++i) {
-                coefy_of(S, 2)[cpad(e[i])] = static_cast<_Float16>(v[i]);
-            }
-            float ad{td[0]}, ar{tr[0]};
-#pragma unroll
-            for (int i{1}; i < 16; ++i) {
-                ad += td[i];
-                ar += tr[i];
-            }
-            const float sums{wave_sum4(ad, ar, 0.0f, 0.0f)};  // lanes 0, 32
-            const float rs{lane_value(sums, 32)};
-            if (lane == 0) {
-                S.cost32 = 1024.0f * sums + 6.0e-4f * rs;
-            }
-        } else {
-            const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16,
-                                          &lines[kLines16 + grp * RowBuf<16>::BS + t16 * RowBuf<16>::RS])};
-            // Frequency (t16, 4 grp + u) in each of the four blocks.
-            const int e0{t16 * 16 + 4 * grp};
-            float w4[4], wi4[4];
-            selection_weights4(g_tables.wsel16, g_tables.wsel_inv16, e0, 0, w4, wi4);
-            float v[16], wq[16], wi[16];
-            int e[16];
-            bool llf[16];
-#pragma unroll
-            for (int i{0}; i < 16; ++i) {
-                e[i] = e0 + (i & 3);
-                v[i] = acc[i];
-                wq[i] = w4[i & 3];
-                wi[i] = wi4[i & 3];
-                llf[i] = lane < 2 && (i & 3) < 2;  // fx, fy < 2
-            }
-            selection_terms(v, llf, wq, wi, prm, td, tr);
-#pragma unroll
-            for (int i{0}; i < 16; ++i) {
-                coefy_of(S, 1)[cpad(256 * (i >> 2) + e[i])] = static_cast<_Float16>(v[i]);
-            }
-            float ad[4], ar[4];
-#pragma unroll
-            for (int q{0}; q < 4; ++q) {
-                ad[q] = td[4 * q];
-                ar[q] = tr[4 * q];
-#pragma unroll
-                for (int u{1}; u < 4; ++u) {
-                    ad[q] += td[4 * q + u];
-                    ar[q] += tr[4 * q + u];
-                }
-            }
-#pragma unroll
-            for (int h{0}; h < 2; ++h) {
-                // Quads 2h (lanes 0, 32) and 2h + 1 (lanes 16, 48).
-                const float sums{wave_sum4(ad[2 * h], ar[2 * h], ad[2 * h + 1], ar[2 * h + 1])};
-                const float d1{lane_value(sums, 16)}, r0{lane_value(sums, 32)}, r1{lane_value(sums, 48)};
-                if (lane == 0) {
-                    S.cost16[2 * h] = 256.0f * sums + 6.0e-4f * r0;
-                    S.cost16[2 * h + 1] = 256.0f * d1 + 6.0e-4f * r1;
-                }
-            }
-        }
-    };
-    const auto cols8 = [&]() {
-        const int job{((wu - 2) << 6) | lane};
-        const int b{job >> 3}, fx{job & 7};
-        const int bx{b & 3}, by{b >> 2};
-        const int base{256 * ((by >> 1) * 2 + (bx >> 1)) + 64 * ((by & 1) * 2 + (bx & 1))};
-        float o[8];
-        dct_line<8, 8>(&lines[kLines8 + b * RowBuf<8>::BS + fx * RowBuf<8>::RS], 0, o);
-        {
-            float wq[8], wi[8], d8[8], r8[8];
-            int e[8];
-            bool llf[8];
-            selection_weights4(g_tables.wsel8, g_tables.wsel_inv8, fx * 8, 0, wq, wi);
-            selection_weights4(g_tables.wsel8, g_tables.wsel_inv8, fx * 8 + 4, 4, wq, wi);
-#pragma unroll
-            for (int f{0}; f < 8; ++f) {
-                e[f] = fx * 8 + f;
-                llf[f] = f == 0 && fx == 0;  // the DC
-            }
-            selection_terms(o, llf, wq, wi, prm, d8, r8);
-#pragma unroll
-            for (int f{0}; f < 8; ++f) {
-                td[f] = d8[f];
-                tr[f] = r8[f];
-                coefy_of(S, 0)[cpad(base + e[f])] = static_cast<_Float16>(o[f]);
-            }
-        }
-        float ad{td[0]}, ar{tr[0]};
-#pragma unroll
-        for (int f{1}; f < 8; ++f) {
-            ad += td[f];
-            ar += tr[f];
-        }
-        float fv{0.0f}, fg{0.0f};
-        if (want_features) {
-#pragma unroll
-            for (int f{0}; f < 8; ++f) {
-                const float c2{o[f] * o[f]};
-                fv += (fx | f) != 0 ? c2 : 0.0f;
-                fg = __builtin_fmaf(grad_weight(fx) + grad_weight(f), c2, fg);
-            }
-        }
+        selection_weights4(g_tables.wsel8, g_tables.wsel_inv8, e0, 0, wq, wi);
+        selection_terms(v, llf, wq, wi, prm, d, rt);
+        store4(coefy_of(S, 0), 256 * wu + 64 * j + e0, c8);
+        const auto column = [&](const float (&x)[4]) {
+            const float top{((x[0] + x[1]) + x[2]) + x[3]};
+            return (((from_row_above(top) + x[0]) + x[1]) + x[2]) + x[3];  // in the odd groups
+        };
         const auto sum8 = [](float x) { return add_down_row<1>(add_down_row<2>(add_down_row<4>(x))); };
-        ad = sum8(ad);
-        ar = sum8(ar);
+        const float ad{sum8(column(d))}, ar{sum8(column(rt))};
+        float fv{0.0f}, fg{0.0f}, dc{0.0f};
         if (want_features) {
+            float c2[4];
+#pragma unroll
+            for (int u{0}; u < 4; ++u) {
+                c2[u] = v[u] * v[u];
+            }
+            const int fx{lane & 7};
+            const auto run = [&](float sv, float sg, float& ov, float& og) {
+#pragma unroll
+                for (int u{0}; u < 4; ++u) {
+                    sv += llf[u] ? 0.0f : c2[u];
+                    sg = __builtin_fmaf(grad_weight(fx) + grad_weight(4 * (grp & 1) + u), c2[u], sg);
+                }
+                ov = sv;
+                og = sg;
+            };
+            float tv, tg;
+            run(0.0f, 0.0f, tv, tg);
+            run(from_row_above(tv), from_row_above(tg), fv, fg);
             fv = sum8(fv);
             fg = sum8(fg);
+            dc = from_row_above(v[0]);
         }
-        if ((lane & 7) == 0) {
-            S.cost8[((by >> 1) * 2 + (bx >> 1)) * 4 + (by & 1) * 2 + (bx & 1)] = 64.0f * ad + 6.0e-4f * ar;
+        if ((lane & 7) == 0 && (grp & 1) != 0) {
+            S.cost8[wu * 4 + j] = 64.0f * ad + 6.0e-4f * ar;
             if (want_features) {
-                feature_store(S, b, fv, fg, ad, ar, o[0]);
+                feature_store(S, (2 * (wu >> 1) + (j >> 1)) * 4 + 2 * (wu & 1) + (j & 1), fv, fg, ad, ar, dc);
             }
+        }
+    };
+    const auto ex_dct16_costs = [&](const f4v& c16) {
+        const int e0{t16 * 16 + 4 * grp};
+        float v[4], wq[4], wi[4], d[4], rt[4];
+        bool llf[4];
+#pragma unroll
+        for (int u{0}; u < 4; ++u) {
+            v[u] = c16[u];
+            llf[u] = u < 2 && lane < 2;  // fx, fy < 2
+        }
+        selection_weights4(g_tables.wsel16, g_tables.wsel_inv16, e0, 0, wq, wi);
+        selection_terms(v, llf, wq, wi, prm, d, rt);
+        const float ad{((d[0] + d[1]) + d[2]) + d[3]}, ar{((rt[0] + rt[1]) + rt[2]) + rt[3]};
+        const float sums{wave_sum4(ad, ar, 0.0f, 0.0f)};  // lanes 0, 32
+        const float rs{lane_value(sums, 32)};
+        if (lane == 0) {
+            S.cost16[wu] = 256.0f * sums + 6.0e-4f * rs;
+        }
+    };
+    const int e32{(qcol + t16) * 32 + qrow + 4 * grp};
+    const auto ex_dct32_terms = [&](const f4v& c32) {
+        float v[4], wq[4], wi[4], d[4], rt[4];
+        bool llf[4];
+#pragma unroll
+        for (int u{0}; u < 4; ++u) {
+            v[u] = c32[u];
+            llf[u] = wu == 0 && lane < 4;  // fx, fy < 4
+        }
+        selection_weights4(g_tables.wsel32, g_tables.wsel_inv32, e32, 0, wq, wi);
+        selection_terms(v, llf, wq, wi, prm, d, rt);
+        *reinterpret_cast<float4*>(S.u.s.t32[0][wu][lane]) = float4{d[0], d[1], d[2], d[3]};
+        *reinterpret_cast<float4*>(S.u.s.t32[1][wu][lane]) = float4{rt[0], rt[1], rt[2], rt[3]};
+    };
+    // Wave 0, after a barrier: the DCT32's cost from the four waves' terms.
+    const auto ex_dct32_cost = [&]() {
+        float s[2];
+#pragma unroll
+        for (int k{0}; k < 2; ++k) {
+#pragma unroll
+            for (int b{0}; b < 4; ++b) {
+                const float4 x{*reinterpret_cast<const float4*>(S.u.s.t32[k][b][lane])};
+                s[k] = b == 0 ? x.x : s[k] + x.x;
+                s[k] += x.y;
+                s[k] += x.z;
+                s[k] += x.w;
+            }
+        }
+        const float sums{wave_sum4(s[0], s[1], 0.0f, 0.0f)};  // lanes 0, 32
+        const float rs{lane_value(sums, 32)};
+        if (lane == 0) {
+            S.cost32 = 1024.0f * sums + 6.0e-4f * rs;
+        }
+        wave_sync();
+    };
+    // The larger candidates: costs, then (every wave has read the Y plane)
+    // their coefficients into its space.
+    const auto ex_big = [&](const f4v& c16, const f4v& c32) {
+        ex_dct16_costs(c16);
+        ex_dct32_terms(c32);
+        __syncthreads();
+        store4(coefy_of(S, 1), 256 * wu + t16 * 16 + 4 * grp, c16);
+        store4(coefy_of(S, 2), e32, c32);
+        if (wu == 0) {
+            ex_dct32_cost();
         }
     };
     // Matrix-core FP16 pieces: wave w transforms quad w as four DCT8s (with
@@ -1382,9 +1410,9 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         }
         selection_weights4(g_tables.wsel8, g_tables.wsel_inv8, e[0], 0, wq, wi);
         selection_terms(v, llf, wq, wi, prm, d, rt);
+        store4(coefy_of(S, 0), 256 * q + 64 * j[0] + e[0], c8);
 #pragma unroll
         for (int u{0}; u < 4; ++u) {
-            coefy_of(S, 0)[cpad(256 * q + 64 * j[u] + e[u])] = static_cast<_Float16>(c8[u]);
             d8 += d[u];
             r8 += rt[u];
             if (want_features) {
@@ -1422,7 +1450,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         __syncthreads();
         float d16{0.0f}, r16{0.0f}, d32{0.0f}, r32{0.0f};
         float v16[4], w16[4], wi16[4], v32[4], w32[4], wi32[4], d[2][4], rt[2][4];
-        int e16[4], e32[4];
+        int e16[4];
         bool llf16[4], llf32[4];
         const int e32_0{(16 * (wu & 1) + t16) * 32 + 16 * (wu >> 1) + 4 * grp};
 #pragma unroll
@@ -1430,7 +1458,6 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
             int j;
             mf_quad_element(lane, u, 16, j, e16[u]);
             v16[u] = c16[u];
-            e32[u] = e32_0 + u;
             v32[u] = c32[0][u];
             llf16[u] = u < 2 && lane < 2;   // fx, fy < 2
             llf32[u] = wu == 0 && lane < 4;  // fx, fy < 4
@@ -1439,12 +1466,12 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         selection_weights4(g_tables.wsel32, g_tables.wsel_inv32, e32_0, 0, w32, wi32);
         selection_terms(v16, llf16, w16, wi16, prm, d[0], rt[0]);
         selection_terms(v32, llf32, w32, wi32, prm, d[1], rt[1]);
+        store4(coefy_of(S, 1), 256 * q + e16[0], c16);
+        store4(coefy_of(S, 2), e32_0, c32[0]);
 #pragma unroll
         for (int u{0}; u < 4; ++u) {
-            coefy_of(S, 1)[cpad(256 * q + e16[u])] = static_cast<_Float16>(c16[u]);
             d16 += d[0][u];
             r16 += rt[0][u];
-            coefy_of(S, 2)[cpad(e32[u])] = static_cast<_Float16>(c32[0][u]);
             d32 += d[1][u];
             r32 += rt[1][u];
         }
@@ -1459,109 +1486,93 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
             S.cost32 = (S.cost32p[0] + S.cost32p[1]) + (S.cost32p[2] + S.cost32p[3]);
         }
     };
-    // The heuristic's decision from the costs (thread 0).
+    // The heuristic's decision from the costs, by wave 0: lane b < 16 decides
+    // the quad of block b (region raster).
     const auto decide = [&]() {
         constexpr float inf{1.0e30f}, eps{1.0e-6f};
         // A forced size (test modes): 1 DCT8, 2 DCT16, 3 DCT32 wherever it fits.
         const std::uint32_t force{(prm.mode & kModeForceMask) >> kModeForceShift};
         const bool fit32{bx0 + 4 <= bw && by0 + 4 <= bh};
         const float c32{fit32 ? S.cost32 : inf};
-        float split{0.0f};
-        int choice[4];
-        for (int q{0}; q < 4; ++q) {
-            const int qx{q & 1}, qy{q >> 1};
-            float sum8{0.0f};
-            bool any8{false};
-            for (int dy{0}; dy < 2; ++dy) {
-                for (int dx{0}; dx < 2; ++dx) {
-                    if (bx0 + 2 * qx + dx < bw && by0 + 2 * qy + dy < bh) {
-                        sum8 += S.cost8[q * 4 + dy * 2 + dx];
-                        any8 = true;
-                    }
-                }
-            }
-            if (!any8) {
-                choice[q] = -1;
-                continue;
-            }
-            const bool fit16{bx0 + 2 * qx + 2 <= bw && by0 + 2 * qy + 2 <= bh};
-            const float c16{fit16 ? S.cost16[q] : inf};
-            if (force != 0 ? (force >= 2 && fit16) : (fit16 && c16 <= sum8 + eps)) {
-                choice[q] = 16;
-                split += c16;
-            } else {
-                choice[q] = 8;
-                split += sum8;
+        const int qx{(lane >> 1) & 1}, qy{(lane >> 3) & 1}, q{2 * qy + qx};
+        float sum8{0.0f};
+        bool any8{false};
+#pragma unroll
+        for (int k{0}; k < 4; ++k) {
+            if (bx0 + 2 * qx + (k & 1) < bw && by0 + 2 * qy + (k >> 1) < bh) {
+                sum8 += S.cost8[q * 4 + k];
+                any8 = true;
             }
         }
+        const bool fit16{bx0 + 2 * qx + 2 <= bw && by0 + 2 * qy + 2 <= bh};
+        const float c16{fit16 ? S.cost16[q] : inf};
+        const bool use16{any8 && (force != 0 ? (force >= 2 && fit16) : (fit16 && c16 <= sum8 + eps))};
+        const float cost{any8 ? (use16 ? c16 : sum8) : 0.0f};
+        // The quads' costs in order (an absent quad adds 0).
+        const float split{((lane_value(cost, 0) + lane_value(cost, 2)) + lane_value(cost, 8)) + lane_value(cost, 10)};
         const bool root32{force != 0 ? (force == 3 && fit32) : (fit32 && c32 <= split + eps)};
-        for (int q{0}; q < 4; ++q) {
-            S.choice[q] = choice[q];
-        }
-        if (root32) {
-            for (int b{0}; b < 16; ++b) {
-                S.acs[b] = b == 0 ? 32 : 0;
+        if (lane < 16) {
+            const bool first{(lane & 5) == 0};  // the quad's first block
+            if (first) {
+                S.choice[q] = any8 ? (use16 ? 16 : 8) : -1;
             }
-        } else {
-            for (int q{0}; q < 4; ++q) {
-                const int ox{2 * (q & 1)}, oy{2 * (q >> 1)};
-                if (choice[q] == 16) {
-                    S.acs[oy * 4 + ox] = 16;
-                    S.acs[oy * 4 + ox + 1] = 0;
-                    S.acs[(oy + 1) * 4 + ox] = 0;
-                    S.acs[(oy + 1) * 4 + ox + 1] = 0;
-                }
-            }
+            S.acs[lane] = root32 ? (lane == 0 ? 32 : 0) : (use16 ? (first ? 16 : 0) : 8);
         }
     };
 
+    [[maybe_unused]] f4v c16{}, c32{};
     if constexpr (!kMf16) {
-        if (wu < 2) {
-            if constexpr (!kLearned) {
-                rows_big();
-            }
+        const float4 b8{*reinterpret_cast<const float4*>(g_tables.ex8[lane])};
+        float p[4];
+        ex_pixels<4>(yp, qrow + t16, qcol, lane, p);
+        if constexpr (kLearned) {
+            ex_dct8_costs(ex_cols(b8, ex_rows(p, b8), f4v{0.0f, 0.0f, 0.0f, 0.0f}));
         } else {
-            rows8();
-        }
-        __syncthreads();
-        CJX_REGION_CUT_AT(7)
-        if (wu >= 2) {
-            cols8();
-        } else if constexpr (!kLearned) {
-            cols_big();
+            const float4 b16{*reinterpret_cast<const float4*>(g_tables.ex16[lane])};
+            const Ex32 a32{ex_basis32(wu >> 1, lane)};
+            f4v t32[2];
+            ex_rows32(yp, ex_basis32(wu & 1, lane), lane, t32);
+            const f4v t8{ex_rows(p, b8)}, r16{ex_rows(p, b16)};
+            const f4v zero{0.0f, 0.0f, 0.0f, 0.0f};
+            c32 = ex_cols32(a32, t32);
+            const f4v c8{ex_cols(b8, t8, zero)};
+            c16 = ex_cols(b16, r16, zero);
+            CJX_REGION_CUT_AT(7)
+            ex_dct8_costs(c8);
+            ex_big(c16, c32);
         }
     } else {
         mf_dct8_costs();
         if constexpr (!kLearned) {
             mf_big();
+            __syncthreads();
         }
     }
-    __syncthreads();
     CJX_REGION_CUT_AT(8)
+    bool fallback{!kLearned};
     if (want_features) {
+        __syncthreads();
         feature_finish(S, tid, bx0, by0, bw, bh);
     }
-    bool fallback{!kLearned};
     if constexpr (kLearned) {
-        fallback = !mlp_decide(S, prm, mlp_regs, lines, tid, bx0, by0, bw, bh);
+        fallback = !mlp_decide(S, prm, mlp_regs, S.u.s.hid, tid, bx0, by0, bw, bh);
         if (fallback) {
             // The heuristic for this region: the larger candidates and the
             // decision from the costs.
             if constexpr (!kMf16) {
-                if (wu < 2) {
-                    rows_big();
-                }
-                __syncthreads();
-                if (wu < 2) {
-                    cols_big();
-                }
+                const float4 b16{*reinterpret_cast<const float4*>(g_tables.ex16[lane])};
+                c16 = ex_quad(yp, qrow, qcol, b16, lane);
+                f4v t32[2];
+                ex_rows32(yp, ex_basis32(wu & 1, lane), lane, t32);
+                c32 = ex_cols32(ex_basis32(wu >> 1, lane), t32);
+                ex_big(c16, c32);
             } else {
                 mf_big();
+                __syncthreads();
             }
-            __syncthreads();
         }
     }
-    if (fallback && tid == 0) {
+    if (fallback && wu == 0) {
         decide();
     }
     __syncthreads();
@@ -1582,246 +1593,123 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
     //    and the CfL partials (frontend_quantize.cu:49-117 on this region).
     const bool need_y{kLearned && !fallback};
     const auto cxb = [&](int ch) { return ch == 0 ? S.p.coef.x : S.p.coef.b; };
-    if constexpr (!kMf16) {
-        const int acs0{__builtin_amdgcn_readfirstlane(S.acs[0])};
-        if (acs0 == 32) {
-            // Waves 0 and 1 transform X and B on the matrix cores (DCT32 as four
-            // 16x16 quadrants), wave 2 Y when it has no coefficients yet.
-            const int ch{wu};
-            float* const cl{lines + ch * RowBuf<32>::BS};
-            const bool active{wu < 2 || (need_y && wu == 2)};
-            if (active) {
-                const int row{16 * (grp & 1) + t16};
-                const v16f acc{mfma_lines<32>(g_tables.basis32 + (16 * (grp >> 1) + t16) * 32,
-                                              plane_of(S, ch == 0 ? 0 : (ch == 1 ? 2 : 1)) + row * kSP, 0,
-                                              sp_swz(row))};
-#pragma unroll
-                for (int b{0}; b < 4; ++b) {
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        cl[(16 * (b >> 1) + 4 * grp + u) * RowBuf<32>::RS + 16 * (b & 1) + t16] = acc[4 * b + u];
-                    }
-                }
-            }
-            __syncthreads();
-            if (active) {
-                const v16f acc{mfma_lines<32>(g_tables.basis32 + (16 * (grp >> 1) + t16) * 32,
-                                              &cl[(16 * (grp & 1) + t16) * RowBuf<32>::RS])};
-                _Float16* const dst{ch < 2 ? cxb(ch) : coefy_of(S, 2)};
-#pragma unroll
-                for (int b{0}; b < 4; ++b) {
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        const int fy{16 * (b >> 1) + 4 * grp + u}, fx{16 * (b & 1) + t16};
-                        dst[cpad(fx * 32 + fy)] = static_cast<_Float16>(acc[4 * b + u]);
-                    }
-                }
-            }
-        } else if (__builtin_amdgcn_readfirstlane(S.acs[2] & S.acs[8] & S.acs[10]) == 16 && acs0 == 16) {
-            // Every quad a DCT16: wave c transforms channel c of the four quads
-            // as one chain (quad q = block q): X, B, then Y when it has no
-            // coefficients yet.
-            constexpr int kChanLines{4 * RowBuf<16>::BS};
-            static_assert(3 * kChanLines <= kScratch, "channel lines");
-            const int nch{need_y ? 3 : 2};
-            float* const cl{lines + wu * kChanLines};
-            const int plane{wu == 0 ? 0 : (wu == 1 ? 2 : 1)};
-            if (wu < nch) {
-                const int row{(grp >> 1) * 16 + t16};
-                const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16, plane_of(S, plane) + row * kSP,
-                                              (grp & 1) * 16, sp_swz(row))};
-#pragma unroll
-                for (int q{0}; q < 4; ++q) {
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        cl[q * RowBuf<16>::BS + (4 * grp + u) * RowBuf<16>::RS + t16] = acc[4 * q + u];
-                    }
-                }
-            }
-            __syncthreads();
-            if (wu < nch) {
-                const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16,
-                                              &cl[grp * RowBuf<16>::BS + t16 * RowBuf<16>::RS])};
-                _Float16* const dst{wu < 2 ? cxb(wu) : coefy_of(S, 1)};
-#pragma unroll
-                for (int q{0}; q < 4; ++q) {
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        dst[cpad(256 * q + t16 * 16 + 4 * grp + u)] = static_cast<_Float16>(acc[4 * q + u]);
-                    }
-                }
-            }
+    // Results stay in registers until every wave has read the planes, whose
+    // space then takes their coefficients.
+    const int acs0{__builtin_amdgcn_readfirstlane(S.acs[0])};
+    const auto dct32 = [&](const float* plane, int fxb, f4v (&c)[2]) {
+        if constexpr (kMf16) {
+            mf_dct32(plane, 16 * fxb, 0, true, lane, c);
         } else {
-            // Wave w transforms quad w: one DCT16 on the matrix cores (block 0 =
-            // X, block 1 = B, block 2 = Y when it has no coefficients yet, else
-            // unused; block 3 unused) or four DCT8s on the VALU (lanes:
-            // channel, block, row).
-            constexpr int kQuadLines{3 * RowBuf<16>::BS};
-            static_assert(kQuadLines >= 2 * 4 * RowBuf<8>::BS && 4 * kQuadLines <= kScratch, "quad lines");
-            float* const ql{lines + wu * kQuadLines};
-            const int q{wu};
-            const int n16{__builtin_amdgcn_readfirstlane(S.acs[(q >> 1) * 8 + (q & 1) * 2])};
-            // Block grp's plane: X, B, then Y (or X again), B again; the
-            // results of repeated blocks are dropped.
-            const int ch16{grp == 2 ? (need_y ? 1 : 0) : (grp & 1) * 2};
-            if (n16 == 16) {
-                const int row{(q >> 1) * 16 + t16};
-                const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16, plane_of(S, ch16) + row * kSP,
-                                              (q & 1) * 16, sp_swz(row))};
-#pragma unroll
-                for (int b{0}; b < 3; ++b) {
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        ql[b * RowBuf<16>::BS + (4 * grp + u) * RowBuf<16>::RS + t16] = acc[4 * b + u];
-                    }
-                }
-            } else {
-                const int ch{lane >> 5}, j{(lane >> 3) & 3}, r{lane & 7};
-                const int bx{2 * (q & 1) + (j & 1)}, by{2 * (q >> 1) + (j >> 1)};
-                float o[8];
-                const int row{by * 8 + r};
-                dct_line<8, 8>(plane_of(S, 2 * ch) + row * kSP, 0, o, bx * 8, sp_swz(row));
-#pragma unroll
-                for (int f{0}; f < 8; ++f) {
-                    ql[(ch * 4 + j) * RowBuf<8>::BS + f * RowBuf<8>::RS + r] = o[f];
-                }
-            }
-            __syncthreads();
-            if (n16 == 16) {
-                const v16f acc{mfma_lines<16>(g_tables.basis16 + t16 * 16,
-                                              &ql[(grp < 3 ? grp : 1) * RowBuf<16>::BS + t16 * RowBuf<16>::RS])};
-#pragma unroll
-                for (int b{0}; b < 3; ++b) {
-                    if (b == 2 && !need_y) {
-                        break;
-                    }
-                    _Float16* const dst{b < 2 ? cxb(b) : coefy_of(S, 1)};
-#pragma unroll
-                    for (int u{0}; u < 4; ++u) {
-                        dst[cpad(256 * q + t16 * 16 + 4 * grp + u)] = static_cast<_Float16>(acc[4 * b + u]);
-                    }
-                }
-            } else {
-                const int ch{lane >> 5}, j{(lane >> 3) & 3}, fx{lane & 7};
-                float o[8];
-                dct_line<8, 8>(&ql[(ch * 4 + j) * RowBuf<8>::BS + fx * RowBuf<8>::RS], 0, o);
-#pragma unroll
-                for (int f{0}; f < 8; ++f) {
-                    cxb(ch)[cpad(256 * q + 64 * j + fx * 8 + f)] = static_cast<_Float16>(o[f]);
-                }
-            }
+            ex_dct32(plane, fxb, lane, c);
+        }
+    };
+    if (acs0 == 32) {
+        // Wave w: channel w % 2 (X, B), horizontal frequencies 16 (w / 2)..;
+        // waves 0-1 also Y's half w when it has no coefficients yet.
+        const int ch{wu & 1}, fxb{wu >> 1};
+        f4v c[2], cy[2];
+        dct32(plane_of(S, 2 * ch), fxb, c);
+        if (need_y && wu < 2) {
+            dct32(plane_of(S, 1), wu, cy);
         }
         __syncthreads();
-    } else {
-        // Matrix-core FP16 form; results in registers until every wave has
-        // read the planes, whose space then takes their coefficients.
-        const int acs0{__builtin_amdgcn_readfirstlane(S.acs[0])};
-        if (acs0 == 32) {
-            // Wave w: channel w % 2 (X, B), horizontal frequencies 16 (w / 2)..;
-            // waves 0-1 also Y's half w when it has no coefficients yet.
-            const int ch{wu & 1}, fx0{16 * (wu >> 1)};
-            f4v c[2], cy[2];
-            mf_dct32(plane_of(S, 2 * ch), fx0, 0, true, lane, c);
+#pragma unroll
+        for (int o{0}; o < 2; ++o) {
+            store4(cxb(ch), (16 * fxb + t16) * 32 + 16 * o + 4 * grp, c[o]);
             if (need_y && wu < 2) {
-                mf_dct32(plane_of(S, 1), 16 * wu, 0, true, lane, cy);
+                store4(coefy_of(S, 2), (16 * wu + t16) * 32 + 16 * o + 4 * grp, cy[o]);
             }
-            __syncthreads();
-#pragma unroll
-            for (int o{0}; o < 2; ++o) {
-#pragma unroll
-                for (int u{0}; u < 4; ++u) {
-                    const int fy{16 * o + 4 * grp + u}, fx{fx0 + t16};
-                    cxb(ch)[cpad(fx * 32 + fy)] = static_cast<_Float16>(c[o][u]);
-                    if (need_y && wu < 2) {
-                        const int fxy{16 * wu + t16};
-                        coefy_of(S, 2)[cpad(fxy * 32 + fy)] = static_cast<_Float16>(cy[o][u]);
-                    }
-                }
-            }
-        } else {
-            // Wave w transforms quad w of X and B (and of Y, when it has no
-            // coefficients yet and takes a DCT16): one DCT16 or four DCT8s.
-            const int q{wu};
-            const int n16{__builtin_amdgcn_readfirstlane(S.acs[(q >> 1) * 8 + (q & 1) * 2])};
-            const int n{n16 == 16 ? 16 : 8};
+        }
+    } else {
+        // Wave w transforms quad w of X and B (and of Y, when it has no
+        // coefficients yet and takes a DCT16): one DCT16 or four DCT8s.
+        const int q{wu};
+        const int n{__builtin_amdgcn_readfirstlane(S.acs[(q >> 1) * 8 + (q & 1) * 2]) == 16 ? 16 : 8};
+        const bool y16{need_y && n == 16};
+        f4v cx, cb, cy{};
+        if constexpr (kMf16) {
             const std::uint16_t* hi{n == 16 ? g_tables.mf16[0] : g_tables.mf8[0]};
             const std::uint16_t* lo{n == 16 ? g_tables.mf16[1] : g_tables.mf8[1]};
-            const int qr{(q >> 1) * 16}, qc{(q & 1) * 16};
-            const f4v cx{mf_quad(plane_of(S, 0), qr, qc, hi, lo, lane)};
-            const f4v cb{mf_quad(plane_of(S, 2), qr, qc, hi, lo, lane)};
-            const bool y16{need_y && n == 16};
-            f4v cy{};
+            cx = mf_quad(plane_of(S, 0), qrow, qcol, hi, lo, lane);
+            cb = mf_quad(plane_of(S, 2), qrow, qcol, hi, lo, lane);
             if (y16) {
-                cy = mf_quad(plane_of(S, 1), qr, qc, hi, lo, lane);
+                cy = mf_quad(plane_of(S, 1), qrow, qcol, hi, lo, lane);
             }
-            __syncthreads();
-#pragma unroll
-            for (int u{0}; u < 4; ++u) {
-                int j, e;
-                mf_quad_element(lane, u, n, j, e);
-                cxb(0)[cpad(256 * q + 64 * j + e)] = static_cast<_Float16>(cx[u]);
-                cxb(1)[cpad(256 * q + 64 * j + e)] = static_cast<_Float16>(cb[u]);
-                if (y16) {
-                    coefy_of(S, 1)[cpad(256 * q + e)] = static_cast<_Float16>(cy[u]);
-                }
+        } else {
+            const float4 b{*reinterpret_cast<const float4*>(n == 16 ? g_tables.ex16[lane] : g_tables.ex8[lane])};
+            cx = ex_quad(plane_of(S, 0), qrow, qcol, b, lane);
+            cb = ex_quad(plane_of(S, 2), qrow, qcol, b, lane);
+            if (y16) {
+                cy = ex_quad(plane_of(S, 1), qrow, qcol, b, lane);
             }
         }
         __syncthreads();
+        int j, e;
+        mf_quad_element(lane, 0, n, j, e);
+        store4(cxb(0), 256 * q + 64 * j + e, cx);
+        store4(cxb(1), 256 * q + 64 * j + e, cb);
+        if (y16) {
+            store4(coefy_of(S, 1), 256 * q + e, cy);
+        }
     }
+    __syncthreads();
 
     CJX_REGION_CUT_AT(5)
+    // Lane l takes coefficients 4 (l % 16) .. + 3 of block k = l / 16 of the
+    // wave's four blocks, (2 (k % 2) + w % 2, 2 (k / 2) + w / 2): one 8-byte
+    // LDS read and one 8-byte store per plane.
     const std::size_t cplane{static_cast<std::size_t>(geo.nblocks) * 64};
-    float acc[3]{0.0f, 0.0f, 0.0f};
-    // Wave w writes blocks (2 (k % 2) + w % 2, 2 (k / 2) + w / 2), k = 0..3,
-    // one coefficient per lane; the block's transform and slot are
-    // wave-uniform (scalar registers).
-    const int acs_root{__builtin_amdgcn_readfirstlane(S.acs[0])};
-#pragma unroll
-    for (int k{0}; k < 4; ++k) {
+    float v[3][4];
+    {
+        const int k{grp}, s4{4 * t16};
         const int bxl{2 * (k & 1) + (wu & 1)}, byl{2 * (k >> 1) + (wu >> 1)};
-        int n{8}, ox{bxl}, oy{byl};
-        if (acs_root == 32) {
-            n = 32;
-            ox = 0;
-            oy = 0;
-        } else if (__builtin_amdgcn_readfirstlane(S.acs[(byl & ~1) * 4 + (bxl & ~1)]) == 16) {
-            n = 16;
-            ox = bxl & ~1;
-            oy = byl & ~1;
+        const bool is32{acs0 == 32};
+        const int n{is32 ? 32 : (S.acs[(byl & ~1) * 4 + (bxl & ~1)] == 16 ? 16 : 8)};
+        const int qc{is32 ? byl * 4 + bxl : (n == 16 ? wu : 0)};
+        const int e{qc * 64 + s4};
+        const int idx{cpad(is32 ? e : 256 * k + 64 * wu + s4)};
+        const h4v hx{*reinterpret_cast<const h4v*>(cxb(0) + idx)};
+        const h4v hy{*reinterpret_cast<const h4v*>((n == 8 ? S.coefy8 : coefy_of(S, is32 ? 2 : 1)) + idx)};
+        const h4v hb{*reinterpret_cast<const h4v*>(cxb(1) + idx)};
+        const bool in{bx0 + bxl < bw && by0 + byl < bh};
+        if (in) {
+            std::uint16_t* const out{coeffs + (static_cast<std::size_t>(by0 + byl) * bw + bx0 + bxl) * 64 + s4};
+            *reinterpret_cast<h4v*>(out) = hx;
+            *reinterpret_cast<h4v*>(out + cplane) = hy;
+            *reinterpret_cast<h4v*>(out + 2 * cplane) = hb;
         }
-        const int qc{(byl - oy) * (n / 8) + (bxl - ox)};
-        const int e{qc * 64 + lane};
-        const int idx{n == 32 ? e : 256 * k + 64 * wu + lane};
-        const int sz{n == 32 ? 2 : (n == 16 ? 1 : 0)};
-        const _Float16 hx{cxb(0)[cpad(idx)]};
-        const _Float16 hy{coefy_of(S, sz)[cpad(idx)]};
-        const _Float16 hb{cxb(1)[cpad(idx)]};
-        float v[3]{0.0f, 0.0f, 0.0f};
-        if (bx0 + bxl < bw && by0 + byl < bh) {
-            std::uint16_t* const out{coeffs + (static_cast<std::size_t>(by0 + byl) * bw + bx0 + bxl) * 64};
-            out[lane] = __builtin_bit_cast(std::uint16_t, hx);
-            out[cplane + lane] = __builtin_bit_cast(std::uint16_t, hy);
-            out[2 * cplane + lane] = __builtin_bit_cast(std::uint16_t, hb);
-            if (!is_llf(e, n)) {
-                const float xr{static_cast<float>(hx)}, yr{static_cast<float>(hy)};
-                const float br{static_cast<float>(hb)};
-                v[0] = xr * yr;
-                v[1] = yr * yr;
-                v[2] = (br - yr) * yr;
-            }
-        }
+        // CfL terms; 0 for the LLF coefficients (the first m of the four
+        // where a row fx < m of the transform starts) and outside the frame.
+        const int m{n >> 3};
+        const int nllf{in ? ((e & (n - 1)) == 0 && e < m * n ? m : 0) : 4};
 #pragma unroll
-        for (int c{0}; c < 3; ++c) {
-            acc[c] = k == 0 ? v[c] : acc[c] + v[c];
+        for (int i{0}; i < 4; ++i) {
+            const float xr{static_cast<float>(hx[i])}, yr{static_cast<float>(hy[i])}, br{static_cast<float>(hb[i])};
+            const bool use{i >= nllf};
+            v[0][i] = use ? xr * yr : 0.0f;
+            v[1][i] = use ? yr * yr : 0.0f;
+            v[2][i] = use ? (br - yr) * yr : 0.0f;
         }
     }
+    // Slot by slot the four blocks in order, then the tree over the 64 slots
+    // (offsets 32 .. 1): after the turn, register k of lane group g holds
+    // slot 4 (l % 16) + g of block k.
     {
-        const float sums{wave_sum4(acc[0], acc[1], acc[2], 0.0f)};  // lanes 0, 32, 16
-        const float s1{lane_value(sums, 32)}, s2{lane_value(sums, 16)};
+        float sum[3];
+#pragma unroll
+        for (int c{0}; c < 3; ++c) {
+            ex_turn(v[c]);
+            float x{((v[c][0] + v[c][1]) + v[c][2]) + v[c][3]};
+            x = add_down_row<8>(x);
+            x = add_down_row<4>(x);
+            x = add_down_row<2>(x);
+            x = add_down_row<1>(x);
+            sum[c] = add_down_16(add_down_32(x));
+        }
         if (lane == 0) {
-            S.cfl[wu][0] = sums;
-            S.cfl[wu][1] = s1;
-            S.cfl[wu][2] = s2;
+            S.cfl[wu][0] = sum[0];
+            S.cfl[wu][1] = sum[1];
+            S.cfl[wu][2] = sum[2];
         }
     }
     __syncthreads();
@@ -2165,7 +2053,7 @@ __global__ __launch_bounds__(256) void dct8_uniform_kernel(
     gaborish_tile(S, tid);
     __syncthreads();
 
-    float* const lines{S.u.scratch};                                     // 16 blocks x RowBuf<8>
+    float* const lines{S.u.scratch};                                     // 16 blocks x RowBuf8
     std::int32_t* const qy{reinterpret_cast<std::int32_t*>(S.u.scratch + 2048)};  // Y's quantized values
     const float ac_scale{prm.qgsf_select};
     const float dcq[3]{4096.0f * prm.dc_scale, 512.0f * prm.dc_scale, 256.0f * prm.dc_scale};
@@ -2181,13 +2069,13 @@ __global__ __launch_bounds__(256) void dct8_uniform_kernel(
             dct_line<8, 8>(plane_of(S, c) + row * kSP, 0, o, (b & 3) * 8, sp_swz(row));
 #pragma unroll
             for (int f{0}; f < 8; ++f) {
-                lines[b * RowBuf<8>::BS + f * RowBuf<8>::RS + sub] = o[f];
+                lines[b * RowBuf8::BS + f * RowBuf8::RS + sub] = o[f];
             }
         }
         __syncthreads();
         if (tid < 128) {
             float o[8];
-            dct_line<8, 8>(&lines[b * RowBuf<8>::BS + sub * RowBuf<8>::RS], 0, o);
+            dct_line<8, 8>(&lines[b * RowBuf8::BS + sub * RowBuf8::RS], 0, o);
 #pragma unroll
             for (int f{0}; f < 8; ++f) {
                 const int e{sub * 8 + f};

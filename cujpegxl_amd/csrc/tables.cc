@@ -171,6 +171,17 @@ DeviceTables build_tables() {
         split_f16(bd, 256, t.mf8[0], t.mf8[1]);
         split_f16(t.basis16, 256, t.mf16[0], t.mf16[1]);
         split_f16(t.basis32, 1024, t.mf32[0], t.mf32[1]);
+        for (int l{0}; l < 64; ++l) {
+            for (int k{0}; k < 8; ++k) {
+                const int c{4 * k + l / 16};
+                if (k < 4) {
+                    t.ex8[l][k] = bd[(l % 16) * 16 + c];
+                    t.ex16[l][k] = t.basis16[(l % 16) * 16 + c];
+                }
+                t.ex32[0][l][k] = t.basis32[(l % 16) * 32 + c];
+                t.ex32[1][l][k] = t.basis32[(16 + l % 16) * 32 + c];
+            }
+        }
     }
     xyb_power_table(t.xyb_tab);
     t.rate[0] = 0.0f;
