@@ -227,7 +227,7 @@ bool BatchEncoder::set_shape(const BatchShape& shape) {
 
 // Coordinate search: the tokenizer and assembly shapes with one workgroup per
 // region first, then the region stage's persistent grids with the best of
-// those (one and two resident rounds of five workgroups per CU).
+// those (one and two resident rounds of six workgroups per CU).
 bool BatchEncoder::tune(int reps, std::string* report) {
     if (!inputs_set_ || reps <= 0) {
         return false;
@@ -238,7 +238,7 @@ bool BatchEncoder::tune(int reps, std::string* report) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device_) != hipSuccess || cus <= 0) {
         cus = 256;
     }
-    const std::uint32_t resident{static_cast<std::uint32_t>(5 * cus) & ~7u};
+    const std::uint32_t resident{static_cast<std::uint32_t>(6 * cus) & ~7u};
     const std::uint32_t kRegionGrids[]{resident, 2 * resident};
     BatchShape best{shape_};
     double best_s{1e30};

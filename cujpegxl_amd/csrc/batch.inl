@@ -32,7 +32,7 @@ __device__ __forceinline__ const FrameJob& batch_job(const FrameJob* __restrict_
 }
 
 template <bool kMf16, bool kLearned>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void region_batch_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void region_batch_kernel(
     const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBRegion, wg)};
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void r
 // contiguous runs of regions per XCD.  Every workgroup leaves once its
 // XCD's share is claimed; no workgroup waits for another.
 template <bool kMf16, bool kLearned>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void region_persistent_batch_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void region_persistent_batch_kernel(
     const FrameJob* __restrict__ jobs, int count, std::uint32_t total, std::uint32_t* __restrict__ counters) {
     __shared__ std::uint32_t claimed;
     const std::uint32_t x{blockIdx.x & 7u};

@@ -106,9 +106,15 @@ __device__ __forceinline__ float clamp01(float v) {
 }
 
 // xyb_impl.cuh:37-70 on the shared numeric primitives (the powers from the
-// table at `tab`, staged in LDS).
+// table at `tab`, staged in LDS).  Both branches are evaluated (the power at
+// the threshold where the line is taken, which keeps its table index in
+// range): a pixel's three curves then overlap instead of waiting for their
+// table reads one after another in divergent branches (region kernel 159 ->
+// 156 us at 3840x2160).
 __device__ __forceinline__ float srgb_to_linear(float e, const float2* tab) {
-    return e <= 0.04045f ? e * (1.0f / 12.92f) : pow24_tab((e + 0.055f) * (1.0f / 1.055f), tab);
+    const float line{e * (1.0f / 12.92f)};
+    const float curve{pow24_tab((fmaxf(e, 0.04045f) + 0.055f) * (1.0f / 1.055f), tab)};
+    return e <= 0.04045f ? line : curve;
 }
 
 // Opsin absorbance bias of the XYB transform.
@@ -340,45 +346,47 @@ __device__ __forceinline__ int cpad(int e) {
 }
 
 // Arrays whose lifetimes do not overlap share storage, which keeps the
-// workgroup under 32 KB of LDS (five resident workgroups per CU):
-// - steps 1-3: the XYB tile, then the AQ terms (step 3) past its end;
-//   step 4: the DCT32's selection terms, the features, the network's hidden
-//   units;
-// - the powers' table and the chroma window in step 1, then the
-//   sharpened planes, from step 2 until their last row pass (Y in
-//   step 4, X and B in step 5); each plane's space then holds coefficients:
-//   X's and B's the chosen transforms (step 5 on), Y's (the last plane, and
-//   512 bytes past it) the DCT16 and DCT32 candidates (step 4 on).  The DCT8
-//   candidates of Y have their own array.
-constexpr int kPlaneHalfs = 2 * 32 * kSP;
-static_assert(kCoefPadded <= kPlaneHalfs, "a coefficient array per plane");
+// workgroup at 23.5 KB of LDS: six resident workgroups per CU (80 VGPRs, no
+// spill).  With a space of their own for the sharpened planes it was 31.7 KB
+// and five per CU, and the kernel took 164 us at 3840x2160 (138 learned +
+// FP16) instead of 159 (134):
+// - `a`: the XYB tile until every thread has read it (its sharpened pixels
+//   wait in registers), then the sharpened planes X, B, Y; Y's space and the
+//   rest past it take the DCT32's selection terms once Y has been
+//   transformed, then X's and B's coefficients of the chosen transforms.
+// - `b`: the powers' table and the chroma window of step 1, then the AQ terms
+//   (steps 2-3), then Y's coefficients of the three candidate sizes, the
+//   features and the network's hidden units.
+struct AqTerms {
+    float cells[64];
+    float ero[64];     // fuzzy erosion of each cell
+    float blk[16][3];  // per block: HF sum, gamma, blue sum
+};
 
 struct RegionShared {
     union {
+        alignas(16) float xyb[3][kTileW * kTileW];  // NV12 -> XYB tile with halo
+        float sharp[3][32 * kSP];
         struct {
-            float xyb[3][kTileW * kTileW];  // NV12 -> XYB tile with halo (steps 1-3)
-            struct {
-                float cells[64];
-                float ero[64];     // fuzzy erosion of each cell
-                float blk[16][3];  // per block: HF sum, gamma, blue sum
-            } aq;                  // AQ terms (step 3)
-        } f;
-        struct {
-            float t32[2][4][64][4];  // DCT32 terms (errors, rates) of each wave's quadrant
-            float feat[112];         // network features (block sums first; learned mode and export)
-            float hid[72];           // the network's hidden units and outputs
-        } s;                         // step 4
-        float scratch[3072];  // dct8_uniform_kernel: row-pass lines, then Y's quantized values
-    } u;
+            float planes[2][32 * kSP];  // X and B
+            union {
+                float t32[2][3][64][4];  // DCT32 terms (errors, rates) of waves 1-3's quadrants
+                _Float16 xb[2][kCoefPadded];
+            } y;
+        } after;
+    } a;
     union {
-        alignas(16) float sharp[3][32 * kSP];
         struct {
-            _Float16 x[kPlaneHalfs];      // X coefficients of the chosen transforms (cpad)
-            _Float16 b[kPlaneHalfs];      // B coefficients of the chosen transforms
-            _Float16 y[2 * kCoefPadded];  // Y coefficients of the DCT16 candidates, then the DCT32 candidate
-        } coef;
-    } p;
-    _Float16 coefy8[kCoefPadded];  // Y coefficients of the DCT8 candidates
+            float2 tab[kXybTabPairs];
+            std::uint32_t win[kChromaW * kChromaW];
+        } in;
+        AqTerms aq;
+        struct {
+            _Float16 y[3][kCoefPadded];  // DCT8, DCT16 and DCT32 candidates
+            float feat[112];             // network features (block sums first; learned mode and export)
+            float hid[72];               // the network's hidden units and outputs
+        } s;
+    } b;
     float cost8[16];       // quad-major
     float cost16[4];
     float cost32;
@@ -389,18 +397,19 @@ struct RegionShared {
     int choice[4];         // the heuristic's choice per quad (export)
     int learned_ok;        // the network's decision was confident
 };
-// LDS is allocated in 1,280-byte blocks: five workgroups per CU (160 KB)
-// need at most 25 blocks each.
-static_assert(sizeof(RegionShared) <= 25 * 1280, "five workgroups per CU");
+// LDS is allocated in 1,280-byte blocks: six workgroups per CU (160 KB) need
+// at most 21 blocks each.
+static_assert(sizeof(RegionShared) <= 21 * 1280, "six workgroups per CU");
+static_assert(offsetof(RegionShared, b) == sizeof(float) * 3 * kTileW * kTileW, "the XYB tile is the largest use of a");
 
 // Sharpened plane of channel c (0 X, 1 Y, 2 B).
 __device__ __forceinline__ float* plane_of(RegionShared& S, int c) {
-    return S.p.sharp[c == 0 ? 0 : (c == 1 ? 2 : 1)];
+    return S.a.sharp[c == 0 ? 0 : (c == 1 ? 2 : 1)];
 }
 
 // Y coefficients of candidate size 8 << sz, element order (cpad).
 __device__ __forceinline__ _Float16* coefy_of(RegionShared& S, int sz) {
-    return sz == 0 ? S.coefy8 : S.p.coef.y + (sz - 1) * kCoefPadded;
+    return S.b.s.y[sz];
 }
 
 // True for the lowest (n/8)^2 frequencies (fx, fy < n/8) of element
@@ -527,10 +536,9 @@ __device__ __forceinline__ void xyb_tile(RegionShared& S, const std::uint8_t* lu
     // The powers' table, then the tile's chroma window: samples
     // (cx0 + j, cy0 + i), clamped to the plane, Cb in the low half-word and
     // Cr in the high one.  Every tap of the tile's pixels (their coordinates
-    // clamped to the frame, the taps to the plane) lands in the window.  Both
-    // live in the sharpened planes' space, which is free until step 2.
-    float2* const tab{reinterpret_cast<float2*>(&S.p.sharp[0][0])};
-    std::uint32_t* const win{reinterpret_cast<std::uint32_t*>(&S.p.sharp[0][0]) + 2 * kXybTabPairs};
+    // clamped to the frame, the taps to the plane) lands in the window.
+    float2* const tab{S.b.in.tab};
+    std::uint32_t* const win{S.b.in.win};
     const int cw{W / 2}, ch{H / 2};
     const int cx0{(px0 >> 1) - 2}, cy0{(py0 >> 1) - 2};
     for (int i{tid}; i < kChromaW * kChromaW; i += 256) {
@@ -583,28 +591,27 @@ __device__ __forceinline__ void xyb_tile(RegionShared& S, const std::uint8_t* lu
             const float yv{static_cast<float>(lcur) * (1.0f / 255.0f)};
             const float cb{static_cast<float>(v & 0xffffu) * kScale - 128.0f / 255.0f};
             const float cr{static_cast<float>(v >> 16) * kScale - 128.0f / 255.0f};
-            pixel_to_xyb(yv, cb, cr, S.u.f.xyb[0][i], S.u.f.xyb[1][i], S.u.f.xyb[2][i], tab, neg_cbrt_bias);
+            pixel_to_xyb(yv, cb, cr, S.a.xyb[0][i], S.a.xyb[1][i], S.a.xyb[2][i], tab, neg_cbrt_bias);
             gy = gy_next;
         }
     }
 }
 
-// Step 2: inverse gaborish of the three channels into the sharpened planes
-// (gaborish.h:16-28; tap order frontend_transform.cu:30-48).
-__device__ __forceinline__ void gaborish_tile(RegionShared& S, int tid) {
+// Step 2: inverse gaborish of the three channels (gaborish.h:16-28; tap order
+// frontend_transform.cu:30-48).  Thread (gy, gx) = (tid / 8, tid % 8) returns
+// the four outputs of row gy, columns 4 gx .. 4 gx + 3 of each channel.
+__device__ __forceinline__ void gaborish_tile(const RegionShared& S, int tid, float4 (&out)[3]) {
     constexpr float k0{-0.09495815671340026f}, k1{-0.041031725066768575f};
     constexpr float k2{0.013710004822696948f}, k3{0.006510206083837737f};
     constexpr float k4{-0.0014789063378272242f};
     constexpr float nm{1.0f / (1.0f + 4.0f * (k0 + k1 + k2 + k4 + 2.0f * k3))};
     constexpr float wc{nm}, wr{nm * k0}, wr2{nm * k2}, wd{nm * k1}, wl{nm * k3}, wd2{nm * k4};
-    // Thread (gy, gx) of each channel: the four outputs of row gy, columns
-    // 4 gx .. 4 gx + 3, from the five input rows gy - 2 .. gy + 2, columns
-    // 4 gx - 2 .. 4 gx + 5 (two aligned 16-byte reads per row; the tile's
-    // row pitch is 36 floats).
+    // From the five input rows gy - 2 .. gy + 2, columns 4 gx - 2 .. 4 gx + 5
+    // (two aligned 16-byte reads per row; the tile's row pitch is 36 floats).
     const int gx{tid & 7}, gy{tid >> 3};
-#pragma unroll 1
+#pragma unroll
     for (int c{0}; c < 3; ++c) {
-        const float* const base{&S.u.f.xyb[c][gy * kTileW + 4 * gx]};
+        const float* const base{&S.a.xyb[c][gy * kTileW + 4 * gx]};
         float r[5][8];
 #pragma unroll
         for (int dy{0}; dy < 5; ++dy) {
@@ -632,7 +639,21 @@ __device__ __forceinline__ void gaborish_tile(RegionShared& S, int tid) {
             o[k] = wc * AT(0, 0) + wr * e + wr2 * r2 + wd * dg + wl * l8 + wd2 * d4;
 #undef AT
         }
-        *reinterpret_cast<float4*>(&plane_of(S, c)[sp_index(gy, 4 * gx)]) = float4{o[0], o[1], o[2], o[3]};
+        out[c] = float4{o[0], o[1], o[2], o[3]};
+        // Computed here: sunk to their use, they would keep all three
+        // channels' inputs (120 registers) alive.
+        asm volatile("" : "+v"(out[c].x), "+v"(out[c].y), "+v"(out[c].z), "+v"(out[c].w));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The outputs into the sharpened planes (every thread has read the XYB tile,
+// whose space they take).
+__device__ __forceinline__ void store_sharp(RegionShared& S, int tid, const float4 (&out)[3]) {
+    const int gx{tid & 7}, gy{tid >> 3};
+#pragma unroll
+    for (int c{0}; c < 3; ++c) {
+        *reinterpret_cast<float4*>(&plane_of(S, c)[sp_index(gy, 4 * gx)]) = out[c];
     }
 }
 
@@ -652,9 +673,9 @@ __device__ __forceinline__ void gaborish_tile(RegionShared& S, int tid) {
 // swaps, no LDS.  A 16 x 16 quad is one tile per pass: a DCT16, or four DCT8s
 // with a block-diagonal basis (a chain's zero steps add +0 to a sum that is
 // never -0).  A DCT32 quadrant takes two row-pass tiles.  Every wave works on
-// one quad and one quadrant.  (Before: K = 1 steps with the DCT32 in wave 0
-// alone, 1,024 clocks a pass, the DCT8s on the VALU, and the row passes
-// through LDS lines; REGION_FIGURES.)
+// one quad and one quadrant.  With K = 1 steps, the DCT32 in wave 0 alone
+// (1,024 clocks a pass), the DCT8s on the VALU and the row passes through LDS
+// lines the region kernel took 179 us at 3840x2160, in this form 164.
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f4v ex_step(float a, float b, f4v acc) {
@@ -940,25 +961,25 @@ __device__ __forceinline__ float grad_weight(int k) {
     return w[k];
 }
 
-// Block b's raw sums (var, grad, dist, rate, mean) into S.u.s.feat[6 b ..]; the
+// Block b's raw sums (var, grad, dist, rate, mean) into S.b.s.feat[6 b ..]; the
 // cost sits in S.cost8.
 __device__ __forceinline__ void feature_store(RegionShared& S, int b, float var, float grad, float dist, float rate,
                                               float mean) {
-    S.u.s.feat[6 * b + 0] = var;
-    S.u.s.feat[6 * b + 1] = grad;
-    S.u.s.feat[6 * b + 3] = dist;
-    S.u.s.feat[6 * b + 4] = rate;
-    S.u.s.feat[6 * b + 5] = mean;
+    S.b.s.feat[6 * b + 0] = var;
+    S.b.s.feat[6 * b + 1] = grad;
+    S.b.s.feat[6 * b + 3] = dist;
+    S.b.s.feat[6 * b + 4] = rate;
+    S.b.s.feat[6 * b + 5] = mean;
 }
 
-// The raw sums -> the 96 features in S.u.s.feat (every thread calls this;
+// The raw sums -> the 96 features in S.b.s.feat (every thread calls this;
 // barriers inside).
 __device__ __forceinline__ void feature_finish(RegionShared& S, int tid, int bx0, int by0, int bw, int bh) {
     float f[6]{};
     if (tid < 16) {
         const int bx{tid & 3}, by{tid >> 2};
         if (bx0 + bx < bw && by0 + by < bh) {
-            const float* s{&S.u.s.feat[6 * tid]};
+            const float* s{&S.b.s.feat[6 * tid]};
             const float c8{S.cost8[((by >> 1) * 2 + (bx >> 1)) * 4 + (by & 1) * 2 + (bx & 1)]};
             f[0] = log2_det(1.0f + 4096.0f * fmaxf(s[0], 0.0f));
             f[1] = log2_det(1.0f + 1024.0f * fmaxf(s[1], 0.0f));
@@ -972,7 +993,7 @@ __device__ __forceinline__ void feature_finish(RegionShared& S, int tid, int bx0
     if (tid < 16) {
 #pragma unroll
         for (int k{0}; k < 6; ++k) {
-            S.u.s.feat[6 * tid + k] = f[k];
+            S.b.s.feat[6 * tid + k] = f[k];
         }
     }
     __syncthreads();
@@ -987,7 +1008,7 @@ __device__ __forceinline__ bool mlp_decide(RegionShared& S, const FrameParams& p
                                            int tid, int bx0, int by0, int bw, int bh) {
     {
         const int j{tid >> 2}, k{tid & 3};
-        const float* const x{&S.u.s.feat[24 * k]};
+        const float* const x{&S.b.s.feat[24 * k]};
         float s{0.0f};
 #pragma unroll
         for (int i{0}; i < 24; i += 8) {
@@ -1074,7 +1095,7 @@ __device__ __forceinline__ void export_features(const RegionShared& S, float* ou
                                                 int by0, int bw, int bh) {
     float* const row{out + static_cast<std::size_t>(region) * kFeatRow};
     if (tid < 96) {
-        row[tid] = S.u.s.feat[tid];
+        row[tid] = S.b.s.feat[tid];
     } else if (tid < 108) {
         const int k{tid - 96};
         float v{0.0f};
@@ -1144,9 +1165,11 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
     __syncthreads();
 
     CJX_REGION_CUT_AT(1)
-    // 2. Inverse gaborish (gaborish.h:16-28; tap order frontend_transform.cu:30-48).
+    // 2. Inverse gaborish (gaborish.h:16-28; tap order frontend_transform.cu:30-48),
+    //    its results kept in registers while the XYB tile is still read.
+    float4 sharp[3];
+    gaborish_tile(S, tid, sharp);
     {
-        gaborish_tile(S, tid);
         // 3a. AQ pre-erosion terms per interior pixel (frontend_fused.cu:118-137)
         //     and their 4x4 cell sums in row order: four lanes per cell, one
         //     per row; row dy continues the running sum of row dy - 1.
@@ -1155,7 +1178,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         float m[4];
 #pragma unroll
         for (int dx{0}; dx < 4; ++dx) {
-            const float* s{&S.u.f.xyb[1][(row + kHalo) * kTileW + col0 + dx + kHalo]};
+            const float* s{&S.a.xyb[1][(row + kHalo) * kTileW + col0 + dx + kHalo]};
             const float yv{s[0]};
             const float base{0.25f * (s[kTileW] + s[-kTileW] + s[-1] + s[1])};
             float diff{ratio_cbrt_gamma(yv + 0.019f, false) * (yv - base)};
@@ -1177,33 +1200,30 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
             }
         }
         if (dy == 3) {
-            S.u.f.aq.cells[cell] = 0.25f * sum;
+            S.b.aq.cells[cell] = 0.25f * sum;
         }
     }
-    __syncthreads();
 
     CJX_REGION_CUT_AT(2)
-    // 3b. Per-block modulation and the quant integer (frontend_fused.cu:117-203).
-    //     The 64 cells' fuzzy erosion and the 16 blocks' final step each run
-    //     once, in parallel lanes; the per-pixel sums are wave sums as before
-    //     (a block's four erosion terms sum as (e0 + e2) + (e1 + e3), which is
-    //     the wave tree over four non-zero lanes).
-    if (tid < 64) {
-        S.u.f.aq.ero[tid] = erosion_cell(S.u.f.aq.cells, tid & 7, tid >> 3, prm);
-    }
+    // 3b. Per-block modulation and the quant integer (frontend_fused.cu:117-203):
+    //     the per-pixel sums as wave sums, then (wave 0, after the barrier)
+    //     the 64 cells' fuzzy erosion and the 16 blocks' final step in
+    //     parallel lanes (a block's four erosion terms sum as
+    //     (e0 + e2) + (e1 + e3), which is the wave tree over four non-zero
+    //     lanes).
 #pragma unroll
     for (int j{0}; j < 4; ++j) {
         const int lb{j * 4 + wu};
         const int lbx{lb & 3}, lby{lb >> 2};
         const int fx{lane & 7}, fy{lane >> 3};
         const int idx{(lby * 8 + fy + kHalo) * kTileW + lbx * 8 + fx + kHalo};
-        const float yv{S.u.f.xyb[1][idx]}, xv{S.u.f.xyb[0][idx]}, bv{S.u.f.xyb[2][idx]};
+        const float yv{S.a.xyb[1][idx]}, xv{S.a.xyb[0][idx]}, bv{S.a.xyb[2][idx]};
         float hf{0.0f};
         if (fx < 7) {
-            hf += fminf(0.0206f, fabsf(yv - S.u.f.xyb[1][idx + 1]));
+            hf += fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + 1]));
         }
         if (fy < 7) {
-            hf += fminf(0.0206f, fabsf(yv - S.u.f.xyb[1][idx + kTileW]));
+            hf += fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + kTileW]));
         }
         const float iny{yv + 0.16f};
         const float gm{ratio_cbrt_gamma(iny - xv, true) + ratio_cbrt_gamma(iny + xv, true)};
@@ -1213,20 +1233,25 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         const float gamma_overall{lane_value(sums, 32) * (0.5f / 64.0f)};
         const float blue_sum{lane_value(sums, 16)};
         if (lane == 0) {
-            S.u.f.aq.blk[lb][0] = sums;
-            S.u.f.aq.blk[lb][1] = gamma_overall;
-            S.u.f.aq.blk[lb][2] = blue_sum;
+            S.b.aq.blk[lb][0] = sums;
+            S.b.aq.blk[lb][1] = gamma_overall;
+            S.b.aq.blk[lb][2] = blue_sum;
         }
     }
-    __syncthreads();
+    __syncthreads();  // the XYB tile is dead from here on
+    store_sharp(S, tid, sharp);
+    if (tid < 64) {
+        S.b.aq.ero[tid] = erosion_cell(S.b.aq.cells, tid & 7, tid >> 3, prm);
+        wave_sync();
+    }
     if (tid < 16) {
         const int lb{tid};
         const int lbx{lb & 3}, lby{lb >> 2};
         if (bx0 + lbx < bw && by0 + lby < bh) {
-            const float e0{S.u.f.aq.ero[(2 * lby) * 8 + 2 * lbx]}, e1{S.u.f.aq.ero[(2 * lby) * 8 + 2 * lbx + 1]};
-            const float e2{S.u.f.aq.ero[(2 * lby + 1) * 8 + 2 * lbx]}, e3{S.u.f.aq.ero[(2 * lby + 1) * 8 + 2 * lbx + 1]};
+            const float e0{S.b.aq.ero[(2 * lby) * 8 + 2 * lbx]}, e1{S.b.aq.ero[(2 * lby) * 8 + 2 * lbx + 1]};
+            const float e2{S.b.aq.ero[(2 * lby + 1) * 8 + 2 * lbx]}, e3{S.b.aq.ero[(2 * lby + 1) * 8 + 2 * lbx + 1]};
             const float aq{(e0 + e2) + (e1 + e3)};
-            float blue_sum{S.u.f.aq.blk[lb][2]};
+            float blue_sum{S.b.aq.blk[lb][2]};
             constexpr float k_limit{0.027121074570634722f};
             if (blue_sum >= 32.0f * k_limit) {
                 blue_sum = 64.0f * k_limit - blue_sum;
@@ -1236,8 +1261,8 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
                 blue_sum = k_max_limit * k_limit;
             }
             float ov{compute_mask(aq)};
-            ov += S.u.f.aq.blk[lb][0] * -0.38f + 0.42f;
-            ov += 0.1005613337192697f * log2_det(S.u.f.aq.blk[lb][1]);
+            ov += S.b.aq.blk[lb][0] * -0.38f + 0.42f;
+            ov += 0.1005613337192697f * log2_det(S.b.aq.blk[lb][1]);
             ov += blue_sum * 0.14207000358439159f;
             const float qval{exp_det(ov) * prm.mul_pb + prm.add_pb};
             int qi{static_cast<int>(qval * prm.inv_global_scale + 0.5f)};
@@ -1255,7 +1280,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
     //    are summed there.  Learned: the DCT8s and their costs, the region's
     //    features and the network first; the DCT16 and DCT32 candidates only
     //    where the network is not confident (the heuristic decides there).
-    __syncthreads();  // the XYB tile is dead from here on
+    __syncthreads();  // the sharpened planes are complete, the AQ terms dead
     CJX_REGION_CUT_AT(6)
     const int grp{lane >> 4}, t16{lane & 15};
     const float* const yp{plane_of(S, 1)};
@@ -1344,6 +1369,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         }
     };
     const int e32{(qcol + t16) * 32 + qrow + 4 * grp};
+    [[maybe_unused]] float own32[2]{0.0f, 0.0f};  // wave 0's terms, summed
     const auto ex_dct32_terms = [&](const f4v& c32) {
         float v[4], wq[4], wi[4], d[4], rt[4];
         bool llf[4];
@@ -1354,18 +1380,23 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         }
         selection_weights4(g_tables.wsel32, g_tables.wsel_inv32, e32, 0, wq, wi);
         selection_terms(v, llf, wq, wi, prm, d, rt);
-        *reinterpret_cast<float4*>(S.u.s.t32[0][wu][lane]) = float4{d[0], d[1], d[2], d[3]};
-        *reinterpret_cast<float4*>(S.u.s.t32[1][wu][lane]) = float4{rt[0], rt[1], rt[2], rt[3]};
+        if (wu == 0) {
+            own32[0] = ((d[0] + d[1]) + d[2]) + d[3];
+            own32[1] = ((rt[0] + rt[1]) + rt[2]) + rt[3];
+        } else {
+            *reinterpret_cast<float4*>(S.a.after.y.t32[0][wu - 1][lane]) = float4{d[0], d[1], d[2], d[3]};
+            *reinterpret_cast<float4*>(S.a.after.y.t32[1][wu - 1][lane]) = float4{rt[0], rt[1], rt[2], rt[3]};
+        }
     };
     // Wave 0, after a barrier: the DCT32's cost from the four waves' terms.
     const auto ex_dct32_cost = [&]() {
-        float s[2];
+        float s[2]{own32[0], own32[1]};
 #pragma unroll
         for (int k{0}; k < 2; ++k) {
 #pragma unroll
-            for (int b{0}; b < 4; ++b) {
-                const float4 x{*reinterpret_cast<const float4*>(S.u.s.t32[k][b][lane])};
-                s[k] = b == 0 ? x.x : s[k] + x.x;
+            for (int b{0}; b < 3; ++b) {
+                const float4 x{*reinterpret_cast<const float4*>(S.a.after.y.t32[k][b][lane])};
+                s[k] += x.x;
                 s[k] += x.y;
                 s[k] += x.z;
                 s[k] += x.w;
@@ -1378,23 +1409,21 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         }
         wave_sync();
     };
-    // The larger candidates: costs, then (every wave has read the Y plane)
-    // their coefficients into its space.
+    // The larger candidates' coefficients and costs, after every wave has
+    // transformed Y (whose space takes the DCT32's terms).
     const auto ex_big = [&](const f4v& c16, const f4v& c32) {
+        store4(coefy_of(S, 1), 256 * wu + t16 * 16 + 4 * grp, c16);
+        store4(coefy_of(S, 2), e32, c32);
         ex_dct16_costs(c16);
         ex_dct32_terms(c32);
         __syncthreads();
-        store4(coefy_of(S, 1), 256 * wu + t16 * 16 + 4 * grp, c16);
-        store4(coefy_of(S, 2), e32, c32);
         if (wu == 0) {
             ex_dct32_cost();
         }
     };
     // Matrix-core FP16 pieces: wave w transforms quad w as four DCT8s (with
     // their costs, from registers) and as one DCT16, and output tile w of the
-    // DCT32 (vertical origin 16 (w / 2), horizontal 16 (w % 2)); the DCT16
-    // and DCT32 results stay in registers until every wave has read the Y
-    // plane, whose space then takes their coefficients.
+    // DCT32 (vertical origin 16 (w / 2), horizontal 16 (w % 2)).
     const auto mf_dct8_costs = [&]() {
         const int q{wu};
         const f4v c8{mf_quad(yp, (q >> 1) * 16, (q & 1) * 16, g_tables.mf8[0], g_tables.mf8[1], lane)};
@@ -1447,7 +1476,6 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         const f4v c16{mf_quad(yp, (q >> 1) * 16, (q & 1) * 16, g_tables.mf16[0], g_tables.mf16[1], lane)};
         f4v c32[2];
         mf_dct32(yp, 16 * (wu & 1), 16 * (wu >> 1), false, lane, c32);
-        __syncthreads();
         float d16{0.0f}, r16{0.0f}, d32{0.0f}, r32{0.0f};
         float v16[4], w16[4], wi16[4], v32[4], w32[4], wi32[4], d[2][4], rt[2][4];
         int e16[4];
@@ -1482,8 +1510,11 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
             S.cost32p[q] = 1024.0f * ds32 + 6.0e-4f * rs32;
         }
         __syncthreads();
-        if (tid == 0) {
-            S.cost32 = (S.cost32p[0] + S.cost32p[1]) + (S.cost32p[2] + S.cost32p[3]);
+        if (wu == 0) {
+            if (lane == 0) {
+                S.cost32 = (S.cost32p[0] + S.cost32p[1]) + (S.cost32p[2] + S.cost32p[3]);
+            }
+            wave_sync();
         }
     };
     // The heuristic's decision from the costs, by wave 0: lane b < 16 decides
@@ -1537,6 +1568,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
             c32 = ex_cols32(a32, t32);
             const f4v c8{ex_cols(b8, t8, zero)};
             c16 = ex_cols(b16, r16, zero);
+            __syncthreads();  // Y is dead from here on
             CJX_REGION_CUT_AT(7)
             ex_dct8_costs(c8);
             ex_big(c16, c32);
@@ -1545,7 +1577,6 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         mf_dct8_costs();
         if constexpr (!kLearned) {
             mf_big();
-            __syncthreads();
         }
     }
     CJX_REGION_CUT_AT(8)
@@ -1555,7 +1586,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         feature_finish(S, tid, bx0, by0, bw, bh);
     }
     if constexpr (kLearned) {
-        fallback = !mlp_decide(S, prm, mlp_regs, S.u.s.hid, tid, bx0, by0, bw, bh);
+        fallback = !mlp_decide(S, prm, mlp_regs, S.b.s.hid, tid, bx0, by0, bw, bh);
         if (fallback) {
             // The heuristic for this region: the larger candidates and the
             // decision from the costs.
@@ -1565,10 +1596,10 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
                 f4v t32[2];
                 ex_rows32(yp, ex_basis32(wu & 1, lane), lane, t32);
                 c32 = ex_cols32(ex_basis32(wu >> 1, lane), t32);
+                __syncthreads();  // Y is dead from here on
                 ex_big(c16, c32);
             } else {
                 mf_big();
-                __syncthreads();
             }
         }
     }
@@ -1592,9 +1623,9 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
     //    DCT32) into the coefficient arrays in element order, then FP16 out
     //    and the CfL partials (frontend_quantize.cu:49-117 on this region).
     const bool need_y{kLearned && !fallback};
-    const auto cxb = [&](int ch) { return ch == 0 ? S.p.coef.x : S.p.coef.b; };
-    // Results stay in registers until every wave has read the planes, whose
-    // space then takes their coefficients.
+    // The coefficients of X and B go to Y's space (and past it): Y is dead
+    // unless a region that the network decided transforms it here.
+    const auto cxb = [&](int ch) { return S.a.after.y.xb[ch]; };
     const int acs0{__builtin_amdgcn_readfirstlane(S.acs[0])};
     const auto dct32 = [&](const float* plane, int fxb, f4v (&c)[2]) {
         if constexpr (kMf16) {
@@ -1612,7 +1643,9 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         if (need_y && wu < 2) {
             dct32(plane_of(S, 1), wu, cy);
         }
-        __syncthreads();
+        if (need_y) {
+            __syncthreads();
+        }
 #pragma unroll
         for (int o{0}; o < 2; ++o) {
             store4(cxb(ch), (16 * fxb + t16) * 32 + 16 * o + 4 * grp, c[o]);
@@ -1643,7 +1676,9 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
                 cy = ex_quad(plane_of(S, 1), qrow, qcol, b, lane);
             }
         }
-        __syncthreads();
+        if (need_y) {
+            __syncthreads();
+        }
         int j, e;
         mf_quad_element(lane, 0, n, j, e);
         store4(cxb(0), 256 * q + 64 * j + e, cx);
@@ -1669,7 +1704,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
         const int e{qc * 64 + s4};
         const int idx{cpad(is32 ? e : 256 * k + 64 * wu + s4)};
         const h4v hx{*reinterpret_cast<const h4v*>(cxb(0) + idx)};
-        const h4v hy{*reinterpret_cast<const h4v*>((n == 8 ? S.coefy8 : coefy_of(S, is32 ? 2 : 1)) + idx)};
+        const h4v hy{*reinterpret_cast<const h4v*>(coefy_of(S, n >> 4) + idx)};
         const h4v hb{*reinterpret_cast<const h4v*>(cxb(1) + idx)};
         const bool in{bx0 + bxl < bw && by0 + byl < bh};
         if (in) {
@@ -1720,7 +1755,7 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
 }
 
 template <bool kMf16, bool kLearned>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void region_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void region_kernel(
     Geometry geo, FrameParams prm, const std::uint8_t* __restrict__ luma, std::size_t luma_pitch,
     const std::uint8_t* __restrict__ chroma, std::size_t chroma_pitch,
     std::uint16_t* __restrict__ coeffs, std::int8_t* __restrict__ acs_out,
@@ -2048,13 +2083,16 @@ __global__ __launch_bounds__(256) void dct8_uniform_kernel(
     const std::size_t nblk{geo.nblocks};
     const std::size_t cplane{nblk * 64};
 
+    __shared__ alignas(16) float lines[16 * RowBuf8::BS];
+    __shared__ std::int32_t qy[1024];  // Y's quantized values
     xyb_tile(S, luma, luma_pitch, chroma, chroma_pitch, rx * 32, ry * 32, W, H, tid);
     __syncthreads();
-    gaborish_tile(S, tid);
+    float4 sharp[3];
+    gaborish_tile(S, tid, sharp);
+    __syncthreads();
+    store_sharp(S, tid, sharp);
     __syncthreads();
 
-    float* const lines{S.u.scratch};                                     // 16 blocks x RowBuf8
-    std::int32_t* const qy{reinterpret_cast<std::int32_t*>(S.u.scratch + 2048)};  // Y's quantized values
     const float ac_scale{prm.qgsf_select};
     const float dcq[3]{4096.0f * prm.dc_scale, 512.0f * prm.dc_scale, 256.0f * prm.dc_scale};
     const int b{tid >> 3}, sub{tid & 7};
