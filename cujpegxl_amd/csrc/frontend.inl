@@ -23,9 +23,9 @@ namespace cjx {
 
 constexpr int kHalo = 2;
 constexpr int kTileW = 32 + 2 * kHalo;  // 36
-// Chroma samples a tile's bilinear taps can reach: (32 + 2 halo) / 2 + 1 on
-// each side.
-constexpr int kChromaW = kTileW / 2 + 2;  // 20
+// Chroma rows a tile's bilinear taps can reach: (32 + 2 halo) / 2 + 1 on each
+// side.
+constexpr int kChromaRows = kTileW / 2 + 2;  // 20
 
 // Orders one wave's LDS accesses: writes before the barrier are seen by
 // every lane's reads after it.
@@ -38,11 +38,13 @@ __device__ __forceinline__ void wave_sync() {
 // (of the frame's workgroups, in a batched launch).
 __device__ __forceinline__ void clear_words(const Clears& c, const Wg& wg) {
     const std::uint32_t stride{wg.nx * wg.ny * blockDim.x};
-    const std::uint32_t t{(wg.y * wg.nx + wg.x) * blockDim.x + threadIdx.x};
+    const std::uint32_t first{(wg.y * wg.nx + wg.x) * blockDim.x};
 #pragma unroll
     for (int k{0}; k < 4; ++k) {
-        for (std::uint32_t i{t}; i < c.words[k]; i += stride) {
-            c.ptr[k][i] = 0;
+        if (first < c.words[k]) {  // a scalar test: most workgroups have nothing to clear
+            for (std::uint32_t i{first + threadIdx.x}; i < c.words[k]; i += stride) {
+                c.ptr[k][i] = 0;
+            }
         }
     }
 }
@@ -105,38 +107,61 @@ __device__ __forceinline__ float clamp01(float v) {
     return fminf(fmaxf(v, 0.0f), 1.0f);
 }
 
-// xyb_impl.cuh:37-70 on the shared numeric primitives (the powers from the
-// table at `tab`, staged in LDS).  Both branches are evaluated (the power at
-// the threshold where the line is taken, which keeps its table index in
-// range): a pixel's three curves then overlap instead of waiting for their
-// table reads one after another in divergent branches (region kernel 159 ->
-// 156 us at 3840x2160).
-__device__ __forceinline__ float srgb_to_linear(float e, const float2* tab) {
+// pow24_tab and cbrt_tab with the series argument's two constants held in
+// registers, so that placing the mantissa bits is one v_and_or_b32.
+struct XybPowers {
+    const float2* tab;
+    std::uint32_t mask, one;
+
+    __device__ __forceinline__ explicit XybPowers(const float2* t) : tab{t}, mask{0x0007ffffu}, one{0x4b000000u} {
+        asm volatile("" : "+s"(mask), "+v"(one));
+    }
+    __device__ __forceinline__ float arg(std::uint32_t u, float r_scaled) const {
+        return (u2f((u & mask) | one) - 8650752.0f) * r_scaled;
+    }
+    __device__ __forceinline__ float pow24(float x) const {
+        const std::uint32_t u{f2u(x)};
+        const float2 e{tab[kXybPow + ((u >> 19) - (122u << 4))]};
+        return pow24_series(e.x, arg(u, e.y));
+    }
+    __device__ __forceinline__ float cbrt(float x) const {
+        const std::uint32_t u{f2u(x)};
+        const float2 e{tab[kXybCbrt + ((u >> 19) - (118u << 4))]};
+        return cbrt_series(e.x, arg(u, e.y));
+    }
+};
+
+// xyb_impl.cuh:37-70 on the shared numeric primitives, clamped to [0, 1] (the
+// line lies there for e in [0, 1]).  Both branches are evaluated: a pixel's
+// three curves then overlap instead of waiting for their table reads one
+// after another in divergent branches (region kernel 159 -> 156 us at
+// 3840x2160).
+__device__ __forceinline__ float srgb_to_linear(float e, const XybPowers& pw) {
     const float line{e * (1.0f / 12.92f)};
-    const float curve{pow24_tab((fmaxf(e, 0.04045f) + 0.055f) * (1.0f / 1.055f), tab)};
+    const float curve{clamp01(pw.pow24((e + 0.055f) * (1.0f / 1.055f)))};
     return e <= 0.04045f ? line : curve;
 }
 
 // Opsin absorbance bias of the XYB transform.
 constexpr float kOpsinBias{0.0037930732552754493f};
 
-// `neg_cbrt_bias` is -cbrt_tab(kOpsinBias, tab), evaluated once by the caller.
+// `neg_cbrt_bias` is -cbrt(kOpsinBias), evaluated once by the caller.
 __device__ __forceinline__ void pixel_to_xyb(float yv, float cb, float cr, float& ox, float& oy, float& ob,
-                                             const float2* tab, float neg_cbrt_bias) {
+                                             const XybPowers& pw, float neg_cbrt_bias) {
     constexpr float m00{0.30f}, m02{0.078f}, m01{1.0f - 0.078f - 0.30f};
     constexpr float m10{0.23f}, m12{0.078f}, m11{1.0f - 0.078f - 0.23f};
     constexpr float m20{0.24342268924547819f}, m21{0.20476744424496821f};
     constexpr float m22{1.0f - 0.24342268924547819f - 0.20476744424496821f};
     constexpr float bias{kOpsinBias};
-    const float r{clamp01(srgb_to_linear(clamp01(yv + 1.5748f * cr), tab))};
-    const float g{clamp01(srgb_to_linear(clamp01(yv - 0.1873242729f * cb - 0.4681242729f * cr), tab))};
-    const float b{clamp01(srgb_to_linear(clamp01(yv + 1.8556f * cb), tab))};
-    float q0{fmaxf(m00 * r + m01 * g + m02 * b + bias, 0.0f)};
-    float q1{fmaxf(m10 * r + m11 * g + m12 * b + bias, 0.0f)};
-    float q2{fmaxf(m20 * r + m21 * g + m22 * b + bias, 0.0f)};
-    q0 = cbrt_tab(q0, tab) + neg_cbrt_bias;
-    q1 = cbrt_tab(q1, tab) + neg_cbrt_bias;
-    q2 = cbrt_tab(q2, tab) + neg_cbrt_bias;
+    const float r{srgb_to_linear(clamp01(yv + 1.5748f * cr), pw)};
+    const float g{srgb_to_linear(clamp01(yv - 0.1873242729f * cb - 0.4681242729f * cr), pw)};
+    const float b{srgb_to_linear(clamp01(yv + 1.8556f * cb), pw)};
+    float q0{m00 * r + m01 * g + m02 * b + bias};  // positive: nothing to clamp
+    float q1{m10 * r + m11 * g + m12 * b + bias};
+    float q2{m20 * r + m21 * g + m22 * b + bias};
+    q0 = pw.cbrt(q0) + neg_cbrt_bias;
+    q1 = pw.cbrt(q1) + neg_cbrt_bias;
+    q2 = pw.cbrt(q2) + neg_cbrt_bias;
     ox = 0.5f * (q0 - q1);
     oy = 0.5f * (q0 + q1);
     ob = q2;
@@ -354,7 +379,7 @@ __device__ __forceinline__ int cpad(int e) {
 //   wait in registers), then the sharpened planes X, B, Y; Y's space and the
 //   rest past it take the DCT32's selection terms once Y has been
 //   transformed, then X's and B's coefficients of the chosen transforms.
-// - `b`: the powers' table and the chroma window of step 1, then the AQ terms
+// - `b`: the chroma rows and the powers' table of step 1, then the AQ terms
 //   (steps 2-3), then Y's coefficients of the three candidate sizes, the
 //   features and the network's hidden units.
 struct AqTerms {
@@ -377,8 +402,8 @@ struct RegionShared {
     } a;
     union {
         struct {
+            std::uint32_t h[kChromaRows * kTileW];
             float2 tab[kXybTabPairs];
-            std::uint32_t win[kChromaW * kChromaW];
         } in;
         AqTerms aq;
         struct {
@@ -526,74 +551,135 @@ __device__ int g_region_cut;
 // cell (coordinate x >> 1) and 1/4 on its neighbour towards the pixel
 // (clamped to the plane), in each direction.  Every partial sum of the
 // float form (products of samples and weights, then their sums) is exact,
-// so the interpolated value is exactly (9 s_kk + 3 s_kn + 3 s_nk + s_nn) / 16:
-// the tile computes that integer sum, for Cb and Cr at once in the two
-// halves of one word (at most 16 * 255 each), and scales it by 1/16, which
-// gives the float form's bits.
+// so the interpolated value is exactly (3 h_k + h_n) / 16 with the horizontal
+// sums h = 3 s_k + s_n of the rows k and n: the tile computes these as
+// integers, for Cb and Cr at once in the two halves of one word (at most
+// 16 * 255 each), and scales by 1/16, which gives the float form's bits.
+//
+// Thread t takes column t % 36 of the tile, for the chroma rows (t / 36 + 7 j)
+// and for the pixels (rows t / 36 + 7 k): the column's taps are computed
+// once, and a row's horizontal sums once for the pixels above and below.  The
+// kernel is bound by VALU issue, so away from the frame's top and bottom,
+// where no row is clamped, every row's address is one of the thread's base
+// registers plus a constant (LDS) or a scalar (planes), and the six luma reads
+// are issued at once.  Other regions, and planes with a pitch that 32-bit
+// offsets do not cover, compute each row's address. 
+// Region kernel at 3840x2160, one address computed per row and tap before:
+// 156 -> 149 us (130.7 -> 124.5 learned + FP16); VALU instructions -9.6%.
 __device__ __forceinline__ void xyb_tile(RegionShared& S, const std::uint8_t* luma, std::size_t luma_pitch,
                                          const std::uint8_t* chroma, std::size_t chroma_pitch, int px0, int py0,
                                          int W, int H, int tid) {
-    // The powers' table, then the tile's chroma window: samples
-    // (cx0 + j, cy0 + i), clamped to the plane, Cb in the low half-word and
-    // Cr in the high one.  Every tap of the tile's pixels (their coordinates
-    // clamped to the frame, the taps to the plane) lands in the window.
     float2* const tab{S.b.in.tab};
-    std::uint32_t* const win{S.b.in.win};
+    std::uint32_t* const h{S.b.in.h};
     const int cw{W / 2}, ch{H / 2};
-    const int cx0{(px0 >> 1) - 2}, cy0{(py0 >> 1) - 2};
-    for (int i{tid}; i < kChromaW * kChromaW; i += 256) {
-        int x{cx0 + i % kChromaW}, y{cy0 + i / kChromaW};
-        x = x < 0 ? 0 : (x >= cw ? cw - 1 : x);
-        y = y < 0 ? 0 : (y >= ch ? ch - 1 : y);
-        const std::uint8_t* p{chroma + static_cast<std::size_t>(static_cast<std::uint32_t>(y)) * chroma_pitch +
-                              2u * static_cast<std::uint32_t>(x)};
-        win[i] = static_cast<std::uint32_t>(p[0]) | (static_cast<std::uint32_t>(p[1]) << 16);
-    }
-    if (tid < kXybTabPairs) {
-        tab[tid] = g_tables.xyb_tab[tid];
-    }
-    __syncthreads();
-    // Thread t converts column t % 36 of the tile, rows t / 36 + 7 k: the
-    // column's luma address and horizontal chroma taps are computed once.
-    if (tid < 7 * kTileW) {
-        const int lx{tid % kTileW};
-        int gx{px0 + lx - kHalo};
-        gx = gx < 0 ? 0 : (gx >= W ? W - 1 : gx);
+    const int cy0{(py0 >> 1) - 2};
+    static_assert(kXybTabPairs == 256, "one table entry per thread");
+    tab[tid] = g_tables.xyb_tab[tid];
+    const int lx{tid % kTileW}, r0{tid / kTileW};
+    const bool active{tid < 7 * kTileW};
+    constexpr std::size_t kMaxPitch{std::size_t{1} << 28};
+    const bool interior{py0 >= kHalo && py0 + 36 <= H && luma_pitch <= kMaxPitch && chroma_pitch <= kMaxPitch};
+    int gx{px0 + lx - kHalo};
+    gx = gx < 0 ? 0 : (gx >= W ? W - 1 : gx);
+    constexpr int kPix{(kTileW + 6) / 7};  // pixel rows of a thread (the last one for r0 = 0 only)
+    std::uint32_t lu[kPix]{};
+    if (active) {
         const int kx{gx >> 1};
         const int nx{(gx & 1) != 0 ? (kx + 1 < cw ? kx + 1 : cw - 1) : (kx > 0 ? kx - 1 : 0)};
-        const int ox{kx - cx0}, onx{nx - cx0};
-        const std::uint8_t* const lcol{luma + static_cast<std::uint32_t>(gx)};
-        const float neg_cbrt_bias{-cbrt_tab(kOpsinBias, tab)};
-        // (1/255) / 16, exact: the 1/16 of the sum folded into the scale.
-        constexpr float kScale{(1.0f / 255.0f) * 0.0625f};
-        const auto row_of = [&](int ly) {
-            const int gy{py0 + ly - kHalo};
-            return gy < 0 ? 0 : (gy >= H ? H - 1 : gy);
-        };
-        const auto luma_at = [&](int gy) {
-            return lcol[static_cast<std::size_t>(static_cast<std::uint32_t>(gy)) * luma_pitch];
-        };
-        // The next row's luma is loaded one iteration ahead (the row past
-        // the tile's last is clamped to the frame, so the load is in bounds).
-        int gy{row_of(tid / kTileW)};
-        std::uint8_t lnext{luma_at(gy)};
-        for (int ly{tid / kTileW}; ly < kTileW; ly += 7) {
-            const int i{ly * kTileW + lx};
-            const std::uint8_t lcur{lnext};
-            const int gy_next{row_of(ly + 7)};
-            lnext = luma_at(gy_next);
-            const int ky{gy >> 1};
-            const int ny{(gy & 1) != 0 ? (ky + 1 < ch ? ky + 1 : ch - 1) : (ky > 0 ? ky - 1 : 0)};
-            const int rk{(ky - cy0) * kChromaW}, rn{(ny - cy0) * kChromaW};
-            const std::uint32_t hk{__umul24(win[rk + ox], 3u) + win[rk + onx]};
-            const std::uint32_t hn{__umul24(win[rn + ox], 3u) + win[rn + onx]};
-            const std::uint32_t v{(hk << 1) + hk + hn};
-            const float yv{static_cast<float>(lcur) * (1.0f / 255.0f)};
-            const float cb{static_cast<float>(v & 0xffffu) * kScale - 128.0f / 255.0f};
-            const float cr{static_cast<float>(v >> 16) * kScale - 128.0f / 255.0f};
-            pixel_to_xyb(yv, cb, cr, S.a.xyb[0][i], S.a.xyb[1][i], S.a.xyb[2][i], tab, neg_cbrt_bias);
-            gy = gy_next;
+        // Chroma pairs (Cb | Cr << 8) at the two taps of up to three rows.
+        constexpr int kRows{(kChromaRows + 6) / 7};
+        std::uint16_t sk[kRows]{}, sn[kRows]{};
+        if (interior) {
+            const std::uint8_t* const lrow{luma + static_cast<std::size_t>(py0 - kHalo) * luma_pitch};
+            const std::uint32_t lo{static_cast<std::uint32_t>(r0) * static_cast<std::uint32_t>(luma_pitch) +
+                                   static_cast<std::uint32_t>(gx)};
+#pragma unroll
+            for (int k{0}; k < kPix; ++k) {
+                if (7 * k + 6 < kTileW || r0 + 7 * k < kTileW) {
+                    lu[k] = (lrow + static_cast<std::size_t>(7 * k) * luma_pitch)[lo];
+                }
+            }
+            const std::uint8_t* const crow{chroma + static_cast<std::size_t>(cy0) * chroma_pitch};
+            const std::uint32_t co{static_cast<std::uint32_t>(r0) * static_cast<std::uint32_t>(chroma_pitch)};
+#pragma unroll
+            for (int j{0}; j < kRows; ++j) {
+                if (7 * j + 6 < kChromaRows || r0 + 7 * j < kChromaRows) {
+                    const std::uint8_t* const row{crow + static_cast<std::size_t>(7 * j) * chroma_pitch};
+                    __builtin_memcpy(&sk[j], row + (co + 2u * static_cast<std::uint32_t>(kx)), 2);
+                    __builtin_memcpy(&sn[j], row + (co + 2u * static_cast<std::uint32_t>(nx)), 2);
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int j{0}; j < kRows; ++j) {
+                if (r0 + 7 * j < kChromaRows) {
+                    int y{cy0 + r0 + 7 * j};
+                    y = y < 0 ? 0 : (y >= ch ? ch - 1 : y);
+                    const std::uint8_t* const row{chroma + static_cast<std::size_t>(static_cast<std::uint32_t>(y)) *
+                                                               chroma_pitch};
+                    std::uint16_t k, n;
+                    __builtin_memcpy(&k, row + 2u * static_cast<std::uint32_t>(kx), 2);
+                    __builtin_memcpy(&n, row + 2u * static_cast<std::uint32_t>(nx), 2);
+                    const auto pair = [](std::uint32_t v) { return (v & 0xffu) | ((v & 0xff00u) << 8); };
+                    h[(r0 + 7 * j) * kTileW + lx] = 3u * pair(k) + pair(n);
+                }
+            }
         }
+        if (interior) {
+#pragma unroll
+            for (int j{0}; j < kRows; ++j) {
+                if (7 * j + 6 < kChromaRows || r0 + 7 * j < kChromaRows) {
+                    const auto pair = [](std::uint32_t v) { return (v & 0xffu) | ((v & 0xff00u) << 8); };
+                    const std::uint32_t k{pair(sk[j])};
+                    h[(r0 + 7 * j) * kTileW + lx] = (k << 1) + k + pair(sn[j]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (!active) {
+        return;
+    }
+    const XybPowers pw{tab};
+    const float neg_cbrt_bias{-pw.cbrt(kOpsinBias)};
+    // (1/255) / 16, exact: the 1/16 of the sum folded into the scale.
+    constexpr float kScale{(1.0f / 255.0f) * 0.0625f};
+    const auto pixel = [&](std::uint32_t l, std::uint32_t hk, std::uint32_t hn, int i) {
+        std::uint32_t kn{hk + hn};
+        asm("" : "+v"(kn));  // two adds, not one quarter-rate v_mad_u64_u32
+        const std::uint32_t v{(hk << 1) + kn};
+        const float yv{static_cast<float>(l) * (1.0f / 255.0f)};
+        const float cb{static_cast<float>(v & 0xffffu) * kScale - 128.0f / 255.0f};
+        const float cr{static_cast<float>(v >> 16) * kScale - 128.0f / 255.0f};
+        pixel_to_xyb(yv, cb, cr, S.a.xyb[0][i], S.a.xyb[1][i], S.a.xyb[2][i], pw, neg_cbrt_bias);
+    };
+    if (interior) {
+        // Tile row ly lies in chroma row (ly + 2) / 2 of the tile's; its
+        // neighbour is the next row for odd ly, the one before for even ly.
+        // Rows r0 + 7 k alternate in parity: two base rows, 7 rows further
+        // every second step.
+        const int ke{((r0 + 2) >> 1) * kTileW + lx}, ko{((r0 + 9) >> 1) * kTileW + lx};
+        const int de{(r0 & 1) != 0 ? kTileW : -kTileW};
+        const int ne{ke + de}, no{ko - de};
+#pragma unroll
+        for (int k{0}; k < kPix; ++k) {
+            if (7 * k + 6 < kTileW || r0 + 7 * k < kTileW) {
+                const int at{(k >> 1) * 7 * kTileW};
+                pixel(lu[k], h[((k & 1) != 0 ? ko : ke) + at], h[((k & 1) != 0 ? no : ne) + at],
+                      r0 * kTileW + lx + 7 * k * kTileW);
+            }
+        }
+        return;
+    }
+#pragma unroll 1
+    for (int ly{r0}; ly < kTileW; ly += 7) {
+        int gy{py0 + ly - kHalo};
+        gy = gy < 0 ? 0 : (gy >= H ? H - 1 : gy);
+        const std::uint32_t l{luma[static_cast<std::size_t>(static_cast<std::uint32_t>(gy)) * luma_pitch +
+                                   static_cast<std::uint32_t>(gx)]};
+        const int ky{gy >> 1};
+        const int ny{(gy & 1) != 0 ? (ky + 1 < ch ? ky + 1 : ch - 1) : (ky > 0 ? ky - 1 : 0)};
+        pixel(l, h[(ky - cy0) * kTileW + lx], h[(ny - cy0) * kTileW + lx], ly * kTileW + lx);
     }
 }
 
@@ -1211,31 +1297,34 @@ __device__ __attribute__((always_inline)) inline void region_kernel_body(const W
     //     parallel lanes (a block's four erosion terms sum as
     //     (e0 + e2) + (e1 + e3), which is the wave tree over four non-zero
     //     lanes).
-#pragma unroll
-    for (int j{0}; j < 4; ++j) {
-        const int lb{j * 4 + wu};
-        const int lbx{lb & 3}, lby{lb >> 2};
+    {
+        // Wave w takes blocks (w, j), j = 0..3, one pixel per lane.
         const int fx{lane & 7}, fy{lane >> 3};
-        const int idx{(lby * 8 + fy + kHalo) * kTileW + lbx * 8 + fx + kHalo};
-        const float yv{S.a.xyb[1][idx]}, xv{S.a.xyb[0][idx]}, bv{S.a.xyb[2][idx]};
-        float hf{0.0f};
-        if (fx < 7) {
-            hf += fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + 1]));
+        const int idx0{(fy + kHalo) * kTileW + wu * 8 + fx + kHalo};
+        float hf[4], gm[4], bl[4];
+#pragma unroll
+        for (int j{0}; j < 4; ++j) {
+            const int idx{idx0 + j * 8 * kTileW};
+            const float yv{S.a.xyb[1][idx]}, xv{S.a.xyb[0][idx]}, bv{S.a.xyb[2][idx]};
+            // Differences inside the block; the tile's halo makes the reads
+            // past its edge valid.
+            const float right{fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + 1]))};
+            const float down{fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + kTileW]))};
+            hf[j] = (fx < 7 ? right : 0.0f) + (fy < 7 ? down : 0.0f);
+            const float iny{yv + 0.16f};
+            gm[j] = ratio_cbrt_gamma(iny - xv, true) + ratio_cbrt_gamma(iny + xv, true);
+            const float pye{yv + 0.084381641171960495f + fabsf(xv)};
+            bl[j] = bv > pye ? fminf(bv - pye, 0.027121074570634722f) : 0.0f;
         }
-        if (fy < 7) {
-            hf += fminf(0.0206f, fabsf(yv - S.a.xyb[1][idx + kTileW]));
-        }
-        const float iny{yv + 0.16f};
-        const float gm{ratio_cbrt_gamma(iny - xv, true) + ratio_cbrt_gamma(iny + xv, true)};
-        const float pye{yv + 0.084381641171960495f + fabsf(xv)};
-        const float bl{bv > pye ? fminf(bv - pye, 0.027121074570634722f) : 0.0f};
-        const float sums{wave_sum4(hf, gm, bl, 0.0f)};  // lanes 0, 32, 16
-        const float gamma_overall{lane_value(sums, 32) * (0.5f / 64.0f)};
-        const float blue_sum{lane_value(sums, 16)};
-        if (lane == 0) {
-            S.b.aq.blk[lb][0] = sums;
-            S.b.aq.blk[lb][1] = gamma_overall;
-            S.b.aq.blk[lb][2] = blue_sum;
+        // Sums of blocks j = 0, 2, 1, 3 in lanes 0, 16, 32, 48.
+        const float hs{wave_sum4(hf[0], hf[1], hf[2], hf[3])};
+        const float gs{wave_sum4(gm[0], gm[1], gm[2], gm[3])};
+        const float bs{wave_sum4(bl[0], bl[1], bl[2], bl[3])};
+        if ((lane & 15) == 0) {
+            const int j{((lane >> 3) & 2) | (lane >> 5)};
+            S.b.aq.blk[4 * j + wu][0] = hs;
+            S.b.aq.blk[4 * j + wu][1] = gs * (0.5f / 64.0f);
+            S.b.aq.blk[4 * j + wu][2] = bs;
         }
     }
     __syncthreads();  // the XYB tile is dead from here on

@@ -87,37 +87,30 @@ CJX_HD float div_by_recip(float a, float b, float r) {
 // {T[k][j], r_j 2^-23} per (k, j), so each power reads one 8-byte entry.
 // m - c_j is exactly D 2^-23 with the integer D = (low 19 mantissa bits of
 // x) - 2^18, so t = D (r_j 2^-23) is the same real product as (m - c_j) r_j
-// and rounds to the same float.
-constexpr int kXybPow = 0;    // [5][16]: x^2.4 for k = -4 .. 0
-constexpr int kXybCbrt = 80;  // [10][16]: x^(1/3) for k = -9 .. 0
-constexpr int kXybTabPairs = 240;
+// and rounds to the same float.  D as a float: the bits placed in the mantissa
+// of 2^23, less 2^23 + 2^18 (exact).
+// x^2.4 for x in [2^-5, 2): the sRGB curve's upper branch takes x in [0.0905, 1]
+// (below it, down to 0.052, the table only has to be readable); x^(1/3) for x
+// in [2^-9, 2): the opsin values, x in [0.0038, 1.004].
+constexpr int kXybPow = 0;    // [6][16]: x^2.4 for k = -5 .. 0
+constexpr int kXybCbrt = 96;  // [10][16]: x^(1/3) for k = -9 .. 0
+constexpr int kXybTabPairs = 256;
 
-CJX_HD float xyb_series_arg(std::uint32_t u, float r_scaled) {
-    return (static_cast<float>(u & 0x0007ffffu) - 262144.0f) * r_scaled;
-}
-
-// x^2.4 for x in [2^-4, 2) (the sRGB curve's upper branch: x in [0.0905, 1]).
-CJX_HD float pow24_tab(float x, const float2* tab) {
-    const std::uint32_t u{f2u(x)};
-    const float2 e{tab[kXybPow + ((u >> 19) - (123u << 4))]};
-    const float t{xyb_series_arg(u, e.y)};
+// T (1 + t)^2.4 and T (1 + t)^(1/3) by their series.
+CJX_HD float pow24_series(float power, float t) {
     float p{0.224f};
     p = __builtin_fmaf(p, t, 1.68f);
     p = __builtin_fmaf(p, t, 2.4f);
     p = __builtin_fmaf(p, t, 1.0f);
-    return e.x * p;
+    return power * p;
 }
 
-// x^(1/3) for x in [2^-9, 2) (the opsin values: x in [0.0038, 1.004]).
-CJX_HD float cbrt_tab(float x, const float2* tab) {
-    const std::uint32_t u{f2u(x)};
-    const float2 e{tab[kXybCbrt + ((u >> 19) - (118u << 4))]};
-    const float t{xyb_series_arg(u, e.y)};
+CJX_HD float cbrt_series(float power, float t) {
     float p{0.0617283951f};
     p = __builtin_fmaf(p, t, -0.111111111f);
     p = __builtin_fmaf(p, t, 0.333333333f);
     p = __builtin_fmaf(p, t, 1.0f);
-    return e.x * p;
+    return power * p;
 }
 
 CJX_HD float exp_det(float x) {

@@ -71,8 +71,8 @@ void xyb_power_table(float2* t) {
         // RN(1 / c) scaled by 2^-23 (exact): the series argument takes the
         // mantissa difference as an integer count of 2^-23 steps.
         const float r{std::ldexp(static_cast<float>(1.0 / c), -23)};
-        for (int k{-4}; k <= 0; ++k) {
-            t[kXybPow + (k + 4) * 16 + j] = float2{static_cast<float>(std::pow(std::ldexp(c, k), 2.4)), r};
+        for (int k{-5}; k <= 0; ++k) {
+            t[kXybPow + (k + 5) * 16 + j] = float2{static_cast<float>(std::pow(std::ldexp(c, k), 2.4)), r};
         }
         for (int k{-9}; k <= 0; ++k) {
             t[kXybCbrt + (k + 9) * 16 + j] = float2{static_cast<float>(std::cbrt(std::ldexp(c, k))), r};

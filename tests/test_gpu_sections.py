@@ -14,6 +14,10 @@ from cujpegxl_amd.synth import synthetic_nv12
 
 pytestmark = pytest.mark.gpu
 
+# Plane addresses and pitches of every alignment (the chroma pairs and the
+# luma bytes are read where they lie).
+PLANES = [(1, 1, 0, 0), (0, 3, 1, 5), (2, 1, 7, 2), (5, 2, 64, 63)]
+
 SIZES = [(2056, 264, 0.8), (264, 2056, 1.5), (2064, 2056, 1.0), (264, 8, 1.0), (4104, 64, 3.0)]
 
 
@@ -59,5 +63,23 @@ def test_more_sections_than_layout_threads(jo):
     dev = cj.DeviceBuffer.from_array(np.concatenate([luma.ravel(), chroma.ravel()]))
     enc = cj.Encoder(w, h, d)
     assert enc.encode_device(dev.ptr, dev.ptr + w * h, w, w) == want
+    enc.close()
+    dev.close()
+
+
+@pytest.mark.parametrize("luma_at,chroma_at,luma_pad,chroma_pad", PLANES)
+def test_unaligned_planes(jo, luma_at, chroma_at, luma_pad, chroma_pad):
+    w, h, d = 296, 136, 1.0
+    luma, chroma = synthetic_nv12(w, h, 5)
+    lp, cp = w + luma_pad, w + chroma_pad
+    base = (luma_at + h * lp + 255) & ~255
+    buf = np.full(base + chroma_at + (h // 2) * cp, 255, np.uint8)
+    for y in range(h):
+        buf[luma_at + y * lp : luma_at + y * lp + w] = luma[y]
+    for y in range(h // 2):
+        buf[base + chroma_at + y * cp : base + chroma_at + y * cp + w] = chroma[y]
+    dev = cj.DeviceBuffer.from_array(buf)
+    enc = cj.Encoder(w, h, d)
+    assert enc.encode_device(dev.ptr + luma_at, dev.ptr + base + chroma_at, lp, cp) == jo.encode_nv12(luma, chroma, w, h, d)
     enc.close()
     dev.close()
