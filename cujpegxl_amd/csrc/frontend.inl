@@ -458,8 +458,8 @@ template <int M>
 __device__ __forceinline__ void selection_terms(const float (&s)[M], const bool (&llf)[M], const float (&wq)[M],
                                                 const float (&wi)[M], const FrameParams& prm, float (&d)[M],
                                                 float (&rt)[M]) {
-    float aq[M];
-    int k[M];
+    float aq[M], r[M];
+    float top{0.0f};
 #pragma unroll
     for (int i{0}; i < M; ++i) {
         const float sv{llf[i] ? 0.0f : s[i]};
@@ -467,18 +467,18 @@ __device__ __forceinline__ void selection_terms(const float (&s)[M], const bool 
         const float err{div_by_recip(q * wq[i], prm.qgsf_select, prm.inv_qgsf_select) - sv};
         d[i] = err * err;
         aq[i] = fabsf(q);
-        k[i] = aq[i] < 256.0f ? static_cast<int>(aq[i]) : 0;
+        top = fmaxf(top, aq[i]);
+        r[i] = g_tables.rate[static_cast<std::uint32_t>(fminf(aq[i], 255.0f))];
     }
-    float r[M];
+    // Past the table (one test for all M).
+    if (__builtin_amdgcn_ballot_w64(top >= 256.0f) != 0) {
 #pragma unroll
-    for (int i{0}; i < M; ++i) {
-        r[i] = g_tables.rate[k[i]];
-    }
-#pragma unroll
-    for (int i{0}; i < M; ++i) {
-        if (aq[i] >= 256.0f) {
-            r[i] = 1.0f + log2_det(1.0f + aq[i]);
+        for (int i{0}; i < M; ++i) {
+            r[i] = aq[i] >= 256.0f ? 1.0f + log2_det(1.0f + aq[i]) : r[i];
         }
+    }
+#pragma unroll
+    for (int i{0}; i < M; ++i) {
         rt[i] = r[i];
     }
 }
