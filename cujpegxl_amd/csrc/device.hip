@@ -47,21 +47,27 @@ bool set_mlp_weights(const std::uint16_t* w1, const float* b1, const std::uint16
     return hipMemcpyToSymbol(HIP_SYMBOL(g_mlp), &m, sizeof(m)) == hipSuccess;
 }
 
+// Workgroups of the network's passes over n regions.
+static std::uint32_t mlp_wgs(std::uint32_t n) {
+    const std::uint32_t tiles{n / kMlpTiles + (n % kMlpTiles != 0 ? 1u : 0u)};
+    return tiles < kMlpMaxWgs ? tiles : kMlpMaxWgs;
+}
+
 std::size_t mlp_partial_floats(std::uint32_t n) {
-    return static_cast<std::size_t>((n + kMlpTiles - 1) / kMlpTiles) * (kMlpParams + 1);
+    return static_cast<std::size_t>((n + kMlpTiles - 1) / kMlpTiles) * (kMlpParams + 1);  // a row per tile is enough
 }
 
 void launch_mlp_step(hipStream_t s, const float* x, const float* labels, std::uint32_t n, float lambda,
                      float* partial, float* grad, float* loss, float* params, float* m, float* v, std::uint32_t step,
                      float lr) {
-    const std::uint32_t rows{(n + kMlpTiles - 1) / kMlpTiles};
-    mlp_grad_kernel<<<rows, 256, 0, s>>>(params, x, labels, n, lambda, partial);
-    mlp_reduce_kernel<<<(kMlpParams + 1 + 255) / 256, 256, 0, s>>>(partial, rows, n, grad, loss, params, m, v, step,
-                                                                   lr);
+    const std::uint32_t rows{mlp_wgs(n)};
+    mlp_grad_kernel<<<rows, kMlpThreads, 0, s>>>(params, x, labels, n, lambda, partial);
+    mlp_reduce_kernel<<<(kMlpParams + 1 + 63) / 64, 64 * kMlpSlices, 0, s>>>(partial, rows, n, grad, loss, params, m, v,
+                                                                             step, lr);
 }
 
 void launch_mlp_forward(hipStream_t s, const float* params, const float* x, std::uint32_t n, float* z) {
-    mlp_forward_kernel<<<(n + 255) / 256, 256, 0, s>>>(params, x, n, z);
+    mlp_forward_kernel<<<mlp_wgs(n), kMlpThreads, 0, s>>>(params, x, n, z);
 }
 
 // One thread per (block position, channel): non-zero AC counts of a
