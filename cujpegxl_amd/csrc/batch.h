@@ -88,16 +88,22 @@ struct BatchShape {
     std::uint32_t region_wgs;
 };
 
-// Stage grids of one frame for a shape and an emission with `band_wgs`
-// workgroups per band (nx, ny only; `first` is the caller's).
-void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32_t band_wgs,
+// Stage grids of one frame of a batch of `blocks` blocks for a shape and an
+// emission with `band_wgs` workgroups per band (nx, ny only; `first` is the
+// caller's).
+void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint64_t blocks, std::uint32_t band_wgs,
                        StageGrid (&grid)[kBStages]);
 
-// Queues the eight batched launches of a batch (all frames in `mode`) on `s`.
-// A persistent region stage (shape.region_wgs != 0) claims its regions
-// through the eight device counters at `counters`, which a one-workgroup
-// launch clears first.
-void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
-                  std::uint32_t mode, const BatchShape& shape, std::uint32_t* counters);
+// Counters of a persistent region stage: one per XCD.
+constexpr int kRegionCounters = 8;
+
+// Queue the batched launches of `count` jobs (all in `mode`) on `s`: the
+// region stage, and the seven stages from its coefficients to the files.  A
+// persistent region stage (shape.region_wgs != 0) claims its regions through
+// the device counters at `counters`, which a one-workgroup launch clears
+// first.
+void launch_batch_regions(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
+                          std::uint32_t mode, const BatchShape& shape, std::uint32_t* counters);
+void launch_batch_files(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages]);
 
 }  // namespace cjx

@@ -126,7 +126,14 @@ __global__ __launch_bounds__(256) void assemble_batch_kernel(const FrameJob* __r
     assemble_kernel_body(wg, j.geo, j.k, j.lay, P, j.out, j.cap);
 }
 
-void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32_t band_wgs,
+// Tokenizer workgroups of a batch, about: two resident rounds of 256 CUs,
+// shared out by the frames' blocks.  A workgroup pays a prologue and writes an
+// 8 KB histogram row that the next stage sums, so a small frame of a large
+// batch gets few: 16 frames of 640x360 to 3840x2160 1253 -> 1175 us against up
+// to 1,024 workgroups for each frame, eight frames of 3840x2160 1804 -> 1778.
+constexpr std::uint64_t kBatchTokenWgs = 4096;
+
+void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint64_t blocks, std::uint32_t band_wgs,
                        StageGrid (&g)[kBStages]) {
     const auto set = [&](BatchStage s, std::uint32_t nx, std::uint32_t ny) {
         g[s] = StageGrid{0, nx > 0 ? nx : 1, ny > 0 ? ny : 1, 0};
@@ -135,9 +142,10 @@ void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32
     set(kBRegion, 8 * ((geo.rw * geo.rh + 7) / 8), 1);
     set(kBQuantize, geo.cmw * geo.cmh, 1);
     const std::uint32_t waves{(3 * geo.nblocks + 3) / 4};
-    std::uint32_t cap{shape.token_cap < static_cast<std::uint32_t>(kTokenGrid) ? shape.token_cap
-                                                                               : static_cast<std::uint32_t>(kTokenGrid)};
-    set(kBTokens, waves < cap ? waves : cap, 1);
+    // A frame's share of the tokenizer's workgroups.
+    const std::uint64_t share{(kBatchTokenWgs * static_cast<std::uint64_t>(geo.nblocks) + blocks - 1) / blocks};
+    const std::uint32_t cap{std::min<std::uint32_t>(shape.token_cap, kTokenGrid)};
+    set(kBTokens, std::min({waves, cap, static_cast<std::uint32_t>(share)}), 1);
     set(kBHistograms, kReduceWgs + dc_wgs, 1);
     set(kBHuffman, kNumClusters + 2 * geo.num_dc, 1);
     set(kBEmit, geo.num_ac * kGroupBands * band_wgs + dc_wgs, 1);
@@ -150,8 +158,8 @@ void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint32
     set(kBAssemble, ag < run_wgs ? static_cast<std::uint32_t>(ag) : run_wgs, 1);
 }
 
-void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
-                  std::uint32_t mode, const BatchShape& shape, std::uint32_t* counters) {
+void launch_batch_regions(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages],
+                          std::uint32_t mode, const BatchShape& shape, std::uint32_t* counters) {
     const bool mf{(mode & kModeMfma16) != 0}, learned{(mode & kModeLearned) != 0};
     if (shape.region_wgs == 0) {
         auto* const region{mf ? (learned ? region_batch_kernel<true, true> : region_batch_kernel<true, false>)
@@ -165,6 +173,9 @@ void launch_batch(hipStream_t s, const FrameJob* jobs, int count, const std::uin
         clear_counters_kernel<<<1, 64, 0, s>>>(counters);
         region<<<shape.region_wgs, 256, 0, s>>>(jobs, count, total[kBRegion], counters);
     }
+}
+
+void launch_batch_files(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages]) {
     quantize_batch_kernel<<<total[kBQuantize], 256, 0, s>>>(jobs, count);
     tokens_batch_kernel<<<total[kBTokens], 256, 0, s>>>(jobs, count);
     histograms_batch_kernel<<<total[kBHistograms], 256, 0, s>>>(jobs, count);

@@ -20,6 +20,7 @@ namespace cjx {
 class BatchEncoder {
 public:
     static constexpr int kMaxBatch = 256;
+    static constexpr int kMaxParts = 3;  // branches of a batch's graph
 
     BatchEncoder() = default;
     ~BatchEncoder();
@@ -61,10 +62,9 @@ private:
     std::vector<std::unique_ptr<Encoder>> frames_;
     std::vector<FrameJob> jobs_;
     std::vector<std::size_t> out_off_, caps_;
-    std::uint32_t total_[kBStages]{};
     void* arena_{nullptr};
     FrameJob* jobs_dev_{nullptr};
-    std::uint32_t* counters_{nullptr};  // the persistent region stage's claim counters (8)
+    std::uint32_t* counters_{nullptr};  // the persistent region stages' claim counters, kRegionCounters a part
     std::uint8_t* out_host_{nullptr};
     std::uint64_t* sizes_host_{nullptr};
     hipStream_t stream_{nullptr};
