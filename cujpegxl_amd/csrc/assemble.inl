@@ -60,15 +60,15 @@ struct Layout {
 // create_huffman_tree's count floors 1, 2, 4, ... are independent trials, so
 // in round r wave w tries floor 2^(8r + w), and the smallest floor whose tree
 // fits 15 bits wins (the serial builder stops at that same floor); floors up
-// to 2^7 take one round.  Floors above 2^15 continue on wave 0.  Wave 0 then
-// builds the codes and the header.
+// to 2^7 take one round.  Wave 0 then builds the codes and the header.
 constexpr int kTrials = 8;
-constexpr int kTrialRounds = 2;
 
 struct HuffmanShared {
     WaveHuffScratch trial[kTrials];
     std::uint8_t trial_depth[kTrials][kHistStride];
-    std::uint32_t trial_max[kTrials];
+    std::uint32_t trial_fits[kTrials];
+    alignas(16) std::uint32_t leaf[kHistStride];  // counts in input order
+    std::uint32_t rank[kHistStride];              // by symbol
     WaveCodeScratch code_scratch;
     std::uint32_t hist[kHistStride];
     std::uint8_t depth[kHistStride];
@@ -84,42 +84,61 @@ __device__ void huffman_depths(HuffmanShared& S, int alpha) {
     if (L.n < 2) {
         return;  // one symbol or none: the simple header, all depths stay 0
     }
+    // Ranks in the stable order of the counts, every wave against its share of
+    // the leaves.
+    constexpr int kShare{64 * R / kTrials};
+    static_assert(kShare % 4 == 0, "four leaves per read");
+    if (w == 0) {
+#pragma unroll
+        for (int r{0}; r < R; ++r) {
+            if (L.cnt[r] != 0) {
+                S.leaf[L.pos[r]] = L.cnt[r];
+            }
+        }
+    }
+    __syncthreads();
+    std::uint32_t rank[R]{};
+    if (kShare * w < L.n) {
+#pragma unroll
+        for (int b{0}; b < kShare; b += 4) {
+            const uint4 x{*reinterpret_cast<const uint4*>(&S.leaf[kShare * w + b])};
+            rank_after<R>(L, x.x, kShare * w + b, rank);
+            rank_after<R>(L, x.y, kShare * w + b + 1, rank);
+            rank_after<R>(L, x.z, kShare * w + b + 2, rank);
+            rank_after<R>(L, x.w, kShare * w + b + 3, rank);
+        }
+#pragma unroll
+        for (int r{0}; r < R; ++r) {
+            if (L.cnt[r] != 0) {
+                atomicAdd(&S.rank[64 * r + lane], rank[r]);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r{0}; r < R; ++r) {
+        rank[r] = S.rank[64 * r + lane];
+    }
     int win{-1};
-    for (int round{0}; round < kTrialRounds && win < 0; ++round) {
+    for (int round{0}; win < 0; ++round) {
         if (round > 0) {
             for (int i{lane}; i < kHistStride; i += 64) {
                 S.trial_depth[w][i] = 0;
             }
             wave_sync();
         }
-        const std::uint32_t maxd{tree_trial<R>(L, 1u << (round * kTrials + w), S.trial_depth[w], S.trial[w])};
+        // A floor of 2^31 makes every count equal: no tree is higher than 8.
+        const bool fits{tree_trial<R, 64 * R>(L, rank, 1u << min(round * kTrials + w, 31), 15, S.trial_depth[w], S.trial[w])};
         if (lane == 0) {
-            S.trial_max[w] = maxd;
+            S.trial_fits[w] = fits ? 1u : 0u;
         }
         __syncthreads();
-        for (int i{0}; i < kTrials; ++i) {
-            if (S.trial_max[i] <= 15u) {
-                win = i;
-                break;
-            }
-        }
+        const std::uint64_t all{__ballot(lane < kTrials && S.trial_fits[lane % kTrials] != 0)};
+        win = all != 0 ? static_cast<int>(__builtin_ctzll(all)) : -1;
         __syncthreads();
     }
-    if (win < 0 && w == 0) {
-        for (std::uint32_t count_limit{1u << (kTrials * kTrialRounds)};; count_limit *= 2) {
-            for (int i{static_cast<int>(threadIdx.x)}; i < kHistStride; i += 64) {
-                S.trial_depth[0][i] = 0;
-            }
-            wave_sync();
-            if (tree_trial<R>(L, count_limit, S.trial_depth[0], S.trial[0]) <= 15u) {
-                break;
-            }
-        }
-    }
-    __syncthreads();
-    const int src{win < 0 ? 0 : win};
     for (int i{static_cast<int>(threadIdx.x)}; i < kHistStride; i += 64 * kTrials) {
-        S.depth[i] = S.trial_depth[src][i];
+        S.depth[i] = S.trial_depth[win][i];
     }
 }
 
@@ -131,6 +150,8 @@ __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const 
     const int w{t >> 6};
     for (int i{t}; i < kHistStride; i += 64 * kTrials) {
         S.hist[i] = hists[h * kHistStride + i];
+        S.leaf[i] = kQueueEnd;  // where no leaf is: after every leaf
+        S.rank[i] = 0;
         S.depth[i] = 0;
         S.code[i] = 0;
     }
@@ -141,13 +162,14 @@ __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const 
         S.hdr[t] = 0;
     }
     __syncthreads();
-    std::uint32_t top{0};
-    for (int i{t & 63}; i < kHistStride; i += 64) {
-        if (S.hist[i] != 0) {
-            top = static_cast<std::uint32_t>(i) + 1u;
+    int alpha{1};
+#pragma unroll
+    for (int r{0}; r < kHistStride / 64; ++r) {
+        const std::uint64_t m{__ballot(S.hist[64 * r + (t & 63)] != 0)};
+        if (m != 0) {
+            alpha = 64 * r + 64 - static_cast<int>(__builtin_clzll(m));
         }
     }
-    const int alpha{static_cast<int>(wave_max_u32(top > 1u ? top : 1u))};
     if (alpha > 1) {
         if (alpha <= 64) {
             huffman_depths<1>(S, alpha);
@@ -158,8 +180,15 @@ __device__ __attribute__((always_inline)) inline void huffman_kernel_body(const 
     __syncthreads();
     std::uint32_t nbits{0};
     if (w == 0 && alpha > 1) {
-        nbits = alpha <= 64 ? wave_finish_code<1>(S.hist, alpha, S.depth, S.code, S.hdr, kHdrWords, S.code_scratch)
-                            : wave_finish_code<4>(S.hist, alpha, S.depth, S.code, S.hdr, kHdrWords, S.code_scratch);
+        nbits = alpha <= 64 ? wave_store_code<1>(S.hist, alpha, S.depth, S.hdr, kHdrWords, S.code_scratch)
+                            : wave_store_code<4>(S.hist, alpha, S.depth, S.hdr, kHdrWords, S.code_scratch);
+    }
+    if (w == 1 && alpha > 1) {  // all depths 0 (one symbol or none): no code
+        if (alpha <= 64) {
+            wave_depths_to_codes<1>(S.depth, alpha, S.code);
+        } else {
+            wave_depths_to_codes<4>(S.depth, alpha, S.code);
+        }
     }
     __syncthreads();
     for (int i{t}; i < kHistStride; i += 64 * kTrials) {

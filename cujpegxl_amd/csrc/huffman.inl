@@ -5,22 +5,26 @@
 // count floor doubled until the depth limit holds, canonical LSB-first codes,
 // simple / code-length-code headers.  The parallel parts:
 //   - leaf positions from ballots, the stable sort as a rank computation over
-//     (count, leaf position);
-//   - the two-queue merge and the top-down depth walk stay sequential, but
-//     their queues live in VGPRs (one value per lane, read with readlane and
-//     written with a lane select at a wave-uniform index), so no step waits on
-//     memory;
+//     (count, leaf position), every wave of a workgroup against its share of
+//     the leaves; a count floor only regroups the ranks;
+//   - the two-queue merge stays sequential, but its queues live in VGPRs (one
+//     value per lane, read and written at a wave-uniform lane), so no step
+//     waits on memory; the depths of up to 64 leaves by pointer jumping, of
+//     more by a top-down walk;
 //   - canonical codes from per-depth ballot ranks;
 //   - the code-length-coded header as a wave scan of per-symbol bit lengths.
 // Every lane runs the same control flow; loop bounds and queue indices are
 // wave-uniform.
+//
+// What bounds it: one wave's chain of instructions (the merge of up to 64
+// leaves, then the header), issued at six to eight cycles each, and the first
+// fetch of its code.  All histograms of a frame run side by side: 9.4 us at
+// 320x240 and 11.2 us at 3840x2160 (15.7 and 19.7 with a merge step of 345
+// cycles, the sort in every wave and the codes before the header).
 
 namespace cjx {
 
 constexpr std::uint32_t kQueueEnd = 0xffffffffu;
-
-// Orders one wave's LDS accesses (its LDS instructions execute in order; this
-// keeps the compiler from moving them across the point).
 
 // R values per lane: element idx lives in register idx / 64 of lane idx % 64.
 template <int R>
@@ -56,20 +60,11 @@ struct LaneArray {
     }
 };
 
-__device__ __forceinline__ std::uint32_t wave_max_u32(std::uint32_t v) {
-#pragma unroll
-    for (int off{32}; off > 0; off >>= 1) {
-        const std::uint32_t o{static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(v), off, 64))};
-        v = o > v ? o : v;
-    }
-    return v;
-}
-
 // LDS scratch of one wave's build.
 struct WaveHuffScratch {
-    std::uint32_t leaf_total[256];  // input order
-    std::uint32_t sorted_total[256];
+    std::uint32_t sorted_total[256 + 1];
     std::uint32_t sorted_symbol[256];
+    std::uint32_t parent[128];  // of leaf i; of internal node k at 64 + k
 };
 
 // Value of x in lane `src` (wave-uniform) of the wave.
@@ -77,89 +72,112 @@ __device__ __forceinline__ std::uint32_t lane_value(std::uint32_t x, int src) {
     return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), src));
 }
 
+// old with lane `lane` (wave-uniform) replaced by x (wave-uniform).
+extern "C" __device__ int cjx_write_lane(int x, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 // The merge and depths below for n <= 64 leaves.  Each queue is one VGPR
-// (lane = queue index) and a merge step has no branch: the two picks are
-// selects on wave-uniform values.  The depths come from the parent links by
-// pointer jumping: every node holds (distance d, ancestor p), initially
-// (1, parent) and (0, root) at the root, and six rounds of d += d[p],
-// p = p[p] leave each node's depth in d (depths are below 64).  Ancestors
-// are internal nodes, so every lookup reads the internal nodes' registers.
+// (lane = queue index); entries that are not there are kQueueEnd.  A merge
+// step takes the two smallest of the two queues' first two (both leaves, both
+// internal nodes, or one of each; leaves first on ties).  One wave issues an
+// instruction every six to eight cycles here, whatever it is, so the step is
+// kept short and has no branch: minima of the four entries give the new node's
+// total, two compares move the leaf queue, the other queue follows from the
+// count of taken entries, and only the leaf queue's position is kept of the
+// picks.  From those each step's lane writes the parent links of the entries
+// it took, and the depths come from the links by pointer jumping: every node
+// holds (distance d, ancestor p), initially (1, parent) and (0, root) at the
+// root, packed as p | d << 8, and six rounds of d += d[p], p = p[p] leave each
+// node's depth in d (depths are below 64).  Ancestors are internal nodes, so
+// every lookup reads the internal nodes' register.
+// (Picks by two selects with child links stored per step: 345 cycles a step;
+// with branches 400; this form: 170.)  kFull: lane numbers may run
+// past the last lane.
+template <bool kFull>
 __device__ std::uint32_t merge_depths_small(WaveHuffScratch& s, int n, std::uint8_t* depth) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
     const std::uint32_t leaf{lane < n ? s.sorted_total[lane] : kQueueEnd};
+    const std::uint32_t leaf1{lane + 1 < n ? s.sorted_total[lane + 1] : kQueueEnd};
     const std::uint32_t sym{lane < n ? s.sorted_symbol[lane] : 0u};
-    // Two-queue merge: leaves (tree index i < n) and internal nodes
-    // (internal k = tree index n + 1 + k), smaller total first, leaf on ties;
-    // internal nodes not yet made read as kQueueEnd.
-    std::uint32_t inner{kQueueEnd}, kid_l{0}, kid_r{0};
-    int i{0}, j{0};
-    for (int k{0}; k < n - 1; ++k) {
-        const std::uint32_t a0{i < n ? lane_value(leaf, i) : kQueueEnd};
-        const std::uint32_t b0{lane_value(inner, j)};
-        const bool leaf0{a0 <= b0};
-        const std::uint32_t t0{leaf0 ? a0 : b0};
-        const int c0{leaf0 ? i : n + 1 + j};
-        i += leaf0 ? 1 : 0;
-        j += leaf0 ? 0 : 1;
-        const std::uint32_t a1{i < n ? lane_value(leaf, i) : kQueueEnd};
-        const std::uint32_t b1{lane_value(inner, j)};
-        const bool leaf1{a1 <= b1};
-        const std::uint32_t t1{leaf1 ? a1 : b1};
-        const int c1{leaf1 ? i : n + 1 + j};
-        i += leaf1 ? 1 : 0;
-        j += leaf1 ? 0 : 1;
-        if (lane == k) {
-            inner = t0 + t1;
-            kid_l = static_cast<std::uint32_t>(c0);
-            kid_r = static_cast<std::uint32_t>(c1);
+    std::uint32_t inner{kQueueEnd}, taken{0};
+    // In scalar registers from the start (a constant may be shared with a
+    // vector's, and the loop moved to vector instructions with it).
+    int i, j, k, both;
+    asm("s_mov_b32 %0, 0" : "=s"(i));
+    asm("s_mov_b32 %0, 0" : "=s"(j));
+    asm("s_mov_b32 %0, 0" : "=s"(k));
+    asm("s_mov_b32 %0, 2" : "=s"(both));  // entries taken after the step
+    for (; k < n - 1; ++k, both += 2) {
+        std::uint32_t a0{lane_value(leaf, i)}, a1{lane_value(leaf1, i)};
+        if constexpr (kFull) {
+            asm("s_cmp_gt_i32 %[i], 63\n\t"
+                "s_cselect_b32 %[a0], -1, %[a0]\n\t"
+                "s_cselect_b32 %[a1], -1, %[a1]"
+                : [a0] "+s"(a0), [a1] "+s"(a1)
+                : [i] "s"(i)
+                : "scc");
         }
+        const std::uint32_t b0{lane_value(inner, j)}, b1{lane_value(inner, j + 1)};
+        std::uint32_t sum, t, u;
+        asm("s_min_u32 %[sum], %[a0], %[b0]\n\t"
+            "s_max_u32 %[t], %[a0], %[b0]\n\t"
+            "s_min_u32 %[u], %[a1], %[b1]\n\t"
+            "s_min_u32 %[t], %[t], %[u]\n\t"
+            "s_add_u32 %[sum], %[sum], %[t]\n\t"
+            "s_cmp_le_u32 %[a1], %[b0]\n\t"   // two leaves
+            "s_addc_u32 %[i], %[i], 1\n\t"
+            "s_cmp_lt_u32 %[b1], %[a0]\n\t"   // no leaf
+            "s_subb_u32 %[i], %[i], 0\n\t"
+            "s_sub_i32 %[j], %[both], %[i]"
+            : [i] "+s"(i), [j] "=&s"(j), [sum] "=&s"(sum), [t] "=&s"(t), [u] "=&s"(u)
+            : [a0] "s"(a0), [a1] "s"(a1), [b0] "s"(b0), [b1] "s"(b1), [both] "s"(both)
+            : "scc");
+        inner = static_cast<std::uint32_t>(cjx_write_lane(static_cast<int>(sum), k, static_cast<int>(inner)));
+        taken = static_cast<std::uint32_t>(cjx_write_lane(i, k, static_cast<int>(taken)));
     }
-    // Parent links in LDS (leaf_total is dead after the sort): node ids are
-    // leaf i -> i, internal k -> 64 + k; the root (internal n - 2) is its own
-    // parent.
-    std::uint32_t* const par{s.leaf_total};
-    const std::uint32_t root{64u + static_cast<std::uint32_t>(n - 2)};
-    if (lane < n - 1) {
-        const std::uint32_t me{64u + static_cast<std::uint32_t>(lane)};
-        const int nn{n};
-        par[kid_l < static_cast<std::uint32_t>(nn) ? kid_l : kid_l - static_cast<std::uint32_t>(nn) - 1u + 64u] = me;
-        par[kid_r < static_cast<std::uint32_t>(nn) ? kid_r : kid_r - static_cast<std::uint32_t>(nn) - 1u + 64u] = me;
+    // Step k took leaves [i0, i1) and internal nodes [2k - i0, 2k + 2 - i1).
+    {
+        const int i1{static_cast<int>(taken)};
+        const int i0{__builtin_amdgcn_update_dpp(0, i1, 0x138, 0xf, 0xf, false)};  // the lane below's; 0 in lane 0
+        const std::uint32_t me{static_cast<std::uint32_t>(lane)};
+        if (lane < n - 1) {
+            if (i1 > i0) {
+                s.parent[i0] = me;
+            }
+            if (i1 > i0 + 1) {
+                s.parent[i0 + 1] = me;
+            }
+            const int j0{2 * lane - i0};
+            if (i1 < i0 + 2) {
+                s.parent[64 + j0] = me;
+            }
+            if (i1 == i0) {
+                s.parent[64 + j0 + 1] = me;
+            }
+        }
+        wave_sync();
     }
-    if (lane == 0) {
-        par[root] = root;
-    }
-    wave_sync();
-    std::uint32_t pa{lane < n ? par[lane] : root};
-    std::uint32_t pb{lane < n - 1 ? par[64 + lane] : root};
-    std::uint32_t da{lane < n ? 1u : 0u};
-    std::uint32_t db{lane < n - 2 ? 1u : 0u};
-    wave_sync();
+    const std::uint32_t up_leaf{s.parent[lane]}, up_inner{s.parent[64 + lane]};
+    const std::uint32_t root{static_cast<std::uint32_t>(n - 2)};
+    std::uint32_t a{lane < n ? (up_leaf | 256u) : root};
+    std::uint32_t b{lane < n - 2 ? (up_inner | 256u) : root};
 #pragma unroll
     for (int r{0}; r < 6; ++r) {
-        const int ia{static_cast<int>(pa - 64u)}, ib{static_cast<int>(pb - 64u)};
-        const std::uint32_t d_a{static_cast<std::uint32_t>(__shfl(static_cast<int>(db), ia, 64))};
-        const std::uint32_t p_a{static_cast<std::uint32_t>(__shfl(static_cast<int>(pb), ia, 64))};
-        const std::uint32_t d_b{static_cast<std::uint32_t>(__shfl(static_cast<int>(db), ib, 64))};
-        const std::uint32_t p_b{static_cast<std::uint32_t>(__shfl(static_cast<int>(pb), ib, 64))};
-        da += d_a;
-        pa = p_a;
-        db += d_b;
-        pb = p_b;
+        const std::uint32_t xa{static_cast<std::uint32_t>(__shfl(static_cast<int>(b), static_cast<int>(a & 255u), 64))};
+        const std::uint32_t xb{static_cast<std::uint32_t>(__shfl(static_cast<int>(b), static_cast<int>(b & 255u), 64))};
+        a = (a & ~255u) + xa;
+        b = (b & ~255u) + xb;
     }
     if (lane < n) {
-        depth[sym] = static_cast<std::uint8_t>(da);
+        depth[sym] = static_cast<std::uint8_t>(a >> 8);
     }
-    return lane < n ? da : 0u;
+    return lane < n ? a >> 8 : 0u;
 }
 
 // Two-queue merge and top-down depths of the n (>= 2) sorted leaves in
 // s.sorted_total / s.sorted_symbol; writes depth[symbol] and returns this
 // lane's largest leaf depth.  Q * 64 >= n.
 template <int Q>
-__device__ std::uint32_t merge_depths(WaveHuffScratch& s, int n, std::uint8_t* depth) {
-    if constexpr (Q == 1) {
-        return merge_depths_small(s, n, depth);
-    }
+__device__ std::uint32_t merge_depths_large(WaveHuffScratch& s, int n, std::uint8_t* depth) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
     LaneArray<Q> leaf{}, sym{};
 #pragma unroll
@@ -262,71 +280,82 @@ __device__ __forceinline__ Leaves<R> wave_leaves(const std::uint32_t* data, int 
     return L;
 }
 
-// One pass of create_huffman_tree's loop (prefix_code.cc:36-96) with count
-// floor `count_limit` for n >= 2 leaves: writes depth[symbol] of every present
-// symbol and returns the largest depth (wave-uniform).
+// Whether each present leaf comes after a leaf of count x at input position
+// `at` in the stable ascending order of the counts, added to its rank.
 template <int R>
-__device__ std::uint32_t tree_trial(const Leaves<R>& L, std::uint32_t count_limit, std::uint8_t* depth,
-                                    WaveHuffScratch& s) {
-    const int lane{static_cast<int>(threadIdx.x) & 63};
-    const int n{L.n};
-    std::uint32_t tot[R];
+__device__ __forceinline__ void rank_after(const Leaves<R>& L, std::uint32_t x, int at, std::uint32_t (&rank)[R]) {
 #pragma unroll
     for (int r{0}; r < R; ++r) {
-        tot[r] = L.cnt[r] > count_limit - 1 ? L.cnt[r] : count_limit - 1;
-        if (L.cnt[r] != 0) {
-            s.leaf_total[L.pos[r]] = tot[r];
-        }
+        rank[r] += x < L.cnt[r] + (at < L.pos[r] ? 1u : 0u) ? 1u : 0u;
     }
-    wave_sync();
-    // Stable ascending sort: rank = smaller totals + equal totals earlier.
-    int rank[R];
-#pragma unroll
-    for (int r{0}; r < R; ++r) {
-        rank[r] = 0;
-    }
-    for (int b{0}; b < n; ++b) {
-        const std::uint32_t t{s.leaf_total[b]};
-#pragma unroll
-        for (int r{0}; r < R; ++r) {
-            rank[r] += (t < tot[r] || (t == tot[r] && b < L.pos[r])) ? 1 : 0;
-        }
-    }
-#pragma unroll
-    for (int r{0}; r < R; ++r) {
-        if (L.cnt[r] != 0) {
-            s.sorted_total[rank[r]] = tot[r];
-            s.sorted_symbol[rank[r]] = static_cast<std::uint32_t>(64 * r + lane);
-        }
-    }
-    wave_sync();
-    const std::uint32_t maxd{n <= 64 ? merge_depths<1>(s, n, depth) : merge_depths<4>(s, n, depth)};
-    wave_sync();
-    return wave_max_u32(maxd);
 }
 
-// create_huffman_tree (prefix_code.cc:36-96) by one wave, floors tried in
-// order.  data[0..length) and depth[0..length) are in LDS; depth is zero on
-// entry for absent symbols.  R * 64 >= length.
-template <int R>
+// One pass of create_huffman_tree's loop (prefix_code.cc:36-96) with count
+// floor `count_limit` for n >= 2 leaves (at most kMost) of the given ranks by
+// (count, input position): writes depth[symbol] of every present symbol and
+// returns whether no depth is above `limit`.
+// (kMost keeps merges that cannot be needed out of the code: the kernel runs
+// once over most of it, so what it is long it also waits to fetch.)
+template <int R, int kMost>
+__device__ bool tree_trial(const Leaves<R>& L, const std::uint32_t (&rank)[R], std::uint32_t count_limit, int limit,
+                           std::uint8_t* depth, WaveHuffScratch& s) {
+    const int lane{static_cast<int>(threadIdx.x) & 63};
+    const int n{L.n};
+    // The floor makes the counts below it equal: those leaves come first, in
+    // input order (descending symbol), the others keep their ranks.
+    const std::uint32_t least{count_limit - 1};
+    const std::uint64_t above{lane == 63 ? 0ull : (~0ull << (lane + 1))};
+    int higher{0};
+#pragma unroll
+    for (int r{R - 1}; r >= 0; --r) {
+        const bool low{L.cnt[r] != 0 && L.cnt[r] <= least};
+        const std::uint64_t lows{__ballot(low)};
+        if (L.cnt[r] != 0) {
+            const std::uint32_t at{low ? static_cast<std::uint32_t>(higher + __popcll(lows & above)) : rank[r]};
+            s.sorted_total[at] = low ? least : L.cnt[r];
+            s.sorted_symbol[at] = static_cast<std::uint32_t>(64 * r + lane);
+        }
+        higher += __popcll(lows);
+    }
+    wave_sync();
+    std::uint32_t maxd{0};
+    if (kMost <= 62 || n <= 62) {
+        maxd = merge_depths_small<false>(s, n, depth);
+    } else if (kMost <= 64 || n <= 64) {
+        maxd = merge_depths_small<true>(s, n, depth);
+    } else {
+        maxd = merge_depths_large<4>(s, n, depth);
+    }
+    wave_sync();
+    return __ballot(maxd > static_cast<std::uint32_t>(limit)) == 0;
+}
+
+// create_huffman_tree (prefix_code.cc:36-96) of at most kMost <= 64 symbols by
+// one wave, floors tried in order.  data[0..length) and depth[0..length) are
+// in LDS; depth is zero on entry for absent symbols.
+template <int kMost>
 __device__ void wave_create_tree(const std::uint32_t* data, int length, int limit, std::uint8_t* depth,
                                  WaveHuffScratch& s) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
-    const Leaves<R> L{wave_leaves<R>(data, length)};
+    const Leaves<1> L{wave_leaves<1>(data, length)};
     if (L.n == 0) {
         return;
     }
     if (L.n == 1) {
-#pragma unroll
-        for (int r{0}; r < R; ++r) {
-            if (L.cnt[r] != 0) {
-                depth[64 * r + lane] = 1;
-            }
+        if (L.cnt[0] != 0) {
+            depth[lane] = 1;
         }
         return;
     }
+    std::uint32_t rank[1]{0};
+#pragma unroll
+    for (int sym{0}; sym < kMost; ++sym) {
+        const std::uint32_t x{lane_value(L.cnt[0], sym)};
+        // Equal counts: the higher symbol first.
+        rank[0] += x - 1u < L.cnt[0] - 1u + (lane < sym ? 1u : 0u) ? 1u : 0u;  // x = 0 is no leaf
+    }
     for (std::uint32_t count_limit{1};; count_limit *= 2) {
-        if (static_cast<int>(tree_trial<R>(L, count_limit, depth, s)) <= limit) {
+        if (tree_trial<1, kMost>(L, rank, count_limit, limit, depth, s)) {
             return;
         }
     }
@@ -336,38 +365,31 @@ __device__ void wave_create_tree(const std::uint32_t* data, int length, int limi
 template <int R>
 __device__ void wave_depths_to_codes(const std::uint8_t* depth, int len, std::uint16_t* bits) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
-    const std::uint64_t below{(1ull << lane) - 1ull};
     int dep[R];
+    std::uint32_t mine[R];
 #pragma unroll
     for (int r{0}; r < R; ++r) {
         const int sym{64 * r + lane};
         dep[r] = sym < len ? depth[sym] : 0;
+        mine[r] = 0;
     }
-    std::uint32_t next[16];
-    {
-        std::uint32_t code{0}, prev{0};
-        next[0] = 0;
-        for (int d{1}; d < 16; ++d) {
-            code = (code + prev) << 1;
-            next[d] = code;
-            std::uint32_t c{0};
+    std::uint32_t next{0};  // the next code of the depth
 #pragma unroll
-            for (int r{0}; r < R; ++r) {
-                c += static_cast<std::uint32_t>(__popcll(__ballot(dep[r] == d)));
-            }
-            prev = c;
-        }
-    }
     for (int d{1}; d < 16; ++d) {
-        std::uint32_t base{next[d]};
 #pragma unroll
         for (int r{0}; r < R; ++r) {
             const std::uint64_t m{__ballot(dep[r] == d)};
-            if (dep[r] == d) {
-                const std::uint32_t c{base + static_cast<std::uint32_t>(__popcll(m & below))};
-                bits[64 * r + lane] = static_cast<std::uint16_t>(__builtin_bitreverse32(c) >> (32 - d));
-            }
-            base += static_cast<std::uint32_t>(__popcll(m));
+            const std::uint32_t code{__builtin_amdgcn_mbcnt_hi(
+                static_cast<std::uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<std::uint32_t>(m), next))};
+            mine[r] = dep[r] == d ? code : mine[r];
+            next += static_cast<std::uint32_t>(__popcll(m));
+        }
+        next <<= 1;
+    }
+#pragma unroll
+    for (int r{0}; r < R; ++r) {
+        if (dep[r] != 0) {
+            bits[64 * r + lane] = static_cast<std::uint16_t>(__builtin_bitreverse32(mine[r]) >> (32 - dep[r]));
         }
     }
 }
@@ -387,45 +409,35 @@ __device__ std::uint32_t wave_store_tree(const std::uint8_t* depth, int num, std
                                          std::uint32_t cap, WaveCodeScratch& s) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
     int dep[R];
-    std::uint32_t last{0};
+    int new_len{0};
 #pragma unroll
     for (int r{0}; r < R; ++r) {
         const int sym{64 * r + lane};
         dep[r] = sym < num ? depth[sym] : 0;
-        if (dep[r] != 0) {
-            last = static_cast<std::uint32_t>(sym) + 1u;
+        const std::uint64_t m{__ballot(dep[r] != 0)};
+        if (m != 0) {
+            new_len = 64 * r + 64 - static_cast<int>(__builtin_clzll(m));
         }
     }
-    const int new_len{static_cast<int>(wave_max_u32(last))};
     // Histogram of depth values over [0, new_len).
-    for (int v{0}; v < 18; ++v) {
-        std::uint32_t c{0};
-#pragma unroll
-        for (int r{0}; r < R; ++r) {
-            c += static_cast<std::uint32_t>(__popcll(__ballot(64 * r + lane < new_len && dep[r] == v)));
-        }
-        if (lane == 0) {
-            s.cl_hist[v] = c;
-        }
-    }
     if (lane < 18) {
+        s.cl_hist[lane] = 0;
         s.cl_depth[lane] = 0;
         s.cl_bits[lane] = 0;
     }
     wave_sync();
-    int num_codes{0}, code{0};
-    for (int i{0}; i < 18; ++i) {
-        if (s.cl_hist[i]) {
-            if (num_codes == 0) {
-                code = i;
-                num_codes = 1;
-            } else if (num_codes == 1) {
-                num_codes = 2;
-                break;
-            }
+#pragma unroll
+    for (int r{0}; r < R; ++r) {
+        if (64 * r + lane < new_len) {
+            atomicAdd(&s.cl_hist[dep[r]], 1u);
         }
     }
-    wave_create_tree<1>(s.cl_hist, 18, 5, s.cl_depth, s.tree);
+    wave_sync();
+    const std::uint32_t uses{lane < 18 ? s.cl_hist[lane] : 0u};
+    const std::uint64_t used{__ballot(uses != 0)};
+    const int num_codes{used == 0 ? 0 : ((used & (used - 1)) == 0 ? 1 : 2)};  // 2: two or more
+    const int code{used == 0 ? 0 : static_cast<int>(__builtin_ctzll(used))};
+    wave_create_tree<18>(s.cl_hist, 18, 5, s.cl_depth, s.tree);
     wave_sync();
     wave_depths_to_codes<1>(s.cl_depth, 18, s.cl_bits);
     wave_sync();
@@ -483,13 +495,12 @@ __device__ std::uint32_t wave_store_tree(const std::uint8_t* depth, int num, std
 
 // build_and_store_huffman_tree (prefix_code.cc:358-397) for hist[0..alpha),
 // alpha >= 2, with depth[] already holding create_huffman_tree's result when
-// more than one symbol is present (all zero otherwise); bits are zeroed by the
-// caller.  One wave.  Returns the header length in bits, or 0 if it would not
-// fit `cap` words.
+// more than one symbol is present (all zero otherwise): the header, by one
+// wave.  (The codes are wave_depths_to_codes' from the same depths.)  Returns
+// the header length in bits, or 0 if it would not fit `cap` words.
 template <int R>
-__device__ std::uint32_t wave_finish_code(const std::uint32_t* hist, int alpha, const std::uint8_t* depth,
-                                          std::uint16_t* bits, std::uint32_t* hdr, std::uint32_t cap,
-                                          WaveCodeScratch& s) {
+__device__ std::uint32_t wave_store_code(const std::uint32_t* hist, int alpha, const std::uint8_t* depth,
+                                         std::uint32_t* hdr, std::uint32_t cap, WaveCodeScratch& s) {
     const int lane{static_cast<int>(threadIdx.x) & 63};
     std::uint64_t present[R];
     int count{0};
@@ -499,7 +510,11 @@ __device__ std::uint32_t wave_finish_code(const std::uint32_t* hist, int alpha, 
         present[r] = __ballot(sym < alpha && hist[sym] != 0);
         count += __popcll(present[r]);
     }
-    // The first four present symbols, ascending.
+    if (count > 4) {
+        const std::uint32_t nb{wave_store_tree<R>(depth, alpha, hdr, cap, s)};
+        return nb <= cap * 32 ? nb : 0u;
+    }
+    // The present symbols, ascending.
     int s4[4]{0, 0, 0, 0};
     {
         int got{0};
@@ -516,22 +531,13 @@ __device__ std::uint32_t wave_finish_code(const std::uint32_t* hist, int alpha, 
     for (int c{alpha - 1}; c; c >>= 1) {
         ++max_bits;
     }
-    if (count <= 1) {
-        std::uint32_t pos{0};
-        if (lane == 0) {
-            BitSink w{hdr, 0, cap * 32};
+    std::uint32_t pos{0};
+    if (lane == 0) {
+        BitSink w{hdr, 0, cap * 32};
+        if (count <= 1) {
             w.write(4, 1);
             w.write(static_cast<std::uint32_t>(max_bits), static_cast<std::uint32_t>(s4[0]));
-            pos = w.ok() ? w.pos : 0u;
-        }
-        return static_cast<std::uint32_t>(__shfl(static_cast<int>(pos), 0, 64));
-    }
-    wave_depths_to_codes<R>(depth, alpha, bits);
-    wave_sync();
-    if (count <= 4) {
-        std::uint32_t pos{0};
-        if (lane == 0) {
-            BitSink w{hdr, 0, cap * 32};
+        } else {
             w.write(2, 1);
             w.write(2, static_cast<std::uint32_t>(count - 1));
             for (int i{0}; i < count; ++i) {
@@ -549,12 +555,10 @@ __device__ std::uint32_t wave_finish_code(const std::uint32_t* hist, int alpha, 
             if (count == 4) {
                 w.write(1, depth[s4[0]] == 1 ? 1u : 0u);
             }
-            pos = w.ok() ? w.pos : 0u;
         }
-        return static_cast<std::uint32_t>(__shfl(static_cast<int>(pos), 0, 64));
+        pos = w.ok() ? w.pos : 0u;
     }
-    const std::uint32_t nb{wave_store_tree<R>(depth, alpha, hdr, cap, s)};
-    return nb <= cap * 32 ? nb : 0u;
+    return static_cast<std::uint32_t>(__shfl(static_cast<int>(pos), 0, 64));
 }
 
 }  // namespace cjx
