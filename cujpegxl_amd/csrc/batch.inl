@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void q
                               ItemList{j.item_list, j.item_count}, j.dc, j.ytox, j.ytob);
 }
 
-__global__ __launch_bounds__(256) void tokens_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
+__global__ __launch_bounds__(kTokenThreads) void tokens_batch_kernel(const FrameJob* __restrict__ jobs, int count) {
     Wg wg;
     const FrameJob& j{batch_job(jobs, count, kBTokens, wg)};
     ac_tokens_kernel_body(wg, j.geo, j.ac, j.acs, j.nz_grid, j.nz_count, j.tokens, j.item_tokens, j.hist_partial,
@@ -141,11 +141,10 @@ void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint64
     const std::uint32_t dc_wgs{dc_chunks_per_group(geo) * geo.num_dc};
     set(kBRegion, 8 * ((geo.rw * geo.rh + 7) / 8), 1);
     set(kBQuantize, geo.cmw * geo.cmh, 1);
-    const std::uint32_t waves{(3 * geo.nblocks + 3) / 4};
     // A frame's share of the tokenizer's workgroups.
     const std::uint64_t share{(kBatchTokenWgs * static_cast<std::uint64_t>(geo.nblocks) + blocks - 1) / blocks};
     const std::uint32_t cap{std::min<std::uint32_t>(shape.token_cap, kTokenGrid)};
-    set(kBTokens, std::min({waves, cap, static_cast<std::uint32_t>(share)}), 1);
+    set(kBTokens, std::min({token_workgroups(geo), cap, static_cast<std::uint32_t>(share)}), 1);
     set(kBHistograms, kReduceWgs + dc_wgs, 1);
     set(kBHuffman, kNumClusters + 2 * geo.num_dc, 1);
     set(kBEmit, geo.num_ac * kGroupBands * band_wgs + dc_wgs, 1);
@@ -177,7 +176,7 @@ void launch_batch_regions(hipStream_t s, const FrameJob* jobs, int count, const 
 
 void launch_batch_files(hipStream_t s, const FrameJob* jobs, int count, const std::uint32_t (&total)[kBStages]) {
     quantize_batch_kernel<<<total[kBQuantize], 256, 0, s>>>(jobs, count);
-    tokens_batch_kernel<<<total[kBTokens], 256, 0, s>>>(jobs, count);
+    tokens_batch_kernel<<<total[kBTokens], kTokenThreads, 0, s>>>(jobs, count);
     histograms_batch_kernel<<<total[kBHistograms], 256, 0, s>>>(jobs, count);
     huffman_batch_kernel<<<total[kBHuffman], 64 * kTrials, 0, s>>>(jobs, count);
     emit_batch_kernel<<<total[kBEmit], kEmitThreads, 0, s>>>(jobs, count);

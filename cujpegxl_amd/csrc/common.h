@@ -113,6 +113,17 @@ constexpr std::uint32_t kModeMask = kModeMfma16 | kModeLearned | kModeForceMask;
 FrameParams make_frame_params(float distance);
 
 // Constant tables (filled once per device by init_device_tables()).
+// The AC tokenizer's lookups, one copy per workgroup in LDS.  Scan entry: raw
+// index of the scan position | its frequency context << 10.  zero_band[r * 32
+// + f]: cluster (within its group of twelve) of a coefficient's token with r
+// non-zeros left at frequency context f.
+struct alignas(16) TokenTables {
+    std::uint16_t scan8[64];
+    std::uint16_t scan16[256];
+    std::uint16_t scan32[1024];
+    std::uint8_t zero_band[64 * 32];
+};
+
 struct DeviceTables {
     float basis8[64];
     float basis16[256];
@@ -132,6 +143,7 @@ struct DeviceTables {
     std::uint16_t order8[64];     // natural scan order, raw index per scan position
     std::uint16_t order16[256];
     std::uint16_t order32[1024];
+    TokenTables tokens;
     double llf2[4];        // T[f][o] = ortho_2(f, o) * resample_scale_2[f]
     double llf4[16];
     float rate[256];       // selection rate term 1 + log2(1 + k) for |q| = k >= 1; 0 for k = 0

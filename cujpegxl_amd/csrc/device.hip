@@ -229,7 +229,7 @@ void launch_ac_tokens(hipStream_t s, const Geometry& geo, const std::int16_t* ac
     // kernel's time for a few waves.
     static const unsigned int resident{[] {
         int per_cu{0}, dev{0}, cus{0};
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ac_tokens_kernel, 256, 0) != hipSuccess ||
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ac_tokens_kernel, kTokenThreads, 0) != hipSuccess ||
             hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             per_cu <= 0 || cus <= 0) {
@@ -238,10 +238,10 @@ void launch_ac_tokens(hipStream_t s, const Geometry& geo, const std::int16_t* ac
         const int n{per_cu * cus};
         return static_cast<unsigned int>(n < kTokenGrid ? n : kTokenGrid);
     }()};
-    const unsigned int waves{(3 * geo.nblocks + 3) / 4};
-    const unsigned int grid{waves < resident ? waves : resident};
-    ac_tokens_kernel<<<grid, 256, 0, s>>>(geo, ac, acs, nz_grid, nz_count, tokens, item_tokens, partial, list.items,
-                                          list.count);
+    const unsigned int pairs{token_workgroups(geo)};
+    const unsigned int grid{pairs < resident ? pairs : resident};
+    ac_tokens_kernel<<<grid, kTokenThreads, 0, s>>>(geo, ac, acs, nz_grid, nz_count, tokens, item_tokens, partial,
+                                                    list.items, list.count);
     const std::uint32_t chunks{dc_chunks_per_group(geo)};
     histograms_kernel<<<kReduceWgs + chunks * geo.num_dc, 256, 0, s>>>(geo, chunks, partial, static_cast<int>(grid),
                                                                        hists, dc, acs, qf, ytox, ytob, fb_count);

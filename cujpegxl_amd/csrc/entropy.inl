@@ -1,13 +1,12 @@
 // Entropy-coding kernels (included into device.hip).
 //
-// AC: one wave tokenizes one block-channel (an "item": first-block x channel
-// in decoder order Y, X, B).  Each 64-coefficient chunk of the block's scan
-// order is classified with one ballot; a lane's remaining-non-zero count and
-// previous-coefficient flag -- the two serial dependencies of the AC context
-// model (entropy.cu:648-681, ac_context.h:78-84) -- come from a popcount of
-// the ballot below it, so every lane forms its token in parallel.  The same
-// tokenizer drives three passes: cluster histograms, per-item bit counts, and
-// bit emission at scanned offsets.
+// AC: half a wave tokenizes one block-channel (an "item": first-block x
+// channel in decoder order Y, X, B), 64 coefficients of the block's scan order
+// at a time, classified with ballots: a lane's remaining-non-zero count, the
+// serial dependency of the AC context model (entropy.cu:648-681,
+// ac_context.h:78-84), comes from popcounts of the ballots below it, so every
+// lane forms its tokens in parallel.  One pass writes the token records, their
+// counts and the cluster histograms; the emission reads the records.
 //
 // DC: a DcGroup section is a list of items (header blobs, DC residual tokens,
 // AcMetadata tokens), each with a known bit length once the codes exist;
@@ -15,46 +14,32 @@
 
 namespace cjx {
 
-__constant__ std::uint8_t c_ctx_map[39]{0, 1, 2, 2, 3,  3,  4,  5,  6,  6,  6,  6,  6,
-                                        7, 8, 9, 9, 10, 11, 12, 13, 14, 14, 14, 14, 14,
-                                        7, 8, 9, 9, 10, 11, 12, 13, 14, 14, 14, 14, 14};
-__constant__ std::uint16_t c_freq_ctx[64]{
-    0,  0,  1,  2,  3,  4,  5,  6,  7,  8,  9,  10, 11, 12, 13, 14, 15, 15, 16, 16, 17, 17,
-    18, 18, 19, 19, 20, 20, 21, 21, 22, 22, 23, 23, 23, 23, 24, 24, 24, 24, 25, 25, 25, 25,
-    26, 26, 26, 26, 27, 27, 27, 27, 28, 28, 28, 28, 29, 29, 29, 29, 30, 30, 30, 30};
-__constant__ std::uint16_t c_nz_ctx[64]{
-    0,   0,   31,  62,  62,  93,  93,  93,  93,  123, 123, 123, 123, 152, 152, 152,
-    152, 152, 152, 152, 152, 180, 180, 180, 180, 180, 180, 180, 180, 180, 180, 180,
-    180, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206,
-    206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206};
+// Block contexts by (channel in order Y, X, B; coefficient order).
+constexpr std::uint8_t kCtxMap[39]{0, 1, 2, 2, 3,  3,  4,  5,  6,  6,  6,  6,  6,
+                                   7, 8, 9, 9, 10, 11, 12, 13, 14, 14, 14, 14, 14,
+                                   7, 8, 9, 9, 10, 11, 12, 13, 14, 14, 14, 14, 14};
 
-// ac_context.h:108-131
-__device__ __forceinline__ int ac_cluster(std::uint32_t ctx) {
-    constexpr std::uint32_t count_contexts{15u * 37u};
-    if (ctx < count_contexts) {
-        const std::uint32_t bucket{ctx / 15u};
-        const int group{static_cast<int>(ctx % 15u) < 7 ? 0 : 1};
-        const int band{bucket < 4 ? 0 : (bucket < 12 ? 1 : (bucket < 24 ? 2 : 3))};
-        return group * 4 + band;
+// The clusters (ac_context.h:108-131) put the block contexts below 7 into one
+// group and the others into a second: with the transforms in use, the Y items
+// are the first group, whatever their transform.
+constexpr bool groups_by_channel() {
+    for (int row{0}; row < 3; ++row) {
+        for (const int ord : {0, 2, 3}) {
+            if ((kCtxMap[row * 13 + ord] < 7) != (row == 0)) {
+                return false;
+            }
+        }
     }
-    const std::uint32_t rel{ctx - count_contexts};
-    const int group{static_cast<int>(rel / 458u) < 7 ? 0 : 1};
-    const std::uint32_t z{rel % 458u};
-    const int band{z < 32    ? 0
-                   : z < 64  ? 1
-                   : z < 96  ? 2
-                   : z < 128 ? 3
-                   : z < 160 ? 4
-                   : z < 200 ? 5
-                   : z < 240 ? 6
-                   : z < 280 ? 7
-                   : z < 328 ? 8
-                   : z < 376 ? 9
-                   : z < 424 ? 10
-                             : 11};
-    return 8 + group * 12 + band;
+    return true;
 }
+static_assert(groups_by_channel(), "an item's cluster group follows from its channel");
 
+// Cluster of an item's zero-count token: the group's band of the predicted
+// count (contexts of 15 blocks per bucket, buckets 8 and up for two counts).
+__device__ __forceinline__ std::uint32_t count_cluster(int c, std::uint32_t pred) {
+    const std::uint32_t bucket{pred < 8 ? pred : 4 + pred / 2};
+    return (c == 1 ? 0u : 4u) + (bucket < 4 ? 0u : (bucket < 12 ? 1u : (bucket < 24 ? 2u : 3u)));
+}
 
 // Inclusive prefix sums over the wave by DPP moves (no LDS crossbar): within
 // each row of 16 lanes by shifts of 1, 2, 4 and 8 (lanes shifted in from
@@ -143,128 +128,117 @@ __device__ __forceinline__ void lds_or_bits(std::uint32_t* words, std::uint32_t 
 }
 
 struct AcItem {
-    int n;             // transform side, 0 if covered
-    int c;             // XYB channel
-    int bx, by;
-    std::uint32_t nz;  // non-zero AC count
-    std::uint32_t nz_ctx;
-    int bctx;
+    std::uint32_t head;  // transform side (0: covered) | XYB channel << 6 | count token's cluster << 8 | AC non-zeros << 16
+    std::uint32_t at;    // block column | block row << 16
+
+    __device__ __forceinline__ int side() const { return static_cast<int>(head & 63u); }
+    __device__ __forceinline__ int channel() const { return static_cast<int>((head >> 6) & 3u); }
+    __device__ __forceinline__ std::uint32_t cluster() const { return (head >> 8) & 7u; }
+    __device__ __forceinline__ std::uint32_t nonzeros() const { return head >> 16; }
+    __device__ __forceinline__ int bx() const { return static_cast<int>(at & 0xffffu); }
+    __device__ __forceinline__ int by() const { return static_cast<int>(at >> 16); }
 };
 
-__device__ __forceinline__ AcItem ac_item(const Geometry& geo, const std::int8_t* acs,
-                                          const std::uint8_t* nz_grid, const std::uint16_t* nz_count,
-                                          std::uint32_t item) {
-    AcItem it{};
-    const std::uint32_t pos{item / 3};
-    const int ci{static_cast<int>(item % 3)};
-    it.c = ci == 0 ? 1 : (ci == 1 ? 0 : 2);
-    it.bx = static_cast<int>(pos % geo.bw);
-    it.by = static_cast<int>(pos / geo.bw);
-    it.n = acs[pos];
-    if (it.n == 0) {
-        return it;
-    }
-    const std::size_t nblk{geo.nblocks};
-    it.nz = nz_count[it.c * nblk + pos];
-    const int ord{it.n == 16 ? 2 : (it.n == 32 ? 3 : 0)};
-    it.bctx = c_ctx_map[(it.c < 2 ? (it.c ^ 1) : 2) * 13 + ord];
-    const bool hl{(it.bx % kAcGroupBlocks) > 0}, ht{(it.by % kAcGroupBlocks) > 0};
-    const int top{ht ? nz_grid[it.c * nblk + pos - geo.bw] : 0};
-    const int left{hl ? nz_grid[it.c * nblk + pos - 1] : 0};
-    std::uint32_t pred{!hl ? (ht ? static_cast<std::uint32_t>(top) : 32u)
-                           : (!ht ? static_cast<std::uint32_t>(left)
-                                  : static_cast<std::uint32_t>((top + left + 1) / 2))};
+// What an item's descriptor is made from, as read: all reads are issued
+// before the first is used.
+struct ItemReads {
+    std::uint32_t pos;
+    int c, n;
+    std::uint32_t nz, top, left;
+    int bx, by;
+};
+
+__device__ __forceinline__ ItemReads read_item(const Geometry& geo, const std::int8_t* acs,
+                                               const std::uint8_t* nz_grid, const std::uint16_t* nz_count,
+                                               std::uint32_t item) {
+    ItemReads r;
+    r.pos = item / 3u;
+    const std::uint32_t ci{item - 3u * r.pos};
+    r.c = ci == 0 ? 1 : (ci == 1 ? 0 : 2);
+    r.by = static_cast<int>(r.pos / geo.bw);
+    r.bx = static_cast<int>(r.pos - static_cast<std::uint32_t>(r.by) * geo.bw);
+    const std::uint32_t at{static_cast<std::uint32_t>(r.c) * geo.nblocks + r.pos};
+    r.n = acs[r.pos];
+    r.nz = nz_count[at];
+    r.top = nz_grid[r.by > 0 ? at - geo.bw : at];
+    r.left = nz_grid[r.bx > 0 ? at - 1 : at];
+    return r;
+}
+
+__device__ __forceinline__ AcItem make_item(const ItemReads& r) {
+    const bool hl{(r.bx % kAcGroupBlocks) > 0}, ht{(r.by % kAcGroupBlocks) > 0};
+    std::uint32_t pred{!hl ? (ht ? r.top : 32u) : (!ht ? r.left : (r.top + r.left + 1) / 2)};
     pred = pred >= 64 ? 64 : pred;
-    it.nz_ctx = (pred < 8 ? pred : 4 + pred / 2) * 15u + static_cast<std::uint32_t>(it.bctx);
+    AcItem it;
+    it.head = static_cast<std::uint32_t>(r.n) | (static_cast<std::uint32_t>(r.c) << 6) |
+              (count_cluster(r.c, pred) << 8) | (r.nz << 16);
+    it.at = static_cast<std::uint32_t>(r.bx) | (static_cast<std::uint32_t>(r.by) << 16);
     return it;
+}
+
+// The tokenizer's tables into LDS, 16 bytes a thread.
+__device__ __forceinline__ void load_token_tables(TokenTables& T) {
+    static_assert(sizeof(TokenTables) % 16 == 0, "whole vectors");
+    for (std::uint32_t i{threadIdx.x}; i < sizeof(TokenTables) / 16; i += blockDim.x) {
+        reinterpret_cast<uint4*>(&T)[i] = reinterpret_cast<const uint4*>(&g_tables.tokens)[i];
+    }
 }
 
 // Tokenizes two items per wave, one per 32-lane half (item `it` of this
 // lane's half, its coefficients staged in `coef` block after block, so that
-// a scan-order entry (block << 6 | position) indexes it directly; `has`
-// false for a half without an item).  `emit(valid, k,
-// cluster, sym, nbits, extra)` is called once per lane per chunk, k being the
-// token's index in the item: 0 for the non-zero-count token (lane 0 of the
-// half, first call), then one token per scan position from the first
-// non-LLF position up to the last non-zero coefficient, so the valid lanes of
-// a chunk are a prefix of the half.  A lane's remaining-non-zero count and
-// previous-coefficient flag (entropy.cu:648-681, ac_context.h:78-84) come
-// from popcounts of the half's ballot bits below it.
-// The tokenizer's lookup tables, staged in LDS once per workgroup (the
-// lookups are per-lane gathers).
-// Zero-density contexts per block context: (nz_ctx[rem] + freq_ctx[k]) * 2 +
-// prev stays below 458 because rem + k <= 64 (ac_context.h:78-84).
-constexpr int kZeroDensityContexts = 458;
-
-struct TokenTables {
-    std::uint16_t order8[64];
-    std::uint16_t order16[256];
-    std::uint16_t order32[1024];
-    std::uint16_t nz_ctx[64];
-    std::uint16_t freq_ctx[64];
-    std::uint8_t zero_band[kZeroDensityContexts];  // ac_cluster's band of each zero-density context
-};
-
-__device__ __forceinline__ void load_token_tables(TokenTables& T) {
-    for (int i{static_cast<int>(threadIdx.x)}; i < 1024; i += static_cast<int>(blockDim.x)) {
-        T.order32[i] = g_tables.order32[i];
-        if (i < 256) {
-            T.order16[i] = g_tables.order16[i];
-        }
-        if (i < 64) {
-            T.order8[i] = g_tables.order8[i];
-            T.nz_ctx[i] = c_nz_ctx[i];
-            T.freq_ctx[i] = c_freq_ctx[i];
-        }
-        if (i < kZeroDensityContexts) {
-            T.zero_band[i] = static_cast<std::uint8_t>(ac_cluster(15u * 37u + static_cast<std::uint32_t>(i)) - 8);
-        }
-    }
-}
-
+// a scan entry's raw index is their index; side 0 for a half without an
+// item).  `emit(valid, k, cluster, sym, nbits, extra)` is called once per lane
+// per chunk, k being the token's index in the item: 0 for the
+// non-zero-count token (lane 0 of the half, first call), then one token per
+// scan position from the first non-LLF position up to the last non-zero
+// coefficient, so the valid lanes of a chunk are a prefix of the half.  A
+// lane's remaining-non-zero count (entropy.cu:648-681, ac_context.h:78-84)
+// comes from popcounts of the half's ballot bits below it; the context's
+// previous-coefficient flag never changes the cluster.  Two chunks of 32
+// positions go side by side: an 8x8 item is one step, and the lookups of a
+// longer item's two chunks wait together.
 template <typename Emit>
 __device__ __forceinline__ void tokenize_item_pair(const TokenTables& T, const std::int16_t* coef, const AcItem& it,
-                                                   bool has, int lane, Emit&& emit) {
+                                                   int lane, Emit&& emit) {
     const int half{lane >> 5}, sub{lane & 31};
+    const int n{it.side()};
+    const std::uint32_t nz{it.nonzeros()};
     {
         std::uint32_t sym{0}, nb{0}, bits{0};
-        hybrid420(it.nz, sym, nb, bits);
-        emit(has && sub == 0, 0u, has ? ac_cluster(it.nz_ctx) : 0, sym, nb, bits);
+        hybrid420(nz, sym, nb, bits);
+        emit(n != 0 && sub == 0, 0u, it.cluster(), sym, nb, bits);
     }
-    const int n{has ? it.n : 8};
-    const int side{n / 8};
-    const std::uint32_t cb{static_cast<std::uint32_t>(side * side)};
-    const std::uint32_t size{static_cast<std::uint32_t>(n * n)};
     const std::uint32_t l2{n == 16 ? 2u : (n == 32 ? 4u : 0u)};
-    const int zgroup{it.bctx < 7 ? 8 : 20};  // 8 + 12 * (block context >= 7)
-    const std::uint16_t* order{n == 32 ? T.order32 : (n == 16 ? T.order16 : T.order8)};
-    std::uint32_t seen{0};
-    std::uint32_t prev_carry{it.nz > size / 16 ? 0u : 1u};
+    const std::uint32_t cb{1u << l2};
+    const std::uint32_t size{64u << l2};
+    const std::uint32_t group{8u + 12u * (it.cluster() >> 2)};
+    const std::uint16_t* const scan{n == 32 ? T.scan32 : (n == 16 ? T.scan16 : T.scan8)};
     const std::uint32_t below{(1u << sub) - 1u};
-    for (std::uint32_t base{cb};; base += 32) {
-        const bool active{has && base < size && seen < it.nz};
-        if (__ballot(active) == 0) {
-            break;
-        }
-        const std::uint32_t k{base + static_cast<std::uint32_t>(sub)};
-        int v{0};
-        if (active && k < size) {
-            v = coef[order[k]];
-        }
-        const std::uint32_t gm{static_cast<std::uint32_t>(__ballot(v != 0) >> (32 * half))};
-        const std::uint32_t before{seen + static_cast<std::uint32_t>(__popc(gm & below))};
-        const std::uint32_t prev{sub == 0 ? prev_carry : ((gm >> (sub - 1)) & 1u)};
-        const bool valid{active && k < size && before < it.nz};
-        std::uint32_t cl{0}, sym{0}, nb{0}, bits{0};
-        if (valid) {
-            const std::uint32_t rem{((it.nz - before) + cb - 1) >> l2};
-            const std::uint32_t kk{k >> l2};
-            cl = static_cast<std::uint32_t>(zgroup + T.zero_band[(T.nz_ctx[rem] + T.freq_ctx[kk]) * 2u + prev]);
-            hybrid420(pack_signed(v), sym, nb, bits);
-        }
-        emit(valid, 1u + (k - cb), static_cast<int>(cl), sym, nb, bits);
-        seen += static_cast<std::uint32_t>(__popc(gm));
-        prev_carry = gm >> 31;
+    const auto half_of{[&](std::uint64_t m) {
+        return half == 0 ? static_cast<std::uint32_t>(m) : static_cast<std::uint32_t>(m >> 32);
+    }};
+    std::uint32_t left{n != 0 ? nz : 0u};  // non-zeros not seen yet
+    for (std::uint32_t base{cb}; __ballot(left != 0 && base < size) != 0; base += 64) {
+        const std::uint32_t k0{base + static_cast<std::uint32_t>(sub)}, k1{k0 + 32};
+        const bool on{left != 0}, on0{on && k0 < size}, on1{on && k1 < size};
+        const std::uint32_t e0{scan[on0 ? k0 : 0]}, e1{scan[on1 ? k1 : 0]};
+        const int c0{coef[e0 & 1023u]}, c1{coef[e1 & 1023u]};
+        const int v0{on0 ? c0 : 0}, v1{on1 ? c1 : 0};
+        const std::uint32_t m0{half_of(__ballot(v0 != 0))}, m1{half_of(__ballot(v1 != 0))};
+        // Non-zeros left at each lane's position.
+        const int left0{static_cast<int>(left) - static_cast<int>(__popc(m0 & below))};
+        const int left1{static_cast<int>(left) - static_cast<int>(__popc(m0) + __popc(m1 & below))};
+        const bool valid0{on0 && left0 > 0}, valid1{on1 && left1 > 0};
+        const std::uint32_t r0{valid0 ? (static_cast<std::uint32_t>(left0) + cb - 1) >> l2 : 0u};
+        const std::uint32_t r1{valid1 ? (static_cast<std::uint32_t>(left1) + cb - 1) >> l2 : 0u};
+        const std::uint32_t band0{T.zero_band[r0 * 32 + (e0 >> 10)]}, band1{T.zero_band[r1 * 32 + (e1 >> 10)]};
+        std::uint32_t sym{0}, nb{0}, bits{0};
+        hybrid420(pack_signed(v0), sym, nb, bits);
+        emit(valid0, 1u + (k0 - cb), group + band0, sym, nb, bits);
+        hybrid420(pack_signed(v1), sym, nb, bits);
+        emit(valid1, 1u + (k1 - cb), group + band1, sym, nb, bits);
+        const std::uint32_t seen{static_cast<std::uint32_t>(__popc(m0) + __popc(m1))};
+        left = seen < left ? left - seen : 0u;
     }
 }
 
@@ -272,9 +246,9 @@ __device__ __forceinline__ void tokenize_item_pair(const TokenTables& T, const s
 // (hybrid-uint extra bits of 16-bit magnitudes fit in 14 bits).  Token k of
 // an item lives in the k-th coefficient slot of the item's covered blocks
 // (an item has at most 1 + n*n - (n/8)^2 <= n*n tokens).
-__device__ __forceinline__ std::uint32_t token_record(int cl, std::uint32_t sym, std::uint32_t nb,
+__device__ __forceinline__ std::uint32_t token_record(std::uint32_t cl, std::uint32_t sym, std::uint32_t nb,
                                                       std::uint32_t extra) {
-    return static_cast<std::uint32_t>(cl) | (sym << 5) | (nb << 13) | (extra << 18);
+    return cl | (sym << 5) | (nb << 13) | (extra << 18);
 }
 
 __device__ __forceinline__ std::size_t token_slot(const Geometry& geo, int c, int bx, int by, int m,
@@ -294,6 +268,16 @@ __device__ __forceinline__ std::size_t token_slot(const Geometry& geo, int c, in
 // the descriptors of 32 pairs are loaded at once (one item per lane), and
 // each pair's coefficient blocks are read as 16-byte vectors while the
 // previous pair is tokenized from its LDS copy.
+// What bounds it: the latency of each wave's chain (descriptor, coefficients,
+// then per 64 positions two LDS lookups, a ballot, another lookup and the LDS
+// atomics), with the four workgroups per CU that 37 KB of LDS leave room for:
+// three take 7 % longer at 7680x4320, two 32 %; one histogram copy (five
+// workgroups) 15 %, more copies of the low symbols only 6 %.  So the first
+// descriptors and coefficients are read while the tables are set up, the
+// context lookups are one byte per (non-zeros left, frequency), an item's
+// descriptor is two words to pass between lanes, and a step takes 64
+// positions.  320x240 16.0 -> 11.0 us, 3840x2160 36.5 -> 28.5, 7680x4320 132
+// -> 80.
 constexpr int kAcSymbols = 64;
 // LDS row stride of a cluster's histogram: one word more than the symbols,
 // so equal symbols of different clusters fall in different banks.
@@ -304,17 +288,17 @@ constexpr int kHistRow = kAcSymbols + 1;
 constexpr int kHistCopy = kNumClusters * kHistRow + 16;
 constexpr int kTokenGrid = 2048;
 constexpr int kTokenBatch = 32;
+constexpr std::uint32_t kTokenThreads = 256;
+
+// Workgroups that leave every wave a pair of items.
+inline std::uint32_t token_workgroups(const Geometry& geo) {
+    constexpr std::uint32_t kItems{2 * kTokenThreads / 64};
+    return (3 * geo.nblocks + kItems - 1) / kItems;
+}
 
 __device__ __forceinline__ AcItem shfl_item(const AcItem& d, int src) {
-    AcItem o;
-    o.n = __shfl(d.n, src, 64);
-    o.c = __shfl(d.c, src, 64);
-    o.bx = __shfl(d.bx, src, 64);
-    o.by = __shfl(d.by, src, 64);
-    o.nz = static_cast<std::uint32_t>(__shfl(static_cast<int>(d.nz), src, 64));
-    o.nz_ctx = static_cast<std::uint32_t>(__shfl(static_cast<int>(d.nz_ctx), src, 64));
-    o.bctx = __shfl(d.bctx, src, 64);
-    return o;
+    return AcItem{static_cast<std::uint32_t>(__shfl(static_cast<int>(d.head), src, 64)),
+                  static_cast<std::uint32_t>(__shfl(static_cast<int>(d.at), src, 64))};
 }
 
 // The m x m coefficient blocks of an item (m = n / 8; 8 to 128 vectors of
@@ -331,16 +315,16 @@ __device__ __forceinline__ int item_vecs(int n) {
 __device__ __forceinline__ uint4 load_item_vec(const std::int16_t* plane, const Geometry& geo, const AcItem& it,
                                                int l2s, int u) {
     const int q{u >> 3};
-    const std::size_t blk{static_cast<std::size_t>(it.by + (q >> l2s)) * geo.bw +
-                          static_cast<std::size_t>(it.bx + (q & ((1 << l2s) - 1)))};
+    const std::size_t blk{static_cast<std::size_t>(it.by() + (q >> l2s)) * geo.bw +
+                          static_cast<std::size_t>(it.bx() + (q & ((1 << l2s) - 1)))};
     return *reinterpret_cast<const uint4*>(plane + blk * 64 + (u & 7) * 8);
 }
 
 __device__ __forceinline__ void load_item_coefs(const Geometry& geo, const std::int16_t* ac, const AcItem& it,
                                                 int sub, ItemVecs& v) {
-    const int l2s{it.n == 32 ? 2 : (it.n == 16 ? 1 : 0)};
-    const int vecs{item_vecs(it.n)};
-    const std::int16_t* plane{ac + static_cast<std::size_t>(it.c) * geo.nblocks * 64};
+    const int l2s{it.side() == 32 ? 2 : (it.side() == 16 ? 1 : 0)};
+    const int vecs{item_vecs(it.side())};
+    const std::int16_t* plane{ac + static_cast<std::size_t>(it.channel()) * geo.nblocks * 64};
     if (sub < vecs) {
         v.r0 = load_item_vec(plane, geo, it, l2s, sub);
     }
@@ -352,7 +336,7 @@ __device__ __forceinline__ void load_item_coefs(const Geometry& geo, const std::
 }
 
 __device__ __forceinline__ void store_item_coefs(std::int16_t* coef, const AcItem& it, int sub, const ItemVecs& v) {
-    const int vecs{item_vecs(it.n)};
+    const int vecs{item_vecs(it.side())};
     if (sub < vecs) {
         *reinterpret_cast<uint4*>(coef + sub * 8) = v.r0;
     }
@@ -361,6 +345,12 @@ __device__ __forceinline__ void store_item_coefs(std::int16_t* coef, const AcIte
         *reinterpret_cast<uint4*>(coef + (sub + 64) * 8) = v.r2;
         *reinterpret_cast<uint4*>(coef + (sub + 96) * 8) = v.r3;
     }
+}
+
+// An item's own index: block * 3 + (0: Y, 1: X, 2: B).
+__device__ __forceinline__ std::uint32_t item_index(const Geometry& geo, const AcItem& it) {
+    return (static_cast<std::uint32_t>(it.by()) * geo.bw + static_cast<std::uint32_t>(it.bx())) * 3u +
+           (it.channel() == 1 ? 0u : (it.channel() == 0 ? 1u : 2u));
 }
 
 __device__ __attribute__((always_inline)) inline void ac_tokens_kernel_body(const Wg& wg, Geometry geo, const std::int16_t* __restrict__ ac,
@@ -372,33 +362,74 @@ __device__ __attribute__((always_inline)) inline void ac_tokens_kernel_body(cons
                                                         std::uint32_t* __restrict__ partial,
                                                         const std::uint32_t* __restrict__ list,
                                                         const std::uint32_t* __restrict__ list_count) {
-    __shared__ std::uint32_t h2[2 * kHistCopy];
+    __shared__ __align__(16) std::uint32_t h2[2 * kHistCopy];
     __shared__ TokenTables T;
-    __shared__ __align__(16) std::int16_t stage[4][2][1024];
-    for (int i{static_cast<int>(threadIdx.x)}; i < 2 * kHistCopy; i += 256) {
-        h2[i] = 0;
-    }
-    load_token_tables(T);
-    __syncthreads();
+    __shared__ __align__(16) std::int16_t stage[kTokenThreads / 64][2][1024];
     const int lane{static_cast<int>(threadIdx.x) & 63};
     const int half{lane >> 5}, sub{lane & 31};
     std::uint32_t* const h{h2 + (lane & 1) * kHistCopy};
     std::int16_t* const coef{stage[threadIdx.x >> 6][half]};
-    const std::uint32_t wave{wg.x * 4 + (threadIdx.x >> 6)};
-    const std::uint32_t stride{2 * wg.nx * 4};
-    // Walk the quantizer's list of items with non-zeros when there is one
-    // (the others follow below; covered blocks' items already have 0
-    // tokens), else every item.
-    const std::uint32_t items{list != nullptr ? list_count[0] : geo.nblocks * 3};
+    const std::uint32_t wave{wg.x * (kTokenThreads / 64) + (threadIdx.x >> 6)};
+    const std::uint32_t stride{2 * wg.nx * (kTokenThreads / 64)};
+    // The list of items with non-zeros from the quantizer when there is one
+    // (covered blocks' items already have 0 tokens), else every item; at the
+    // list's end the first blocks' items without non-zeros.  The wave's first
+    // items and the thread's first item without non-zeros are read while the
+    // tables are set up: entries past the list's ends are read too (they are
+    // in the buffer), but not used.
+    const std::uint32_t all{3u * geo.nblocks}, last{all - 1u};
+    const auto item_at{[&](std::uint32_t base) {
+        return base + stride * static_cast<std::uint32_t>(lane >> 1) + static_cast<std::uint32_t>(lane & 1);
+    }};
+    const std::uint32_t li{item_at(2 * wave)};
+    const std::uint32_t zi{wg.x * kTokenThreads + threadIdx.x};
+    std::uint32_t first{li}, zero{0};
+    std::uint32_t items{all}, zeros{0};
+    if (list != nullptr) {
+        items = list_count[0];
+        zeros = list_count[1];
+        first = list[li < all ? li : 0u];
+        zero = list[zi < all ? last - zi : 0u];
+    }
+    for (std::uint32_t i{threadIdx.x}; i < 2 * kHistCopy / 4; i += kTokenThreads) {
+        reinterpret_cast<uint4*>(h2)[i] = uint4{0, 0, 0, 0};
+    }
+    static_assert(2 * kHistCopy % 4 == 0, "whole vectors");
+    const ItemReads first_reads{read_item(geo, acs, nz_grid, nz_count, li < items ? first : 0u)};
+    const ItemReads zero_reads{read_item(geo, acs, nz_grid, nz_count, zi < zeros ? zero : 0u)};
+    load_token_tables(T);
+    AcItem d{make_item(first_reads)};
+    d.head = li < items ? d.head : 0u;
+    AcItem cur{shfl_item(d, half)};
+    ItemVecs v{};
+    load_item_coefs(geo, ac, cur, sub, v);
+    __syncthreads();
+    // First blocks without non-zero coefficients, one per thread: their one
+    // token is the zero count, in the count's context.
+    {
+        AcItem it{make_item(zero_reads)};
+        for (std::uint32_t i{zi}; i < zeros; i += wg.nx * kTokenThreads) {
+            if (i != zi) {
+                it = make_item(read_item(geo, acs, nz_grid, nz_count, list[last - i]));
+            }
+            std::uint32_t sym{0}, nb{0}, bits{0};
+            hybrid420(0u, sym, nb, bits);
+            atomicAdd(&h[it.cluster() * kHistRow + (sym & (kAcSymbols - 1))], 1u);
+            tokens[token_slot(geo, it.channel(), it.bx(), it.by(), 1, 0)] = token_record(it.cluster(), sym, nb, bits);
+            item_tokens[item_index(geo, it)] = 1;
+        }
+    }
     for (std::uint32_t base{2 * wave}; base < items; base += stride * kTokenBatch) {
-        const std::uint32_t li{base + stride * static_cast<std::uint32_t>(lane >> 1) +
-                               static_cast<std::uint32_t>(lane & 1)};
-        const AcItem d{li < items ? ac_item(geo, acs, nz_grid, nz_count, list != nullptr ? list[li] : li) : AcItem{}};
+        if (base != 2 * wave) {
+            const std::uint32_t i{item_at(base)};
+            const ItemReads r{read_item(geo, acs, nz_grid, nz_count, i < items ? (list != nullptr ? list[i] : i) : 0u)};
+            d = make_item(r);
+            d.head = i < items ? d.head : 0u;
+            cur = shfl_item(d, half);
+            load_item_coefs(geo, ac, cur, sub, v);
+        }
         const int npairs{static_cast<int>(min(static_cast<std::uint32_t>(kTokenBatch),
                                               (items - base + stride - 1) / stride))};
-        AcItem cur{shfl_item(d, half)};
-        ItemVecs v{};
-        load_item_coefs(geo, ac, cur, sub, v);
         for (int t{0}; t < npairs; ++t) {
             const std::uint32_t item{base + stride * static_cast<std::uint32_t>(t) + static_cast<std::uint32_t>(half)};
             wave_sync();
@@ -409,63 +440,46 @@ __device__ __attribute__((always_inline)) inline void ac_tokens_kernel_body(cons
                 nx = shfl_item(d, 2 * (t + 1) + half);
                 load_item_coefs(geo, ac, nx, sub, v);
             }
-            const bool has{cur.n != 0};
             std::uint32_t count{0};
-            if (__ballot(has) != 0) {
+            if (__ballot(cur.side() != 0) != 0) {
                 const AcItem it{cur};
-                const std::uint32_t m{has ? static_cast<std::uint32_t>(it.n / 8) : 1u};
-                const std::uint32_t l2m{m >> 1};
+                const std::uint32_t l2m{it.side() == 32 ? 2u : (it.side() == 16 ? 1u : 0u)};
+                const std::uint32_t m{1u << l2m};
                 // token_slot in 32 bits (3 * blocks * 64 < 2^32 for the
                 // at most 32 DC groups a frame may have).
-                const std::uint32_t slot0{static_cast<std::uint32_t>(token_slot(geo, has ? it.c : 0, it.bx, it.by, 1, 0))};
+                const std::uint32_t slot0{static_cast<std::uint32_t>(
+                    token_slot(geo, it.channel(), it.bx(), it.by(), 1, 0))};
                 const std::uint32_t row{geo.bw * 64};
-                tokenize_item_pair(T, coef, it, has, lane,
-                                   [&](bool valid, std::uint32_t k, int cl, std::uint32_t sym, std::uint32_t nb,
-                                       std::uint32_t extra) {
+                tokenize_item_pair(T, coef, it, lane,
+                                   [&](bool valid, std::uint32_t k, std::uint32_t cl, std::uint32_t sym,
+                                       std::uint32_t nb, std::uint32_t extra) {
                                        if (valid) {
                                            atomicAdd(&h[cl * kHistRow + (sym & (kAcSymbols - 1))], 1u);
                                            const std::uint32_t q{k >> 6};
                                            tokens[slot0 + (q >> l2m) * row + ((q & (m - 1)) << 6) + (k & 63u)] =
                                                token_record(cl, sym, nb, extra);
                                        }
+                                       const std::uint64_t ballot{__ballot(valid)};
                                        count += static_cast<std::uint32_t>(
-                                           __popc(static_cast<std::uint32_t>(__ballot(valid) >> (32 * half))));
+                                           __popc(half == 0 ? static_cast<std::uint32_t>(ballot)
+                                                            : static_cast<std::uint32_t>(ballot >> 32)));
                                    });
             }
             if (sub == 0 && item < items) {
-                // The item's own index: block * 3 + (0: Y, 1: X, 2: B).
-                const std::uint32_t own{(static_cast<std::uint32_t>(cur.by) * geo.bw + static_cast<std::uint32_t>(cur.bx)) * 3u +
-                                        (cur.c == 1 ? 0u : (cur.c == 0 ? 1u : 2u))};
-                item_tokens[own] = static_cast<std::uint16_t>(count);
+                item_tokens[item_index(geo, cur)] = static_cast<std::uint16_t>(count);
             }
             cur = nx;
         }
     }
-    // First blocks without non-zero coefficients, one per thread: their one
-    // token is the zero count, in the count's context.
-    if (list != nullptr) {
-        const std::uint32_t zeros{list_count[1]};
-        const std::uint32_t last{3u * geo.nblocks - 1u};
-        for (std::uint32_t i{wg.x * 256u + threadIdx.x}; i < zeros; i += wg.nx * 256u) {
-            const AcItem it{ac_item(geo, acs, nz_grid, nz_count, list[last - i])};
-            std::uint32_t sym{0}, nb{0}, bits{0};
-            hybrid420(0u, sym, nb, bits);
-            const int cl{ac_cluster(it.nz_ctx)};
-            atomicAdd(&h[cl * kHistRow + (sym & (kAcSymbols - 1))], 1u);
-            tokens[token_slot(geo, it.c, it.bx, it.by, 1, 0)] = token_record(cl, sym, nb, bits);
-            item_tokens[(static_cast<std::uint32_t>(it.by) * geo.bw + static_cast<std::uint32_t>(it.bx)) * 3u +
-                        (it.c == 1 ? 0u : (it.c == 0 ? 1u : 2u))] = 1;
-        }
-    }
     __syncthreads();
     std::uint32_t* mine{partial + static_cast<std::size_t>(wg.x) * kNumClusters * kAcSymbols};
-    for (int i{static_cast<int>(threadIdx.x)}; i < kNumClusters * kAcSymbols; i += 256) {
+    for (int i{static_cast<int>(threadIdx.x)}; i < kNumClusters * kAcSymbols; i += kTokenThreads) {
         const int r{(i >> 6) * kHistRow + (i & (kAcSymbols - 1))};
         mine[i] = h2[r] + h2[kHistCopy + r];
     }
 }
 
-__global__ __launch_bounds__(256) void ac_tokens_kernel(Geometry geo, const std::int16_t* __restrict__ ac,
+__global__ __launch_bounds__(kTokenThreads) void ac_tokens_kernel(Geometry geo, const std::int16_t* __restrict__ ac,
                                                         const std::int8_t* __restrict__ acs,
                                                         const std::uint8_t* __restrict__ nz_grid,
                                                         const std::uint16_t* __restrict__ nz_count,

@@ -91,6 +91,42 @@ void selection_weights(int n, const float* dct8_y, float* out) {
     }
 }
 
+// Contexts of the zero-density model by frequency (scan position over the
+// covered blocks) and by non-zeros left (ac_context.h:78-84).
+constexpr std::uint8_t kFreqCtx[64]{
+    0,  0,  1,  2,  3,  4,  5,  6,  7,  8,  9,  10, 11, 12, 13, 14, 15, 15, 16, 16, 17, 17,
+    18, 18, 19, 19, 20, 20, 21, 21, 22, 22, 23, 23, 23, 23, 24, 24, 24, 24, 25, 25, 25, 25,
+    26, 26, 26, 26, 27, 27, 27, 27, 28, 28, 28, 28, 29, 29, 29, 29, 30, 30, 30, 30};
+constexpr std::uint8_t kNzCtx[64]{
+    0,   0,   31,  62,  62,  93,  93,  93,  93,  123, 123, 123, 123, 152, 152, 152,
+    152, 152, 152, 152, 152, 180, 180, 180, 180, 180, 180, 180, 180, 180, 180, 180,
+    180, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206,
+    206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206, 206};
+// Bands of the zero-density contexts z = (nz + freq) * 2 + prev
+// (ac_context.h:108-131): every bound is even, so the previous coefficient's
+// flag never moves a token to another band.
+constexpr int kZeroBandBounds[11]{32, 64, 96, 128, 160, 200, 240, 280, 328, 376, 424};
+
+void token_tables(const DeviceTables& t, TokenTables& k) {
+    const auto scan{[](const std::uint16_t* order, int n, std::uint16_t* out) {
+        for (int i{0}; i < n * n; ++i) {
+            out[i] = static_cast<std::uint16_t>(order[i] | (kFreqCtx[i / (n * n / 64)] << 10));
+        }
+    }};
+    scan(t.order8, 8, k.scan8);
+    scan(t.order16, 16, k.scan16);
+    scan(t.order32, 32, k.scan32);
+    for (int left{0}; left < 64; ++left) {
+        for (int freq{0}; freq < 32; ++freq) {
+            int band{0};
+            for (const int bound : kZeroBandBounds) {
+                band += (kNzCtx[left] + freq) * 2 >= bound ? 1 : 0;
+            }
+            k.zero_band[left * 32 + freq] = static_cast<std::uint8_t>(band);
+        }
+    }
+}
+
 // coeff_order.cc:10-43: diagonal zig-zag with the LLF corner first.
 void natural_order(int n, std::uint16_t* out) {
     const int cx{n / 8};
@@ -148,6 +184,7 @@ DeviceTables build_tables() {
     natural_order(8, t.order8);
     natural_order(16, t.order16);
     natural_order(32, t.order32);
+    token_tables(t, t.tokens);
     llf_table(2, t.llf2);
     llf_table(4, t.llf4);
     auto recip = [](const float* w, float* r, int n) {
