@@ -185,8 +185,5 @@ __device__ __forceinline__ float dequant_inv_of(int n, int c, int e) {
     return n == 32 ? g_tables.dequant_inv32[c][e]
                    : (n == 16 ? g_tables.dequant_inv16[c][e] : g_tables.dequant_inv8[c][e]);
 }
-__device__ __forceinline__ const std::uint16_t* order_of(int n) {
-    return n == 32 ? g_tables.order32 : (n == 16 ? g_tables.order16 : g_tables.order8);
-}
 
 }  // namespace cjx

@@ -437,18 +437,9 @@ __device__ __forceinline__ _Float16* coefy_of(RegionShared& S, int sz) {
     return S.b.s.y[sz];
 }
 
-// True for the lowest (n/8)^2 frequencies (fx, fy < n/8) of element
-// e = fx * n + fy of an n x n transform, n = 8, 16 or 32 (shifts, not a
-// division by a runtime n).
-__device__ __forceinline__ bool is_llf(int e, int n) {
-    const int l2{n == 32 ? 5 : (n == 16 ? 4 : 3)};
-    const int m{n >> 3};
-    return (e >> l2) < m && (e & (n - 1)) < m;
-}
-
 // Selection terms of M Y coefficients of one lane (transform_select_impl.cuh:
 // 49-108): squared quantization error and rate proxy; LLF coefficients
-// (llf[i], from the callers' closed forms of is_llf for their lane layouts)
+// (llf[i], from the callers' closed forms for their lane layouts)
 // contribute 0, which the terms of a zero coefficient are exactly (q = 0,
 // err = 0, rate[0] = 0).  The two quotients are the correctly rounded ones,
 // by reciprocals.  The weights come in as arguments (read four at a time by
@@ -1858,31 +1849,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void r
 struct TileShared {
     unsigned int nz[64][3];
     int own[64];              // packed owner: local position | (n << 8)
+    float2 scale[64];         // the block's quantizer q and RN(1 / q)
     float maps[2];
     // LLF coefficients: (fx, fy) of the transform at local position op in
     // slot op + 8 fx + fy (the blocks it covers, so no two transforms meet).
     float llf[3][64];
     double resample[4 + 16];  // g_tables.llf2, llf4
 };
-
-__device__ __forceinline__ int owner_in_tile(const std::int8_t* acs, int bw, int bx, int by, int& ox,
-                                             int& oy) {
-    const int rxb{bx & ~3}, ryb{by & ~3};
-    if (acs[static_cast<std::size_t>(ryb) * bw + rxb] == 32) {
-        ox = rxb;
-        oy = ryb;
-        return 32;
-    }
-    const int qx{bx & ~1}, qy{by & ~1};
-    if (acs[static_cast<std::size_t>(qy) * bw + qx] == 16) {
-        ox = qx;
-        oy = qy;
-        return 16;
-    }
-    ox = bx;
-    oy = by;
-    return 8;
-}
 
 // DC coefficient of channel c of the block at local position p of a tile
 // (frontend_quantize.cu:181-199, dc_from_llf_strided): the owner transform's
@@ -1907,6 +1880,14 @@ __device__ __forceinline__ float block_dc(const TileShared& S, int p, int c) {
     return static_cast<float>(static_cast<double>(m) * sum);
 }
 
+// What bounds it: at 3840x2160 vector instructions (10.3 M, 21 us of issue) and
+// 100 MB in and out (19 us at a copy's rate), in one resident round of eight
+// waves per SIMD, 36.4 us.  Owners, quantizers and reciprocals are set up once
+// per block, one 32-bit offset serves a step's reads and writes, the LLF
+// coefficients are masked after packing and non-zeros are counted in packed
+// halves (12.4 M instructions, 40.4 us with a quotient, a test and a 64-bit
+// address for each of those; 320x240 10.1 -> 8.7 us, 7680x4320 150 -> 113).
+// The next step's coefficients read ahead gain nothing (36.8).
 __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(const Wg& wg, 
     Geometry geo, FrameParams prm, const std::uint16_t* __restrict__ coeffs,
     const std::int8_t* __restrict__ acs, const std::int32_t* __restrict__ qf,
@@ -1926,11 +1907,25 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
     if (tid < 64) {
         S.nz[tid][0] = S.nz[tid][1] = S.nz[tid][2] = 0u;
         const int bx{tx * 8 + (tid & 7)}, by{ty * 8 + (tid >> 3)};
-        int ox{bx}, oy{by}, n{8};
+        // The transform that covers the block: the 32x32 or 16x16 one whose
+        // first block its aligned square starts with, else its own.  Every
+        // candidate is read before any is looked at.
+        int op{tid}, n{8};
+        float quant{1.0f};  // of blocks past the frame, which no lane uses
         if (bx < bw && by < bh) {
-            n = owner_in_tile(acs, bw, bx, by, ox, oy);
+            const std::uint32_t row{static_cast<std::uint32_t>(bw)};
+            const std::uint32_t at8{static_cast<std::uint32_t>(by) * row + static_cast<std::uint32_t>(bx)};
+            const std::uint32_t at16{static_cast<std::uint32_t>(by & ~1) * row + static_cast<std::uint32_t>(bx & ~1)};
+            const std::uint32_t at32{static_cast<std::uint32_t>(by & ~3) * row + static_cast<std::uint32_t>(bx & ~3)};
+            const int n32{acs[at32]}, n16{acs[at16]};
+            const std::int32_t f8{qf[at8]}, f16{qf[at16]}, f32{qf[at32]};
+            n = n32 == 32 ? 32 : (n16 == 16 ? 16 : 8);
+            op = n == 32 ? tid & 0x24 : (n == 16 ? tid & 0x36 : tid);
+            quant = static_cast<float>(n == 32 ? f32 : (n == 16 ? f16 : f8));
         }
-        S.own[tid] = ((oy - ty * 8) * 8 + (ox - tx * 8)) | (n << 8);
+        S.own[tid] = op | (n << 8);
+        const float qgsf{quant * prm.global_scale_float};
+        S.scale[tid] = float2{qgsf, 1.0f / qgsf};
     }
     if (tid >= 128 && tid < 148) {
         const int i{tid - 128};
@@ -1955,17 +1950,42 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
     // 16-byte reads.  y_round = qy wy / qgsf is the correctly rounded
     // quotient, by the block's RN(1 / qgsf).
     const int grp{lane >> 4}, e4{4 * (lane & 15)};
+    // Weights and reciprocals of a transform size at one distance, so that
+    // one offset serves both; 32-bit offsets (an accepted frame's plane has
+    // at most 2^28 bytes).
+    constexpr std::uint32_t kInverse{offsetof(DeviceTables, dequant_inv8) - offsetof(DeviceTables, dequant8)};
     static_assert(offsetof(DeviceTables, dequant8) % 16 == 0 && offsetof(DeviceTables, dequant16) % 16 == 0 &&
-                      offsetof(DeviceTables, dequant32) % 16 == 0 && offsetof(DeviceTables, dequant_inv8) % 16 == 0 &&
-                      offsetof(DeviceTables, dequant_inv16) % 16 == 0 &&
-                      offsetof(DeviceTables, dequant_inv32) % 16 == 0,
+                      offsetof(DeviceTables, dequant32) % 16 == 0 && kInverse % 16 == 0 &&
+                      offsetof(DeviceTables, dequant_inv16) == offsetof(DeviceTables, dequant16) + kInverse &&
+                      offsetof(DeviceTables, dequant_inv32) == offsetof(DeviceTables, dequant32) + kInverse,
                   "16-byte weight reads");
+    const auto* const weights{reinterpret_cast<const std::uint8_t*>(&g_tables.dequant8[0][0])};
+    const auto* const inverses{reinterpret_cast<const std::uint8_t*>(&g_tables.dequant_inv8[0][0])};
+    const auto* const in0{reinterpret_cast<const std::uint8_t*>(coeffs)};
+    const auto* const in1{reinterpret_cast<const std::uint8_t*>(coeffs + cplane)};
+    const auto* const in2{reinterpret_cast<const std::uint8_t*>(coeffs + 2 * cplane)};
+    auto* const out0{reinterpret_cast<std::uint8_t*>(ac)};
+    auto* const out1{reinterpret_cast<std::uint8_t*>(ac + cplane)};
+    auto* const out2{reinterpret_cast<std::uint8_t*>(ac + 2 * cplane)};
     const auto f16_at = [](uint2 h, int i) {
         const std::uint32_t wd{i < 2 ? h.x : h.y};
         return static_cast<float>(
             __builtin_bit_cast(_Float16, static_cast<std::uint16_t>((i & 1) != 0 ? wd >> 16 : wd & 0xffffu)));
     };
     const auto f4_at = [](const float4& v, int i) { return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w)); };
+    // The low halves of two integers in one word.
+    const auto pair = [](int lo, int hi) {
+        return __builtin_amdgcn_perm(static_cast<std::uint32_t>(hi), static_cast<std::uint32_t>(lo), 0x05040100u);
+    };
+    // Non-zeros among four 16-bit values.
+    const auto nonzeros = [](std::uint32_t a, std::uint32_t b) {
+        using u16x2 = std::uint16_t __attribute__((ext_vector_type(2)));
+        const u16x2 one{1, 1};
+        const u16x2 n{__builtin_elementwise_min(__builtin_bit_cast(u16x2, a), one) +
+                      __builtin_elementwise_min(__builtin_bit_cast(u16x2, b), one)};
+        const std::uint32_t both{__builtin_bit_cast(std::uint32_t, n)};
+        return (both & 0xffffu) + (both >> 16);
+    };
 #pragma unroll 1
     for (int j{0}; j < 4; ++j) {
         const int p{16 * j + 4 * grp + w};
@@ -1976,19 +1996,32 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
         // Non-zeros among the lane's four: X | Y << 8 | B << 16.
         std::uint32_t cnt{0};
         if (in) {
-            const int ox{tx * 8 + (op & 7)}, oy{ty * 8 + (op >> 3)};
             const int m{n >> 3};
-            const int e0{((by - oy) * m + (bx - ox)) * 64 + e4};
-            const std::size_t slot{(static_cast<std::size_t>(by) * bw + bx) * 64 + e4};
-            const uint2 hx{*reinterpret_cast<const uint2*>(coeffs + slot)};
-            const uint2 hy{*reinterpret_cast<const uint2*>(coeffs + cplane + slot)};
-            const uint2 hb{*reinterpret_cast<const uint2*>(coeffs + 2 * cplane + slot)};
-            const float qgsf{static_cast<float>(qf[static_cast<std::size_t>(oy) * bw + ox]) *
-                             prm.global_scale_float};
-            const float rq{1.0f / qgsf};
+            const int e0{(((p >> 3) - (op >> 3)) * m + ((p & 7) - (op & 7))) * 64 + e4};
+            const std::uint32_t at{2u * ((static_cast<std::uint32_t>(by) * static_cast<std::uint32_t>(bw) +
+                                          static_cast<std::uint32_t>(bx)) * 64u + static_cast<std::uint32_t>(e4))};
+            const uint2 hx{*reinterpret_cast<const uint2*>(in0 + at)};
+            const uint2 hy{*reinterpret_cast<const uint2*>(in1 + at)};
+            const uint2 hb{*reinterpret_cast<const uint2*>(in2 + at)};
+            const std::uint32_t next{4u * static_cast<std::uint32_t>(n * n)};
+            const std::uint32_t wx_at{
+                (n == 32 ? static_cast<std::uint32_t>(offsetof(DeviceTables, dequant32) - offsetof(DeviceTables, dequant8))
+                         : (n == 16 ? static_cast<std::uint32_t>(offsetof(DeviceTables, dequant16) -
+                                                                 offsetof(DeviceTables, dequant8))
+                                    : 0u)) +
+                4u * static_cast<std::uint32_t>(e0)};
+            const std::uint32_t wy_at{wx_at + next}, wb_at{wy_at + next};
+            const float4 wx4{*reinterpret_cast<const float4*>(weights + wx_at)};
+            const float4 wy4{*reinterpret_cast<const float4*>(weights + wy_at)};
+            const float4 wb4{*reinterpret_cast<const float4*>(weights + wb_at)};
+            const float4 ix4{*reinterpret_cast<const float4*>(inverses + wx_at)};
+            const float4 iy4{*reinterpret_cast<const float4*>(inverses + wy_at)};
+            const float4 ib4{*reinterpret_cast<const float4*>(inverses + wb_at)};
+            const float qgsf{S.scale[p].x}, rq{S.scale[p].y};
             // The lane's LLF coefficients (the first m of its four, in the
-            // rows fx < m) to where block_dc reads them.
+            // rows fx < m) to where block_dc reads them; they are no items'.
             const int fx{e0 >> (n == 32 ? 5 : (n == 16 ? 4 : 3))};
+            std::uint32_t keep0{~0u}, keep1{~0u};
             if ((e0 & (n - 1)) == 0 && fx < m) {
 #pragma unroll
                 for (int i{0}; i < 4; ++i) {
@@ -1998,42 +2031,28 @@ __device__ __attribute__((always_inline)) inline void tile_quantize_kernel_body(
                         S.llf[2][op + 8 * fx + i] = f16_at(hb, i);
                     }
                 }
+                keep0 = m == 1 ? 0xffff0000u : 0u;
+                keep1 = m == 4 ? 0u : ~0u;
             }
-            const int cs{n * n};
-            const float* const wt{n == 32 ? &g_tables.dequant32[0][0]
-                                          : (n == 16 ? &g_tables.dequant16[0][0] : &g_tables.dequant8[0][0])};
-            const float* const wit{n == 32 ? &g_tables.dequant_inv32[0][0]
-                                           : (n == 16 ? &g_tables.dequant_inv16[0][0] : &g_tables.dequant_inv8[0][0])};
-            const float4 wx4{*reinterpret_cast<const float4*>(wt + e0)};
-            const float4 wy4{*reinterpret_cast<const float4*>(wt + cs + e0)};
-            const float4 wb4{*reinterpret_cast<const float4*>(wt + 2 * cs + e0)};
-            const float4 ix4{*reinterpret_cast<const float4*>(wit + e0)};
-            const float4 iy4{*reinterpret_cast<const float4*>(wit + cs + e0)};
-            const float4 ib4{*reinterpret_cast<const float4*>(wit + 2 * cs + e0)};
-            std::uint32_t q0[2]{0u, 0u}, q1[2]{0u, 0u}, q2[2]{0u, 0u};
+            int a0[4], a1[4], a2[4];
 #pragma unroll
             for (int i{0}; i < 4; ++i) {
-                std::int16_t a0{0}, a1{0}, a2{0};
-                if (!is_llf(e0 + i, n)) {
-                    const float wy{f4_at(wy4, i)};
-                    const int qy{static_cast<int>(
-                        __builtin_rintf(div_by_recip(f16_at(hy, i) * qgsf, wy, f4_at(iy4, i))))};
-                    const float y_round{div_by_recip(static_cast<float>(qy) * wy, qgsf, rq)};
-                    a0 = static_cast<std::int16_t>(static_cast<int>(__builtin_rintf(div_by_recip(
-                        (f16_at(hx, i) - yx * y_round) * qgsf, f4_at(wx4, i), f4_at(ix4, i)))));
-                    a1 = static_cast<std::int16_t>(qy);
-                    a2 = static_cast<std::int16_t>(static_cast<int>(__builtin_rintf(div_by_recip(
-                        (f16_at(hb, i) - yb * y_round) * qgsf, f4_at(wb4, i), f4_at(ib4, i)))));
-                }
-                const int sh{16 * (i & 1)};
-                q0[i >> 1] |= static_cast<std::uint32_t>(static_cast<std::uint16_t>(a0)) << sh;
-                q1[i >> 1] |= static_cast<std::uint32_t>(static_cast<std::uint16_t>(a1)) << sh;
-                q2[i >> 1] |= static_cast<std::uint32_t>(static_cast<std::uint16_t>(a2)) << sh;
-                cnt += (a0 != 0 ? 1u : 0u) | (a1 != 0 ? 0x100u : 0u) | (a2 != 0 ? 0x10000u : 0u);
+                const float wy{f4_at(wy4, i)};
+                const float qy{__builtin_rintf(div_by_recip(f16_at(hy, i) * qgsf, wy, f4_at(iy4, i)))};
+                const float y_round{div_by_recip(qy * wy, qgsf, rq)};
+                a0[i] = static_cast<int>(__builtin_rintf(
+                    div_by_recip((f16_at(hx, i) - yx * y_round) * qgsf, f4_at(wx4, i), f4_at(ix4, i))));
+                a1[i] = static_cast<int>(qy);
+                a2[i] = static_cast<int>(__builtin_rintf(
+                    div_by_recip((f16_at(hb, i) - yb * y_round) * qgsf, f4_at(wb4, i), f4_at(ib4, i))));
             }
-            *reinterpret_cast<uint2*>(ac + slot) = uint2{q0[0], q0[1]};
-            *reinterpret_cast<uint2*>(ac + cplane + slot) = uint2{q1[0], q1[1]};
-            *reinterpret_cast<uint2*>(ac + 2 * cplane + slot) = uint2{q2[0], q2[1]};
+            const uint2 q0{pair(a0[0], a0[1]) & keep0, pair(a0[2], a0[3]) & keep1};
+            const uint2 q1{pair(a1[0], a1[1]) & keep0, pair(a1[2], a1[3]) & keep1};
+            const uint2 q2{pair(a2[0], a2[1]) & keep0, pair(a2[2], a2[3]) & keep1};
+            cnt = nonzeros(q0.x, q0.y) | (nonzeros(q1.x, q1.y) << 8) | (nonzeros(q2.x, q2.y) << 16);
+            *reinterpret_cast<uint2*>(out0 + at) = q0;
+            *reinterpret_cast<uint2*>(out1 + at) = q1;
+            *reinterpret_cast<uint2*>(out2 + at) = q2;
         }
         // The block's counts into lane 0 of its row of 16 lanes (row
         // shifts; lanes shifted in from outside the row read 0).
