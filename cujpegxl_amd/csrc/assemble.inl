@@ -714,7 +714,8 @@ __device__ __attribute__((always_inline)) inline void assemble_kernel_body(const
                                                                            const Layout* __restrict__ lay,
                                                                            const Sources& P,
                                                                            std::uint32_t* __restrict__ out_words,
-                                                                           std::uint64_t cap_bytes) {
+                                                                           std::uint64_t cap_bytes,
+                                                                           const FileHead& head) {
     if (lay->overflow != 0) {
         return;
     }
@@ -784,6 +785,9 @@ __device__ __attribute__((always_inline)) inline void assemble_kernel_body(const
             if (w >= w1) {
                 continue;
             }
+            if (w < head.words) {
+                head.to[w] = v;
+            }
             if ((w + 1) * 4 <= cap_bytes) {
                 out_words[w] = v;
             } else {
@@ -799,8 +803,8 @@ __device__ __attribute__((always_inline)) inline void assemble_kernel_body(const
 __global__ __launch_bounds__(256) void assemble_kernel(Geometry geo, const Constants* __restrict__ k,
                                                        const Layout* __restrict__ lay, Sources P,
                                                        std::uint32_t* __restrict__ out_words,
-                                                       std::uint64_t cap_bytes) {
-    assemble_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, lay, P, out_words, cap_bytes);
+                                                       std::uint64_t cap_bytes, FileHead head) {
+    assemble_kernel_body(Wg{blockIdx.x, blockIdx.y, gridDim.x, gridDim.y}, geo, k, lay, P, out_words, cap_bytes, head);
 }
 
 }  // namespace cjx

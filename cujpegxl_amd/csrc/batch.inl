@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void assemble_batch_kernel(const FrameJob* __r
     const FrameJob& j{batch_job(jobs, count, kBAssemble, wg)};
     const Sources P{j.dc_staging, j.chunk_bits, j.dc_chunks,
                     j.ac_staging, j.ac_run_bits, j.dc_group_bits, j.dc_base, j.ac_base};
-    assemble_kernel_body(wg, j.geo, j.k, j.lay, P, j.out, j.cap);
+    assemble_kernel_body(wg, j.geo, j.k, j.lay, P, j.out, j.cap, FileHead{nullptr, 0});
 }
 
 // Tokenizer workgroups of a batch, about: two resident rounds of 256 CUs,

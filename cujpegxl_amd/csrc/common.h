@@ -113,6 +113,13 @@ constexpr std::uint32_t kModeMask = kModeMfma16 | kModeLearned | kModeForceMask;
 FrameParams make_frame_params(float distance);
 
 // Constant tables (filled once per device by init_device_tables()).
+// Where the assembly also writes the file's first `words` words (mapped host
+// memory), for a host that copies them on.
+struct FileHead {
+    std::uint32_t* to;
+    std::uint64_t words;
+};
+
 // The AC tokenizer's lookups, one copy per workgroup in LDS.  Scan entry: raw
 // index of the scan position | its frequency context << 10.  zero_band[r * 32
 // + f]: cluster (within its group of twelve) of a coefficient's token with r

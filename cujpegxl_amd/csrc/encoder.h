@@ -7,10 +7,12 @@
 #include <array>
 #include <cstddef>
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "batch.h"
 #include "common.h"
+#include "copy_team.h"
 
 namespace cjx {
 
@@ -133,7 +135,7 @@ private:
     // null) unless they are already those of (global_scale, quant_dc).
     bool build_constants(std::uint32_t global_scale, std::uint32_t quant_dc, hipStream_t s = nullptr);
     // `listed`: the quantizer listed the non-empty items for the tokenizer.
-    bool run_entropy(std::uint8_t* out, std::size_t cap, bool listed, bool size_event = true);
+    bool run_entropy(std::uint8_t* out, std::size_t cap, bool listed, bool size_event);
     std::uint8_t* mapped_output(std::uint8_t* dst) const;
     Clears entropy_clears() const;
     // Queues a frame after the work on `caller` (null: the null stream);
@@ -141,7 +143,7 @@ private:
     bool submit_nv12(const std::uint8_t* luma, std::size_t luma_pitch, const std::uint8_t* chroma,
                      std::size_t chroma_pitch, hipStream_t caller, bool release_caller, std::uint8_t* dst,
                      std::size_t cap);
-    bool queue_readback(std::uint8_t* direct);
+    void queue_readback(std::uint8_t* direct);
     bool stage_chunk(int slot, std::size_t n);
     bool upload_nv12(const std::uint8_t* luma, std::size_t luma_pitch, const std::uint8_t* chroma,
                      std::size_t chroma_pitch);
@@ -164,7 +166,6 @@ private:
     hipEvent_t ev_caller_{nullptr}, ev_input_free_{nullptr};  // ordering against a caller's stream
     bool pending_{false};            // a frame's readback is queued, finish() not yet called
     std::size_t staged_{0};          // output bytes queued into the staging chunks
-    std::size_t stage_len_[2]{0, 0};
     std::uint8_t* direct_dst_{nullptr};  // page-locked output the assembly wrote the file into
     std::uint8_t* input_{nullptr};   // device NV12 frame for host input (allocated on first use)
     int profiling_{0};
@@ -213,7 +214,14 @@ private:
     // Readback: the file is copied in chunks through two pinned slots, the
     // device-to-host copy of one chunk overlapping the host copy of the last.
     static constexpr std::size_t kStageChunk = 512 * 1024;
-    std::uint8_t* stage_host_{nullptr};   // pinned, 2 * kStageChunk
+    std::uint8_t* stage_host_{nullptr};   // pinned and mapped, 2 * kStageChunk
+    std::uint8_t* stage_dev_{nullptr};    // its device address
+    // Copies the rows of a host frame to the staging chunks, with helper
+    // threads for frames of kTeamBytes or more.
+    static constexpr std::size_t kTeamBytes = 1024 * 1024;
+    static constexpr unsigned int kTeamHelpers = 3;
+    std::unique_ptr<CopyTeam> copy_team_;
+    bool team_shared_{false};
     std::array<hipEvent_t, 2> stage_ready_{};
     std::vector<void*> allocations_{};
 };

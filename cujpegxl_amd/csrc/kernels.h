@@ -106,6 +106,9 @@ void launch_assemble(hipStream_t s, const Geometry& geo, const Constants* k, con
                      const std::uint32_t* dc_staging, const std::uint32_t* ac_staging, const std::uint64_t* dc_bits,
                      const std::uint16_t* ac_run_bits, const std::uint32_t* chunk_off, const std::uint64_t* dc_base,
                      const std::uint64_t* ac_base, std::uint8_t* out, std::uint64_t cap_bytes,
-                     hipEvent_t done = nullptr);
+                     const FileHead& head = FileHead{nullptr, 0}, hipEvent_t done = nullptr);
+// `bytes` (a multiple of 8, at 8-byte addresses) of mapped host memory to the
+// device; `done` is bound to the copy's completion.
+void launch_copy_in(hipStream_t s, std::uint8_t* dst, const std::uint8_t* src, std::size_t bytes, hipEvent_t done);
 
 }  // namespace cjx
