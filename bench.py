@@ -142,9 +142,9 @@ def mixed_batch(cj, synthetic_nv12, frames: int = 64, seed: int = 4) -> dict:
                   "p50_ms": round(float(np.percentile(lat_ms, 50)), 4),
                   "p99_ms": round(float(np.percentile(lat_ms, 99)), 4), "bytes": nbytes,
                   "launches": "one synchronous encode per frame (eight launches each)"}
-    # The same 64 frames as one batch: every stage one launch over all
-    # frames, the eight launches replayed from a captured hipGraph, launch
-    # shapes chosen by the autotuner first.
+    # The same 64 frames as one batch: every stage one launch over the frames
+    # of a graph branch (eight launches each, up to three branches), replayed
+    # from a captured hipGraph, launch shapes chosen by the autotuner first.
     batch = cj.Batch([MIXED_SIZES[p] for p in picks], [float(d) for d in dists])
     batch.set_inputs([(bufs[p].ptr, bufs[p].ptr + MIXED_SIZES[p][0] * MIXED_SIZES[p][1], MIXED_SIZES[p][0],
                        MIXED_SIZES[p][0]) for p in picks])
@@ -166,7 +166,7 @@ def mixed_batch(cj, synthetic_nv12, frames: int = 64, seed: int = 4) -> dict:
                "frame_latency_p99_ms": round(float(np.percentile(lat_b, 99)), 4), "bytes": batch_bytes,
                "bytes_equal_sequential": batch_bytes == nbytes,
                "tuned": tune.strip().splitlines()[-1],
-               "launches": "one launch per stage over the 64 frames (eight per batch), replayed from a hipGraph"}
+               "launches": "eight launches per graph branch (up to three), each over the branch's frames, replayed from a hipGraph"}
     return {"frames": frames, "sizes": "640x360 .. 3840x2160 uniform, d ~ U[0.8, 3.0], seed 4",
             "sequential": sequential, "batched": batched,
             "batched_vs_sequential": round(batched["fps"] / sequential["fps"], 3)}

@@ -434,24 +434,6 @@ void Encoder::carve(Get& get) {
     get(dc_base_, geo_.num_dc * sizeof(std::uint64_t));
 }
 
-bool Encoder::alloc() {
-    out_cap_ = (max_output_size(geo_.width, geo_.height) + 64 + 3) & ~static_cast<std::size_t>(3);
-    bool ok{true};
-    auto get = [&](auto*& p, std::size_t bytes) {
-        void* q{nullptr};
-        if (ok && !injected_alloc_failure() && hipMalloc(&q, bytes < 256 ? 256 : bytes) == hipSuccess) {
-            allocations_.push_back(q);
-            p = static_cast<std::remove_reference_t<decltype(p)>>(q);
-        } else {
-            ok = false;
-        }
-    };
-    carve(get);
-    get(out_, out_cap_);
-    const_gs_ = const_qdc_ = 0;
-    return ok;
-}
-
 // Consecutive 256-byte aligned ranges from offset 0 of a workspace (`base`
 // null: sizing only).
 namespace {
@@ -465,6 +447,32 @@ struct Bump {
     }
 };
 }  // namespace
+
+// One allocation holds every buffer: a program that creates an encoder for a
+// single frame pays for each allocation, mapped on creation and unmapped on
+// destruction (one-shot encode of a host frame with 31 allocations and with
+// one: 1920x1080 3,790 and 1,270 us, 3840x2160 5,170 and 2,540).
+bool Encoder::alloc() {
+    out_cap_ = (max_output_size(geo_.width, geo_.height) + 64 + 3) & ~static_cast<std::size_t>(3);
+    const_gs_ = const_qdc_ = 0;
+    Bump size{nullptr};
+    carve(size);
+    size(out_, out_cap_);
+    void* arena{nullptr};
+    if (hipMalloc(&arena, size.used) != hipSuccess) {
+        return false;
+    }
+    allocations_.push_back(arena);
+    bool ok{true};
+    Bump place{static_cast<std::uint8_t*>(arena)};
+    auto get = [&](auto*& p, std::size_t bytes) {
+        ok = ok && !injected_alloc_failure();
+        place(p, bytes);
+    };
+    carve(get);
+    get(out_, out_cap_);
+    return ok;
+}
 
 std::size_t Encoder::workspace_bytes(std::uint32_t width, std::uint32_t height) {
     Encoder probe;

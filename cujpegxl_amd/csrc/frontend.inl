@@ -522,7 +522,7 @@ __device__ __forceinline__ void tile_partials(const Geometry& geo, const float* 
 // Profiling builds only (CJX_REGION_CUT, never the shipped libraries): the
 // region kernel returns, uniformly, at the start of step k + 1 when the
 // device word says k (k = 6, 7, 8 cut the transform selection after its
-// opening barrier, its row passes and its column passes), so that the time
+// opening barrier, its transforms and its rate-distortion terms), so that the time
 // and instruction counts of each step are differences of two cut builds.
 #ifdef CJX_REGION_CUT
 __device__ int g_region_cut;

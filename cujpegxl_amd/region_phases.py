@@ -27,16 +27,16 @@ import statistics
 import sys
 
 # Cut k returns at the start of step k + 1; 6, 7 and 8 cut the transform
-# selection after its opening barrier, its row passes and its column passes
-# (7 exists in the plain form only); 0 is the whole kernel.
+# selection after its opening barrier, its transforms (7 exists in the plain
+# form only) and its rate-distortion terms; 0 is the whole kernel.
 CUTS = (1, 2, 3, 6, 7, 8, 4, 5, 0)
 STEPS = {
     1: "1 NV12 -> XYB (36x36 tile)",
     2: "2 inverse gaborish + 3a AQ cells",
     3: "3b AQ blocks and the quant field",
     6: "4a selection: opening barrier (3b's tail)",
-    7: "4b selection: row passes",
-    8: "4c selection: column passes, RD terms, costs",
+    7: "4b selection: transforms on the matrix cores",
+    8: "4c selection: RD terms, costs (learned: the transforms too)",
     4: "4d decision (and the network, learned)",
     5: "5 chosen DCTs of X and B",
     0: "6 FP16 coefficients out + CfL partials",

@@ -107,8 +107,10 @@ typedef struct cujpegxl_nv12_host_input {
 } cujpegxl_nv12_host_input;
 
 /* Synchronous encode of a host-resident NV12 frame: the planes are uploaded
- * into a device frame the encoder owns (through its pinned staging buffer, or
- * by direct DMA when both planes are pinned host memory), then encoded as
+ * into a device frame the encoder owns (through its pinned staging buffer,
+ * frames of 1 MiB or more with up to three helper threads of the encoder for
+ * the host copy, or by direct DMA when both planes are pinned host memory),
+ * then encoded as
  * cujpegxl_encoder_encode does.  Same validation and statuses. */
 cujpegxl_status cujpegxl_encoder_encode_host(cujpegxl_encoder* encoder,
                                              const cujpegxl_nv12_host_input* input,

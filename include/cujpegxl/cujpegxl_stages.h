@@ -94,8 +94,9 @@ int cjx_mlp_default_weights(int32_t device);
 
 /* Batches of frames of uneven sizes and distances (no counterpart in the
  * reference, whose encoder takes one frame at a time): every stage runs as
- * one launch over all the batch's frames, the batch's eight launches are
- * captured once as a hipGraph and replayed, and the launches' shapes come
+ * one launch over all the batch's frames (a large batch as up to three
+ * branches of about equal blocks), the launches are captured once as a
+ * hipGraph and replayed, and the launches' shapes come
  * from an autotuner (cjx_batch_tune).  Files land in page-locked host memory
  * the library owns (cjx_batch_result gives each file's address and size,
  * valid until the next run).  `mode`: 0 or CJX_MODE_MFMA16 / CJX_MODE_LEARNED
