@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <utility>
 
 #include "kernels.h"
 #include "prefix.h"
@@ -200,29 +201,32 @@ bool injected_alloc_failure() {
     return false;
 }
 
-// Idle streams of destroyed encoders, at most four per device (a process has
-// four hardware queues), for the next ones: creating a stream takes the
-// runtime up to 0.8 ms, most of the creation of a small encoder (640x360
-// one-shot encodes 950 -> 325 us).
+// The stream of a destroyed encoder, one per device, for the next one:
+// creating a stream takes the runtime up to 0.8 ms, most of the creation of a
+// small encoder (640x360 one-shot encodes 950 -> 325 us).  Only one, because a
+// stream keeps its hardware queue (of four): two kept streams may share one,
+// and two frames in flight then run one after the other (2560x1440 352 -> 375
+// us with four kept), while new streams take the least used queues.
 class StreamPool {
 public:
     hipStream_t take(int device) {
+        hipStream_t s{nullptr};
         if (device < kDevices) {
             const std::lock_guard<std::mutex> lock{mutex_};
-            if (count_[device] > 0) {
-                return idle_[device][--count_[device]];
-            }
+            std::swap(s, idle_[device]);
         }
-        hipStream_t s{nullptr};
-        return hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess ? s : nullptr;
+        if (s == nullptr && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
+            return nullptr;
+        }
+        return s;
     }
 
     // `s` has nothing queued.
     void give(int device, hipStream_t s) {
         if (device >= 0 && device < kDevices) {
             const std::lock_guard<std::mutex> lock{mutex_};
-            if (count_[device] < kIdle) {
-                idle_[device][count_[device]++] = s;
+            if (idle_[device] == nullptr) {
+                std::swap(s, idle_[device]);
                 return;
             }
         }
@@ -230,10 +234,9 @@ public:
     }
 
 private:
-    static constexpr int kDevices{64}, kIdle{4};
+    static constexpr int kDevices{64};
     std::mutex mutex_;
-    hipStream_t idle_[kDevices][kIdle]{};
-    int count_[kDevices]{};
+    hipStream_t idle_[kDevices]{};
 };
 
 // Never destroyed: encoders may be destroyed after this file's statics.
