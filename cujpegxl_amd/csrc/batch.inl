@@ -107,7 +107,7 @@ __global__ __launch_bounds__(kEmitThreads) void emit_batch_kernel(const FrameJob
     const FrameJob& j{batch_job(jobs, count, kBEmit, wg)};
     emit_kernel_body(wg, j.geo, EmitArgs{j.acs, j.item_tokens, j.tokens, j.codes, j.k, j.fb_count, j.dc, j.qf, j.ytox,
                                          j.ytob, j.ac_staging, j.ac_run_bits, j.dc_staging, j.chunk_bits,
-                                         j.dc_chunks, wg.nx - j.dc_chunks * j.geo.num_dc});
+                                         j.dc_chunks, wg.nx - j.dc_chunks * j.geo.num_dc, false});
 }
 
 __global__ __launch_bounds__(kLayoutThreads) void layout_batch_kernel(const FrameJob* __restrict__ jobs, int count) {

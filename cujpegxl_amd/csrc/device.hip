@@ -317,9 +317,11 @@ void launch_emit(hipStream_t s, const Geometry& geo, const std::int8_t* acs, con
     const std::uint32_t chunks{dc_chunks_per_group(geo)};
     const std::uint32_t bands{geo.num_ac * kGroupBands};
     const std::uint32_t ac_wgs{bands * emit_band_wgs(bands)};
-    emit_kernel<<<ac_wgs + chunks * geo.num_dc, kEmitThreads, 0, s>>>(
+    const std::uint32_t wgs{ac_wgs + chunks * geo.num_dc};
+    constexpr std::uint32_t kResident{8 * 256};  // eight workgroups on each of 256 CUs
+    emit_kernel<<<wgs, kEmitThreads, 0, s>>>(
         geo, EmitArgs{acs, item_tokens, tokens, cs, k, fb_count, dc, qf, ytox, ytob, ac_staging, ac_run_bits,
-                      dc_staging, chunk_bits, chunks, ac_wgs});
+                      dc_staging, chunk_bits, chunks, ac_wgs, wgs <= kResident});
 }
 
 void launch_layout(hipStream_t s, const Geometry& geo, const Constants* k, const CodeSet* cs,
