@@ -187,8 +187,9 @@ void modular_prefix(HostBits& w, int predictor) {
 std::once_flag g_tables_once[64];
 bool g_tables_ok[64];
 
-// Test hook: the allocation that brings the countdown from 1 to 0 fails as
-// if the device were out of memory (0: no failure pending).
+// Test hook: the runtime object (stream, event, page-locked or device memory)
+// whose creation brings the countdown from 1 to 0 is refused as if there were
+// none left (0: no failure pending).
 std::atomic<int> g_fail_alloc_countdown{0};
 
 bool injected_alloc_failure() {
@@ -199,6 +200,24 @@ bool injected_alloc_failure() {
         }
     }
     return false;
+}
+
+// Everything an encoder creates comes from the four calls below, so that the
+// hook can refuse each of them.
+bool create_stream(hipStream_t* s) {
+    return !injected_alloc_failure() && hipStreamCreateWithFlags(s, hipStreamNonBlocking) == hipSuccess;
+}
+
+bool create_event(hipEvent_t* e, unsigned int flags = hipEventDefault) {
+    return !injected_alloc_failure() && hipEventCreateWithFlags(e, flags) == hipSuccess;
+}
+
+bool alloc_host(void** p, std::size_t bytes, unsigned int flags) {
+    return !injected_alloc_failure() && hipHostMalloc(p, bytes, flags) == hipSuccess;
+}
+
+bool alloc_device(void** p, std::size_t bytes) {
+    return !injected_alloc_failure() && hipMalloc(p, bytes) == hipSuccess;
 }
 
 // The stream of a destroyed encoder, one per device, for the next one:
@@ -215,10 +234,7 @@ public:
             const std::lock_guard<std::mutex> lock{mutex_};
             std::swap(s, idle_[device]);
         }
-        if (s == nullptr && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
-            return nullptr;
-        }
-        return s;
+        return s != nullptr || create_stream(&s) ? s : nullptr;
     }
 
     // `s` has nothing queued.
@@ -413,30 +429,30 @@ bool Encoder::setup(int device) {
         return false;
     }
     for (hipEvent_t* e : {&ev_done_, &ev_caller_, &ev_input_free_}) {
-        if (hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) {
+        if (!create_event(e, hipEventDisableTiming)) {
             return false;
         }
     }
     // Bound to kernels' completion at launch (timing-capable events).
     for (hipEvent_t* e : {&ev_size_, &ev_end_}) {
-        if (hipEventCreate(e) != hipSuccess) {
+        if (!create_event(e)) {
             return false;
         }
     }
     for (hipEvent_t& e : events_) {
-        if (hipEventCreate(&e) != hipSuccess) {
+        if (!create_event(&e)) {
             return false;
         }
     }
-    if (hipHostMalloc(reinterpret_cast<void**>(&total_host_), sizeof(std::uint64_t)) != hipSuccess ||
+    if (!alloc_host(reinterpret_cast<void**>(&total_host_), sizeof(std::uint64_t), hipHostMallocDefault) ||
         hipHostGetDevicePointer(reinterpret_cast<void**>(&total_dev_), total_host_, 0) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&stage_host_), 2 * kStageChunk, hipHostMallocMapped) != hipSuccess ||
+        !alloc_host(reinterpret_cast<void**>(&stage_host_), 2 * kStageChunk, hipHostMallocMapped) ||
         hipHostGetDevicePointer(reinterpret_cast<void**>(&stage_dev_), stage_host_, 0) != hipSuccess) {
         return false;
     }
     // Also bound to the upload's copies (timing-capable events).
     for (hipEvent_t& e : stage_ready_) {
-        if (hipEventCreate(&e) != hipSuccess) {
+        if (!create_event(&e)) {
             return false;
         }
     }
@@ -507,19 +523,14 @@ bool Encoder::alloc() {
     carve(size);
     size(out_, out_cap_);
     void* arena{nullptr};
-    if (hipMalloc(&arena, size.used) != hipSuccess) {
+    if (!alloc_device(&arena, size.used)) {
         return false;
     }
     allocations_.push_back(arena);
-    bool ok{true};
     Bump place{static_cast<std::uint8_t*>(arena)};
-    auto get = [&](auto*& p, std::size_t bytes) {
-        ok = ok && !injected_alloc_failure();
-        place(p, bytes);
-    };
-    carve(get);
-    get(out_, out_cap_);
-    return ok;
+    carve(place);
+    place(out_, out_cap_);
+    return true;
 }
 
 std::size_t Encoder::workspace_bytes(std::uint32_t width, std::uint32_t height) {
@@ -994,7 +1005,7 @@ bool Encoder::upload_nv12(const std::uint8_t* luma, std::size_t luma_pitch, cons
     const std::size_t w{geo_.width}, h{geo_.height};
     if (input_ == nullptr) {
         void* p{nullptr};
-        if (hipMalloc(&p, w * h * 3 / 2) != hipSuccess) {
+        if (!alloc_device(&p, w * h * 3 / 2)) {
             return false;
         }
         allocations_.push_back(p);
@@ -1184,7 +1195,7 @@ bool Encoder::export_features(bool on) {
     }
     if (on && features_ == nullptr) {
         void* p{nullptr};
-        if (hipMalloc(&p, static_cast<std::size_t>(geo_.rw) * geo_.rh * 108 * sizeof(float)) != hipSuccess) {
+        if (!alloc_device(&p, static_cast<std::size_t>(geo_.rw) * geo_.rh * 108 * sizeof(float))) {
             return false;
         }
         allocations_.push_back(p);

@@ -231,7 +231,8 @@ bool device_has_matrix_cores(int ordinal);
 // The constant tables (and the default network weights) on `device`, once;
 // the device must be current.
 bool ensure_device_tables(int device);
-// Test hook: the n-th device allocation from now fails (0 cancels).
+// Test hook: the n-th stream, event or memory block that an encoder creates
+// from now on is refused (0 cancels).
 void fail_allocation_after(int n);
 
 }  // namespace cjx

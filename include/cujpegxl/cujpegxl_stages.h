@@ -177,9 +177,10 @@ int cjx_stage_encode_cycle(cujpegxl_encoder* encoder, const cujpegxl_nv12_input*
 int cjx_stage_build_codes(int32_t device_ordinal, const uint32_t* hists, uint32_t count, uint32_t* alpha,
                           uint8_t* depth, uint16_t* bits, uint32_t* hdr_words, uint32_t* hdr_bits);
 
-/* Test hook for the failure paths: the n-th device allocation an encoder
- * makes from now on (create, configure) fails as if the device were out of
- * memory; 0 cancels.  No counterpart in the reference. */
+/* Test hook for the failure paths: the n-th stream, event, page-locked or
+ * device memory block that an encoder creates from now on (create, configure,
+ * the first host-input encode, feature export) is refused as if there were
+ * none left; 0 cancels.  No counterpart in the reference. */
 void cjx_stage_fail_allocation_after(int n);
 
 /* Device memory for harnesses that have no other allocator. */
