@@ -5,14 +5,17 @@
 // page-locked staging chunks.  The owner of a team opens a job of numbered
 // pieces, releases pieces in order as their destination becomes free, works
 // on pieces itself and closes the job; the helpers take pieces while a job is
-// open and sleep otherwise.  A team without helpers is the plain copy.  One
-// thread at a time may use a team.
+// open and sleep otherwise, also within a job once no piece has been released
+// for kIdle (a GPU busy with other work can hold a staging chunk for as long as
+// that work takes).  A team without helpers is the plain copy.  One thread at a
+// time may use a team.
 #pragma once
 
 #include <pthread.h>
 #include <signal.h>
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdint>
 #include <functional>
@@ -84,7 +87,10 @@ public:
     }
 
     // Pieces below `n` may be copied.
-    void release(std::uint32_t n) { released_.store(n, std::memory_order_release); }
+    void release(std::uint32_t n) {
+        released_.store(n);
+        wake_sleeping();
+    }
 
     // Copies pieces until all of group g, which has been released, are done.
     void finish_group(std::uint32_t g) {
@@ -105,12 +111,29 @@ public:
             open_ = false;
         }
         next_.store(pieces_);
+        wake_sleeping();
         while (busy_.load(std::memory_order_acquire) != 0) {
             __builtin_ia32_pause();
         }
     }
 
 private:
+    // How long a helper polls for the next piece of an open job: ten times what
+    // a staging chunk of 512 KB takes to come free on an idle device (19 us), so
+    // that only a held-up upload pays for a wake-up.
+    static constexpr std::chrono::microseconds kIdle{200};
+
+    // After a change to next_ or released_.  A helper counts itself into
+    // sleeping_ before it looks at them for the last time, so one of the two
+    // sees the other's write; the lock keeps the call out of the time between
+    // that look and the wait.
+    void wake_sleeping() {
+        if (sleeping_.load() != 0) {
+            { const std::lock_guard<std::mutex> lock{mutex_}; }
+            wake_.notify_all();
+        }
+    }
+
     // One released piece, if any is left.
     bool take() {
         std::uint32_t i{next_.load()};
@@ -135,9 +158,23 @@ private:
             seen = job_;
             busy_.fetch_add(1);
             lock.unlock();
-            while (next_.load() < pieces_) {
-                if (!take()) {
-                    __builtin_ia32_pause();
+            auto last{std::chrono::steady_clock::now()};  // this helper's last piece
+            for (unsigned int polls{1}; next_.load() < pieces_; ++polls) {
+                if (take()) {
+                    last = std::chrono::steady_clock::now();
+                    continue;
+                }
+                __builtin_ia32_pause();
+                if (polls % 64 == 0 && std::chrono::steady_clock::now() - last >= kIdle) {
+                    lock.lock();
+                    sleeping_.fetch_add(1);
+                    wake_.wait(lock, [&] {
+                        const std::uint32_t i{next_.load()};
+                        return i >= pieces_ || i < released_.load();
+                    });
+                    sleeping_.fetch_sub(1);
+                    lock.unlock();
+                    last = std::chrono::steady_clock::now();
                 }
             }
             busy_.fetch_sub(1, std::memory_order_release);
@@ -151,7 +188,7 @@ private:
     std::uint64_t job_{0};
     std::function<void(std::uint32_t)> copy_;
     std::uint32_t pieces_{0}, group_{1};
-    std::atomic<std::uint32_t> next_{0}, released_{0}, busy_{0};
+    std::atomic<std::uint32_t> next_{0}, released_{0}, busy_{0}, sleeping_{0};
     std::atomic<std::uint32_t> done_[kGroups]{};
     std::vector<std::thread> threads_;  // last: started with every other member in place
 };
