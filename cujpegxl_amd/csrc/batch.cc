@@ -8,6 +8,8 @@
 #include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
+#include <utility>
 
 #include "kernels.h"
 
@@ -121,6 +123,23 @@ bool BatchEncoder::configure(int n, const std::uint32_t* w, const std::uint32_t*
     return apply_shape(shape_);
 }
 
+// Every frame's stage grids for `shape` (`first` 0).
+std::vector<BatchEncoder::FrameGrids> BatchEncoder::frame_grids(const BatchShape& shape) const {
+    std::uint32_t bands{0};
+    std::uint64_t blocks{0};
+    for (const FrameJob& j : jobs_) {
+        bands += j.geo.num_ac * ac_group_bands();
+        blocks += j.geo.nblocks;
+    }
+    std::vector<FrameGrids> grids(jobs_.size());
+    for (std::size_t i{0}; i < jobs_.size(); ++i) {
+        StageGrid g[kBStages];
+        batch_stage_grids(jobs_[i].geo, shape, blocks, emit_band_wgs(bands), g);
+        std::copy(std::begin(g), std::end(g), grids[i].begin());
+    }
+    return grids;
+}
+
 // Stage grids and first workgroups for `shape`, the jobs on the device, and
 // a fresh graph of the batch's launches.
 //
@@ -139,12 +158,11 @@ bool BatchEncoder::apply_shape(const BatchShape& shape) {
         return false;
     }
     shape_ = shape;
-    std::uint32_t bands{0};
     std::uint64_t blocks{0};
     for (const FrameJob& j : jobs_) {
-        bands += j.geo.num_ac * ac_group_bands();
         blocks += j.geo.nblocks;
     }
+    const std::vector<FrameGrids> grids{frame_grids(shape)};
     constexpr std::uint64_t kPartBlocks{80000};
     const std::uint64_t wanted{std::clamp<std::uint64_t>(blocks / kPartBlocks, 1, kMaxParts)};
     const int n{static_cast<int>(jobs_.size())};
@@ -157,7 +175,7 @@ bool BatchEncoder::apply_shape(const BatchShape& shape) {
         if (seen * wanted >= (part + 1) * blocks) {
             first[++part] = i;
         }
-        batch_stage_grids(j.geo, shape_, blocks, emit_band_wgs(bands), j.grid);
+        std::copy(grids[i].begin(), grids[i].end(), std::begin(j.grid));
         for (int s{0}; s < kBStages; ++s) {
             j.grid[s].first = total[part][s];
             total[part][s] += j.grid[s].nx * j.grid[s].ny;
@@ -272,7 +290,12 @@ bool BatchEncoder::set_shape(const BatchShape& shape) {
 
 // Coordinate search: the tokenizer and assembly shapes with one workgroup per
 // region first, then the region stage's persistent grids with the best of
-// those (one and two resident rounds of six workgroups per CU).
+// those (one and two resident rounds of six workgroups per CU).  Shapes with
+// the same launches are timed once and share that time, the first of them
+// being taken: a frame's share of the tokenizer's workgroups and the runs of
+// its file bound its grids, so several caps may stand for one launch (eight
+// frames of 3840x2160: token caps from 512 up, 4 and 16 words), and a choice
+// between their timings would be by noise.
 bool BatchEncoder::tune(int reps, std::string* report) {
     if (!inputs_set_ || reps <= 0) {
         return false;
@@ -288,15 +311,27 @@ bool BatchEncoder::tune(int reps, std::string* report) {
     BatchShape best{shape_};
     double best_s{1e30};
     char line[192];
+    struct Timed {
+        std::uint32_t region_wgs;
+        std::vector<FrameGrids> grids;
+        double seconds;
+    };
+    std::vector<Timed> timed;
     const auto trial = [&](const BatchShape& c) {
-        if (!apply_shape(c)) {
-            return false;
-        }
+        std::vector<FrameGrids> grids{frame_grids(c)};
+        const auto same{std::find_if(timed.begin(), timed.end(), [&](const Timed& t) {
+            return t.region_wgs == c.region_wgs && t.grids == grids;
+        })};
         double s{0.0};
-        if (!run(2, nullptr) || !run(reps, &s)) {
-            return false;
+        if (same != timed.end()) {
+            s = same->seconds;
+        } else {
+            if (!apply_shape(c) || !run(2, nullptr) || !run(reps, &s)) {
+                return false;
+            }
+            s /= reps;
+            timed.push_back(Timed{c.region_wgs, std::move(grids), s});
         }
-        s /= reps;
         std::snprintf(line, sizeof(line), "token_cap=%u assemble_words=%u region_wgs=%u batch_ms=%.4f\n",
                       c.token_cap, c.assemble_words, c.region_wgs, 1e3 * s);
         if (report != nullptr) {

@@ -32,6 +32,8 @@ struct StageGrid {
     std::uint32_t first;  // the frame's first workgroup in the batched launch
     std::uint32_t nx, ny;  // the frame's own grid
     std::uint32_t pad;
+
+    bool operator==(const StageGrid& o) const { return first == o.first && nx == o.nx && ny == o.ny; }
 };
 
 struct FrameJob {

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstdint>
 #include <memory>
 #include <string>
@@ -54,6 +55,8 @@ public:
 
 private:
     void release();
+    using FrameGrids = std::array<StageGrid, kBStages>;
+    std::vector<FrameGrids> frame_grids(const BatchShape& shape) const;
     bool apply_shape(const BatchShape& shape);
 
     int device_{-1};

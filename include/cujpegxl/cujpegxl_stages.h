@@ -119,7 +119,9 @@ int cjx_batch_result(const cjx_batch* batch, uint32_t index, const uint8_t** dat
  * tokenizer workgroups per frame x output words per assembly thread with one
  * workgroup per region, then the region stage as a persistent grid (one and
  * two resident rounds) with the best of those; one line per candidate, then
- * the choice, into `report`. */
+ * the choice, into `report`.  Candidates that come to the same launches are
+ * timed once and share the time; the first of them is the one that may be
+ * chosen. */
 int cjx_batch_tune(cjx_batch* batch, int32_t reps, char* report, size_t cap);
 /* Sets a launch shape directly: tokenizer workgroups per frame (>= 1),
  * output words per assembly thread (>= 1), and region_wgs = 0 for one
