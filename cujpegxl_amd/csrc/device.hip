@@ -54,7 +54,7 @@ static std::uint32_t mlp_wgs(std::uint32_t n) {
 }
 
 std::size_t mlp_partial_floats(std::uint32_t n) {
-    return static_cast<std::size_t>((n + kMlpTiles - 1) / kMlpTiles) * (kMlpParams + 1);  // a row per tile is enough
+    return static_cast<std::size_t>(mlp_wgs(n)) * (kMlpParams + 1);  // a row per workgroup
 }
 
 void launch_mlp_step(hipStream_t s, const float* x, const float* labels, std::uint32_t n, float lambda,
