@@ -126,11 +126,14 @@ __global__ __launch_bounds__(256) void assemble_batch_kernel(const FrameJob* __r
     assemble_kernel_body(wg, j.geo, j.k, j.lay, P, j.out, j.cap, FileHead{nullptr, 0});
 }
 
-// Tokenizer workgroups of a batch, about: two resident rounds of 256 CUs,
-// shared out by the frames' blocks.  A workgroup pays a prologue and writes an
-// 8 KB histogram row that the next stage sums, so a small frame of a large
-// batch gets few: 16 frames of 640x360 to 3840x2160 1253 -> 1175 us against up
-// to 1,024 workgroups for each frame, eight frames of 3840x2160 1804 -> 1778.
+// Tokenizer workgroups of a batch, about: four times the 1,024 that are
+// resident (four workgroups on each of 256 CUs), shared out by the frames'
+// blocks.  A workgroup pays a prologue and writes an 8 KB histogram row that
+// the next stage sums, so a small frame of a large batch gets few: 16 frames of
+// 640x360 to 3840x2160 1253 -> 1175 us against up to 1,024 workgroups for each
+// frame, eight frames of 3840x2160 1804 -> 1778.  (A branch of the batch
+// launches its frames' part, which is no whole number of resident rounds: 1,536
+// for three of the eight.)
 constexpr std::uint64_t kBatchTokenWgs = 4096;
 
 void batch_stage_grids(const Geometry& geo, const BatchShape& shape, std::uint64_t blocks, std::uint32_t band_wgs,

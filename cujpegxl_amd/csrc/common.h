@@ -112,7 +112,6 @@ constexpr std::uint32_t kModeMask = kModeMfma16 | kModeLearned | kModeForceMask;
 
 FrameParams make_frame_params(float distance);
 
-// Constant tables (filled once per device by init_device_tables()).
 // Where the assembly also writes the file's first `words` words (mapped host
 // memory), for a host that copies them on.
 struct FileHead {
@@ -131,6 +130,7 @@ struct alignas(16) TokenTables {
     std::uint8_t zero_band[64 * 32];
 };
 
+// Constant tables (filled once per device by init_device_tables()).
 struct DeviceTables {
     float basis8[64];
     float basis16[256];
@@ -154,7 +154,7 @@ struct DeviceTables {
     double llf2[4];        // T[f][o] = ortho_2(f, o) * resample_scale_2[f]
     double llf4[16];
     float rate[256];       // selection rate term 1 + log2(1 + k) for |q| = k >= 1; 0 for k = 0
-    float2 xyb_tab[kXybTabPairs];  // {power, segment reciprocal} pairs of pow24_tab / cbrt_tab
+    float2 xyb_tab[kXybTabPairs];  // {power, segment reciprocal} pairs of the XYB powers
     // FP16 operands of the matrix-core DCT form: [0] = RN16(a), [1] =
     // RN16(a - [0]) of every basis entry a (FP16 bit patterns, row-major):
     // blockdiag(A8, A8) (a 16x16 quad of four DCT8s), A16 and A32.

@@ -827,8 +827,9 @@ bool Encoder::spin_on(hipEvent_t e) {
 
 // The end of a frame: the assembly kernel's own completion when it writes
 // the output and ends the frame, else an event after the last copy.  The
-// host polls (only tens of microseconds of work remain): polling saves the
-// wake-up latency of a blocking wait, which is of the same order.
+// host polls it, and so would the runtime's own wait: hipEventSynchronize takes
+// the thread's whole time on events of either kind (60 ms of 60, also with
+// hipEventBlockingSync).
 bool Encoder::wait_done() {
     if (end_bound_) {
         end_bound_ = false;
@@ -847,10 +848,9 @@ bool Encoder::finish(std::uint8_t* dst, std::size_t cap, std::size_t* size) {
     }
     pending_ = false;
     // Poll for the size, or for the frame's end when no size event was bound
-    // (the assembly writes the file into `dst`): a blocking wait would add
-    // its wake-up latency, and the event's interrupt, to the frame, and an
-    // event in mid-chain for a first blocking wait costs about 5 us of idle
-    // device time after the kernel that carries it.
+    // (the assembly writes the file into `dst`): an event in mid-chain, to wait
+    // for in two parts, costs about 5 us of idle device time after the kernel
+    // that carries it.
     const bool ended{!size_bound_};
     if (!(ended ? wait_done() : spin_on(ev_size_))) {
         return false;

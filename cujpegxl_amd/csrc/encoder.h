@@ -21,8 +21,8 @@ enum class Stage : int {
     kQuantize,     // CfL maps, quantization, DC, non-zero counts
     kHistograms,   // AC cluster, DC and AcMetadata histograms
     kCodes,        // prefix codes and code headers
-    kSizes,        // per-item bits, group scans, section layout
-    kEmit,         // zero fill, headers, AC and DC token emission
+    kSizes,        // AC and DC token emission with their bit counts, section layout
+    kEmit,         // assembly of the file
     kReadback,     // size and bytes to the host
     kCount
 };

@@ -9,8 +9,10 @@
 // counts and the cluster histograms; the emission reads the records.
 //
 // DC: a DcGroup section is a list of items (header blobs, DC residual tokens,
-// AcMetadata tokens), each with a known bit length once the codes exist;
-// chunked scans give every item its bit offset and the emitter ORs its bits in.
+// AcMetadata tokens), each with a known bit length once the codes exist.  A
+// workgroup writes a chunk of 1,024 items at chunk-relative bits into a slot of
+// its own, with its bit count; the layout scans the counts and the assembly
+// joins the chunks.
 
 namespace cjx {
 
@@ -52,13 +54,6 @@ __device__ __forceinline__ std::uint32_t dpp_u32(std::uint32_t x) {
         __builtin_amdgcn_update_dpp(0, static_cast<int>(x), kCtrl, kRowMask, 0xf, kCtrl < 0x140));
 }
 
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ std::uint64_t dpp_u64(std::uint64_t x) {
-    const std::uint32_t lo{dpp_u32<kCtrl, kRowMask>(static_cast<std::uint32_t>(x))};
-    const std::uint32_t hi{dpp_u32<kCtrl, kRowMask>(static_cast<std::uint32_t>(x >> 32))};
-    return (static_cast<std::uint64_t>(hi) << 32) | lo;
-}
-
 __device__ __forceinline__ std::uint32_t wave_incl_scan_u32(std::uint32_t x) {
     x += dpp_u32<0x111, 0xf>(x);
     x += dpp_u32<0x112, 0xf>(x);
@@ -66,15 +61,6 @@ __device__ __forceinline__ std::uint32_t wave_incl_scan_u32(std::uint32_t x) {
     x += dpp_u32<0x118, 0xf>(x);
     x += dpp_u32<0x142, 0xa>(x);
     return x + dpp_u32<0x143, 0xc>(x);
-}
-
-__device__ __forceinline__ std::uint64_t wave_incl_scan_u64(std::uint64_t x) {
-    x += dpp_u64<0x111, 0xf>(x);
-    x += dpp_u64<0x112, 0xf>(x);
-    x += dpp_u64<0x114, 0xf>(x);
-    x += dpp_u64<0x118, 0xf>(x);
-    x += dpp_u64<0x142, 0xa>(x);
-    return x + dpp_u64<0x143, 0xc>(x);
 }
 
 // Sum over the wave, in every lane (the scan's last lane, read as a scalar).
@@ -86,27 +72,6 @@ __device__ __forceinline__ int wave_sum_int(int v) {
 __device__ __forceinline__ int wave_excl_scan(int v, int lane) {
     (void)lane;
     return static_cast<int>(wave_incl_scan_u32(static_cast<std::uint32_t>(v)) - static_cast<std::uint32_t>(v));
-}
-
-// ORs `len` (<= 32) bits of `value` at absolute bit position `pos`; words at
-// or beyond `cap_words` are never touched (the layout makes that unreachable;
-// the check keeps an inconsistent layout from writing out of bounds).
-__device__ __forceinline__ void or_bits(std::uint32_t* words, std::uint64_t cap_words, std::uint64_t pos,
-                                        std::uint32_t value, std::uint32_t len) {
-    if (len == 0) {
-        return;
-    }
-    if (len < 32) {
-        value &= (1u << len) - 1u;
-    }
-    const std::uint64_t wi{pos >> 5};
-    const std::uint32_t b{static_cast<std::uint32_t>(pos & 31u)};
-    if (wi < cap_words) {
-        atomicOr(&words[wi], value << b);
-    }
-    if (b + len > 32 && wi + 1 < cap_words) {
-        atomicOr(&words[wi + 1], value >> (32 - b));
-    }
 }
 
 // ORs `len` (<= 32) bits at bit `pos` of an LDS word buffer of `cap` words.
@@ -506,31 +471,6 @@ __device__ __forceinline__ void ac_hist_reduce_body(const Wg& wg, const std::uin
     if (sum != 0) {
         atomicAdd(&hist[(bin / kAcSymbols) * kHistStride + bin % kAcSymbols], sum);
     }
-}
-
-// Block-wide exclusive scan of one value per thread (blockDim.x multiple of 64).
-__device__ std::uint64_t block_excl_scan(std::uint64_t v, std::uint64_t* sh, std::uint64_t& total) {
-    const int tid{static_cast<int>(threadIdx.x)};
-    const int lane{tid & 63}, wv{tid >> 6}, nw{static_cast<int>(blockDim.x) >> 6};
-    const std::uint64_t x{wave_incl_scan_u64(v)};
-    if (lane == 63) {
-        sh[wv] = x;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        std::uint64_t run{0};
-        for (int i{0}; i < nw; ++i) {
-            const std::uint64_t t{sh[i]};
-            sh[i] = run;
-            run += t;
-        }
-        sh[nw] = run;
-    }
-    __syncthreads();
-    const std::uint64_t r{sh[wv] + x - v};
-    total = sh[nw];
-    __syncthreads();
-    return r;
 }
 
 // Exclusive scan of one value per thread over a workgroup of kWaves waves:

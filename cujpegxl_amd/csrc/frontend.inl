@@ -107,7 +107,7 @@ __device__ __forceinline__ float clamp01(float v) {
     return fminf(fmaxf(v, 0.0f), 1.0f);
 }
 
-// pow24_tab and cbrt_tab with the series argument's two constants held in
+// The table-driven powers with the series argument's two constants held in
 // registers, so that placing the mantissa bits is one v_and_or_b32.
 struct XybPowers {
     const float2* tab;
@@ -554,7 +554,7 @@ __device__ int g_region_cut;
 // where no row is clamped, every row's address is one of the thread's base
 // registers plus a constant (LDS) or a scalar (planes), and the six luma reads
 // are issued at once.  Other regions, and planes with a pitch that 32-bit
-// offsets do not cover, compute each row's address. 
+// offsets do not cover, compute each row's address.
 // Region kernel at 3840x2160, one address computed per row and tap before:
 // 156 -> 149 us (130.7 -> 124.5 learned + FP16); VALU instructions -9.6%.
 __device__ __forceinline__ void xyb_tile(RegionShared& S, const std::uint8_t* luma, std::size_t luma_pitch,

@@ -25,8 +25,8 @@
 namespace cjx {
 
 // Holds the buffers of every accepted shape (at most 4096 on a side and
-// 1920 x 1088 pixels; the largest need, 100 MiB, is a narrow frame crossing
-// many AC groups, e.g. 520 x 4016).
+// 1920 x 1088 pixels; the largest need, 97.9 MiB, is a narrow frame crossing
+// many AC groups, 536 x 3896).
 constexpr std::size_t kNoAllocScratchBytes = CUJPEGXL_NOALLOC_SCRATCH_BYTES;
 
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];

@@ -63,7 +63,7 @@ void split_f16(const float* a, int count, std::uint16_t* hi, std::uint16_t* lo) 
     }
 }
 
-// The table of pow24_tab / cbrt_tab (numeric.h): per exponent k and segment j,
+// The table of the XYB powers (numeric.h): per exponent k and segment j,
 // {RN((2^k c_j)^a), RN(1 / c_j)} with c_j = 1 + (j + 1/2) / 16, in double.
 void xyb_power_table(float2* t) {
     for (int j{0}; j < 16; ++j) {
