@@ -59,8 +59,9 @@ int cjx_stage_encode_dct8_uniform(cujpegxl_encoder* encoder, const cujpegxl_nv12
                                   cujpegxl_output* output);
 
 /* Per-stage device time of the following encodes (HIP events on the
- * encoder's stream): region, quantize, histograms, codes, sizes, emit,
- * readback.  `ms` receives 7 floats for the last encode.  `on`: 0 off,
+ * encoder's stream): region, quantize, histograms (tokens and histograms),
+ * codes, sizes (token emission and the file's layout), emit (assembly of the
+ * file), readback.  `ms` receives 7 floats for the last encode.  `on`: 0 off,
  * 1 every stage, 2 the region kernel only (one event pair; the others read
  * 0).  Each timed event adds a few microseconds of idle device time. */
 int cjx_stage_set_profiling(cujpegxl_encoder* encoder, int on);
